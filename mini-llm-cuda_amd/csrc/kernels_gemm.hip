@@ -1,6 +1,6 @@
 // MFMA GEMM for prefill and batched decode on gfx950:
 //
-//     C[M, N] = A[M, K] . B[N, K]^T  (+ R[M, N])        C, R fp32;  A and B both fp32 or both bf16
+//     C[M, N] = A[M, K] . B[N, K]^T  (+ R[M, N])        C, R fp32;  A and B both fp32, bf16 or IEEE half
 //
 // A holds activations (one token per row), B a weight matrix in the checkpoint's row-major [out, in]
 // order -- both operands are K-contiguous, which is what the MFMA operand layout wants: for the
@@ -9,9 +9,8 @@
 // feeding four v_mfma_f32_32x32x2_f32 steps).  This replaces the cublasGemmEx calls of
 // inference.cu:401-465, 487-507, 582-602, 624-695 and 723-743 for L > 1 columns.
 //
-// Tiling: 128 x 128 output tile per 256-thread workgroup (2 x 2 waves of 64 x 64), K in slices of
-// 128 bytes per row.  Slices go global -> registers -> LDS (rows padded to 144 bytes: conflict-free
-// 16-byte reads), the next slice's global loads fly while the current one is multiplied.
+// Here: the 256 x 256-tile kernel of the long two-byte products (k_gemm_tn_w4), the weight-streaming kernels of decode batches
+// (k_gemm_skinny*) and the dispatch; kernels_tile.hip has what lies between, and every longer fp32 product.
 #include <string.h>
 
 #include <algorithm>
@@ -28,8 +27,6 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 #define GKB 128           // bytes of K per row and slice
-#define GLD 144           // padded LDS row pitch in bytes
-#define GTHREADS 256
 
 template <typename T> struct GemmTraits;
 template <> struct GemmTraits<float> {
@@ -85,366 +82,9 @@ __device__ __forceinline__ void gemm_tile_of(int id, int tilesM, int tilesN, int
 #define GEMM_EPI_PLAIN 0  // C = acc (+ R), fp32
 #define GEMM_EPI_SWIGLU 1 // columns 2j, 2j+1 are gate and up of unit j: U[m, j] = silu(gate) * up, stored as T
 
-// lda/ldb in elements; K * sizeof(T) must be a multiple of 128.  R may be null, and may alias C.
-// BM x BN 32x32 blocks per wave, waves arranged 2 x 2: the workgroup tile is 64 BM x 64 BN.
-template <typename T, int BM, int BN, int EPI>
-__global__ void __launch_bounds__(GTHREADS) k_gemm_tn(const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb,
-                                                      void* Cv, int ldc, const float* R, int ldr, int M, int N, int K, int tilesM, int tilesN, float alpha) {
-    constexpr int TM = 64 * BM, TN = 64 * BN;
-    constexpr int PA = TM / 32, PB = TN / 32; // 16-byte pieces per thread and slice
-    extern __shared__ __attribute__((aligned(16))) unsigned char gsm[];
-    unsigned char* As = gsm;
-    unsigned char* Bs = gsm + TM * GLD;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    int tm, tn;
-    gemm_tile_of(blockIdx.x, tilesM, tilesN, tm, tn);
-    if (tm < 0) return;
-    const int m0 = tm * TM, n0 = tn * TN;
-    const int nslices = (int)(((size_t)K * sizeof(T)) / GKB);
-    const unsigned char* Ab = reinterpret_cast<const unsigned char*>(A);
-    const unsigned char* Bb = reinterpret_cast<const unsigned char*>(B);
-    const size_t ldaB = (size_t)lda * sizeof(T), ldbB = (size_t)ldb * sizeof(T);
-
-    // global -> register staging; rows past the edge repeat the last row, their results are never stored
-    const int piece = tid & 7, srow = tid >> 3; // piece i of a thread is row srow + 32 i
-    u32x4 ra[PA], rb[PB];
-    auto load_slice = [&](int s) {
-#pragma unroll
-        for (int i = 0; i < PA; i++)
-            ra[i] = *reinterpret_cast<const u32x4*>(Ab + (size_t)min(m0 + srow + 32 * i, M - 1) * ldaB + (size_t)s * GKB + piece * 16);
-#pragma unroll
-        for (int i = 0; i < PB; i++)
-            rb[i] = *reinterpret_cast<const u32x4*>(Bb + (size_t)min(n0 + srow + 32 * i, N - 1) * ldbB + (size_t)s * GKB + piece * 16);
-    };
-    auto store_slice = [&]() {
-#pragma unroll
-        for (int i = 0; i < PA; i++) *reinterpret_cast<u32x4*>(As + (srow + 32 * i) * GLD + piece * 16) = ra[i];
-#pragma unroll
-        for (int i = 0; i < PB; i++) *reinterpret_cast<u32x4*>(Bs + (srow + 32 * i) * GLD + piece * 16) = rb[i];
-    };
-
-    f32x16 acc[BM][BN];
-#pragma unroll
-    for (int i = 0; i < BM; i++)
-#pragma unroll
-        for (int j = 0; j < BN; j++) acc[i][j] = (f32x16)(0.f);
-
-    load_slice(0);
-    store_slice();
-    __syncthreads();
-    const int half = lane >> 5, lrow = lane & 31;
-    for (int s = 0; s < nslices; s++) {
-        if (s + 1 < nslices) load_slice(s + 1);
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            u32x4 fa[BM], fb[BN];
-#pragma unroll
-            for (int b = 0; b < BM; b++) fa[b] = *reinterpret_cast<const u32x4*>(As + (wm * 32 * BM + b * 32 + lrow) * GLD + (2 * jj + half) * 16);
-#pragma unroll
-            for (int b = 0; b < BN; b++) fb[b] = *reinterpret_cast<const u32x4*>(Bs + (wn * 32 * BN + b * 32 + lrow) * GLD + (2 * jj + half) * 16);
-#pragma unroll
-            for (int bm = 0; bm < BM; bm++)
-#pragma unroll
-                for (int bn = 0; bn < BN; bn++) GemmTraits<T>::mma(fa[bm], fb[bn], acc[bm][bn]);
-        }
-        __syncthreads();
-        if (s + 1 < nslices) {
-            store_slice();
-            __syncthreads();
-        }
-    }
-
-    // accumulator layout of the 32x32 tile: element i of lane l is row 8*(i/4) + 4*(l/32) + i%4, column l%32
-#pragma unroll
-    for (int bm = 0; bm < BM; bm++)
-#pragma unroll
-        for (int bn = 0; bn < BN; bn++) {
-            const int col = n0 + wn * 32 * BN + bn * 32 + lrow;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int row = m0 + wm * 32 * BM + bm * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-                float v = acc[bm][bn][i] * alpha;
-                if (EPI == GEMM_EPI_SWIGLU) {
-                    const float o = __shfl_xor(v, 1, 64); // the up value sits in the odd neighbour lane
-                    if (!(lane & 1) && row < M && col < N) GemmTraits<T>::put((T*)Cv + (size_t)row * ldc + (col >> 1), (v / (1.0f + expf(-v))) * o);
-                } else if (row < M && col < N) {
-                    if (R) v += R[(size_t)row * ldr + col];
-                    ((float*)Cv)[(size_t)row * ldc + col] = v;
-                }
-            }
-        }
-}
-
 // ----------------------------------------------------------------------------
-// Large-tile variant for long M (prefill): 256 x 256 output tile per 512-thread workgroup, each of the
-// 2 x 4 waves owning 128 x 64 (eight 32x32 accumulators).  K slices of 128 bytes per row go from global
-// memory straight into LDS (no register staging), two stages deep: the loads of slice s+1 are in
-// flight while slice s is multiplied, and one barrier per slice separates the stages.
-//
-// A direct load puts lane i's 16 bytes at (wave-uniform base) + 16 i, so rows cannot be padded.  The
-// 8 pieces of a 128-byte row are stored permuted instead: slot j of row r holds piece j ^ ((r >> 1) & 7)
-// -- the lane picks which piece it fetches, not where it lands.  The LDS serves 256 bytes (64 banks) per
-// cycle, i.e. sixteen lanes of a 16-byte read; two consecutive rows fill the 64 banks once, so sixteen
-// consecutive rows reading the same piece touch sixteen different 16-byte bank groups: even and odd rows
-// lie in different halves of the banks, and rows of equal parity differ in (r >> 1) & 7.
-// ----------------------------------------------------------------------------
-#define GB_T 256
-#define GB_STAGE (2 * GB_T * GKB) // bytes per stage: A rows then B rows
-
-#define GB_THREADS 512 // 8 waves: 2 along M x 4 along N, each 128 x 64 (two waves per SIMD keep LDS and MFMA busy in turn)
-#define GB_BN 2        // 32-wide column blocks per wave
-
-template <typename T, int EPI>
-__global__ void __launch_bounds__(GB_THREADS) k_gemm_tn_big(const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb,
-                                                            void* Cv, int ldc, const float* R, int ldr, int M, int N, int K, int tilesM, int tilesN, float alpha) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char gsm[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 2, wn = wave & 3;
-    // A workgroup walks the tiles id, id + gridDim.x, ... (one workgroup per compute unit): the first slice of the next
-    // tile is fetched during the last slice of the current one and the epilogue's stores drain under the next tile's
-    // first slices, so a tile boundary costs the epilogue's issue time, not a kernel launch, a cold start and a drain.
-    int id = blockIdx.x, tm, tn;
-    gemm_tile_of(id, tilesM, tilesN, tm, tn);
-    if (tm < 0) return;
-    const int nslices = (int)(((size_t)K * sizeof(T)) / GKB);
-    const size_t ldaB = (size_t)lda * sizeof(T), ldbB = (size_t)ldb * sizeof(T);
-
-    // A loading wave fills 64 rows of A and of B, eight rows per load instruction.  A load's address is
-    // a scalar base (the tile's first row, advanced by one slice per trip on the scalar unit) plus a 32-bit lane offset
-    // that changes only from tile to tile, and its LDS target is scalar too: issuing a slice's loads takes no vector-ALU
-    // instruction, so it does not queue behind the MFMAs of the other wave on the SIMD.
-    // Only the first wave of every SIMD (waves 0..3) loads, for its own rows and for those of the SIMD's second wave:
-    // the load path takes an instruction every ~50 ns per SIMD and a wave starts its MFMAs only when its loads are
-    // out, so the second wave multiplies while the first one feeds the load path.  (Spreading the loads between the
-    // MFMAs instead, by quarters or one per MFMA pair, measured 5-9 % slower.)
-    unsigned goffA[8], goffB[8];
-    auto uniform_base = [](const void* p) { // wave-uniform pointer into global memory, kept in scalar registers
-        unsigned long long v = (unsigned long long)p;
-        asm("" : "+s"(v));
-        return (const unsigned char*)(__attribute__((address_space(1))) const unsigned char*)v;
-    };
-    const unsigned char *baseA, *baseB;
-    auto aim = [&](int tm_, int tn_) { // lane offsets and scalar bases of tile (tm_, tn_)
-        const int m0_ = tm_ * GB_T, n0_ = tn_ * GB_T;
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const int r = (wave & 3) * 64 + q * 8 + (lane >> 3);
-            const int pc = (lane & 7) ^ ((r >> 1) & 7);
-            goffA[q] = (unsigned)((size_t)(min(m0_ + r, M - 1) - m0_) * ldaB) + pc * 16; // rows past the end: the last row again
-            goffB[q] = (unsigned)((size_t)(min(n0_ + r, N - 1) - n0_) * ldbB) + pc * 16;
-        }
-        baseA = uniform_base(reinterpret_cast<const unsigned char*>(A) + (size_t)m0_ * ldaB);
-        baseB = uniform_base(reinterpret_cast<const unsigned char*>(B) + (size_t)n0_ * ldbB);
-    };
-    // (written as the instruction itself: through the builtin the compiler either re-forms 64-bit lane addresses or
-    // copies the offsets, one vector-ALU instruction per load either way)
-    auto dma16 = [](unsigned long long sbase, unsigned laneOff, unsigned ldsAddr) {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(ldsAddr), "v"(laneOff), "s"(sbase) : "memory", "m0");
-    };
-    const unsigned ldsBase = (unsigned)(unsigned long long)gsm + (unsigned)((wave & 3) * 64 * GKB);
-    auto issue = [&](int s, int stage) {
-        if (wave >= 4) return;
-        const unsigned dst = ldsBase + (unsigned)(stage * GB_STAGE);
-        const unsigned long long sa = (unsigned long long)baseA + (unsigned long long)s * GKB, sb = (unsigned long long)baseB + (unsigned long long)s * GKB;
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            dma16(sa, goffA[q], dst + q * 8 * GKB);
-            dma16(sb, goffB[q], dst + GB_T * GKB + q * 8 * GKB);
-        }
-    };
-
-    const int half = lane >> 5, lrow = lane & 31;
-    // row offsets and swizzle keys of this lane's operand rows ((row >> 1) & 7 does not depend on the 32-row block)
-    const int keyA = ((wm * 128 + lrow) >> 1) & 7, keyB = ((wn * 32 * GB_BN + lrow) >> 1) & 7;
-    const int offA = (wm * 128 + lrow) * GKB, offB = GB_T * GKB + (wn * 32 * GB_BN + lrow) * GKB;
-
-    aim(tm, tn);
-    issue(0, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    int gs = 0; // slices consumed so far, over all tiles: slice gs sits in stage gs & 1
-  for (;;) {
-    const int m0 = tm * GB_T, n0 = tn * GB_T;
-    int tmN, tnN;
-    gemm_tile_of(id + (int)gridDim.x, tilesM, tilesN, tmN, tnN);
-    const bool more = tmN >= 0;
-    f32x16 acc[4][GB_BN];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < GB_BN; j++) acc[i][j] = (f32x16)(0.f);
-    for (int s = 0; s < nslices; s++, gs++) {
-        const int stage = gs & 1;
-        const unsigned char* base = gsm + stage * GB_STAGE;
-        // operand fragments one 16-wide step ahead of the MFMAs that use them
-        u32x4 fa[2][4], fb[2][GB_BN];
-        auto frags = [&](int jj, int buf) {
-            const int pa = ((2 * jj + half) ^ keyA) * 16, pb = ((2 * jj + half) ^ keyB) * 16;
-#pragma unroll
-            for (int b = 0; b < 4; b++) fa[buf][b] = *reinterpret_cast<const u32x4*>(base + offA + b * 32 * GKB + pa);
-#pragma unroll
-            for (int b = 0; b < GB_BN; b++) fb[buf][b] = *reinterpret_cast<const u32x4*>(base + offB + b * 32 * GKB + pb);
-        };
-        frags(0, 0); // before the loads: the first operands cross the LDS latency while the loads go out
-        __builtin_amdgcn_sched_barrier(0);
-        if (s + 1 < nslices) issue(s + 1, stage ^ 1);
-        else if (more) { aim(tmN, tnN); issue(0, stage ^ 1); } // the tile's own slices are all out: the next tile's first one
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            // the reads of step jj+1 go out in the middle of step jj's MFMAs: early enough to have landed when
-            // they are needed, late enough that waiting for step jj's operands does not wait for them too.
-            // The scheduling barriers pin that order (the scheduler would sink every read to its first use).
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int bm = 0; bm < 2; bm++)
-#pragma unroll
-                for (int bn = 0; bn < GB_BN; bn++) GemmTraits<T>::mma(fb[jj & 1][bn], fa[jj & 1][bm], acc[bm][bn]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (jj < 3) frags(jj + 1, (jj + 1) & 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int bm = 2; bm < 4; bm++)
-#pragma unroll
-                for (int bn = 0; bn < GB_BN; bn++) GemmTraits<T>::mma(fb[jj & 1][bn], fa[jj & 1][bm], acc[bm][bn]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the slice after this one has landed
-        __syncthreads();                                  // ... for every wave, and everyone is done with this one
-    }
-    unsigned char* const freeStage = gsm + ((gs - 1) & 1) * GB_STAGE; // the stage consumed last: the epilogue's patches live there
-
-    // Epilogue.  The product was formed transposed (weights as the first MFMA operand), so lane (lrow, half) holds, for
-    // every 32 x 32 block, row lrow of C and the columns 8 g + 4 half + 0..3 in acc[..][4 g + 0..3]: the gate and up value
-    // of a SwiGLU pair sit in one lane.  A block then goes through a patch of LDS of the wave's own (the stages are free:
-    // the loop ended with a barrier) and is read back with several lanes per row, so that a store instruction writes whole
-    // rows of 64 or 128 bytes instead of 64 scattered pieces; the residual is read the same way.
-    {
-        constexpr int EP = 144;                                  // patch row pitch in bytes (16-byte aligned, rows 4 banks apart)
-        typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
-        typedef __attribute__((address_space(3))) uint32_t lds_u32;
-        typedef __attribute__((address_space(3))) float lds_f32;
-        const unsigned patch = (unsigned)(unsigned long long)freeStage + wave * (32 * EP); // 8 x 4.5 KB inside the 64 KB stage
-        const int mW = m0 + wm * 128, nW = n0 + wn * 32 * GB_BN;
-        if (EPI == GEMM_EPI_PLAIN) {
-            const bool vec = ((ldc & 3) == 0) && (!R || (ldr & 3) == 0) && (((unsigned long long)Cv & 15) == 0) && (((unsigned long long)R & 15) == 0);
-            const unsigned wr = patch + lrow * EP + half * 16, rd = patch + (lane >> 3) * EP + (lane & 7) * 16;
-#pragma unroll
-            for (int bm = 0; bm < 4; bm++)
-#pragma unroll
-                for (int bn = 0; bn < GB_BN; bn++) {
-                    const unsigned pb = 0;
-#pragma unroll
-                    for (int g = 0; g < 4; g++) {
-                        f32x4 v;
-                        v.x = acc[bm][bn][4 * g] * alpha; v.y = acc[bm][bn][4 * g + 1] * alpha; v.z = acc[bm][bn][4 * g + 2] * alpha; v.w = acc[bm][bn][4 * g + 3] * alpha;
-                        *(lds_f32x4*)(wr + pb + g * 32) = v;
-                    }
-                    const int rowb = mW + bm * 32 + (lane >> 3), col = nW + bn * 32 + (lane & 7) * 4;
-                    f32x4 v[4];
-#pragma unroll
-                    for (int k = 0; k < 4; k++) v[k] = *(const lds_f32x4*)(rd + pb + k * 8 * EP);
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const int row = rowb + 8 * k;
-                        if (row >= M || col >= N) continue;
-                        float* cp = (float*)Cv + (size_t)row * ldc + col;
-                        if (vec && col + 3 < N) {
-                            if (R) v[k] += *reinterpret_cast<const f32x4*>(R + (size_t)row * ldr + col);
-                            *reinterpret_cast<f32x4*>(cp) = v[k];
-                        } else {
-                            const float* rp = R ? R + (size_t)row * ldr + col : nullptr;
-                            cp[0] = v[k].x + (rp ? rp[0] : 0.f);
-                            if (col + 1 < N) cp[1] = v[k].y + (rp ? rp[1] : 0.f);
-                            if (col + 2 < N) cp[2] = v[k].z + (rp ? rp[2] : 0.f);
-                            if (col + 3 < N) cp[3] = v[k].w + (rp ? rp[3] : 0.f);
-                        }
-                    }
-                }
-        } else { // SwiGLU: columns 2 j, 2 j + 1 of the product are gate and up of unit j; U[m, j] = silu(gate) * up in the operand type
-            constexpr int ES = (int)sizeof(T);                   // 2 or 4
-            constexpr int OUTW = 16 * GB_BN;                     // units per row of the wave's tile
-            constexpr int LPR = OUTW * ES / 16;                  // lanes per row when reading back 16 bytes each
-            constexpr int RPP = 64 / LPR;                        // rows per pass
-            const bool vec = (((size_t)ldc * ES) & 15) == 0 && (((unsigned long long)Cv & 15) == 0);
-            const int jW = nW >> 1, NU = N >> 1;
-#pragma unroll
-            for (int bm = 0; bm < 4; bm++) {
-                const unsigned pb = 0;
-#pragma unroll
-                for (int bn = 0; bn < GB_BN; bn++)
-#pragma unroll
-                    for (int g = 0; g < 4; g++) {
-                        const float g0 = acc[bm][bn][4 * g] * alpha, u0 = acc[bm][bn][4 * g + 1] * alpha;
-                        const float g1 = acc[bm][bn][4 * g + 2] * alpha, u1 = acc[bm][bn][4 * g + 3] * alpha;
-                        const float o0 = (g0 / (1.0f + expf(-g0))) * u0, o1 = (g1 / (1.0f + expf(-g1))) * u1;
-                        const unsigned at = patch + pb + lrow * EP + (bn * 16 + 4 * g + 2 * half) * ES;
-                        if (ES == 2) {
-                            *(lds_u32*)at = GemmTraits<T>::bits(o0) | (GemmTraits<T>::bits(o1) << 16);
-                        } else {
-                            *(lds_f32*)at = o0;
-                            *(lds_f32*)(at + 4) = o1;
-                        }
-                    }
-#pragma unroll
-                for (int k = 0; k < 32 / RPP; k++) {
-                    const int rl = (lane / LPR) + RPP * k, piece = lane % LPR;
-                    const f32x4 v = *(const lds_f32x4*)(patch + pb + rl * EP + piece * 16);
-                    const int row = mW + bm * 32 + rl, j = jW + piece * (16 / ES);
-                    if (row >= M || j >= NU) continue;
-                    T* up = (T*)Cv + (size_t)row * ldc + j;
-                    if (vec && j + 16 / ES - 1 < NU) {
-                        *reinterpret_cast<f32x4*>(up) = v;
-                    } else {
-                        const uint32_t w[4] = {__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
-#pragma unroll
-                        for (int e = 0; e < 16 / ES; e++)
-                            if (j + e < NU) {
-                                if (ES == 2) reinterpret_cast<uint16_t*>(up)[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
-                                else reinterpret_cast<uint32_t*>(up)[e] = w[e];
-                            }
-                    }
-                }
-            }
-        }
-    }
-    if (!more) break;
-    __syncthreads(); // every wave is done with its patch: the stage may be fetched into again
-    id += (int)gridDim.x; tm = tmN; tn = tnN;
-  }
-}
-
-template <typename T>
-static hipError_t launch_gemm_big(hipStream_t stream, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                                  const float* R, int ldr, int M, int N, int K, float alpha) {
-    const int tilesM = (M + GB_T - 1) / GB_T, tilesN = (N + GB_T - 1) / GB_T;
-    static int numCUs = 0;
-    if (!numCUs) {
-        hipDeviceProp_t prop;
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess) return hipErrorInvalidDevice;
-        numCUs = std::max(8, (prop.multiProcessorCount / 8) * 8);
-    }
-    const unsigned grid = (unsigned)std::min(numCUs, ((tilesM * tilesN + 7) / 8) * 8); // one workgroup per compute unit walks its tiles
-    const size_t lds = 2 * GB_STAGE;
-    static std::atomic<bool> attr{false}; // set-up is idempotent: two threads that race here both do it
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_tn_big<T, GEMM_EPI_PLAIN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_tn_big<T, GEMM_EPI_SWIGLU>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
-    if (epi == GEMM_EPI_SWIGLU)
-        hipLaunchKernelGGL((k_gemm_tn_big<T, GEMM_EPI_SWIGLU>), dim3(grid), dim3(GB_THREADS), lds, stream, (const T*)A, lda, (const T*)B, ldb, C, ldc, R, ldr, M, N, K, tilesM, tilesN, alpha);
-    else
-        hipLaunchKernelGGL((k_gemm_tn_big<T, GEMM_EPI_PLAIN>), dim3(grid), dim3(GB_THREADS), lds, stream, (const T*)A, lda, (const T*)B, ldb, C, ldc, R, ldr, M, N, K, tilesM, tilesN, alpha);
-    return hipGetLastError();
-}
-
-// ----------------------------------------------------------------------------
-// Large-tile kernel for two-byte operands (the prefill path of a bf16 model): the same 256 x 256 tile, K slices and
-// LDS layout as k_gemm_tn_big, but FOUR waves per workgroup, one per SIMD, each owning 128 x 128 of the tile in 256
-// accumulator registers, multiplied with v_mfma_f32_16x16x32 (64 blocks of 16 x 16 per wave, two 32-wide steps per
+// Large-tile kernel for two-byte operands (the prefill path of a bf16 model): 256 x 256 output tile per workgroup of
+// four waves, one per SIMD, each owning 128 x 128 of the tile in 256 accumulator registers, multiplied with v_mfma_f32_16x16x32 (64 blocks of 16 x 16 per wave, two 32-wide steps per
 // slice).  On operand data that toggles the multipliers the part is limited by power, not by issue slots, and the
 // 16 x 16 x 32 form does a given product on less of it than 32 x 32 x 16 (an accumulator is read and written once per
 // 32 products instead of once per 16): a register-only loop of either form sustains 1.95 against 1.70 PFLOP/s on
@@ -461,8 +101,15 @@ static hipError_t launch_gemm_big(hipStream_t stream, int epi, const void* A, in
 // The load cursor runs ahead of the multiply position and crosses tile boundaries by itself: a workgroup walks its
 // tiles in one launch and the next tile's first two slices are in flight while the epilogue runs.  The epilogue uses a
 // patch of LDS per wave outside the two stages.  Per slice and wave: 128 MFMAs, 32 LDS reads, 16 loads -- a third fewer
-// LDS bytes per flop than the 8-wave kernel (128 x 128 per wave instead of 128 x 64).
+// LDS bytes per flop than with eight waves of 128 x 64.
+// K slices of 128 bytes per row go from global memory straight into LDS, two stages deep.  A direct load puts lane i's
+// 16 bytes at (wave-uniform base) + 16 i, so rows cannot be padded; the eight pieces of a row are stored permuted
+// instead: slot j of row r holds piece j ^ ((r >> 1) & 7) -- the lane picks which piece it fetches, not where it lands.
+// The LDS serves 256 bytes (64 banks) per cycle, i.e. sixteen lanes of a 16-byte read; two consecutive rows fill the banks
+// once, and sixteen rows reading the same piece touch sixteen different 16-byte bank groups.
 // ----------------------------------------------------------------------------
+#define GB_T 256
+#define GB_STAGE (2 * GB_T * GKB) // bytes per stage: A rows then B rows
 #define GW_THREADS 256
 #define GW_FPOS 40     // MFMA index within a slice (0..127) in front of which F sits
 #define GW_RPOS 96     // ... and R
@@ -796,7 +443,7 @@ __global__ void __launch_bounds__(GW_THREADS) k_gemm_tn_w4(const T* __restrict__
 
 // Compute units of the current device, rounded down to a multiple of eight (one workgroup per unit, the same number
 // on every XCD); 0 when the device cannot be asked.
-static int gemm_num_cus() {
+int mlh_gemm_num_cus(void) {
     static std::atomic<int> numCUs{0};
     if (!numCUs) {
         hipDeviceProp_t prop;
@@ -811,7 +458,7 @@ template <typename T>
 static hipError_t launch_gemm_w4(hipStream_t stream, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
                                  const float* R, int ldr, int M, int N, int K, float alpha) {
     const int tilesM = (M + GB_T - 1) / GB_T, tilesN = (N + GB_T - 1) / GB_T;
-    const int numCUs = gemm_num_cus();
+    const int numCUs = mlh_gemm_num_cus();
     if (!numCUs) return hipErrorInvalidDevice;
     const unsigned grid = (unsigned)std::min(numCUs, ((tilesM * tilesN + 7) / 8) * 8); // one workgroup per compute unit walks its tiles
     const size_t lds = GW_LDS;
@@ -836,27 +483,12 @@ static hipError_t launch_gemm_w4(hipStream_t stream, int epi, const void* A, int
     return hipGetLastError();
 }
 
-template <typename T, int BM, int BN>
-static hipError_t launch_gemm(hipStream_t stream, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                              const float* R, int ldr, int M, int N, int K, float alpha) {
-    constexpr int TM = 64 * BM, TN = 64 * BN;
-    const int tilesM = (M + TM - 1) / TM, tilesN = (N + TN - 1) / TN;
-    const int total = tilesM * tilesN;
-    const unsigned grid = (unsigned)(((total + 7) / 8) * 8);
-    const size_t lds = (size_t)(TM + TN) * GLD;
-    static std::atomic<bool> attr[2] = {{false}, {false}};
-    if (lds > 64 * 1024 && !attr[epi]) {
-        hipError_t e = hipFuncSetAttribute(epi ? reinterpret_cast<const void*>(&k_gemm_tn<T, BM, BN, GEMM_EPI_SWIGLU>)
-                                               : reinterpret_cast<const void*>(&k_gemm_tn<T, BM, BN, GEMM_EPI_PLAIN>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        attr[epi] = true;
-    }
-    if (epi == GEMM_EPI_SWIGLU)
-        hipLaunchKernelGGL((k_gemm_tn<T, BM, BN, GEMM_EPI_SWIGLU>), dim3(grid), dim3(GTHREADS), lds, stream, (const T*)A, lda, (const T*)B, ldb, C, ldc, R, ldr, M, N, K, tilesM, tilesN, alpha);
-    else
-        hipLaunchKernelGGL((k_gemm_tn<T, BM, BN, GEMM_EPI_PLAIN>), dim3(grid), dim3(GTHREADS), lds, stream, (const T*)A, lda, (const T*)B, ldb, C, ldc, R, ldr, M, N, K, tilesM, tilesN, alpha);
-    return hipGetLastError();
+// Expected microseconds of launch_gemm_w4: rounds of one tile per compute unit, a K slice of 1.22 us and an epilogue of 4.5 us
+// where few units work, 1.5 and 12 us where all do (the epilogue's stores then share the memory, the MFMAs the power).
+static double w4_us(int M, int N, int K, int cus) {
+    const int tiles = ((M + GB_T - 1) / GB_T) * ((N + GB_T - 1) / GB_T), full = tiles / cus;
+    const double slices = K / 64.0, load = (double)(tiles - full * cus) / cus;
+    return full * (1.5 * slices + 12.0) + (load > 0 ? (1.22 + 0.28 * load) * slices + 4.5 + 7.5 * load : 0.0);
 }
 
 // ----------------------------------------------------------------------------
@@ -882,7 +514,7 @@ __device__ __forceinline__ void g_ast(float* p, float v) {
     __hip_atomic_store(reinterpret_cast<unsigned*>(p), __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-#define GSK_COUNTERS 1024 // tiles a split-K launch may have (N <= 32768)
+#define GSK_COUNTERS MLH_GEMM_WS_COUNTERS // tiles a split-K launch may have (N <= 32768)
 #define GSK_WAVES 8       // waves of a skinny-GEMM workgroup: they split K, and each keeps two chunks of loads in flight --
                           // with few waves the kernel waits on memory latency chunk after chunk, not on bandwidth
 
@@ -1440,7 +1072,7 @@ static hipError_t launch_gemm_skinny16(hipStream_t stream, int epi, const void* 
 }
 
 // Workspace for split-K: GSK_COUNTERS zeroed counters, then the partial tiles.
-size_t mlh_gemm_workspace_bytes(void) { return (size_t)GSK_COUNTERS * 4 + (size_t)256 * 8 * 2 * 16 * 64 * 4; }
+size_t mlh_gemm_workspace_bytes(void) { return (size_t)GSK_COUNTERS * 4 + (size_t)MLH_GEMM_WS_PARTIALS * 4; }
 
 template <typename T, int MB>
 static hipError_t launch_gemm_skinny(hipStream_t stream, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
@@ -1479,13 +1111,14 @@ bool mlh_gemm_norm_fusable(int dtype, int M, int N, int K) {
 
 hipError_t mlh_gemm_tn_epi(hipStream_t stream, int dtype, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
                            const float* R, int ldr, int M, int N, int K, void* ws, float alpha, const float* normGain) {
-    const size_t esz = dtype == MLH_DTYPE_F32 ? 4 : 2;
+    const size_t esz = dtype == MLH_GEMM_P3 ? 6 : dtype == MLH_DTYPE_F32 ? 4 : 2;
+    if (dtype == MLH_GEMM_P3 && (M <= 0 || N <= 0 || K <= 0 || K % 32 || lda % 32 || ldb % 32)) return hipErrorInvalidValue;
+    if (dtype == MLH_GEMM_P3) return mlh_gemm_tile(stream, dtype, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha);
     if (M <= 0 || N <= 0 || K <= 0 || ((size_t)K * esz) % GKB != 0 || ((size_t)lda * esz) % 16 != 0 || ((size_t)ldb * esz) % 16 != 0)
         return hipErrorInvalidValue;
     if (epi == GEMM_EPI_SWIGLU && (N & 1)) return hipErrorInvalidValue;
     if (normGain && !mlh_gemm_norm_fusable(dtype, M, N, K)) return hipErrorInvalidValue;
-    // M <= 64 (one row per sequence of a decode batch): weight-streaming skinny kernel; long M: 256 x 256 tiles
-    // fed by direct-to-LDS loads; in between: 128 x 128 tiles
+    // M <= 64 (one row per sequence of a decode batch): weight-streaming skinny kernel; more rows: tiles
 #define GEMM_BY_TYPE(call_f32, call_bf16, call_f16) \
     return dtype == MLH_DTYPE_BF16 ? (call_bf16) : dtype == MLH_GEMM_F16 ? (call_f16) : (call_f32)
     if (M <= 32 && normGain && dtype == MLH_GEMM_F16 && skinny_norm8_fits(M, K))
@@ -1503,38 +1136,28 @@ hipError_t mlh_gemm_tn_epi(hipStream_t stream, int dtype, int epi, const void* A
         GEMM_BY_TYPE((launch_gemm_skinny<float, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)),
                      (launch_gemm_skinny<bf16_t, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)),
                      (launch_gemm_skinny<f16_t, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)));
-    if (M > 128 && N <= 128 && dtype != MLH_DTYPE_F32 && epi == GEMM_EPI_PLAIN) { // a narrow strip of columns: 64-row tiles put every compute unit to work
-        if (dtype == MLH_GEMM_F16) return launch_gemm<f16_t, 1, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha);
-        return launch_gemm<bf16_t, 1, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha);
-    }
-    if (M > 128 && dtype != MLH_DTYPE_F32 && epi == GEMM_EPI_PLAIN && N > GB_T && N % GB_T != 0 && N % GB_T <= 128) {
-        // A last column of tiles that is less than half full: when taking it away saves the tile walkers a whole round
-        // (every compute unit one 256 x 256 tile: K x 31 ns) and the strip kernel does those columns in less than that
-        // (5 us + 180 TFLOP/s, measured), the product runs as two launches.
-        const int rem = N % GB_T, cus = gemm_num_cus(), tilesM = (M + GB_T - 1) / GB_T;
-        if (!cus) return hipErrorInvalidDevice;
-        const int roundsAll = (tilesM * (N / GB_T + 1) + cus - 1) / cus, roundsMain = (tilesM * (N / GB_T) + cus - 1) / cus;
-        if (roundsMain < roundsAll && 5.0 + 2.0 * M * rem * K / 180e6 < 0.031 * K) {
-            const int Nm = N - rem;
+    if (dtype == MLH_DTYPE_F32) return hipErrorInvalidValue; // longer fp32 products take their operands as planes (MLH_GEMM_P3)
+    // Two-byte operands: 256 x 256 tiles walked by one workgroup per unit where there are enough of them, smaller tiles
+    // (kernels_tile.hip) otherwise: the estimates decide.
+    const int cus = mlh_gemm_num_cus();
+    if (!cus) return hipErrorInvalidDevice;
+    const double usTile = mlh_gemm_tile_us(dtype, M, N, K, cus, ws != nullptr), usW4 = w4_us(M, N, K, cus);
+    if (usTile <= usW4) return mlh_gemm_tile(stream, dtype, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha);
+    const int rem = N % GB_T;
+    if (epi == GEMM_EPI_PLAIN && N > GB_T && rem != 0 && rem <= 128) {
+        // A last column of tiles that is less than half full: the product runs as two launches when taking those columns
+        // away saves the tile walkers more (a round) than they cost as a strip of their own.
+        const int Nm = N - rem;
+        if (w4_us(M, Nm, K, cus) + mlh_gemm_tile_us(dtype, M, rem, K, cus, ws != nullptr) < usW4) {
             const hipError_t e = mlh_gemm_tn_epi(stream, dtype, epi, A, lda, B, ldb, C, ldc, R, ldr, M, Nm, K, ws, alpha, nullptr);
             if (e != hipSuccess) return e;
-            return mlh_gemm_tn_epi(stream, dtype, epi, A, lda, (const unsigned char*)B + (size_t)Nm * ldb * esz, ldb, (float*)C + Nm, ldc,
-                                   R ? R + Nm : nullptr, ldr, M, rem, K, ws, alpha, nullptr);
+            return mlh_gemm_tile(stream, dtype, epi, A, lda, (const unsigned char*)B + (size_t)Nm * ldb * esz, ldb, (float*)C + Nm, ldc,
+                                 R ? R + Nm : nullptr, ldr, M, rem, K, ws, alpha);
         }
     }
-    if (M > 128)
-        GEMM_BY_TYPE((launch_gemm_big<float>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha)),
-                     (launch_gemm_w4<bf16_t>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha)),
-                     (launch_gemm_w4<f16_t>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha)));
-    GEMM_BY_TYPE((launch_gemm<float, 2, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha)),
-                 (launch_gemm<bf16_t, 2, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha)),
-                 (launch_gemm<f16_t, 2, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha)));
+    return dtype == MLH_DTYPE_BF16 ? launch_gemm_w4<bf16_t>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha)
+                                   : launch_gemm_w4<f16_t>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha);
 #undef GEMM_BY_TYPE
-}
-
-hipError_t mlh_gemm_tn(hipStream_t stream, int dtype, const void* A, int lda, const void* B, int ldb, float* C, int ldc,
-                       const float* R, int ldr, int M, int N, int K) {
-    return mlh_gemm_tn_epi(stream, dtype, GEMM_EPI_PLAIN, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, nullptr, 1.0f);
 }
 
 static void host_to_bf16(const float* src, bf16_t* dst, size_t n) {
@@ -1558,15 +1181,18 @@ static void host_to_f16(const float* src, f16_t* dst, size_t n) {
 // dtype says so), result back on the host, mean launch time over `iters` launches from HIP events.
 extern "C" int mlh_selftest_gemm(int dtypeAndEpilogue, int M, int N, int K, const float* A, const float* B, const float* R, float* C,
                                  int iters, double* avgUs) {
-    const int dtype = dtypeAndEpilogue & 0xff;
+    int dtype = dtypeAndEpilogue & 0xff;
+    if (dtype == MLH_DTYPE_F32 && M > 64) dtype = MLH_GEMM_P3; // as the prefill pass does
+    const bool p3 = dtype == MLH_GEMM_P3;
     const bool swiglu = (dtypeAndEpilogue & MLH_SELFTEST_SWIGLU) != 0; // C is then [M, N / 2]: silu(gate) * up of the column pairs
     if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0 || (swiglu && (R || (N & 1)))) return -1;
     if (mlh_device_count() <= 0) return -1;
-    const size_t esz = dtype == MLH_DTYPE_F32 ? 4 : 2;
-    const int NC = swiglu ? N / 2 : N;
+    if (p3 && K % 32) return -1;
+    const size_t esz = p3 ? 6 : dtype == MLH_DTYPE_F32 ? 4 : 2;
+    const int NC = !swiglu ? N : p3 ? (N / 2 + 31) / 32 * 32 : N / 2; // (rows of planes are whole blocks)
     const size_t csz = swiglu ? esz : 4; // the SwiGLU epilogue writes the operand type
     void *dA = nullptr, *dB = nullptr, *dW = nullptr, *dC = nullptr;
-    float* dR = nullptr;
+    float *dR = nullptr, *dF = nullptr;
     int rc = 0;
     std::vector<bf16_t> ha, hb;
     std::vector<uint16_t> hc;
@@ -1586,8 +1212,17 @@ extern "C" int mlh_selftest_gemm(int dtypeAndEpilogue, int M, int N, int K, cons
     ST(hipMalloc(&dA, (size_t)M * K * esz)); ST(hipMalloc(&dB, (size_t)N * K * esz));
     ST(hipMalloc(&dC, (size_t)M * NC * csz));
     if (R) { ST(hipMalloc((void**)&dR, (size_t)M * N * 4)); ST(hipMemcpy(dR, R, (size_t)M * N * 4, hipMemcpyHostToDevice)); }
-    ST(hipMemcpy(dA, srcA, (size_t)M * K * esz, hipMemcpyHostToDevice));
-    ST(hipMemcpy(dB, srcB, (size_t)N * K * esz, hipMemcpyHostToDevice));
+    if (p3) {
+        ST(hipMalloc((void**)&dF, (size_t)std::max(M, N) * K * 4));
+        ST(hipMemcpy(dF, A, (size_t)M * K * 4, hipMemcpyHostToDevice));
+        ST(mlh_split_p3(nullptr, dF, K, dA, K, M, K));
+        ST(hipDeviceSynchronize());
+        ST(hipMemcpy(dF, B, (size_t)N * K * 4, hipMemcpyHostToDevice));
+        ST(mlh_split_p3(nullptr, dF, K, dB, K, N, K));
+    } else {
+        ST(hipMemcpy(dA, srcA, (size_t)M * K * esz, hipMemcpyHostToDevice));
+        ST(hipMemcpy(dB, srcB, (size_t)N * K * esz, hipMemcpyHostToDevice));
+    }
     ST(hipMalloc(&dW, mlh_gemm_workspace_bytes()));
     ST(hipMemset(dW, 0, mlh_gemm_workspace_bytes()));
     ST(mlh_gemm_tn_epi(nullptr, dtype, epi, dA, K, dB, K, dC, NC, dR, N, M, N, K, dW));
@@ -1604,6 +1239,16 @@ extern "C" int mlh_selftest_gemm(int dtypeAndEpilogue, int M, int N, int K, cons
     }
     if (csz == 4) {
         ST(hipMemcpy(C, dC, (size_t)M * NC * 4, hipMemcpyDeviceToHost));
+    } else if (p3) { // the sum of the planes is the fp32 result
+        hc.resize((size_t)M * NC * 3);
+        ST(hipMemcpy(hc.data(), dC, hc.size() * 2, hipMemcpyDeviceToHost));
+        for (int m = 0; m < M; m++)
+            for (int j = 0; j < N / 2; j++) {
+                const uint16_t* b = hc.data() + ((size_t)m * (NC / 32) + j / 32) * 96 + j % 32;
+                float v = 0.f;
+                for (int p = 2; p >= 0; p--) { const uint32_t u = (uint32_t)b[32 * p] << 16; float f; memcpy(&f, &u, 4); v += f; }
+                C[(size_t)m * (N / 2) + j] = v;
+            }
     } else { // half or bf16 results back as floats
         hc.resize((size_t)M * NC);
         ST(hipMemcpy(hc.data(), dC, hc.size() * 2, hipMemcpyDeviceToHost));
@@ -1616,7 +1261,7 @@ extern "C" int mlh_selftest_gemm(int dtypeAndEpilogue, int M, int N, int K, cons
 done:
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
-    (void)hipFree(dA); (void)hipFree(dB); (void)hipFree(dC); (void)hipFree(dR); (void)hipFree(dW);
+    (void)hipFree(dA); (void)hipFree(dB); (void)hipFree(dC); (void)hipFree(dR); (void)hipFree(dW); (void)hipFree(dF);
     return rc;
 }
 

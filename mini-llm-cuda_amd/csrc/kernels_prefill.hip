@@ -10,12 +10,14 @@
 //
 // and at the end the LM head runs for the last row of every segment only (the reference computes
 // logits for all L columns, inference.cu:723-743, and uses the last one).  With bf16 weights the GEMM
-// inputs (normed activations, mixing output, FFN activations) are rounded to bf16; accumulation, the
+// inputs (normed activations, mixing output, FFN activations) are rounded to half; with fp32 weights they and the
+// weights are stored as three bf16 planes that add up to the fp32 value (p3.h).  Accumulation, the
 // residual stream, K/V and GDN states stay fp32.  This is what runInference(L) (inference.cu:376-751)
 // does for L columns, minus the columns that are already in the cache.
 #include <algorithm>
 
 #include "mlh_internal.h"
+#include "p3.h"
 #include "sample.h"
 
 #define PWG 256
@@ -72,6 +74,9 @@ template <> __device__ __forceinline__ void put<f16_t>(f16_t* p, float v) { // s
     const _Float16 h = (_Float16)fminf(fmaxf(v, -65504.0f), 65504.0f);
     p->bits = __builtin_bit_cast(uint16_t, h);
 }
+// element `col` of row `row` of a GEMM input matrix (leading dimension ld in elements; fp32 models: three bf16 planes, p3.h)
+template <typename AT> __device__ __forceinline__ void put_at(void* base, size_t row, int ld, int col, float v) { put<AT>((AT*)base + row * ld + col, v); }
+template <> __device__ __forceinline__ void put_at<p3_t>(void* base, size_t row, int ld, int col, float v) { p3_put((unsigned char*)base + row * ld * 6, col, v); }
 template <typename WT> __device__ __forceinline__ float getw(const WT* p);
 template <> __device__ __forceinline__ float getw<float>(const float* p) { return *p; }
 template <> __device__ __forceinline__ float getw<bf16_t>(const bf16_t* p) { return __uint_as_float(((uint32_t)*p) << 16); }
@@ -102,8 +107,11 @@ template <> __device__ __forceinline__ void put4<f16_t>(f16_t* o, float a, float
     *reinterpret_cast<uint2*>(o) = w;
 }
 
+template <typename AT> __device__ __forceinline__ void put4_at(void* base, size_t row, int ld, int col, float a, float b, float c, float d) { put4<AT>((AT*)base + row * ld + col, a, b, c, d); }
+template <> __device__ __forceinline__ void put4_at<p3_t>(void* base, size_t row, int ld, int col, float a, float b, float c, float d) { p3_put4((unsigned char*)base + row * ld * 6, col, a, b, c, d); }
+
 template <typename AT>
-__global__ void __launch_bounds__(PWG) k_pf_rmsnorm(const float* __restrict__ X, const float* __restrict__ gamma, AT* out, int n, int d) {
+__global__ void __launch_bounds__(PWG) k_pf_rmsnorm(const float* __restrict__ X, const float* __restrict__ gamma, void* out, int n, int d) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= n) return;
     const float* x = X + (size_t)row * d;
@@ -127,12 +135,12 @@ __global__ void __launch_bounds__(PWG) k_pf_rmsnorm(const float* __restrict__ X,
         const int i = lane * 4 + k * 256;
         if (i < d) {
             const f32x4 v = keep[k], g = *reinterpret_cast<const f32x4*>(gamma + i);
-            put4<AT>(out + (size_t)row * d + i, g.x * (v.x / r), g.y * (v.y / r), g.z * (v.z / r), g.w * (v.w / r));
+            put4_at<AT>(out, (size_t)row, d, i, g.x * (v.x / r), g.y * (v.y / r), g.z * (v.z / r), g.w * (v.w / r));
         }
     }
     for (int i = lane * 4 + KEEP * 256; i < d; i += 256) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(x + i), g = *reinterpret_cast<const f32x4*>(gamma + i);
-        put4<AT>(out + (size_t)row * d + i, g.x * (v.x / r), g.y * (v.y / r), g.z * (v.z / r), g.w * (v.w / r));
+        put4_at<AT>(out, (size_t)row, d, i, g.x * (v.x / r), g.y * (v.y / r), g.z * (v.z / r), g.w * (v.w / r));
     }
 }
 
@@ -289,7 +297,7 @@ __global__ void __launch_bounds__(PWG) k_pf_attn(PfArgs P, LayerDev L) {
             const int dcol = h * HD + lane + 64 * ee;
             float v = acc[qq][ee] / l[qq];
             if (a.gating) v = v * pf_sigmoid(P.QKV[row * P.qkvLd + L.offG + dcol]);
-            put<AT>((AT*)P.Amix + row * P.aLd + dcol, v);
+            put_at<AT>(P.Amix, row, P.aLd, dcol, v);
         }
     }
 }
@@ -686,7 +694,7 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
             const float w = wn * rk * ainv;
 #pragma unroll
             for (int e = 0; e < CPT; e++) S[e] = fmaf(w, kk[e], S[e]);
-            if (cg == 0) put<AT>((AT*)P.Amix + (size_t)(row0 + t0 + c) * P.aLd + h * DV + r0 + r, alpha * p + wn * kqn);
+            if (cg == 0) put_at<AT>(P.Amix, (size_t)(row0 + t0 + c), P.aLd, h * DV + r0 + r, alpha * p + wn * kqn);
         }
     }
 #pragma unroll
@@ -1157,7 +1165,7 @@ __global__ void k_pf_ple(PfArgs P, LayerDev L) {
     const int row = blockIdx.x, j = threadIdx.x;
     if (j >= P.a.ple) return;
     const float g = P.QKV[(size_t)row * P.qkvLd + L.offPle + j];
-    put<AT>((AT*)P.Amix + (size_t)row * P.aLd + L.ad + j, pf_silu(g) * getw<WT>((const WT*)L.pleTable + (size_t)P.ids[row] * P.a.ple + j));
+    put_at<AT>(P.Amix, (size_t)row, P.aLd, L.ad + j, pf_silu(g) * getw<WT>((const WT*)L.pleTable + (size_t)P.ids[row] * P.a.ple + j));
 }
 
 // residual of the last row of every segment -> decode slot buffer x[slot]
@@ -1295,10 +1303,22 @@ static int build_mirror(mlh_ctx* c, const void* src, size_t n, const void** dst,
     return 0;
 }
 
+// An fp32 matrix as three bf16 planes, what the tiled products of the prefill multiply.
+static int build_planes(mlh_ctx* c, const void* src, int rows, int cols, const void** dst) {
+    void* buf = nullptr;
+    MLH_CHECK(c, hipMalloc(&buf, (size_t)rows * cols * 6));
+    c->mirrorAllocs.push_back(buf);
+    MLH_CHECK(c, mlh_split_p3(c->stream, (const float*)src, cols, buf, cols, rows, cols));
+    *dst = buf;
+    return 0;
+}
+
 int mlh_build_gemm_operands(mlh_ctx* c) {
     const mlh_hparams& hp = c->hp;
-    const bool mirror = hp.weightDtype == MLH_DTYPE_BF16 && mlh_prefill_gemm_supported(c);
+    const bool supported = mlh_prefill_gemm_supported(c), mirror = hp.weightDtype == MLH_DTYPE_BF16 && supported;
+    const bool planes = hp.weightDtype == MLH_DTYPE_F32 && supported;
     c->gemmDtype = mirror ? MLH_GEMM_F16 : hp.weightDtype;
+    c->pfDtype = planes ? MLH_GEMM_P3 : c->gemmDtype;
     c->f16Inexact = 0;
     for (void* p : c->mirrorAllocs) (void)hipFree(p); // a repeated finalize rebuilds them
     c->mirrorAllocs.clear();
@@ -1319,15 +1339,21 @@ int mlh_build_gemm_operands(mlh_ctx* c) {
             wo = cat;
             L.WoG = cat;
         }
+        if (planes && ((rc = build_planes(c, L.Wa, L.rowsA, (int)d, &L.WaP)) || (rc = build_planes(c, wo, (int)d, L.ad + (int)pl, &L.WoP)) ||
+                       (rc = build_planes(c, L.W13, 2 * (int)F, (int)d, &L.W13P)) || (rc = build_planes(c, L.W2, (int)d, (int)F, &L.W2P))))
+            break;
         if (!mirror) continue;
         if ((rc = build_mirror(c, L.Wa, (size_t)L.rowsA * d, &L.WaG, &L.sWa, d_scratch)) ||
             (rc = build_mirror(c, wo, d * (L.ad + pl), &L.WoG, &L.sWo, d_scratch)) ||
             (rc = build_mirror(c, L.W13, 2 * F * d, &L.W13G, &L.sW13, d_scratch)) ||
             (rc = build_mirror(c, L.W2, d * F, &L.W2G, &L.sW2, d_scratch)))
             break;
+        L.WaP = L.WaG; L.WoP = L.WoG; L.W13P = L.W13G; L.W2P = L.W2G;
     }
     c->EG = c->E; c->sE = 1.0f;
     if (rc == 0 && mirror) rc = build_mirror(c, c->E, (size_t)hp.vocabSize * hp.dim, &c->EG, &c->sE, d_scratch);
+    c->EP = c->EG;
+    if (rc == 0 && planes) rc = build_planes(c, c->E, hp.vocabSize, hp.dim, &c->EP);
     if (d_scratch) (void)hipFree(d_scratch);
     return rc;
 }
@@ -1341,7 +1367,7 @@ int mlh_init_prefill_kernels(mlh_ctx* c) {
     MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gdn_scan<64>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * GdLayout<64>::image));
     MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gdn_scan<128>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * GdLayout<128>::image));
     const int lds = (2 * 64 * 132 + PF_QB * 128) * 4;
-    MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_attn<128, float>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_attn<128, p3_t>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     return 0;
 }
 
@@ -1354,7 +1380,7 @@ static int ensure_prefill_buffers(mlh_ctx* c, int rows) {
     c->pfRows = 0;
     for (int g = 0; g < 2; g++) // captured batched steps hold the old buffer addresses
         if (c->graphExec[g]) { (void)hipGraphExecDestroy(c->graphExec[g]); c->graphExec[g] = nullptr; }
-    const size_t n = (size_t)rows, wb = c->wbytes;
+    const size_t n = (size_t)rows, wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 6; // GEMM input elements: halves, or three bf16 planes
     auto alloc = [&](void** p, size_t bytes) -> int {
         MLH_CHECK(c, hipMalloc(p, std::max<size_t>(bytes, 16)));
         c->pfAllocs.push_back(*p);
@@ -1375,6 +1401,17 @@ static int ensure_prefill_buffers(mlh_ctx* c, int rows) {
     return 0;
 }
 
+// Split-K workspace of the GEMMs; its launches are ordered on the context's stream.
+static int ensure_gemm_workspace(mlh_ctx* c) {
+    if (c->gemmWs) return 0;
+    void* ws = nullptr;
+    MLH_CHECK(c, hipMalloc(&ws, mlh_gemm_workspace_bytes()));
+    c->allocs.push_back(ws);
+    MLH_CHECK(c, hipMemset(ws, 0, mlh_gemm_workspace_bytes()));
+    c->gemmWs = ws;
+    return 0;
+}
+
 #define PF_DISPATCH_WT(c, expr_f32, expr_bf16) do { if ((c)->hp.weightDtype == MLH_DTYPE_BF16) { expr_bf16; } else { expr_f32; } } while (0)
 
 // Appends lens[s] tokens to sequence seqs[s] for every segment s (token ids concatenated in `ids`).
@@ -1384,6 +1421,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     int n = 0;
     for (int s = 0; s < nseg; s++) n += lens[s];
     int rc = ensure_prefill_buffers(c, n);
+    if (rc == 0) rc = ensure_gemm_workspace(c);
     if (rc) return rc;
     // ---- metadata ----
     const bool mfmaAttn = hp.weightDtype == MLH_DTYPE_BF16; // bf16 models: bf16 MFMA attention, 128 queries per workgroup
@@ -1450,10 +1488,10 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     for (int s = 0; s < nseg; s++) fresh = fresh && segPos0[s] == 0;
     P.Kh = mfmaAttn && fresh ? c->pfKh : nullptr;
     P.Vh = mfmaAttn && fresh ? c->pfVh : nullptr;
-    const int d_ = hp.dim, F = hp.ffnDim, dt = c->gemmDtype;
+    const int d_ = hp.dim, F = hp.ffnDim, dt = c->pfDtype;
 #define GEMM(A, lda, B, alpha, ldb, C, ldc, R, ldr, M, N, K)                                                \
     do {                                                                                                    \
-        hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, nullptr, alpha); \
+        hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, c->gemmWs, alpha); \
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; } \
     } while (0)
 
@@ -1461,29 +1499,29 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
                    hipLaunchKernelGGL((k_pf_embed<bf16_t>), dim3(cdiv(d_, PWG), n), dim3(PWG), 0, st, P));
     for (int t = hp.transformers - 1; t >= 0; t--) { // file block 0 is the top (inference.cu:384-385)
         const LayerDev& L = c->layers[t];
-        PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, L.g1, (float*)P.Xn, n, d_),
-                       hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, L.g1, (f16_t*)P.Xn, n, d_));
-        GEMM(P.Xn, d_, L.WaG, L.sWa, d_, P.QKV, P.qkvLd, nullptr, 0, n, L.rowsA, d_);
+        PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<p3_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, L.g1, P.Xn, n, d_),
+                       hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, L.g1, P.Xn, n, d_));
+        GEMM(P.Xn, d_, L.WaP, L.sWa, d_, P.QKV, P.qkvLd, nullptr, 0, n, L.rowsA, d_);
         if (L.kind == MLH_KIND_ATTENTION) {
             if (hp.headDim == 64) {
                 hipLaunchKernelGGL((k_pf_qk_rope_kv<64>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<64, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<64, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
-                else hipLaunchKernelGGL((k_pf_attn<64, float>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 68 + PF_QB * 64) * 4, st, P, L);
+                else hipLaunchKernelGGL((k_pf_attn<64, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 68 + PF_QB * 64) * 4, st, P, L);
             } else {
                 hipLaunchKernelGGL((k_pf_qk_rope_kv<128>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<128, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<128, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
-                else hipLaunchKernelGGL((k_pf_attn<128, float>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 132 + PF_QB * 128) * 4, st, P, L);
+                else hipLaunchKernelGGL((k_pf_attn<128, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 132 + PF_QB * 128) * 4, st, P, L);
             }
         } else {
             const int skipFrom = nchunk > 0 ? GD_C : 0x7fffffff;
             const dim3 gr(hp.gdnHeads, nseg, hp.gdnDv / PF_GR);
             if (hp.gdnDk == 64) {
-                PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<64, float>), gr, dim3(PWG), 0, st, P, L, skipFrom),
+                PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<64, p3_t>), gr, dim3(PWG), 0, st, P, L, skipFrom),
                                hipLaunchKernelGGL((k_pf_gdn<64, f16_t>), gr, dim3(PWG), 0, st, P, L, skipFrom));
             } else {
-                PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<128, float>), gr, dim3(PWG), 0, st, P, L, skipFrom),
+                PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<128, p3_t>), gr, dim3(PWG), 0, st, P, L, skipFrom),
                                hipLaunchKernelGGL((k_pf_gdn<128, f16_t>), gr, dim3(PWG), 0, st, P, L, skipFrom));
             }
             if (nchunk > 0) {
@@ -1498,22 +1536,22 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
             }
         }
         if (hp.pleDim > 0)
-            PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_ple<float, float>), dim3(n), dim3(std::max(64, hp.pleDim)), 0, st, P, L),
+            PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_ple<float, p3_t>), dim3(n), dim3(std::max(64, hp.pleDim)), 0, st, P, L),
                            hipLaunchKernelGGL((k_pf_ple<bf16_t, f16_t>), dim3(n), dim3(std::max(64, hp.pleDim)), 0, st, P, L));
-        GEMM(P.Amix, P.aLd, L.WoG, L.sWo, L.ad + hp.pleDim, P.H1, d_, P.X, d_, n, d_, L.ad + hp.pleDim); // Wo . a + pleUp . e + x
-        PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.H1, L.g2, (float*)P.Xn, n, d_),
-                       hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.H1, L.g2, (f16_t*)P.Xn, n, d_));
+        GEMM(P.Amix, P.aLd, L.WoP, L.sWo, L.ad + hp.pleDim, P.H1, d_, P.X, d_, n, d_, L.ad + hp.pleDim); // Wo . a + pleUp . e + x
+        PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<p3_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.H1, L.g2, P.Xn, n, d_),
+                       hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.H1, L.g2, P.Xn, n, d_));
         { // gate/up projection with SiLU(gate) * up in the epilogue (inference.cu:262-281): U comes out in the GEMM input type
-            hipError_t e_ = mlh_gemm_tn_epi(st, dt, 1, P.Xn, d_, L.W13G, d_, P.U, F, nullptr, 0, n, 2 * F, d_, nullptr, L.sW13);
+            hipError_t e_ = mlh_gemm_tn_epi(st, dt, 1, P.Xn, d_, L.W13P, d_, P.U, F, nullptr, 0, n, 2 * F, d_, c->gemmWs, L.sW13);
             if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
         }
-        GEMM(P.U, F, L.W2G, L.sW2, F, P.X, d_, P.H1, d_, n, d_, F);
+        GEMM(P.U, F, L.W2P, L.sW2, F, P.X, d_, P.H1, d_, n, d_, F);
     }
 #undef GEMM
     if (allLogits) { // final RMSNorm + tied LM head for every row (inference.cu:705-743 computes all L columns)
-        PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, c->gF, (float*)P.Xn, n, d_),
-                       hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, c->gF, (f16_t*)P.Xn, n, d_));
-        hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, P.Xn, d_, c->EG, d_, allLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_, nullptr, c->sE);
+        PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<p3_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, c->gF, P.Xn, n, d_),
+                       hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, c->gF, P.Xn, n, d_));
+        hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, P.Xn, d_, c->EP, d_, allLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_, c->gemmWs, c->sE);
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
     }
     hipLaunchKernelGGL(k_pf_gather_last, dim3(cdiv(d_, PWG), nseg), dim3(PWG), 0, st, P);
@@ -1657,11 +1695,7 @@ int mlh_prepare_batch_step(mlh_ctx* c, int nseq) {
     if (!mlh_batch_step_applicable(c, nseq)) return 0;
     int rc = ensure_prefill_buffers(c, std::max(nseq, 64));
     if (rc) return rc;
-    if (!c->gemmWs) {
-        MLH_CHECK(c, hipMalloc(&c->gemmWs, mlh_gemm_workspace_bytes()));
-        c->allocs.push_back(c->gemmWs);
-        MLH_CHECK(c, hipMemset(c->gemmWs, 0, mlh_gemm_workspace_bytes()));
-    }
+    if ((rc = ensure_gemm_workspace(c))) return rc;
     if (!c->pfLogits) {
         MLH_CHECK(c, hipMalloc((void**)&c->pfLogits, (size_t)64 * c->hp.vocabSize * 4));
         c->allocs.push_back(c->pfLogits);
@@ -1691,8 +1725,8 @@ int mlh_launch_batch_step(mlh_ctx* c, int nseq, const int* tokPtr) {
         if (mlh_gemm_norm_fusable(dt, n, L.rowsA, d_)) {
             GEMMN(0, c->x, d_, L.WaG, L.sWa, d_, c->qkv, c->maxRowsA, nullptr, 0, n, L.rowsA, d_, L.g1);
         } else {
-            if (bf) hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, L.g1, (f16_t*)c->pfXn, n, d_);
-            else hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, L.g1, (float*)c->pfXn, n, d_);
+            if (bf) hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, L.g1, c->pfXn, n, d_);
+            else hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, L.g1, c->pfXn, n, d_);
             GEMM(0, c->pfXn, d_, L.WaG, L.sWa, d_, c->qkv, c->maxRowsA, nullptr, 0, n, L.rowsA, d_);
         }
         const bool gdn = L.kind != MLH_KIND_ATTENTION;
@@ -1713,14 +1747,14 @@ int mlh_launch_batch_step(mlh_ctx* c, int nseq, const int* tokPtr) {
         if (mlh_gemm_norm_fusable(dt, n, 2 * F, d_)) {
             GEMMN(1, c->h1, d_, L.W13G, L.sW13, d_, c->pfU, F, nullptr, 0, n, 2 * F, d_, L.g2);
         } else {
-            if (bf) hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->h1, L.g2, (f16_t*)c->pfXn, n, d_);
-            else hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->h1, L.g2, (float*)c->pfXn, n, d_);
+            if (bf) hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->h1, L.g2, c->pfXn, n, d_);
+            else hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->h1, L.g2, c->pfXn, n, d_);
             GEMM(1, c->pfXn, d_, L.W13G, L.sW13, d_, c->pfU, F, nullptr, 0, n, 2 * F, d_);
         }
         GEMM(0, c->pfU, F, L.W2G, L.sW2, F, c->x, d_, c->h1, d_, n, d_, F);
     }
-    if (bf) hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, c->gF, (f16_t*)c->pfXn, n, d_);
-    else hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, c->gF, (float*)c->pfXn, n, d_);
+    if (bf) hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, c->gF, c->pfXn, n, d_);
+    else hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, c->gF, c->pfXn, n, d_);
     GEMM(0, c->pfXn, d_, c->EG, c->sE, d_, c->pfLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_);
 #undef GEMM
 #undef GEMMN

@@ -17,6 +17,9 @@ typedef uint16_t bf16_t;
 // IEEE half, as the MFMA path stores weights and activations of bf16 models (see MLH_GEMM_F16)
 struct f16_t { uint16_t bits; };
 #define MLH_GEMM_F16 2 // GEMM operand type code beside MLH_DTYPE_F32 / MLH_DTYPE_BF16
+#define MLH_GEMM_P3 3  // ... and for fp32 operands stored as three bf16 planes (p3.h)
+#define MLH_GEMM_WS_COUNTERS 1024 // tile counters at the head of a split-K workspace ...
+#define MLH_GEMM_WS_PARTIALS (256 * 8 * 2 * 16 * 64) // ... and the partial sums (floats) behind them
 #define MLH_SELFTEST_SWIGLU 0x100 // mlh_selftest_gemm: flag beside the operand type, selects the SwiGLU epilogue
 
 // Device-side description of one transformer block.
@@ -43,6 +46,7 @@ struct LayerDev {
     // mirrors scaled by a power of two (exact), with the inverse scale applied to the product.
     // WoG is [dim, ad + pleDim]: Wo with pleUp appended along K, so that h1 = [a | e] . WoG^T is one product.
     const void *WaG, *WoG, *W13G, *W2G;
+    const void *WaP, *WoP, *W13P, *W2P; // the same for the prefill's tiled products: fp32 models as three bf16 planes (p3.h)
     float sWa, sWo, sW13, sW2;
 };
 
@@ -170,7 +174,9 @@ struct mlh_ctx {
     size_t pfGdnChunks = 0;
     const void* EG = nullptr;  // LM-head matrix as the MFMA path reads it (see LayerDev::WaG)
     float sE = 1.0f;
-    int gemmDtype = MLH_DTYPE_F32; // operand type of the MFMA path: MLH_DTYPE_F32 or MLH_GEMM_F16
+    const void* EP = nullptr;  // the same for the prefill's tiled products
+    int gemmDtype = MLH_DTYPE_F32; // operand type of the batched step's products: MLH_DTYPE_F32 or MLH_GEMM_F16
+    int pfDtype = MLH_DTYPE_F32;   // ... and of the prefill's: MLH_GEMM_P3 or MLH_GEMM_F16
     std::vector<void*> mirrorAllocs;
     long f16Inexact = 0;       // bf16 weights that had no exact scaled-half representation (reported at finalize)
     void* gemmWs = nullptr;    // split-K workspace of the skinny GEMM
@@ -196,9 +202,8 @@ int mlh_launch_probs(mlh_ctx* c, int seq);
 int mlh_init_kernels(mlh_ctx* c);
 
 // kernels_gemm.hip
-hipError_t mlh_gemm_tn(hipStream_t stream, int dtype, const void* A, int lda, const void* B, int ldb, float* C, int ldc,
-                       const float* R, int ldr, int M, int N, int K);
-// epi 0: as above.  epi 1 (SwiGLU): columns 2j / 2j+1 of the product are gate / up of unit j and
+// C[M,N] = A[M,K] . B[N,K]^T (+ R[M,N]); dtype: operand type code (fp32 operands: M <= 64; MLH_GEMM_P3 has no limit).
+// epi 0: C, R fp32.  epi 1 (SwiGLU): columns 2j / 2j+1 of the product are gate / up of unit j and
 // C is [M, N/2] in the operand type: C[m, j] = silu(gate) * up.
 // ws: zero-initialised workspace of mlh_gemm_workspace_bytes() or null; with it, M <= 64 products of matrices
 // with few rows are split along K over workgroups (deterministically reduced).
@@ -208,6 +213,12 @@ hipError_t mlh_gemm_tn(hipStream_t stream, int dtype, const void* A, int lda, co
 // eps 1e-8 inside the root), without a pass that writes the normalised rows.
 hipError_t mlh_gemm_tn_epi(hipStream_t stream, int dtype, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
                            const float* R, int ldr, int M, int N, int K, void* ws, float alpha = 1.0f, const float* normGain = nullptr);
+// kernels_tile.hip: the same product in 128 x 128 / 64 x 64 tiles (operands half, bf16 or P3), and fp32 -> P3 rows
+hipError_t mlh_gemm_tile(hipStream_t stream, int dtype, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
+                         const float* R, int ldr, int M, int N, int K, void* ws, float alpha);
+double mlh_gemm_tile_us(int dtype, int M, int N, int K, int cus, bool ws); // what that product is expected to take
+int mlh_gemm_num_cus(void); // kernels_gemm.hip: compute units of the current device, a multiple of eight; 0: unknown
+hipError_t mlh_split_p3(hipStream_t stream, const float* src, int lds, void* dst, int ldd, int rows, int cols);
 bool mlh_gemm_norm_fusable(int dtype, int M, int N, int K);
 size_t mlh_gemm_workspace_bytes(void);
 extern "C" int mlh_gemm_device_init(int device);
