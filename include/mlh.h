@@ -182,7 +182,8 @@ int mlh_set_graph(mlh_ctx* ctx, int stepsPerGraph);
  * head size 64 (attention heads; gated-delta-net heads with 64 x 64 states, as many as attention heads;
  * per-layer embeddings of a width that is a multiple of 8) and attention-only models with head size 128 (the
  * reference's compiled-in shape, network_meta.h:3-20: 6 heads x 128) on a 256-unit device
- * (mlh_xcd_decode_supported), and falls back to mode 1 otherwise.  Mode 3 is the default.
+ * (mlh_xcd_decode_supported); other models run as the kernel sequence (widths multiples of 32 fp32 / 64 bf16) or as mode 1.
+ * Mode 3 is the default.
  * Both need every compute unit for themselves and all their waits are bounded: when a launch gives up (units held
  * by other work), the sequence is as it was before the launch (position, token and tags are written at a kernel's
  * normal end only; the XCD-rank kernel keeps gated-delta-net states in LDS until then, the barrier kernel's are put

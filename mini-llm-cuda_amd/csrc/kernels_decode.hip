@@ -16,6 +16,7 @@
 #include <type_traits>
 #include "mlh_internal.h"
 #include "persist_common.h"
+#include "rows.h"
 #include "sample.h"
 
 #define WG 256
@@ -485,29 +486,25 @@ __global__ void __launch_bounds__(AttnCfg<HD>::NW * 64) k_attn(StepArgs a, Layer
     for (int w = 0; w < NW; w++) M = fmaxf(M, comb[w * (HD + 2) + HD]);
     if (a.mixRows && a.nsplit == 1) {
         // batched step, one workgroup per (head, sequence): the finished mixing output (inference.cu:549-573), gated
-        // (inference.cu:241-250), goes straight into the output-projection GEMM's input row; the workgroup of head 0
+        // (inference.cu:241-250), goes straight into the planes the output projection multiplies (rows.h); the workgroup of head 0
         // appends the PLE columns e = silu(gate) * P[tok]
         float l = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; w++) l += expf(comb[w * (HD + 2) + HD] - M) * comb[w * (HD + 2) + HD + 1];
-        const size_t row = (size_t)slot * a.mixRowsLd;
-        auto put_row = [&](size_t col, float v) {
-            if (a.mixRowsHalf) ((_Float16*)a.mixRows)[row + col] = (_Float16)fminf(fmaxf(v, -65504.0f), 65504.0f); // saturating
-            else ((float*)a.mixRows)[row + col] = v;
-        };
+        auto put_row = [&](int col, float v) { rows_put(a.mixRows, col, slot, a.mixLay, a.wbytes == 2, v); };
         for (int i = tid; i < HD; i += NW * 64) {
             float s = 0.f;
 #pragma unroll
             for (int w = 0; w < NW; w++) s += expf(comb[w * (HD + 2) + HD] - M) * comb[w * (HD + 2) + i];
             float v = s / l;
             if (a.gating) v = v * sigmoidf_ref(qkv[L.offG + h * HD + i]);
-            put_row((size_t)h * HD + i, v);
+            put_row(h * HD + i, v);
         }
         if (h == 0)
             for (int j = tid; j < a.ple; j += NW * 64) {
                 const size_t e = (size_t)a.tok[slot] * a.ple + j;
                 const float pv = a.wbytes == 2 ? __uint_as_float(((uint32_t)((const uint16_t*)L.pleTable)[e]) << 16) : ((const float*)L.pleTable)[e];
-                put_row((size_t)a.heads * HD + j, siluf_ref(qkv[L.offPle + j]) * pv);
+                put_row(a.heads * HD + j, siluf_ref(qkv[L.offPle + j]) * pv);
             }
         return;
     }
@@ -599,19 +596,15 @@ __global__ void __launch_bounds__(WG) k_gdn(StepArgs a, LayerDev L) {
         if (cg == 0) a.mix[(size_t)slot * (a.gdnHeads * DV) + h * DV + r] = oacc;
         return;
     }
-    // batched step: the read-out is a row segment of the output-projection GEMM's input; the workgroup of head 0 also
+    // row step: the read-out goes into the planes the output projection multiplies; the workgroup of head 0 also
     // appends the PLE columns e = silu(gate) * P[tok] behind the gdnHeads * DV read-out columns
-    const size_t row = (size_t)slot * a.mixRowsLd;
-    auto put_row = [&](size_t col, float v) {
-        if (a.mixRowsHalf) ((_Float16*)a.mixRows)[row + col] = (_Float16)fminf(fmaxf(v, -65504.0f), 65504.0f); // saturating
-        else ((float*)a.mixRows)[row + col] = v;
-    };
-    if (cg == 0) put_row((size_t)h * DV + r, oacc);
+    auto put_row = [&](int col, float v) { rows_put(a.mixRows, col, slot, a.mixLay, a.wbytes == 2, v); };
+    if (cg == 0) put_row(h * DV + r, oacc);
     if (h == 0 && blockIdx.z == 0)
         for (int j = tid; j < a.ple; j += WG) {
             const size_t e = (size_t)a.tok[slot] * a.ple + j;
             const float p = a.wbytes == 2 ? __uint_as_float(((uint32_t)((const uint16_t*)L.pleTable)[e]) << 16) : ((const float*)L.pleTable)[e];
-            put_row((size_t)a.gdnHeads * DV + j, siluf_ref(qkv[L.offPle + j]) * p);
+            put_row(a.gdnHeads * DV + j, siluf_ref(qkv[L.offPle + j]) * p);
         }
 }
 
@@ -929,7 +922,7 @@ void mlh_fill_args(mlh_ctx* c, StepArgs& a, int nseq, const int* tokPtr) {
     a.nseq = nseq; a.sidx = c->d_sidx; a.tok = tokPtr; a.pos = c->d_pos;
     a.pageTable = c->d_pageTable; a.pagesPerSeq = c->pagesPerSeq; a.nsplit = c->nsplit;
     a.x = c->x; a.qkv = c->qkv; a.qkvStride = c->maxRowsA; a.part = c->part; a.mix = c->mix;
-    a.mixRows = c->mixRows; a.mixRowsLd = c->mixRowsLd; a.mixRowsHalf = c->mixRowsHalf; a.wbytes = c->wbytes;
+    a.mixRows = c->mixRows; a.mixLay = c->mixLay; a.wbytes = c->wbytes;
     a.temperature = c->temperature; a.sampleSeed = c->sampleSeed;
     a.h1 = c->h1; a.u = c->u; a.logits = c->logits; a.amaxVal = c->amaxVal; a.amaxIdx = c->amaxIdx;
     a.amaxParts = c->amaxParts; a.rope = c->rope; a.E = c->E; a.gF = c->gF;
@@ -1003,7 +996,7 @@ static size_t attn_lds_bytes(int hd) {
 // Nothing to set up: no decode kernel needs more LDS than a launch may use without opting in.
 int mlh_init_kernels(mlh_ctx*) { return 0; }
 
-static int launch_mix(mlh_ctx* c, const StepArgs& a, const LayerDev& L) {
+int mlh_launch_mix(mlh_ctx* c, const StepArgs& a, const LayerDev& L) {
     hipStream_t st = c->stream;
     if (L.kind == MLH_KIND_ATTENTION) {
         if (a.hd == 64) {
@@ -1034,9 +1027,9 @@ static int launch_mix(mlh_ctx* c, const StepArgs& a, const LayerDev& L) {
     return 0;
 }
 
-// Enqueues one decode step on the context's stream (no synchronisation).
-int mlh_launch_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead) {
-    if (lmHead && !c->profEvents && mlh_batch_step_applicable(c, nseq)) return mlh_launch_batch_step(c, nseq, tokPtr);
+// Enqueues one decode step on the context's stream (no synchronisation).  embedded, embedNext: of a run of steps, see mlh_rows_step.
+int mlh_launch_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool embedded, bool embedNext) {
+    if (!c->profEvents && mlh_rows_applicable(c, nseq)) return mlh_rows_step(c, nseq, tokPtr, lmHead, embedded, embedNext);
     StepArgs a;
     mlh_fill_args(c, a, nseq, tokPtr);
     hipStream_t st = c->stream;
@@ -1058,7 +1051,7 @@ int mlh_launch_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead) {
         const LayerDev& L = c->layers[t];
         launch_gemv(c, MLH_K_QKV, a, L);
         mark(MLH_K_QKV);
-        if (launch_mix(c, a, L) != 0) return -1;
+        if (mlh_launch_mix(c, a, L) != 0) return -1;
         mark(L.kind == MLH_KIND_ATTENTION ? MLH_K_ATTN : MLH_K_GDN);
         launch_gemv(c, MLH_K_OPROJ, a, L);
         mark(MLH_K_OPROJ);
@@ -1096,11 +1089,11 @@ int mlh_launch_one(mlh_ctx* c, int kernel, int layer, int nseq) {
             break;
         case MLH_K_ATTN:
             if (L.kind != MLH_KIND_ATTENTION) { c->err = "layer is not an attention layer"; return -1; }
-            if (launch_mix(c, a, L) != 0) return -1;
+            if (mlh_launch_mix(c, a, L) != 0) return -1;
             break;
         case MLH_K_GDN:
             if (L.kind != MLH_KIND_GDN) { c->err = "layer is not a GDN layer"; return -1; }
-            if (launch_mix(c, a, L) != 0) return -1;
+            if (mlh_launch_mix(c, a, L) != 0) return -1;
             break;
         case MLH_K_COPY:
             return mlh_launch_copy(c);

@@ -9,8 +9,8 @@
 // feeding four v_mfma_f32_32x32x2_f32 steps).  This replaces the cublasGemmEx calls of
 // inference.cu:401-465, 487-507, 582-602, 624-695 and 723-743 for L > 1 columns.
 //
-// Here: the 256 x 256-tile kernel of the long two-byte products (k_gemm_tn_w4), the weight-streaming kernels of decode batches
-// (k_gemm_skinny*) and the dispatch; kernels_tile.hip has what lies between, and every longer fp32 product.
+// Here: the 256 x 256-tile kernel of the long two-byte products (k_gemm_tn_w4), the weight-streaming kernels for up to
+// 64 rows (k_gemm_skinny*) and the dispatch; kernels_tile.hip has what lies between, and every longer fp32 product.
 #include <string.h>
 
 #include <algorithm>
@@ -492,7 +492,7 @@ static double w4_us(int M, int N, int K, int cus) {
 }
 
 // ----------------------------------------------------------------------------
-// Skinny variant for M <= 64 (batched decode: one row per sequence).  The weight matrix is the big
+// Skinny variant for M <= 64.  The weight matrix is the big
 // operand and is read exactly once: a workgroup owns 32 weight rows and (with split-K) one slice of
 // K, its four waves take 128-byte chunks of that slice in turn and multiply straight out of global
 // memory -- the MFMA operand layout (lane = row, 16 bytes of K) is also a reasonable load pattern:
@@ -642,9 +642,6 @@ __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny(const T* __restr
 // x K = 768 take one unit 5.8 us -- and a matrix of a few thousand rows in 32-row tiles occupies a third of the chip:
 // tiles of 16 rows double the units at work.  Lane l holds weight row l % 16 (token l % 16 of a block) and the
 // 16 bytes at K offset (l / 16) * 16 of each 64-byte half chunk; element e of those vectors meets element e.
-// With NORM the rows of A are RMS-normalised on the way in (inference.cu:24-50): C = (gain * A / rms(A)) . B^T.  The gain
-// multiplies the elements as they are loaded, the sum of squares of a row is gathered from the same loads, and
-// 1 / rms scales the finished product, so the normalised activations are never written to memory (gridDim.y = 1).
 // The activation rows take the way through LDS: the operand layout wants 16 different rows in 16 neighbouring lanes,
 // and a load of that shape touches 16 cache lines for 64 bytes each -- the L1 then fills at 36 GB/s per compute unit
 // instead of 112 GB/s with eight lanes per 128-byte line (measured with a load-only probe), and at 64 tokens the
@@ -653,14 +650,12 @@ __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny(const T* __restr
 // private buffer and reads the operands from there; only the 16 weight rows still load row per lane.
 #define SK16_ABUF (64 * GKB)                          // one chunk of A: 64 token rows x 128 bytes
 #define SK16_LDS (GSK_WAVES * SK16_ABUF)              // bytes of dynamic LDS per workgroup
-template <int EPI, bool NORM>
+template <int EPI>
 __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny16(const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb,
                                                                    void* Cv, int ldc, const float* R, int ldr, int M, int N, int K,
-                                                                   unsigned* counters, float* partials, float alpha,
-                                                                   const float* __restrict__ gain) {
+                                                                   unsigned* counters, float* partials, float alpha) {
     extern __shared__ __attribute__((aligned(16))) unsigned char sk16_lds[];
     float (*red)[4][4][64] = reinterpret_cast<float (*)[4][4][64]>(sk16_lds); // [GSK_WAVES], over the A buffers once they are done
-    __shared__ float ssred[GSK_WAVES][4][16];
     __shared__ int lastFlag;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n0 = blockIdx.x * 16, n16 = lane & 15, kq = lane >> 4;
@@ -685,16 +680,10 @@ __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny16(const float* _
     f32x4 acc[4];
 #pragma unroll
     for (int tb = 0; tb < 4; tb++) acc[tb] = (f32x4)(0.f);
-    f32x4 fb[2][2], fa[4][2], fg[2][2];
-    float ss[4] = {0.f, 0.f, 0.f, 0.f}; // NORM: this lane's share of the sums of squares of its four tokens
-    const unsigned char* grow = reinterpret_cast<const unsigned char*>(gain) + kq * 16;
-    auto load = [&](int c, int buf) { // buf names the registers of the weight rows and the gain; A has one LDS buffer
+    f32x4 fb[2][2], fa[4][2];
+    auto load = [&](int c, int buf) { // buf names the registers of the weight rows; A has one LDS buffer
 #pragma unroll
         for (int p = 0; p < 2; p++) fb[buf][p] = *reinterpret_cast<const f32x4*>(brow + (size_t)c * GKB + p * 64);
-        if (NORM) {
-#pragma unroll
-            for (int p = 0; p < 2; p++) fg[buf][p] = *reinterpret_cast<const f32x4*>(grow + (size_t)c * GKB + p * 64);
-        }
         const unsigned char* src = abase + (size_t)c * GKB;
 #pragma unroll
         for (int j = 0; j < 8; j++) __builtin_amdgcn_global_load_lds(src + aoff[j], wbuf + j * 8 * GKB, 16, 0, 0);
@@ -706,7 +695,7 @@ __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny16(const float* _
     // its back get their target registers copied before the data has landed.)
     auto mul = [&](int buf, int cnext) { // cnext < 0: nothing more to fetch
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): this chunk's weight rows, gain and A rows have landed
+        __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): this chunk's weight rows and A rows have landed
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         const unsigned char* rd = wbuf + ardoff;
@@ -719,16 +708,6 @@ __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny16(const float* _
         __builtin_amdgcn_sched_barrier(0);
         if (cnext >= 0) load(cnext, buf ^ 1);
         __builtin_amdgcn_sched_barrier(0);
-        if (NORM) {
-#pragma unroll
-            for (int tb = 0; tb < 4; tb++)
-#pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    const f32x4 x = fa[tb][p];
-                    ss[tb] = fmaf(x.x, x.x, ss[tb]); ss[tb] = fmaf(x.y, x.y, ss[tb]); ss[tb] = fmaf(x.z, x.z, ss[tb]); ss[tb] = fmaf(x.w, x.w, ss[tb]);
-                    fa[tb][p] = x * fg[buf][p];
-                }
-        }
 #pragma unroll
         for (int p = 0; p < 2; p++)
 #pragma unroll
@@ -752,15 +731,6 @@ __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny16(const float* _
     for (int tb = 0; tb < 4; tb++)
 #pragma unroll
         for (int r = 0; r < 4; r++) red[wave][tb][r][lane] = acc[tb][r];
-    if (NORM) { // lanes n16, n16 + 16, + 32, + 48 hold the four K quarters of token n16
-#pragma unroll
-        for (int tb = 0; tb < 4; tb++) {
-            float t = ss[tb];
-            t += __shfl_xor(t, 16, 64);
-            t += __shfl_xor(t, 32, 64);
-            if (lane < 16) ssred[wave][tb][lane] = t;
-        }
-    }
     __syncthreads();
     auto wsum = [&](int tb, int r) { // fixed order
         float t = 0.f;
@@ -799,14 +769,6 @@ __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny16(const float* _
         }
     }
     const int m = tb * 16 + n16, n = n0 + 4 * kq; // accumulator element r: weight row 4 (lane / 16) + r, token lane % 16
-    if (NORM) {
-        float t = 0.f;
-#pragma unroll
-        for (int w = 0; w < GSK_WAVES; w++) t += ssred[w][tb][n16];
-        const float ri = 1.0f / sqrtf(t / (float)K + 1e-8f);
-#pragma unroll
-        for (int r = 0; r < 4; r++) v[r] *= ri;
-    }
     if (m >= M) return;
     if (EPI == GEMM_EPI_SWIGLU) {
 #pragma unroll
@@ -823,229 +785,12 @@ __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny16(const float* _
     }
 }
 
-// The weight-streaming kernel for M <= 32 with the RMSNorm of the activation rows fused in (one 32-row tile, no split
-// over K): A holds the fp32 residual rows; a lane multiplies its elements by the gain on the way into the operand
-// registers (rounded to half for half weights), adds up their squares, and 1 / rms scales the result:
-//   W . (g (.) x / rms(x)) = (W . (g (.) x)) / rms(x),   rms(x) = sqrt(sum x^2 / K + 1e-8)   (inference.cu:24-50, 83-95)
-// T is the weight operand type (float, or f16_t for the half mirrors of a bf16 model).
-template <typename T, int EPI>
-__global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny_norm(const float* __restrict__ A, int lda, const T* __restrict__ B, int ldb,
-                                                               void* Cv, int ldc, const float* R, int ldr, int M, int N, int K,
-                                                               float alpha, const float* __restrict__ gain) {
-    constexpr int EPC = GKB / (int)sizeof(T), HPC = EPC / 2, NV = HPC / 4; // elements per chunk, per lane half, 16-byte loads of fp32
-    __shared__ float red[GSK_WAVES][1][16][64];
-    __shared__ float ssq[GSK_WAVES][64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n0 = blockIdx.x * 32, n32 = lane & 31, half = lane >> 5;
-    const int nchunks = (int)(((size_t)K * sizeof(T)) / GKB);
-    const unsigned char* brow = reinterpret_cast<const unsigned char*>(B) + (size_t)min(n0 + n32, N - 1) * ldb * sizeof(T) + half * 64;
-    const float* arow = A + (size_t)min(n32, M - 1) * lda + half * HPC;
-    const float* grow = gain + half * HPC;
-    f32x16 acc = (f32x16)(0.f);
-    float ss = 0.f;
-    u32x4 fb[2][4];
-    f32x4 xa[2][NV], ga[2][NV];
-    auto load = [&](int c, int buf) {
-#pragma unroll
-        for (int p = 0; p < 4; p++) fb[buf][p] = *reinterpret_cast<const u32x4*>(brow + (size_t)c * GKB + p * 16);
-#pragma unroll
-        for (int q = 0; q < NV; q++) {
-            xa[buf][q] = *reinterpret_cast<const f32x4*>(arow + (size_t)c * EPC + 4 * q);
-            ga[buf][q] = *reinterpret_cast<const f32x4*>(grow + (size_t)c * EPC + 4 * q);
-        }
-    };
-    auto half2 = [](float lo, float hi) { // two floats -> two IEEE halves, saturating
-        const _Float16 a = (_Float16)fminf(fmaxf(lo, -65504.0f), 65504.0f), b = (_Float16)fminf(fmaxf(hi, -65504.0f), 65504.0f);
-        return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
-    };
-    auto mul = [&](int buf) {
-#pragma unroll
-        for (int p = 0; p < 4; p++) {
-            u32x4 fa;
-            if constexpr (sizeof(T) == 4) {
-                const f32x4 x = xa[buf][p], g = ga[buf][p];
-                ss = fmaf(x.x, x.x, ss); ss = fmaf(x.y, x.y, ss); ss = fmaf(x.z, x.z, ss); ss = fmaf(x.w, x.w, ss);
-                fa.x = __float_as_uint(g.x * x.x); fa.y = __float_as_uint(g.y * x.y); fa.z = __float_as_uint(g.z * x.z); fa.w = __float_as_uint(g.w * x.w);
-            } else {
-                const f32x4 x0 = xa[buf][2 * p], x1 = xa[buf][2 * p + 1], g0 = ga[buf][2 * p], g1 = ga[buf][2 * p + 1];
-                ss = fmaf(x0.x, x0.x, ss); ss = fmaf(x0.y, x0.y, ss); ss = fmaf(x0.z, x0.z, ss); ss = fmaf(x0.w, x0.w, ss);
-                ss = fmaf(x1.x, x1.x, ss); ss = fmaf(x1.y, x1.y, ss); ss = fmaf(x1.z, x1.z, ss); ss = fmaf(x1.w, x1.w, ss);
-                fa.x = half2(g0.x * x0.x, g0.y * x0.y); fa.y = half2(g0.z * x0.z, g0.w * x0.w);
-                fa.z = half2(g1.x * x1.x, g1.y * x1.y); fa.w = half2(g1.z * x1.z, g1.w * x1.w);
-            }
-            GemmTraits<T>::mma(fb[buf][p], fa, acc);
-        }
-    };
-    int c = wave;
-    if (c < nchunks) load(c, 0);
-    for (; c < nchunks; c += 2 * GSK_WAVES) { // two chunks per trip so the buffers are addressed statically
-        if (c + GSK_WAVES < nchunks) load(c + GSK_WAVES, 1);
-        mul(0);
-        if (c + GSK_WAVES < nchunks) {
-            if (c + 2 * GSK_WAVES < nchunks) load(c + 2 * GSK_WAVES, 0);
-            mul(1);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 16; i++) red[wave][0][i][lane] = acc[i];
-    ssq[wave][lane] = ss;
-    __syncthreads();
-    // token m = n32: the squares of its row are spread over the waves and the two lane halves (fixed summation order)
-    float tot = 0.f;
-#pragma unroll
-    for (int w = 0; w < GSK_WAVES; w++) tot += ssq[w][n32] + ssq[w][n32 + 32];
-    const float scale = alpha / sqrtf(tot / (float)K + 1e-8f);
-    for (int g = wave; g < 4; g += GSK_WAVES) {
-        const int i4 = g;
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = red_sum(red, 0, 4 * i4 + j, lane) * scale;
-        const int m = n32, n = n0 + 8 * i4 + 4 * half; // accumulator element i: weight row 8 (i / 4) + 4 half + i % 4, column m
-        if (m >= M) continue;
-        if (EPI == GEMM_EPI_SWIGLU) {
-#pragma unroll
-            for (int j = 0; j < 4; j += 2)
-                if (n + j + 1 < N) GemmTraits<T>::put((T*)Cv + (size_t)m * ldc + ((n + j) >> 1), (v[j] / (1.0f + expf(-v[j]))) * v[j + 1]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (n + j < N) {
-                    float o = v[j];
-                    if (R) o += R[(size_t)m * ldr + n + j];
-                    ((float*)Cv)[(size_t)m * ldc + n + j] = o;
-                }
-        }
-    }
-}
-
-// The same for at most GSK_WAVES rows and half weights, with the normalised-up-to-1/rms rows staged in LDS: wave w
-// turns row w into halves of g (.) x once (sum of squares from the same pass), the product then reads its token
-// operand from LDS instead of holding fp32 rows and gains in registers -- this keeps the register need of the plain
-// kernel, so two workgroups share a compute unit and a matrix of several hundred row blocks still takes one round.
-// LDS rows are K halves + 16 bytes apart (rows four banks apart: the eight rows a read touches do not collide).
-template <int EPI>
-__global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny_norm8(const float* __restrict__ A, int lda, const f16_t* __restrict__ B, int ldb,
-                                                                void* Cv, int ldc, const float* R, int ldr, int M, int N, int K,
-                                                                float alpha, const float* __restrict__ gain) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char a16[]; // [M][2 K + 16] bytes
-    __shared__ float red[GSK_WAVES][1][16][64];
-    __shared__ float rinv[GSK_WAVES];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n0 = blockIdx.x * 32, n32 = lane & 31, half = lane >> 5;
-    const int nchunks = (int)(((size_t)K * 2) / GKB);
-    const int pitch = 2 * K + 16;
-    const unsigned char* brow = reinterpret_cast<const unsigned char*>(B) + (size_t)min(n0 + n32, N - 1) * ldb * 2 + half * 64;
-    f32x16 acc = (f32x16)(0.f);
-    u32x4 fb[2][4];
-    auto loadw = [&](int c, int buf) {
-#pragma unroll
-        for (int p = 0; p < 4; p++) fb[buf][p] = *reinterpret_cast<const u32x4*>(brow + (size_t)c * GKB + p * 16);
-    };
-    int c = wave;
-    if (c < nchunks) loadw(c, 0); // the first weights are on their way while the rows are staged
-    if (wave < M) {
-        const float* xr = A + (size_t)wave * lda;
-        float ss = 0.f;
-        for (int k = lane * 8; k < K; k += 64 * 8) {
-            const f32x4 x0 = *reinterpret_cast<const f32x4*>(xr + k), x1 = *reinterpret_cast<const f32x4*>(xr + k + 4);
-            const f32x4 g0 = *reinterpret_cast<const f32x4*>(gain + k), g1 = *reinterpret_cast<const f32x4*>(gain + k + 4);
-            ss = fmaf(x0.x, x0.x, ss); ss = fmaf(x0.y, x0.y, ss); ss = fmaf(x0.z, x0.z, ss); ss = fmaf(x0.w, x0.w, ss);
-            ss = fmaf(x1.x, x1.x, ss); ss = fmaf(x1.y, x1.y, ss); ss = fmaf(x1.z, x1.z, ss); ss = fmaf(x1.w, x1.w, ss);
-            auto h2 = [](float lo, float hi) {
-                const _Float16 a = (_Float16)fminf(fmaxf(lo, -65504.0f), 65504.0f), b = (_Float16)fminf(fmaxf(hi, -65504.0f), 65504.0f);
-                return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
-            };
-            u32x4 w;
-            w.x = h2(g0.x * x0.x, g0.y * x0.y); w.y = h2(g0.z * x0.z, g0.w * x0.w);
-            w.z = h2(g1.x * x1.x, g1.y * x1.y); w.w = h2(g1.z * x1.z, g1.w * x1.w);
-            *reinterpret_cast<u32x4*>(a16 + (size_t)wave * pitch + 2 * k) = w;
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-        if (lane == 0) rinv[wave] = 1.0f / sqrtf(ss / (float)K + 1e-8f);
-    }
-    __syncthreads();
-    const unsigned char* arow = a16 + (size_t)min(n32, M - 1) * pitch + half * 64;
-    auto mul = [&](int cc, int buf) {
-#pragma unroll
-        for (int p = 0; p < 4; p++) {
-            const u32x4 fa = *reinterpret_cast<const u32x4*>(arow + (size_t)cc * GKB + p * 16);
-            GemmTraits<f16_t>::mma(fb[buf][p], fa, acc);
-        }
-    };
-    for (; c < nchunks; c += 2 * GSK_WAVES) { // two chunks per trip so the buffers are addressed statically
-        if (c + GSK_WAVES < nchunks) loadw(c + GSK_WAVES, 1);
-        mul(c, 0);
-        if (c + GSK_WAVES < nchunks) {
-            if (c + 2 * GSK_WAVES < nchunks) loadw(c + 2 * GSK_WAVES, 0);
-            mul(c + GSK_WAVES, 1);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 16; i++) red[wave][0][i][lane] = acc[i];
-    __syncthreads();
-    const float scale = alpha * rinv[min(n32, M - 1)];
-    for (int g = wave; g < 4; g += GSK_WAVES) {
-        const int i4 = g;
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = red_sum(red, 0, 4 * i4 + j, lane) * scale;
-        const int m = n32, n = n0 + 8 * i4 + 4 * half; // accumulator element i: weight row 8 (i / 4) + 4 half + i % 4, column m
-        if (m >= M) continue;
-        if (EPI == GEMM_EPI_SWIGLU) {
-#pragma unroll
-            for (int j = 0; j < 4; j += 2)
-                if (n + j + 1 < N) GemmTraits<f16_t>::put((f16_t*)Cv + (size_t)m * ldc + ((n + j) >> 1), (v[j] / (1.0f + expf(-v[j]))) * v[j + 1]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (n + j < N) {
-                    float o = v[j];
-                    if (R) o += R[(size_t)m * ldr + n + j];
-                    ((float*)Cv)[(size_t)m * ldc + n + j] = o;
-                }
-        }
-    }
-}
-
-// rows that k_gemm_skinny_norm8 can stage: at most one per wave, and 40 KB of LDS beside the reduction buffer (two workgroups per unit)
-static bool skinny_norm8_fits(int M, int K) { return M <= GSK_WAVES && (size_t)M * (2 * (size_t)K + 16) <= 40 * 1024 && K % 512 == 0; }
-
-static hipError_t launch_gemm_skinny_norm8(hipStream_t stream, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                                           const float* R, int ldr, int M, int N, int K, float alpha, const float* normGain) {
-    const dim3 grid((N + 31) / 32);
-    const size_t lds = (size_t)M * (2 * (size_t)K + 16);
-    static std::atomic<bool> attr{false}; // set-up is idempotent: two threads that race here both do it // static + dynamic LDS pass 64 KB
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_skinny_norm8<GEMM_EPI_PLAIN>), hipFuncAttributeMaxDynamicSharedMemorySize, 40 * 1024);
-        if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_skinny_norm8<GEMM_EPI_SWIGLU>), hipFuncAttributeMaxDynamicSharedMemorySize, 40 * 1024);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
-    if (epi == GEMM_EPI_SWIGLU)
-        hipLaunchKernelGGL((k_gemm_skinny_norm8<GEMM_EPI_SWIGLU>), grid, dim3(GSK_WAVES * 64), lds, stream, (const float*)A, lda, (const f16_t*)B, ldb, C, ldc, R, ldr, M, N, K, alpha, normGain);
-    else
-        hipLaunchKernelGGL((k_gemm_skinny_norm8<GEMM_EPI_PLAIN>), grid, dim3(GSK_WAVES * 64), lds, stream, (const float*)A, lda, (const f16_t*)B, ldb, C, ldc, R, ldr, M, N, K, alpha, normGain);
-    return hipGetLastError();
-}
-
-template <typename T>
-static hipError_t launch_gemm_skinny_norm(hipStream_t stream, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                                          const float* R, int ldr, int M, int N, int K, float alpha, const float* normGain) {
-    const dim3 grid((N + 31) / 32);
-    if (epi == GEMM_EPI_SWIGLU)
-        hipLaunchKernelGGL((k_gemm_skinny_norm<T, GEMM_EPI_SWIGLU>), grid, dim3(GSK_WAVES * 64), 0, stream, (const float*)A, lda, (const T*)B, ldb, C, ldc, R, ldr, M, N, K, alpha, normGain);
-    else
-        hipLaunchKernelGGL((k_gemm_skinny_norm<T, GEMM_EPI_PLAIN>), grid, dim3(GSK_WAVES * 64), 0, stream, (const float*)A, lda, (const T*)B, ldb, C, ldc, R, ldr, M, N, K, alpha, normGain);
-    return hipGetLastError();
-}
-
 static hipError_t launch_gemm_skinny16(hipStream_t stream, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                                       const float* R, int ldr, int M, int N, int K, void* ws, float alpha, const float* normGain) {
+                                       const float* R, int ldr, int M, int N, int K, void* ws, float alpha) {
     const int nblocks = (N + 15) / 16;
     const int nchunks = (int)(((size_t)K * 4) / GKB);
     int ks = 1;
-    if (ws && !normGain && nblocks <= 64 && nchunks >= 32) { // few rows, long K: also split K over workgroups (see launch_gemm_skinny)
+    if (ws && nblocks <= 64 && nchunks >= 32) { // few rows, long K: also split K over workgroups (see launch_gemm_skinny)
         ks = std::min(std::min(8, 256 / nblocks), std::max(1, nchunks / GSK_WAVES));
         if ((size_t)nblocks * ks > 256 * 8) ks = 1;
     }
@@ -1054,19 +799,17 @@ static hipError_t launch_gemm_skinny16(hipStream_t stream, int epi, const void* 
     float* partials = ws ? (float*)((unsigned char*)ws + (size_t)GSK_COUNTERS * 4) : nullptr;
     static std::atomic<bool> attr{false}; // set-up is idempotent: two threads that race here both do it
     if (!attr) {
-        const void* fns[4] = {reinterpret_cast<const void*>(&k_gemm_skinny16<GEMM_EPI_PLAIN, false>), reinterpret_cast<const void*>(&k_gemm_skinny16<GEMM_EPI_PLAIN, true>),
-                              reinterpret_cast<const void*>(&k_gemm_skinny16<GEMM_EPI_SWIGLU, false>), reinterpret_cast<const void*>(&k_gemm_skinny16<GEMM_EPI_SWIGLU, true>)};
+        const void* fns[2] = {reinterpret_cast<const void*>(&k_gemm_skinny16<GEMM_EPI_PLAIN>), reinterpret_cast<const void*>(&k_gemm_skinny16<GEMM_EPI_SWIGLU>)};
         for (const void* f : fns) {
             const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, SK16_LDS);
             if (e != hipSuccess) return e;
         }
         attr = true;
     }
-#define SK16(EPI_, NORM_)                                                                                                     \
-    hipLaunchKernelGGL((k_gemm_skinny16<EPI_, NORM_>), grid, dim3(GSK_WAVES * 64), SK16_LDS, stream, (const float*)A, lda, (const float*)B, ldb, \
-                       C, ldc, R, ldr, M, N, K, counters, partials, alpha, normGain)
-    if (epi == GEMM_EPI_SWIGLU) { if (normGain) SK16(GEMM_EPI_SWIGLU, true); else SK16(GEMM_EPI_SWIGLU, false); }
-    else { if (normGain) SK16(GEMM_EPI_PLAIN, true); else SK16(GEMM_EPI_PLAIN, false); }
+#define SK16(EPI_)                                                                                                            \
+    hipLaunchKernelGGL((k_gemm_skinny16<EPI_>), grid, dim3(GSK_WAVES * 64), SK16_LDS, stream, (const float*)A, lda, (const float*)B, ldb, \
+                       C, ldc, R, ldr, M, N, K, counters, partials, alpha)
+    if (epi == GEMM_EPI_SWIGLU) SK16(GEMM_EPI_SWIGLU); else SK16(GEMM_EPI_PLAIN);
 #undef SK16
     return hipGetLastError();
 }
@@ -1100,38 +843,23 @@ static hipError_t launch_gemm_skinny(hipStream_t stream, int epi, const void* A,
 // epi = GEMM_EPI_PLAIN: C fp32 [M, N] (+ R).  epi = GEMM_EPI_SWIGLU: C is [M, N/2] in the operand type.
 // ws: optional zero-initialised workspace of mlh_gemm_workspace_bytes() (enables split-K for M <= 64); launches that
 // share a workspace must be ordered on one stream.
-// True when mlh_gemm_tn_epi can take `normGain` for this shape (the RMSNorm of A's rows fused into the product).
-bool mlh_gemm_norm_fusable(int dtype, int M, int N, int K) {
-    // k_gemm_skinny_norm (A is the fp32 residual for both operand types).  With half weights its register need allows
-    // one workgroup per compute unit, where the plain kernel runs two: a matrix of more than 256 row blocks would
-    // take two rounds and lose more than the saved RMSNorm launch brings -- unless the rows fit k_gemm_skinny_norm8's LDS.
-    if (M <= 32) return dtype == MLH_DTYPE_F32 || (dtype == MLH_GEMM_F16 && ((N + 31) / 32 <= 256 || skinny_norm8_fits(M, K)));
-    return dtype == MLH_DTYPE_F32 && M > 32 && M <= 64 && N <= 16 * GSK_COUNTERS && (N + 31) / 32 < 200;
-}
-
 hipError_t mlh_gemm_tn_epi(hipStream_t stream, int dtype, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                           const float* R, int ldr, int M, int N, int K, void* ws, float alpha, const float* normGain) {
+                           const float* R, int ldr, int M, int N, int K, void* ws, float alpha) {
     const size_t esz = dtype == MLH_GEMM_P3 ? 6 : dtype == MLH_DTYPE_F32 ? 4 : 2;
     if (dtype == MLH_GEMM_P3 && (M <= 0 || N <= 0 || K <= 0 || K % 32 || lda % 32 || ldb % 32)) return hipErrorInvalidValue;
     if (dtype == MLH_GEMM_P3) return mlh_gemm_tile(stream, dtype, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha);
     if (M <= 0 || N <= 0 || K <= 0 || ((size_t)K * esz) % GKB != 0 || ((size_t)lda * esz) % 16 != 0 || ((size_t)ldb * esz) % 16 != 0)
         return hipErrorInvalidValue;
     if (epi == GEMM_EPI_SWIGLU && (N & 1)) return hipErrorInvalidValue;
-    if (normGain && !mlh_gemm_norm_fusable(dtype, M, N, K)) return hipErrorInvalidValue;
-    // M <= 64 (one row per sequence of a decode batch): weight-streaming skinny kernel; more rows: tiles
+    // M <= 64 (short prefills of bf16 models, mlh_gemm_device): weight-streaming skinny kernel; more rows: tiles
 #define GEMM_BY_TYPE(call_f32, call_bf16, call_f16) \
     return dtype == MLH_DTYPE_BF16 ? (call_bf16) : dtype == MLH_GEMM_F16 ? (call_f16) : (call_f32)
-    if (M <= 32 && normGain && dtype == MLH_GEMM_F16 && skinny_norm8_fits(M, K))
-        return launch_gemm_skinny_norm8(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha, normGain);
-    if (M <= 32 && normGain)
-        return dtype == MLH_GEMM_F16 ? launch_gemm_skinny_norm<f16_t>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha, normGain)
-                                     : launch_gemm_skinny_norm<float>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha, normGain);
     if (M <= 32)
         GEMM_BY_TYPE((launch_gemm_skinny<float, 1>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)),
                      (launch_gemm_skinny<bf16_t, 1>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)),
                      (launch_gemm_skinny<f16_t, 1>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)));
     if (M > 32 && M <= 64 && dtype == MLH_DTYPE_F32 && N <= 16 * GSK_COUNTERS && (N + 31) / 32 < 200) // the 32-row tiles would leave compute units idle
-        return launch_gemm_skinny16(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha, normGain);
+        return launch_gemm_skinny16(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha);
     if (M <= 64)
         GEMM_BY_TYPE((launch_gemm_skinny<float, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)),
                      (launch_gemm_skinny<bf16_t, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)),
@@ -1149,7 +877,7 @@ hipError_t mlh_gemm_tn_epi(hipStream_t stream, int dtype, int epi, const void* A
         // away saves the tile walkers more (a round) than they cost as a strip of their own.
         const int Nm = N - rem;
         if (w4_us(M, Nm, K, cus) + mlh_gemm_tile_us(dtype, M, rem, K, cus, ws != nullptr) < usW4) {
-            const hipError_t e = mlh_gemm_tn_epi(stream, dtype, epi, A, lda, B, ldb, C, ldc, R, ldr, M, Nm, K, ws, alpha, nullptr);
+            const hipError_t e = mlh_gemm_tn_epi(stream, dtype, epi, A, lda, B, ldb, C, ldc, R, ldr, M, Nm, K, ws, alpha);
             if (e != hipSuccess) return e;
             return mlh_gemm_tile(stream, dtype, epi, A, lda, (const unsigned char*)B + (size_t)Nm * ldb * esz, ldb, (float*)C + Nm, ldc,
                                  R ? R + Nm : nullptr, ldr, M, rem, K, ws, alpha);

@@ -1317,8 +1317,7 @@ int mlh_build_gemm_operands(mlh_ctx* c) {
     const mlh_hparams& hp = c->hp;
     const bool supported = mlh_prefill_gemm_supported(c), mirror = hp.weightDtype == MLH_DTYPE_BF16 && supported;
     const bool planes = hp.weightDtype == MLH_DTYPE_F32 && supported;
-    c->gemmDtype = mirror ? MLH_GEMM_F16 : hp.weightDtype;
-    c->pfDtype = planes ? MLH_GEMM_P3 : c->gemmDtype;
+    c->pfDtype = planes ? MLH_GEMM_P3 : mirror ? MLH_GEMM_F16 : hp.weightDtype;
     c->f16Inexact = 0;
     for (void* p : c->mirrorAllocs) (void)hipFree(p); // a repeated finalize rebuilds them
     c->mirrorAllocs.clear();
@@ -1327,7 +1326,7 @@ int mlh_build_gemm_operands(mlh_ctx* c) {
     int rc = 0;
     const size_t d = hp.dim, F = hp.ffnDim, pl = hp.pleDim, wb = c->wbytes;
     for (LayerDev& L : c->layers) {
-        L.WaG = L.Wa; L.WoG = L.Wo; L.W13G = L.W13; L.W2G = L.W2;
+        L.WaP = L.Wa; L.WoP = L.Wo; L.W13P = L.W13; L.W2P = L.W2;
         L.sWa = L.sWo = L.sW13 = L.sW2 = 1.0f;
         const void* wo = L.Wo;
         if (pl > 0) { // [Wo | pleUp] along K, in the storage type
@@ -1337,22 +1336,20 @@ int mlh_build_gemm_operands(mlh_ctx* c) {
             MLH_CHECK(c, hipMemcpy2D(cat, (L.ad + pl) * wb, L.Wo, L.ad * wb, L.ad * wb, d, hipMemcpyDeviceToDevice));
             MLH_CHECK(c, hipMemcpy2D((char*)cat + L.ad * wb, (L.ad + pl) * wb, L.pleUp, pl * wb, pl * wb, d, hipMemcpyDeviceToDevice));
             wo = cat;
-            L.WoG = cat;
         }
+        L.WoR = wo;
         if (planes && ((rc = build_planes(c, L.Wa, L.rowsA, (int)d, &L.WaP)) || (rc = build_planes(c, wo, (int)d, L.ad + (int)pl, &L.WoP)) ||
                        (rc = build_planes(c, L.W13, 2 * (int)F, (int)d, &L.W13P)) || (rc = build_planes(c, L.W2, (int)d, (int)F, &L.W2P))))
             break;
         if (!mirror) continue;
-        if ((rc = build_mirror(c, L.Wa, (size_t)L.rowsA * d, &L.WaG, &L.sWa, d_scratch)) ||
-            (rc = build_mirror(c, wo, d * (L.ad + pl), &L.WoG, &L.sWo, d_scratch)) ||
-            (rc = build_mirror(c, L.W13, 2 * F * d, &L.W13G, &L.sW13, d_scratch)) ||
-            (rc = build_mirror(c, L.W2, d * F, &L.W2G, &L.sW2, d_scratch)))
+        if ((rc = build_mirror(c, L.Wa, (size_t)L.rowsA * d, &L.WaP, &L.sWa, d_scratch)) ||
+            (rc = build_mirror(c, wo, d * (L.ad + pl), &L.WoP, &L.sWo, d_scratch)) ||
+            (rc = build_mirror(c, L.W13, 2 * F * d, &L.W13P, &L.sW13, d_scratch)) ||
+            (rc = build_mirror(c, L.W2, d * F, &L.W2P, &L.sW2, d_scratch)))
             break;
-        L.WaP = L.WaG; L.WoP = L.WoG; L.W13P = L.W13G; L.W2P = L.W2G;
     }
-    c->EG = c->E; c->sE = 1.0f;
-    if (rc == 0 && mirror) rc = build_mirror(c, c->E, (size_t)hp.vocabSize * hp.dim, &c->EG, &c->sE, d_scratch);
-    c->EP = c->EG;
+    c->EP = c->E; c->sE = 1.0f;
+    if (rc == 0 && mirror) rc = build_mirror(c, c->E, (size_t)hp.vocabSize * hp.dim, &c->EP, &c->sE, d_scratch);
     if (rc == 0 && planes) rc = build_planes(c, c->E, hp.vocabSize, hp.dim, &c->EP);
     if (d_scratch) (void)hipFree(d_scratch);
     return rc;
@@ -1429,7 +1426,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     std::vector<int> rowSeq(n), rowPos(n), segStart(nseg), segPos0(nseg), blkSeg, blkQ0, chunkSeg, chunkT0, chunkBase(nseg, 0);
     bool anyGdn = false;
     for (const LayerDev& L : c->layers) anyGdn = anyGdn || L.kind == MLH_KIND_GDN;
-    const bool gdnChunked = anyGdn && c->gemmDtype == MLH_GEMM_F16; // segments of 64 tokens or more: chunk-parallel MFMA path
+    const bool gdnChunked = anyGdn && c->pfDtype == MLH_GEMM_F16; // segments of 64 tokens or more: chunk-parallel MFMA path
     int r = 0;
     for (int s = 0; s < nseg; s++) {
         segStart[s] = r;
@@ -1561,205 +1558,5 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     if (e != hipSuccess) { c->err = std::string("prefill launch: ") + hipGetErrorString(e); return -2; }
     MLH_CHECK(c, hipStreamSynchronize(st));
     for (int s = 0; s < nseg; s++) c->h_len[seqs[s]] += lens[s];
-    return 0;
-}
-
-// ----------------------------------------------------------------------------
-// Batched decode step (8 or more sequences, one new token each): the same row pipeline with the
-// skinny MFMA GEMM -- every weight matrix is streamed once per step whatever the batch size -- and
-// the decode path's own attention / GDN kernels, whose split-KV partials are combined here.
-// Everything stays on the device and on the stream (no allocation, no host round trip), so a
-// step can be captured into a graph like the GEMV step.
-// ----------------------------------------------------------------------------
-#define MLH_BATCH_GEMM_MIN_SEQS 8
-
-template <typename WT>
-__global__ void k_bd_embed(StepArgs a) {
-    const int slot = blockIdx.y, i = blockIdx.x * PWG + threadIdx.x;
-    if (slot == 0 && i == 0) *a.stepCounter += 1; // steps started; k_bd_finish logs into row (counter - 1)
-    if (i >= a.dim) return;
-    a.x[(size_t)slot * a.dim + i] = getw<WT>((const WT*)a.E + (size_t)a.tok[slot] * a.dim + i);
-}
-
-// Mixing output rows in the GEMM input type: attention layers combine the split-KV partials of the decode
-// attention kernel and apply the sigmoid gate (inference.cu:241-250); GDN layers convert the read-out.
-// PLE rows e = silu(gate) * P[tok] are appended to the row (column L.ad on).
-template <typename WT, typename AT>
-__global__ void __launch_bounds__(PWG) k_bd_mix(StepArgs a, LayerDev L, AT* Amix, int aLd) {
-    const int slot = blockIdx.x, tid = threadIdx.x;
-    const float* qkv = a.qkv + (size_t)slot * a.qkvStride;
-    // the row is dealt to the gridDim.y workgroups of the slot in contiguous pieces (one workgroup per slot would
-    // walk every head's partials alone)
-    const int piece = (L.ad + (int)gridDim.y - 1) / (int)gridDim.y, i0 = (int)blockIdx.y * piece, i1 = min(L.ad, i0 + piece);
-    if (L.kind == MLH_KIND_ATTENTION) {
-        const int hd = a.hd;
-        for (int i = i0 + tid; i < i1; i += PWG) {
-            const int h = i / hd, e = i - h * hd;
-            const float* pp = a.part + (((size_t)slot * a.nsplit) * a.heads + h) * (hd + 2);
-            const size_t sstride = (size_t)a.heads * (hd + 2);
-            float M = -1.0e30f;
-            for (int s = 0; s < a.nsplit; s++) M = fmaxf(M, pp[s * sstride + hd]);
-            float num = 0.f, den = 0.f;
-            for (int s = 0; s < a.nsplit; s++) {
-                const float w = expf(pp[s * sstride + hd] - M);
-                num = fmaf(w, pp[s * sstride + e], num);
-                den = fmaf(w, pp[s * sstride + hd + 1], den);
-            }
-            float v = num / den;
-            if (a.gating) v = v * pf_sigmoid(qkv[L.offG + i]);
-            put<AT>(Amix + (size_t)slot * aLd + i, v);
-        }
-    } else {
-        for (int i = i0 + tid; i < i1; i += PWG) put<AT>(Amix + (size_t)slot * aLd + i, a.mix[(size_t)slot * L.ad + i]);
-    }
-    if (blockIdx.y == 0)
-        for (int j = tid; j < a.ple; j += PWG)
-        put<AT>(Amix + (size_t)slot * aLd + L.ad + j, pf_silu(qkv[L.offPle + j]) * getw<WT>((const WT*)L.pleTable + (size_t)a.tok[slot] * a.ple + j));
-}
-
-// One workgroup per slot: argmax of the slot's logits (lowest index on ties), logits copied to the
-// sequence's row, bookkeeping of k_finish (next token, id log, position).
-__global__ void __launch_bounds__(PWG) k_bd_finish(StepArgs a, const float* lg, int* tokOut) {
-    __shared__ float sv[PWG];
-    __shared__ int si[PWG];
-    __shared__ double sd[PWG + 1];
-    const int slot = blockIdx.x, tid = threadIdx.x, seq = a.sidx[slot];
-    const float* row = lg + (size_t)slot * a.vocab;
-    float* dst = a.logits + (size_t)seq * a.vocab;
-    if (a.temperature > 0.f) { // draw instead of argmax
-        for (int i = tid; i < a.vocab; i += PWG) dst[i] = row[i];
-        const int nxt = mlh_sample_row<PWG>(row, a.vocab, a.temperature, mlh_sample_uniform(a.sampleSeed, seq, a.pos[seq] + 1), sd, si);
-        __syncthreads();
-        if (tid == 0) {
-            const int step = *a.stepCounter - 1;
-            tokOut[slot] = nxt;
-            a.nextTok[seq] = nxt;
-            if (step >= 0 && step < a.outCapacity) a.outIds[(size_t)step * a.nseq + slot] = nxt;
-            a.pos[seq] += 1;
-        }
-        return;
-    }
-    float v = -3.0e38f;
-    int idx = 0x7fffffff;
-    if ((a.vocab & 3) == 0) { // 16 bytes per lane, four loads in flight before the first store (row and dst do not overlap)
-        const f32x4* row4 = reinterpret_cast<const f32x4*>(row);
-        f32x4* dst4 = reinterpret_cast<f32x4*>(dst);
-        const int n4 = a.vocab >> 2;
-        for (int i0 = tid; i0 < n4; i0 += 4 * PWG) {
-            f32x4 x[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) x[k] = row4[min(i0 + k * PWG, n4 - 1)];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int i = i0 + k * PWG;
-                if (i < n4) {
-                    dst4[i] = x[k];
-                    // i ascends per thread and the four elements are taken in order: ties keep the lower index
-                    if (x[k].x > v) { v = x[k].x; idx = 4 * i; }
-                    if (x[k].y > v) { v = x[k].y; idx = 4 * i + 1; }
-                    if (x[k].z > v) { v = x[k].z; idx = 4 * i + 2; }
-                    if (x[k].w > v) { v = x[k].w; idx = 4 * i + 3; }
-                }
-            }
-        }
-    } else {
-        for (int i = tid; i < a.vocab; i += PWG) {
-            const float x = row[i];
-            dst[i] = x;
-            if (x > v) { v = x; idx = i; } // i ascends: ties keep the lower index
-        }
-    }
-    sv[tid] = v; si[tid] = idx;
-    __syncthreads();
-    for (int s = PWG / 2; s > 0; s >>= 1) {
-        if (tid < s && (sv[tid + s] > sv[tid] || (sv[tid + s] == sv[tid] && si[tid + s] < si[tid]))) { sv[tid] = sv[tid + s]; si[tid] = si[tid + s]; }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        int nxt = si[0];
-        if (nxt < 0 || nxt >= a.vocab) nxt = 0;
-        const int step = *a.stepCounter - 1;
-        tokOut[slot] = nxt;
-        a.nextTok[seq] = nxt;
-        if (step >= 0 && step < a.outCapacity) a.outIds[(size_t)step * a.nseq + slot] = nxt;
-        a.pos[seq] += 1;
-    }
-}
-
-bool mlh_batch_step_applicable(const mlh_ctx* c, int nseq) {
-    return c->prefillMode == 0 && nseq >= MLH_BATCH_GEMM_MIN_SEQS && nseq <= 64 && mlh_prefill_gemm_supported(c);
-}
-
-// Allocations the batched step needs; call outside graph capture.
-int mlh_prepare_batch_step(mlh_ctx* c, int nseq) {
-    if (!mlh_batch_step_applicable(c, nseq)) return 0;
-    int rc = ensure_prefill_buffers(c, std::max(nseq, 64));
-    if (rc) return rc;
-    if ((rc = ensure_gemm_workspace(c))) return rc;
-    if (!c->pfLogits) {
-        MLH_CHECK(c, hipMalloc((void**)&c->pfLogits, (size_t)64 * c->hp.vocabSize * 4));
-        c->allocs.push_back(c->pfLogits);
-    }
-    return 0;
-}
-
-int mlh_launch_batch_step(mlh_ctx* c, int nseq, const int* tokPtr) {
-    const mlh_hparams& hp = c->hp;
-    if (c->pfRows < nseq || !c->pfLogits) { c->err = "batched step buffers not prepared"; return -1; }
-    StepArgs a;
-    mlh_fill_args(c, a, nseq, tokPtr);
-    hipStream_t st = c->stream;
-    const int d_ = hp.dim, F = hp.ffnDim, dt = c->gemmDtype, n = nseq;
-    const bool bf = hp.weightDtype == MLH_DTYPE_BF16;
-#define GEMMN(epi, A, lda, B, alpha, ldb, C, ldc, R, ldr, M, N, K, G)                                                 \
-    do {                                                                                                            \
-        hipError_t e_ = mlh_gemm_tn_epi(st, dt, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, c->gemmWs, alpha, G);  \
-        if (e_ != hipSuccess) { c->err = std::string("batched step GEMM: ") + hipGetErrorString(e_); return -2; }    \
-    } while (0)
-#define GEMM(epi, A, lda, B, alpha, ldb, C, ldc, R, ldr, M, N, K) GEMMN(epi, A, lda, B, alpha, ldb, C, ldc, R, ldr, M, N, K, nullptr)
-    if (bf) hipLaunchKernelGGL((k_bd_embed<bf16_t>), dim3(cdiv(d_, PWG), n), dim3(PWG), 0, st, a);
-    else hipLaunchKernelGGL((k_bd_embed<float>), dim3(cdiv(d_, PWG), n), dim3(PWG), 0, st, a);
-    for (int t = hp.transformers - 1; t >= 0; t--) {
-        const LayerDev& L = c->layers[t];
-        // (fp32, 33..64 sequences: the RMSNorm rides in the product, see mlh_gemm_norm_fusable)
-        if (mlh_gemm_norm_fusable(dt, n, L.rowsA, d_)) {
-            GEMMN(0, c->x, d_, L.WaG, L.sWa, d_, c->qkv, c->maxRowsA, nullptr, 0, n, L.rowsA, d_, L.g1);
-        } else {
-            if (bf) hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, L.g1, c->pfXn, n, d_);
-            else hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, L.g1, c->pfXn, n, d_);
-            GEMM(0, c->pfXn, d_, L.WaG, L.sWa, d_, c->qkv, c->maxRowsA, nullptr, 0, n, L.rowsA, d_);
-        }
-        const bool gdn = L.kind != MLH_KIND_ATTENTION;
-        // The GDN kernel writes its read-out and the PLE columns straight into the GEMM's input rows (mlh_launch_one
-        // reads the step's tokens from the context's own buffer, hence the second condition).
-        // The attention kernel does the same when one workgroup holds all keys of a (head, sequence) pair.
-        const bool direct = (gdn || c->nsplit == 1) && tokPtr == c->d_tok;
-        if (direct) { c->mixRows = c->pfA; c->mixRowsLd = c->maxAd + hp.pleDim; c->mixRowsHalf = bf ? 1 : 0; }
-        int rc = mlh_launch_one(c, gdn ? MLH_K_GDN : MLH_K_ATTN, t, nseq);
-        c->mixRows = nullptr;
-        if (rc) return rc;
-        if (!direct) { // attention: combine the split-KV partials, gate; PLE columns
-            const dim3 mg(n, std::max(1, (L.ad + PWG - 1) / PWG * (n <= 16 ? 4 : 1))); // few slots: more workgroups per row
-            if (bf) hipLaunchKernelGGL((k_bd_mix<bf16_t, f16_t>), mg, dim3(PWG), 0, st, a, L, (f16_t*)c->pfA, c->maxAd + hp.pleDim);
-            else hipLaunchKernelGGL((k_bd_mix<float, float>), mg, dim3(PWG), 0, st, a, L, (float*)c->pfA, c->maxAd + hp.pleDim);
-        }
-        GEMM(0, c->pfA, c->maxAd + hp.pleDim, L.WoG, L.sWo, L.ad + hp.pleDim, c->h1, d_, c->x, d_, n, d_, L.ad + hp.pleDim);
-        if (mlh_gemm_norm_fusable(dt, n, 2 * F, d_)) {
-            GEMMN(1, c->h1, d_, L.W13G, L.sW13, d_, c->pfU, F, nullptr, 0, n, 2 * F, d_, L.g2);
-        } else {
-            if (bf) hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->h1, L.g2, c->pfXn, n, d_);
-            else hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->h1, L.g2, c->pfXn, n, d_);
-            GEMM(1, c->pfXn, d_, L.W13G, L.sW13, d_, c->pfU, F, nullptr, 0, n, 2 * F, d_);
-        }
-        GEMM(0, c->pfU, F, L.W2G, L.sW2, F, c->x, d_, c->h1, d_, n, d_, F);
-    }
-    if (bf) hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, c->gF, c->pfXn, n, d_);
-    else hipLaunchKernelGGL((k_pf_rmsnorm<float>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, c->x, c->gF, c->pfXn, n, d_);
-    GEMM(0, c->pfXn, d_, c->EG, c->sE, d_, c->pfLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_);
-#undef GEMM
-#undef GEMMN
-    hipLaunchKernelGGL(k_bd_finish, dim3(n), dim3(PWG), 0, st, a, c->pfLogits, c->d_tok);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) { c->err = std::string("batched step launch: ") + hipGetErrorString(e); return -2; }
     return 0;
 }

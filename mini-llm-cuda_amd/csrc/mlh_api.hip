@@ -391,6 +391,7 @@ extern "C" int mlh_finalize(mlh_ctx* c) {
     int rc = mlh_init_kernels(c);
     if (rc == 0) rc = mlh_init_prefill_kernels(c);
     if (rc == 0) rc = mlh_build_gemm_operands(c);
+    if (rc == 0 && mlh_prefill_gemm_supported(c)) rc = mlh_rows_prepare(c);
     if (rc) return rc;
     MLH_CHECK(c, hipMemcpy(c->d_layers, c->layers.data(), c->layers.size() * sizeof(LayerDev), hipMemcpyHostToDevice));
     // function attributes and occupancy of the single-launch decode kernels, here and not on every launch
@@ -587,7 +588,7 @@ static int ensure_graph(mlh_ctx* c, int slot, int nseq, int k) {
     hipGraph_t g = nullptr;
     MLH_CHECK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int rc = 0;
-    for (int i = 0; i < k && rc == 0; i++) rc = mlh_launch_step(c, nseq, c->d_tok, true);
+    for (int i = 0; i < k && rc == 0; i++) rc = mlh_launch_step(c, nseq, c->d_tok, true, i > 0, i + 1 < k);
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
     if (e != hipSuccess) { c->err = std::string("hipStreamEndCapture: ") + hipGetErrorString(e); return -2; }
@@ -601,7 +602,11 @@ static int ensure_graph(mlh_ctx* c, int slot, int nseq, int k) {
 
 static bool use_persistent(const mlh_ctx* c, int nseq) {
     // (the single-launch kernels fuse the argmax only: sampling runs through the kernel sequence)
-    return nseq == 1 && c->usePersistent && c->temperature <= 0.f && mlh_persistent_supported(c);
+    if (nseq != 1 || !c->usePersistent || c->temperature > 0.f) return false;
+    // mode 3 on a model the XCD-rank kernel does not cover: the row step where it applies (its launches cost less than the
+    // barrier kernel's phases), else the barrier kernel
+    if (c->usePersistent == 3) return mlh_xcd_supported(c) || (!mlh_rows_applicable(c, 1) && mlh_persistent_supported(c));
+    return mlh_persistent_supported(c);
 }
 
 // After the stream has drained: a single-launch decode that gave up a bounded wait leaves its flag set.  The sequence
@@ -645,7 +650,7 @@ static int run_steps(mlh_ctx* c, int nseq, int steps) {
         }
     } else {
         for (int i = 0; i < steps; i++)
-            if ((rc = mlh_launch_step(c, nseq, c->d_tok, true))) return rc;
+            if ((rc = mlh_launch_step(c, nseq, c->d_tok, true, i > 0, i + 1 < steps))) return rc;
     }
     return 0;
 }
@@ -661,7 +666,6 @@ static int check_decode(mlh_ctx* c, const int32_t* ids, int nseq, int steps) {
         if (ids[s] < 0 || ids[s] >= hp.vocabSize) { c->err = "token id out of range"; return -1; }
         if (c->h_len[s] + steps > hp.maxL) { c->err = "sequence would exceed maxL"; return -1; }
     }
-    if ((rc = mlh_prepare_batch_step(c, nseq))) return rc;
     return set_identity_slots(c, nseq);
 }
 

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "mlh.h"
+#include "rows.h"
 
 #define MLH_KV_PAGE 64      // positions per KV page; equals the attention key tile
 #define MLH_ATTN_WG_KEYS 256 // keys one attention workgroup covers (4 waves x one 64-key tile)
@@ -42,12 +43,12 @@ struct LayerDev {
     int kind;
     int rowsA, offK, offV, offG, offPle, offGa, offGb;
     int ad;               // width of the mixing output fed to Wo
-    // What the MFMA path multiplies: the matrices themselves for fp32 models; for bf16 models IEEE-half
+    // What the prefill's products multiply: fp32 matrices as three bf16 planes (p3.h); for bf16 models IEEE-half
     // mirrors scaled by a power of two (exact), with the inverse scale applied to the product.
-    // WoG is [dim, ad + pleDim]: Wo with pleUp appended along K, so that h1 = [a | e] . WoG^T is one product.
-    const void *WaG, *WoG, *W13G, *W2G;
-    const void *WaP, *WoP, *W13P, *W2P; // the same for the prefill's tiled products: fp32 models as three bf16 planes (p3.h)
+    // WoP is [dim, ad + pleDim]: Wo with pleUp appended along K, so that h1 = [a | e] . WoP^T is one product.
+    const void *WaP, *WoP, *W13P, *W2P;
     float sWa, sWo, sW13, sW2;
+    const void *WaR, *WoR, *W13R, *W2R; // for the row step: the matrices ([Wo | pleUp] as one) in its fetch order (rows.h)
 };
 
 // Arguments shared by all kernels of a decode step.
@@ -70,9 +71,8 @@ struct StepArgs {
     int qkvStride;
     float* part;          // [slots, nsplit, heads, hd + 2] attention partials (m, l, acc)
     float* mix;           // [slots, maxAd] GDN read-out
-    void* mixRows;        // batched step: if set, the GDN read-out and the PLE columns go straight into the rows of the
-    int mixRowsLd;        //   output-projection GEMM (leading dimension in elements, fp32 or IEEE half) instead of `mix`
-    int mixRowsHalf;
+    unsigned char* mixRows; // row step: if set, the mixing output and the PLE columns go straight into the planes the output
+    RowsLayout mixLay;    //   projection multiplies (rows.h) instead of `mix` and `part`
     int wbytes;           // bytes per weight element (PLE table rows)
     float temperature;    // > 0: the next token is drawn from softmax(logits / temperature) instead of the argmax
     unsigned long long sampleSeed;
@@ -108,8 +108,11 @@ struct mlh_ctx {
     float* gF = nullptr;
     float* rope = nullptr;
 
-    void* mixRows = nullptr; // see StepArgs::mixRows; set by the batched step around its GDN launches
-    int mixRowsLd = 0, mixRowsHalf = 0;
+    unsigned char* mixRows = nullptr; // see StepArgs::mixRows; set by the row step
+    RowsLayout mixLay = {1, 1};
+    void* rowsBuf = nullptr; // row step (kernels_rows.hip): planes of the residual rows x and h1, the mixing output and the FFN units, partial sums of squares
+    unsigned char *rowsX = nullptr, *rowsH = nullptr, *rowsMix = nullptr, *rowsU = nullptr;
+    float *rowsSsqX = nullptr, *rowsSsqH = nullptr;
     int pagesPerSeq = 0;
     int nsplit = 1;
     int maxRowsA = 0, maxAd = 0;
@@ -172,15 +175,13 @@ struct mlh_ctx {
     void* pfGdnWs = nullptr;   // chunk operands of the chunk-parallel GDN prefill
     float* pfGdnG = nullptr;
     size_t pfGdnChunks = 0;
-    const void* EG = nullptr;  // LM-head matrix as the MFMA path reads it (see LayerDev::WaG)
+    const void* EP = nullptr;  // LM-head matrix as the prefill's products read it (see LayerDev::WaP)
     float sE = 1.0f;
-    const void* EP = nullptr;  // the same for the prefill's tiled products
-    int gemmDtype = MLH_DTYPE_F32; // operand type of the batched step's products: MLH_DTYPE_F32 or MLH_GEMM_F16
-    int pfDtype = MLH_DTYPE_F32;   // ... and of the prefill's: MLH_GEMM_P3 or MLH_GEMM_F16
+    const void* ER = nullptr;  // ... and in the row step's fetch order
+    int pfDtype = MLH_DTYPE_F32; // operand type of those: MLH_GEMM_P3 or MLH_GEMM_F16
     std::vector<void*> mirrorAllocs;
     long f16Inexact = 0;       // bf16 weights that had no exact scaled-half representation (reported at finalize)
     void* gemmWs = nullptr;    // split-K workspace of the skinny GEMM
-    float* pfLogits = nullptr; // [64, vocab] logits of a batched decode step in slot order
 
     std::vector<int> h_len; // host mirror of d_pos
     int identityNseq = 0;   // d_sidx currently holds 0..identityNseq-1 (0 = unknown)
@@ -192,7 +193,8 @@ struct mlh_ctx {
 };
 
 // kernels_decode.hip
-int mlh_launch_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead);
+int mlh_launch_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool embedded = false, bool embedNext = false);
+int mlh_launch_mix(mlh_ctx* c, const StepArgs& a, const LayerDev& L);
 int mlh_launch_one(mlh_ctx* c, int kernel, int layer, int nseq);
 double mlh_kernel_bytes(mlh_ctx* c, int kernel, int layer, int nseq);
 void mlh_fill_args(mlh_ctx* c, StepArgs& a, int nseq, const int* tokPtr);
@@ -208,18 +210,14 @@ int mlh_init_kernels(mlh_ctx* c);
 // ws: zero-initialised workspace of mlh_gemm_workspace_bytes() or null; with it, M <= 64 products of matrices
 // with few rows are split along K over workgroups (deterministically reduced).
 // alpha scales the product before the epilogue (the power of two an fp16 weight mirror was scaled by, inverted).
-// normGain (M <= 64 for fp32 operands, M <= 32 for half operands, see mlh_gemm_norm_fusable): A holds the raw fp32
-// rows -- also when the weights are half -- and the product is taken of gain * A / rms(A) (the RMSNorm of the rows,
-// eps 1e-8 inside the root), without a pass that writes the normalised rows.
 hipError_t mlh_gemm_tn_epi(hipStream_t stream, int dtype, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                           const float* R, int ldr, int M, int N, int K, void* ws, float alpha = 1.0f, const float* normGain = nullptr);
+                           const float* R, int ldr, int M, int N, int K, void* ws, float alpha = 1.0f);
 // kernels_tile.hip: the same product in 128 x 128 / 64 x 64 tiles (operands half, bf16 or P3), and fp32 -> P3 rows
 hipError_t mlh_gemm_tile(hipStream_t stream, int dtype, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
                          const float* R, int ldr, int M, int N, int K, void* ws, float alpha);
 double mlh_gemm_tile_us(int dtype, int M, int N, int K, int cus, bool ws); // what that product is expected to take
 int mlh_gemm_num_cus(void); // kernels_gemm.hip: compute units of the current device, a multiple of eight; 0: unknown
 hipError_t mlh_split_p3(hipStream_t stream, const float* src, int lds, void* dst, int ldd, int rows, int cols);
-bool mlh_gemm_norm_fusable(int dtype, int M, int N, int K);
 size_t mlh_gemm_workspace_bytes(void);
 extern "C" int mlh_gemm_device_init(int device);
 
@@ -230,11 +228,13 @@ void mlh_set_thread_error(const std::string& msg);
 bool mlh_prefill_gemm_supported(const mlh_ctx* c);
 int mlh_init_prefill_kernels(mlh_ctx* c);
 int mlh_build_gemm_operands(mlh_ctx* c); // at finalize: fp16 mirrors for bf16 models
-bool mlh_batch_step_applicable(const mlh_ctx* c, int nseq);
-int mlh_prepare_batch_step(mlh_ctx* c, int nseq);
-int mlh_launch_batch_step(mlh_ctx* c, int nseq, const int* tokPtr);
 int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_t* ids, const int32_t* lens, float* allLogits);
 int mlh_launch_softmax_rows(mlh_ctx* c, const float* logits, float* probs, const int* target, float* nll, int rows);
+
+// kernels_rows.hip: the decode step of up to 64 sequences
+bool mlh_rows_applicable(const mlh_ctx* c, int nseq);
+int mlh_rows_prepare(mlh_ctx* c);
+int mlh_rows_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool embedded, bool embedNext);
 
 // kernels_persistent.hip
 bool mlh_persistent_supported(const mlh_ctx* c);
