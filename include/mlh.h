@@ -137,10 +137,11 @@ int mlh_prefill_batch(mlh_ctx* ctx, int nseg, const int32_t* seqs, const int32_t
  * vocabScores_DEVICE / vocabScores_postSoftmax_DEVICE, inference.cu:723-749); either may be
  * null.  mean_nll (may be null) receives the mean over positions 0..n-2 of
  * -log max(p(ids[i+1] | ids[0..i]), 1e-4), the sequence loss processSequence prints
- * (training_orchestrator.cu:289-359, clamp at :343-347).  Allocates its own staging buffers per call. */
+ * (training_orchestrator.cu:289-359, clamp at :343-347).  Result buffers up to
+ * 512 MB stay with the context for the next call; from 4 MB of results on, four host threads live for the call. */
 int mlh_forward_full(mlh_ctx* ctx, int seq, const int32_t* ids, int n, float* logits_out, float* probs_out, float* mean_nll);
 
-/* 0 (default): GEMM prefill when the call has 16 or more tokens and dim, ffnDim,
+/* 0 (default): MFMA products when the call has two or more tokens and dim, ffnDim,
  * pleDim and the mixing widths are multiples of 32 (fp32) / 64 (bf16);
  * 1: always token by token through the decode kernels. */
 int mlh_set_prefill_mode(mlh_ctx* ctx, int mode);

@@ -14,9 +14,12 @@
 // weights are stored as three bf16 planes that add up to the fp32 value (p3.h).  Accumulation, the
 // residual stream, K/V and GDN states stay fp32.  This is what runInference(L) (inference.cu:376-751)
 // does for L columns, minus the columns that are already in the cache.
+#include <string.h>
+
 #include <algorithm>
 
 #include "mlh_internal.h"
+#include "sample.h"
 #include "p3.h"
 #include "sample.h"
 
@@ -46,6 +49,9 @@ struct PfArgs {
     void* U;           // [n, ffn]
     uint16_t* Kh;      // [n, dim] IEEE-half copies of this call's K and V rows (after norm and RoPE), or null: what the MFMA
     uint16_t* Vh;      //          attention reads when every segment starts at position 0 (all of its keys are rows of the call)
+    unsigned char* rows; // short calls: the mixing output goes into the planes of the row products (rows.h) instead of Amix
+    RowsLayout lay;
+    int half;            // bf16 weights
 };
 
 __device__ __forceinline__ float pf_wave_sum(float v) {
@@ -77,6 +83,11 @@ template <> __device__ __forceinline__ void put<f16_t>(f16_t* p, float v) { // s
 // element `col` of row `row` of a GEMM input matrix (leading dimension ld in elements; fp32 models: three bf16 planes, p3.h)
 template <typename AT> __device__ __forceinline__ void put_at(void* base, size_t row, int ld, int col, float v) { put<AT>((AT*)base + row * ld + col, v); }
 template <> __device__ __forceinline__ void put_at<p3_t>(void* base, size_t row, int ld, int col, float v) { p3_put((unsigned char*)base + row * ld * 6, col, v); }
+// element `col` of a token's mixing output (behind it: its PLE columns)
+template <typename AT> __device__ __forceinline__ void put_mix(const PfArgs& P, size_t row, int col, float v) {
+    if (P.rows) rows_put(P.rows, col, (int)row, P.lay, P.half != 0, v);
+    else put_at<AT>(P.Amix, row, P.aLd, col, v);
+}
 template <typename WT> __device__ __forceinline__ float getw(const WT* p);
 template <> __device__ __forceinline__ float getw<float>(const float* p) { return *p; }
 template <> __device__ __forceinline__ float getw<bf16_t>(const bf16_t* p) { return __uint_as_float(((uint32_t)*p) << 16); }
@@ -297,7 +308,7 @@ __global__ void __launch_bounds__(PWG) k_pf_attn(PfArgs P, LayerDev L) {
             const int dcol = h * HD + lane + 64 * ee;
             float v = acc[qq][ee] / l[qq];
             if (a.gating) v = v * pf_sigmoid(P.QKV[row * P.qkvLd + L.offG + dcol]);
-            put_at<AT>(P.Amix, row, P.aLd, dcol, v);
+            put_mix<AT>(P, row, dcol, v);
         }
     }
 }
@@ -561,6 +572,7 @@ __global__ void __launch_bounds__(PWG, H16 ? 2 : 1) k_pf_attn_mfma(PfArgs P, Lay
                 const f32x4 gt = *reinterpret_cast<const f32x4*>(P.QKV + row * P.qkvLd + L.offG + dcol);
                 o.x *= pf_sigmoid(gt.x); o.y *= pf_sigmoid(gt.y); o.z *= pf_sigmoid(gt.z); o.w *= pf_sigmoid(gt.w);
             }
+            if (P.rows) { rows_put4(P.rows, dcol, (int)row, P.lay, true, o.x, o.y, o.z, o.w); continue; }
             u32x2 w; w.x = pack_f16(o.x, o.y); w.y = pack_f16(o.z, o.w);
             *reinterpret_cast<u32x2*>((bf16_t*)P.Amix + row * P.aLd + dcol) = w;
         }
@@ -694,7 +706,7 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
             const float w = wn * rk * ainv;
 #pragma unroll
             for (int e = 0; e < CPT; e++) S[e] = fmaf(w, kk[e], S[e]);
-            if (cg == 0) put_at<AT>(P.Amix, (size_t)(row0 + t0 + c), P.aLd, h * DV + r0 + r, alpha * p + wn * kqn);
+            if (cg == 0) put_mix<AT>(P, (size_t)(row0 + t0 + c), h * DV + r0 + r, alpha * p + wn * kqn);
         }
     }
 #pragma unroll
@@ -1165,46 +1177,43 @@ __global__ void k_pf_ple(PfArgs P, LayerDev L) {
     const int row = blockIdx.x, j = threadIdx.x;
     if (j >= P.a.ple) return;
     const float g = P.QKV[(size_t)row * P.qkvLd + L.offPle + j];
-    put_at<AT>(P.Amix, (size_t)row, P.aLd, L.ad + j, pf_silu(g) * getw<WT>((const WT*)L.pleTable + (size_t)P.ids[row] * P.a.ple + j));
+    put_mix<AT>(P, (size_t)row, L.ad + j, pf_silu(g) * getw<WT>((const WT*)L.pleTable + (size_t)P.ids[row] * P.a.ple + j));
 }
 
-// residual of the last row of every segment -> decode slot buffer x[slot]
-__global__ void k_pf_gather_last(PfArgs P) {
-    const int seg = blockIdx.y, i = blockIdx.x * PWG + threadIdx.x;
-    if (i >= P.a.dim) return;
-    const int row = P.segStart[seg] + P.segLen[seg] - 1;
-    P.a.x[(size_t)seg * P.a.dim + i] = P.X[(size_t)row * P.a.dim + i];
-}
-
-// argmax over the LM-head partials of every segment's last row; sequence lengths advance by the segment length
-__global__ void __launch_bounds__(PWG) k_pf_finish(PfArgs P, int nparts, int* tokOut) {
+// One workgroup per segment: argmax over the LM head's partial maxima of its last row (lowest index on ties); the
+// sequence's length advances by the segment's.  picks: pinned host memory, by sequence.
+__global__ void __launch_bounds__(PWG) k_pf_finish(PfArgs P, int nparts, int* picks) {
     __shared__ float sv[PWG];
     __shared__ int si[PWG];
+    __shared__ double sd[PWG + 1];
     const StepArgs& a = P.a;
-    const int tid = threadIdx.x;
-    for (int seg = 0; seg < P.nseg; seg++) {
-        float v = -3.0e38f;
-        int idx = 0x7fffffff;
-        for (int i = tid; i < nparts; i += PWG) {
-            const float v2 = a.amaxVal[(size_t)seg * a.amaxParts + i];
-            const int i2 = a.amaxIdx[(size_t)seg * a.amaxParts + i];
-            if (v2 > v || (v2 == v && i2 < idx)) { v = v2; idx = i2; }
-        }
-        sv[tid] = v; si[tid] = idx;
+    const int tid = threadIdx.x, seg = blockIdx.x;
+    if (P.n < MLH_PREFILL_GEMM_MIN_ROWS && a.temperature > 0.f) { // short calls draw, as the decode step they take the place of does
+        const int seq = P.segSeq[seg], end = P.segPos0[seg] + P.segLen[seg];
+        const int nxt = mlh_sample_row<PWG>(a.logits + (size_t)seq * a.vocab, a.vocab, a.temperature, mlh_sample_uniform(a.sampleSeed, seq, end), sd, si);
+        if (tid == 0) { a.nextTok[seq] = nxt; picks[seq] = nxt; a.pos[seq] = end; }
+        return;
+    }
+    float v = -3.0e38f;
+    int idx = 0x7fffffff;
+    for (int i = tid; i < nparts; i += PWG) {
+        const float v2 = a.amaxVal[(size_t)seg * a.amaxParts + i];
+        const int i2 = a.amaxIdx[(size_t)seg * a.amaxParts + i];
+        if (v2 > v || (v2 == v && i2 < idx)) { v = v2; idx = i2; }
+    }
+    sv[tid] = v; si[tid] = idx;
+    __syncthreads();
+    for (int s = PWG / 2; s > 0; s >>= 1) {
+        if (tid < s && (sv[tid + s] > sv[tid] || (sv[tid + s] == sv[tid] && si[tid + s] < si[tid]))) { sv[tid] = sv[tid + s]; si[tid] = si[tid + s]; }
         __syncthreads();
-        for (int s = PWG / 2; s > 0; s >>= 1) {
-            if (tid < s && (sv[tid + s] > sv[tid] || (sv[tid + s] == sv[tid] && si[tid + s] < si[tid]))) { sv[tid] = sv[tid + s]; si[tid] = si[tid + s]; }
-            __syncthreads();
-        }
-        if (tid == 0) {
-            int nxt = si[0];
-            if (nxt < 0 || nxt >= a.vocab) nxt = 0;
-            const int seq = P.segSeq[seg];
-            tokOut[seg] = nxt;
-            a.nextTok[seq] = nxt;
-            a.pos[seq] += P.segLen[seg];
-        }
-        __syncthreads();
+    }
+    if (tid == 0) {
+        int nxt = si[0];
+        if (nxt < 0 || nxt >= a.vocab) nxt = 0; // only reachable with non-finite logits
+        const int seq = P.segSeq[seg];
+        a.nextTok[seq] = nxt;
+        picks[seq] = nxt;
+        a.pos[seq] += P.segLen[seg];
     }
 }
 
@@ -1365,6 +1374,7 @@ int mlh_init_prefill_kernels(mlh_ctx* c) {
     MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gdn_scan<128>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * GdLayout<128>::image));
     const int lds = (2 * 64 * 132 + PF_QB * 128) * 4;
     MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_attn<128, p3_t>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_attn<128, f16_t>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     return 0;
 }
 
@@ -1384,17 +1394,17 @@ static int ensure_prefill_buffers(mlh_ctx* c, int rows) {
         return 0;
     };
     int rc;
-    const int nblk = cdiv(rows, PF_QB) + hp.maxSeqs, nchunk = cdiv(rows, GD_C) + hp.maxSeqs;
+    const size_t nblk = cdiv(rows, PF_QB) + hp.maxSeqs, nchunk = cdiv(rows, GD_C) + hp.maxSeqs;
+    const size_t meta = 3 * n + 5 * (size_t)hp.maxSeqs + 2 * nblk + 2 * nchunk; // ids, sequence and position of every row; segments; attention blocks; GDN chunks
     if ((rc = alloc((void**)&c->pfX, n * hp.dim * 4)) || (rc = alloc(&c->pfXn, n * hp.dim * wb)) ||
         (rc = alloc((void**)&c->pfQKV, n * c->maxRowsA * 4)) || (rc = alloc(&c->pfA, n * (c->maxAd + hp.pleDim) * wb)) ||
         (rc = alloc((void**)&c->pfH1, n * hp.dim * 4)) ||
         (rc = alloc(&c->pfU, n * hp.ffnDim * wb)) ||
         (hp.weightDtype == MLH_DTYPE_BF16 && ((rc = alloc((void**)&c->pfKh, n * hp.dim * 2)) || (rc = alloc((void**)&c->pfVh, n * hp.dim * 2)))) ||
-        (rc = alloc((void**)&c->pfMeta, (3 * n + 4 * (size_t)hp.maxSeqs + 2 * (size_t)nblk + 2 * (size_t)nchunk + hp.maxSeqs) * 4)))
+        (rc = alloc((void**)&c->pfMeta, meta * 4)))
         return rc;
+    if ((rc = mlh_pin(c, c->pinMeta, meta * 4)) || (rc = mlh_pin(c, c->pinNext, (size_t)hp.maxSeqs * 4))) return rc;
     c->pfRows = rows;
-    c->pfBlkCap = nblk;
-    c->pfChunkCap = nchunk;
     return 0;
 }
 
@@ -1411,6 +1421,13 @@ static int ensure_gemm_workspace(mlh_ctx* c) {
 
 #define PF_DISPATCH_WT(c, expr_f32, expr_bf16) do { if ((c)->hp.weightDtype == MLH_DTYPE_BF16) { expr_bf16; } else { expr_f32; } } while (0)
 
+// Calls of up to this many tokens run through the row kernels: fewer launches (norms and embedding ride along) and, for bf16
+// models, fp32 precision of the activations.  Measured against the tiled products (us per call): 12 fp32 layers of dim 768, 5 / 16 / 64
+// tokens 461 / 510 / 771 -- 672 / 724 / 1012, and beyond 64 rows the weights would be fetched once more; 24 bf16 layers of dim 2048,
+// 16 / 32 / 48 tokens 1511 / 2155 / 3767 -- 1953 / 2255 / 2723: three plane products against one of halves.
+#define MLH_ROWS_PREFILL_F32 64
+#define MLH_ROWS_PREFILL_BF16 32
+
 // Appends lens[s] tokens to sequence seqs[s] for every segment s (token ids concatenated in `ids`).
 // allLogits: null, or a device buffer [rows, vocab] that receives the logits of every position.
 int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_t* ids, const int32_t* lens, float* allLogits) {
@@ -1420,25 +1437,32 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     int rc = ensure_prefill_buffers(c, n);
     if (rc == 0) rc = ensure_gemm_workspace(c);
     if (rc) return rc;
-    // ---- metadata ----
-    const bool mfmaAttn = hp.weightDtype == MLH_DTYPE_BF16; // bf16 models: bf16 MFMA attention, 128 queries per workgroup
+    const bool rowsPath = n <= (hp.weightDtype == MLH_DTYPE_F32 ? MLH_ROWS_PREFILL_F32 : MLH_ROWS_PREFILL_BF16);
+    // ---- metadata: laid out in pinned memory as on the device, one copy ----
+    // bf16 models: fp16 MFMA attention, 128 queries per workgroup; below 16 tokens as precise as the token-by-token path
+    const bool mfmaAttn = hp.weightDtype == MLH_DTYPE_BF16 && n >= MLH_PREFILL_GEMM_MIN_ROWS;
     const int qb = mfmaAttn ? PF_MQB : PF_QB;
-    std::vector<int> rowSeq(n), rowPos(n), segStart(nseg), segPos0(nseg), blkSeg, blkQ0, chunkSeg, chunkT0, chunkBase(nseg, 0);
-    bool anyGdn = false;
+    bool anyGdn = false, fresh = true; // fresh: every segment starts its sequence, all keys of the call are rows of the call
     for (const LayerDev& L : c->layers) anyGdn = anyGdn || L.kind == MLH_KIND_GDN;
-    const bool gdnChunked = anyGdn && c->pfDtype == MLH_GEMM_F16; // segments of 64 tokens or more: chunk-parallel MFMA path
-    int r = 0;
+    const bool gdnChunked = anyGdn && c->pfDtype == MLH_GEMM_F16 && !rowsPath; // segments of 64 tokens or more: chunk-parallel MFMA path
+    int nblk = 0, nchunk = 0;
     for (int s = 0; s < nseg; s++) {
-        segStart[s] = r;
-        segPos0[s] = c->h_len[seqs[s]];
-        for (int i = 0; i < lens[s]; i++, r++) { rowSeq[r] = seqs[s]; rowPos[r] = segPos0[s] + i; }
-        for (int q0 = 0; q0 < lens[s]; q0 += qb) { blkSeg.push_back(s); blkQ0.push_back(q0); }
-        chunkBase[s] = (int)chunkSeg.size();
-        if (gdnChunked && lens[s] >= GD_C)
-            for (int t0 = 0; t0 < lens[s]; t0 += GD_C) { chunkSeg.push_back(s); chunkT0.push_back(t0); }
+        nblk += cdiv(lens[s], qb);
+        if (gdnChunked && lens[s] >= GD_C) nchunk += cdiv(lens[s], GD_C);
     }
-    const int nblk = (int)blkSeg.size(), nchunk = (int)chunkSeg.size();
-    if (nblk > c->pfBlkCap) { c->err = "prefill: too many attention blocks"; return -1; }
+    int* const h = c->pinMeta.p;
+    int *h_ids = h, *h_rowSeq = h + n, *h_rowPos = h + 2 * n, *h_seg = h + 3 * n, *h_blk = h_seg + 5 * nseg, *h_chunk = h_blk + 2 * nblk;
+    const size_t metaInts = (size_t)(h_chunk - h) + 2 * (size_t)nchunk;
+    memcpy(h_ids, ids, (size_t)n * 4);
+    for (int s = 0, r = 0, b = 0, k = 0; s < nseg; s++) { // segStart, segLen, segSeq, segPos0, chunkBase; blkSeg, blkQ0; chunkSeg, chunkT0
+        const int pos0 = c->h_len[seqs[s]];
+        h_seg[s] = r; h_seg[nseg + s] = lens[s]; h_seg[2 * nseg + s] = seqs[s]; h_seg[3 * nseg + s] = pos0; h_seg[4 * nseg + s] = k;
+        fresh = fresh && pos0 == 0;
+        for (int q0 = 0; q0 < lens[s]; q0 += qb, b++) { h_blk[b] = s; h_blk[nblk + b] = q0; }
+        if (gdnChunked && lens[s] >= GD_C)
+            for (int t0 = 0; t0 < lens[s]; t0 += GD_C, k++) { h_chunk[k] = s; h_chunk[nchunk + k] = t0; }
+        for (int i = 0; i < lens[s]; i++, r++) { h_rowSeq[r] = seqs[s]; h_rowPos[r] = pos0 + i; }
+    }
     if (nchunk > 0) {
         const size_t per = (size_t)hp.gdnHeads * (hp.gdnDk == 64 ? GdLayout<64>::total : GdLayout<128>::total);
         if ((size_t)nchunk > c->pfGdnChunks) {
@@ -1450,41 +1474,22 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         }
     }
     int* d = c->pfMeta;
-    int* d_ids = d; int* d_rowSeq = d + n; int* d_rowPos = d + 2 * n;
-    int* d_seg = d + 3 * n; // segStart, segLen, segSeq, segPos0 (maxSeqs each)
-    int* d_blk = d_seg + 4 * hp.maxSeqs;
-    int* d_chunk = d_blk + 2 * c->pfBlkCap; // chunkSeg, chunkT0 (pfChunkCap each), chunkBase (maxSeqs)
+    int *d_seg = d + 3 * n, *d_blk = d_seg + 5 * nseg, *d_chunk = d_blk + 2 * nblk;
     hipStream_t st = c->stream;
-    MLH_CHECK(c, hipMemcpyAsync(d_ids, ids, (size_t)n * 4, hipMemcpyHostToDevice, st));
-    MLH_CHECK(c, hipMemcpyAsync(d_rowSeq, rowSeq.data(), (size_t)n * 4, hipMemcpyHostToDevice, st));
-    MLH_CHECK(c, hipMemcpyAsync(d_rowPos, rowPos.data(), (size_t)n * 4, hipMemcpyHostToDevice, st));
-    MLH_CHECK(c, hipMemcpyAsync(d_seg, segStart.data(), (size_t)nseg * 4, hipMemcpyHostToDevice, st));
-    MLH_CHECK(c, hipMemcpyAsync(d_seg + hp.maxSeqs, lens, (size_t)nseg * 4, hipMemcpyHostToDevice, st));
-    MLH_CHECK(c, hipMemcpyAsync(d_seg + 2 * hp.maxSeqs, seqs, (size_t)nseg * 4, hipMemcpyHostToDevice, st));
-    MLH_CHECK(c, hipMemcpyAsync(d_seg + 3 * hp.maxSeqs, segPos0.data(), (size_t)nseg * 4, hipMemcpyHostToDevice, st));
-    MLH_CHECK(c, hipMemcpyAsync(d_blk, blkSeg.data(), (size_t)nblk * 4, hipMemcpyHostToDevice, st));
-    MLH_CHECK(c, hipMemcpyAsync(d_blk + c->pfBlkCap, blkQ0.data(), (size_t)nblk * 4, hipMemcpyHostToDevice, st));
-    if (nchunk > 0) {
-        if (nchunk > c->pfChunkCap) { c->err = "prefill: too many GDN chunks"; return -1; }
-        MLH_CHECK(c, hipMemcpyAsync(d_chunk, chunkSeg.data(), (size_t)nchunk * 4, hipMemcpyHostToDevice, st));
-        MLH_CHECK(c, hipMemcpyAsync(d_chunk + c->pfChunkCap, chunkT0.data(), (size_t)nchunk * 4, hipMemcpyHostToDevice, st));
-        MLH_CHECK(c, hipMemcpyAsync(d_chunk + 2 * c->pfChunkCap, chunkBase.data(), (size_t)nseg * 4, hipMemcpyHostToDevice, st));
-    }
-    MLH_CHECK(c, hipMemcpyAsync(c->d_sidx, seqs, (size_t)nseg * 4, hipMemcpyHostToDevice, st));
-    MLH_CHECK(c, hipStreamSynchronize(st)); // the host vectors above go out of scope
-    c->identityNseq = 0;
+    MLH_CHECK(c, hipMemcpyAsync(d, h, metaInts * 4, hipMemcpyHostToDevice, st)); // (the call ends with a synchronisation: the pinned copy is free again)
 
     PfArgs P;
     mlh_fill_args(c, P.a, nseg, c->d_tok);
-    P.n = n; P.nseg = nseg; P.ids = d_ids; P.rowSeq = d_rowSeq; P.rowPos = d_rowPos;
-    P.segStart = d_seg; P.segLen = d_seg + hp.maxSeqs; P.segSeq = d_seg + 2 * hp.maxSeqs; P.segPos0 = d_seg + 3 * hp.maxSeqs;
-    P.blkSeg = d_blk; P.blkQ0 = d_blk + c->pfBlkCap;
+    P.n = n; P.nseg = nseg; P.ids = d; P.rowSeq = d + n; P.rowPos = d + 2 * n;
+    P.segStart = d_seg; P.segLen = d_seg + nseg; P.segSeq = d_seg + 2 * nseg; P.segPos0 = d_seg + 3 * nseg;
+    P.blkSeg = d_blk; P.blkQ0 = d_blk + nblk;
     P.X = c->pfX; P.Xn = c->pfXn; P.QKV = c->pfQKV; P.qkvLd = c->maxRowsA; P.Amix = c->pfA; P.aLd = c->maxAd + hp.pleDim;
     P.H1 = c->pfH1; P.U = c->pfU;
-    bool fresh = true; // every segment starts its sequence: all keys of the call are rows of the call
-    for (int s = 0; s < nseg; s++) fresh = fresh && segPos0[s] == 0;
     P.Kh = mfmaAttn && fresh ? c->pfKh : nullptr;
     P.Vh = mfmaAttn && fresh ? c->pfVh : nullptr;
+    P.lay = rows_layout(std::min(n, 64)); P.rows = rowsPath ? c->rowsMix : nullptr; P.half = hp.weightDtype == MLH_DTYPE_BF16;
+    RowsArgs base = {};
+    base.M = n; base.lay = P.lay; base.normDim = hp.dim;
     const int d_ = hp.dim, F = hp.ffnDim, dt = c->pfDtype;
 #define GEMM(A, lda, B, alpha, ldb, C, ldc, R, ldr, M, N, K)                                                \
     do {                                                                                                    \
@@ -1492,23 +1497,32 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; } \
     } while (0)
 
-    PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_embed<float>), dim3(cdiv(d_, PWG), n), dim3(PWG), 0, st, P),
+    if (rowsPath) mlh_rows_embed(c, P.ids, n, P.X, P.lay);
+    else PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_embed<float>), dim3(cdiv(d_, PWG), n), dim3(PWG), 0, st, P),
                    hipLaunchKernelGGL((k_pf_embed<bf16_t>), dim3(cdiv(d_, PWG), n), dim3(PWG), 0, st, P));
     for (int t = hp.transformers - 1; t >= 0; t--) { // file block 0 is the top (inference.cu:384-385)
         const LayerDev& L = c->layers[t];
-        PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<p3_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, L.g1, P.Xn, n, d_),
-                       hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, L.g1, P.Xn, n, d_));
-        GEMM(P.Xn, d_, L.WaP, L.sWa, d_, P.QKV, P.qkvLd, nullptr, 0, n, L.rowsA, d_);
+        if (rowsPath) {
+            RowsArgs R = base;
+            R.K = d_; R.A = c->rowsX; R.ssqIn = c->rowsSsqX; R.nparts = t == hp.transformers - 1 ? 1 : d_ / RW_TILE; R.C = P.QKV; R.ldc = P.qkvLd;
+            mlh_rows_gemm(c, RW_PLAIN, L.WaR, L.rowsA, R);
+        } else {
+            PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<p3_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, L.g1, P.Xn, n, d_),
+                           hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, L.g1, P.Xn, n, d_));
+            GEMM(P.Xn, d_, L.WaP, L.sWa, d_, P.QKV, P.qkvLd, nullptr, 0, n, L.rowsA, d_);
+        }
         if (L.kind == MLH_KIND_ATTENTION) {
             if (hp.headDim == 64) {
                 hipLaunchKernelGGL((k_pf_qk_rope_kv<64>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<64, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<64, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
+                else if (P.half) hipLaunchKernelGGL((k_pf_attn<64, f16_t>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 68 + PF_QB * 64) * 4, st, P, L);
                 else hipLaunchKernelGGL((k_pf_attn<64, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 68 + PF_QB * 64) * 4, st, P, L);
             } else {
                 hipLaunchKernelGGL((k_pf_qk_rope_kv<128>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<128, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<128, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
+                else if (P.half) hipLaunchKernelGGL((k_pf_attn<128, f16_t>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 132 + PF_QB * 128) * 4, st, P, L);
                 else hipLaunchKernelGGL((k_pf_attn<128, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 132 + PF_QB * 128) * 4, st, P, L);
             }
         } else {
@@ -1522,7 +1536,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
                                hipLaunchKernelGGL((k_pf_gdn<128, f16_t>), gr, dim3(PWG), 0, st, P, L, skipFrom));
             }
             if (nchunk > 0) {
-                const int* dcs = d_chunk; const int* dct = d_chunk + c->pfChunkCap; const int* dcb = d_chunk + 2 * c->pfChunkCap;
+                const int *dcs = d_chunk, *dct = d_chunk + nchunk, *dcb = d_seg + 4 * nseg;
                 if (hp.gdnDk == 64) {
                     hipLaunchKernelGGL((k_gdn_prep<64>), dim3(nchunk, hp.gdnHeads), dim3(128), gdn_prep_lds(64), st, P, L, dcs, dct, (unsigned char*)c->pfGdnWs, c->pfGdnG);
                     hipLaunchKernelGGL((k_gdn_scan<64>), dim3(hp.gdnHeads, nseg), dim3(128), (size_t)2 * GdLayout<64>::image, st, P, L, dcb, (const unsigned char*)c->pfGdnWs, c->pfGdnG);
@@ -1535,6 +1549,10 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         if (hp.pleDim > 0)
             PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_ple<float, p3_t>), dim3(n), dim3(std::max(64, hp.pleDim)), 0, st, P, L),
                            hipLaunchKernelGGL((k_pf_ple<bf16_t, f16_t>), dim3(n), dim3(std::max(64, hp.pleDim)), 0, st, P, L));
+        if (rowsPath) {
+            mlh_rows_rest_of_layer(c, t, base, P.X, P.H1);
+            continue;
+        }
         GEMM(P.Amix, P.aLd, L.WoP, L.sWo, L.ad + hp.pleDim, P.H1, d_, P.X, d_, n, d_, L.ad + hp.pleDim); // Wo . a + pleUp . e + x
         PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<p3_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.H1, L.g2, P.Xn, n, d_),
                        hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.H1, L.g2, P.Xn, n, d_));
@@ -1545,18 +1563,26 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         GEMM(P.U, F, L.W2P, L.sW2, F, P.X, d_, P.H1, d_, n, d_, F);
     }
 #undef GEMM
-    if (allLogits) { // final RMSNorm + tied LM head for every row (inference.cu:705-743 computes all L columns)
+    if (allLogits && rowsPath) { // tied LM head of every normalised row (inference.cu:705-743 computes all L columns)
+        RowsArgs R = base;
+        R.K = d_; R.A = c->rowsX; R.ssqIn = c->rowsSsqX; R.nparts = d_ / RW_TILE; R.C = allLogits; R.ldc = hp.vocabSize;
+        mlh_rows_gemm(c, RW_PLAIN, c->ER, hp.vocabSize, R);
+    } else if (allLogits) {
         PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<p3_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, c->gF, P.Xn, n, d_),
                        hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, c->gF, P.Xn, n, d_));
         hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, P.Xn, d_, c->EP, d_, allLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_, c->gemmWs, c->sE);
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
     }
-    hipLaunchKernelGGL(k_pf_gather_last, dim3(cdiv(d_, PWG), nseg), dim3(PWG), 0, st, P);
-    if ((rc = mlh_launch_one(c, MLH_K_LMHEAD, 0, nseg))) return rc;
-    hipLaunchKernelGGL(k_pf_finish, dim3(1), dim3(PWG), 0, st, P, c->amaxParts, c->d_tok);
+    for (int s0 = 0; s0 < nseg; s0 += 64)
+        mlh_rows_lm_head(c, std::min(64, nseg - s0), P.X, P.segStart + s0, P.segLen + s0, P.segSeq + s0, c->amaxVal + (size_t)s0 * c->amaxParts, c->amaxIdx + (size_t)s0 * c->amaxParts);
+    hipLaunchKernelGGL(k_pf_finish, dim3(nseg), dim3(PWG), 0, st, P, cdiv(hp.vocabSize, RW_TILE), c->pinNext.p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { c->err = std::string("prefill launch: ") + hipGetErrorString(e); return -2; }
     MLH_CHECK(c, hipStreamSynchronize(st));
-    for (int s = 0; s < nseg; s++) c->h_len[seqs[s]] += lens[s];
+    for (int s = 0; s < nseg; s++) {
+        c->h_len[seqs[s]] += lens[s];
+        c->h_next[seqs[s]] = c->pinNext.p[seqs[s]];
+        c->h_nextKnown[seqs[s]] = 1;
+    }
     return 0;
 }

@@ -27,29 +27,6 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 #define RW_WAVES 8
 #define RW_THREADS (RW_WAVES * 64)
-#define RW_TILE 16 // weight rows per workgroup
-enum { RW_PLAIN, RW_RESID, RW_SWIGLU, RW_LOGITS };
-
-struct RowsArgs {
-    const unsigned char* W;         // in fetch order (rows.h)
-    int M, N, K, tiles;
-    RowsLayout lay;                 // of the plane buffers
-    const unsigned char* A;         // planes of the input rows
-    const float* ssqIn;             // [nparts][64] partial sums of squares of the rows behind A, or null: no normalisation
-    int nparts, normDim;
-    float* C;                       // RW_PLAIN, RW_RESID: [M, ldc] fp32; RW_LOGITS: row sidx[m] of [*, ldc]
-    int ldc;
-    const float* R;                 // RW_RESID: added to the product, [M, ldc]
-    unsigned char* out;             // RW_RESID: planes of outGain (.) C; RW_SWIGLU: planes of silu(gate) * up
-    const float* outGain;
-    float* ssqOut;                  // RW_RESID: [workgroup][64]
-    const int* sidx;
-    float* amaxVal;                 // RW_LOGITS: [M, amaxParts] largest logit of each workgroup's rows and its index
-    int* amaxIdx;
-    int amaxParts;
-    int* stepCounter;               // RW_LOGITS: counted up once
-};
-
 template <typename WT> struct RowsW;
 template <> struct RowsW<float> {
     static constexpr int KE = 32, SUB = 1; // K per chunk, 32-wide steps per chunk
@@ -182,7 +159,7 @@ __device__ __forceinline__ void rows_epilogue(const RowsArgs& P, const RowsShare
                     if (n + e < P.N) c[e] = v[e];
         }
         if (EPI == RW_LOGITS) { // largest of the 16 rows, lowest index on ties
-            if (tile == 0 && tb0 == 0 && threadIdx.x == 0) *P.stepCounter += 1; // steps begun: the finish logs into row (counter - 1)
+            if (P.stepCounter && tile == 0 && tb0 == 0 && threadIdx.x == 0) *P.stepCounter += 1; // steps begun: the finish logs into row (counter - 1)
             float best = -3.0e38f;
             int bi = 0x7fffffff;
 #pragma unroll
@@ -340,25 +317,26 @@ template <typename WT> __device__ __forceinline__ float rw_get(const WT* p);
 template <> __device__ __forceinline__ float rw_get<float>(const float* p) { return *p; }
 template <> __device__ __forceinline__ float rw_get<bf16_t>(const bf16_t* p) { return __uint_as_float(((uint32_t)*p) << 16); }
 
-struct RowsEmbed { // what the embedding of a row writes besides the residual row itself
+struct RowsEmbed { // what the embedding of a row writes
+    float* x;           // residual rows
     unsigned char* out; // planes of gain (.) row
     const float* gain;  // of the first applied layer
     float* ssq;         // partial sums of squares [.][64]: the row's whole sum in the first
     RowsLayout lay;
 };
 
-// residual row of token id `tok` for `slot`: every thread of a 256-thread workgroup calls it (inference.cu:9-22)
-template <typename WT>
-__device__ __forceinline__ void rows_embed(const StepArgs& a, const RowsEmbed& e, int slot, int tok, float* sh) {
+// Residual row `slot` from the fp32 or weight-typed row src: its copy, its planes and its sum of squares.  Every thread of a
+// 256-thread workgroup calls it; half: bf16 weights.
+template <typename ST>
+__device__ __forceinline__ void rows_begin(const RowsEmbed& e, int dim, bool half, int slot, const ST* src, float* sh) {
     const int tid = threadIdx.x;
-    const WT* src = (const WT*)a.E + (size_t)tok * a.dim;
     float s = 0.f;
-    for (int i = tid * 4; i < a.dim; i += 1024) {
+    for (int i = tid * 4; i < dim; i += 1024) {
         f32x4 v;
-        v.x = rw_get<WT>(src + i); v.y = rw_get<WT>(src + i + 1); v.z = rw_get<WT>(src + i + 2); v.w = rw_get<WT>(src + i + 3);
-        *reinterpret_cast<f32x4*>(a.x + (size_t)slot * a.dim + i) = v;
+        v.x = rw_get<ST>(src + i); v.y = rw_get<ST>(src + i + 1); v.z = rw_get<ST>(src + i + 2); v.w = rw_get<ST>(src + i + 3);
+        if (e.x) *reinterpret_cast<f32x4*>(e.x + (size_t)slot * dim + i) = v;
         const f32x4 g = *reinterpret_cast<const f32x4*>(e.gain + i);
-        rows_put4(e.out, i, slot, e.lay, sizeof(WT) == 2, g.x * v.x, g.y * v.y, g.z * v.z, g.w * v.w);
+        rows_put4(e.out, i, slot, e.lay, half, g.x * v.x, g.y * v.y, g.z * v.z, g.w * v.w);
         s = fmaf(v.x, v.x, s); s = fmaf(v.y, v.y, s); s = fmaf(v.z, v.z, s); s = fmaf(v.w, v.w, s);
     }
 #pragma unroll
@@ -368,10 +346,17 @@ __device__ __forceinline__ void rows_embed(const StepArgs& a, const RowsEmbed& e
     if (tid == 0) e.ssq[slot] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
+// the embedding of a token (inference.cu:9-22)
 template <typename WT>
 __global__ void __launch_bounds__(256) k_rows_embed(StepArgs a, RowsEmbed e) {
     __shared__ float sh[4];
-    rows_embed<WT>(a, e, blockIdx.x, a.tok[blockIdx.x], sh);
+    rows_begin<WT>(e, a.dim, sizeof(WT) == 2, blockIdx.x, (const WT*)a.E + (size_t)a.tok[blockIdx.x] * a.dim, sh);
+}
+
+// the last row of every segment of a prefill, for the LM head: segment seg0 + x becomes row x
+__global__ void __launch_bounds__(256) k_rows_last(RowsEmbed e, const float* X, int dim, bool half, const int* segStart, const int* segLen) {
+    __shared__ float sh[4];
+    rows_begin<float>(e, dim, half, blockIdx.x, X + (size_t)(segStart[blockIdx.x] + segLen[blockIdx.x] - 1) * dim, sh);
 }
 
 // Attention over several workgroups per (head, sequence): their partial results combined, gated (inference.cu:241-250) and,
@@ -441,7 +426,7 @@ __global__ void __launch_bounds__(256) k_rows_finish(StepArgs a, RowsEmbed e, in
         if (step >= 0 && step < a.outCapacity) a.outIds[(size_t)step * a.nseq + slot] = nxt;
         a.pos[seq] += 1;
     }
-    if (embedNext) rows_embed<WT>(a, e, slot, nxt, sv);
+    if (embedNext) rows_begin<WT>(e, a.dim, sizeof(WT) == 2, slot, (const WT*)a.E + (size_t)nxt * a.dim, sv);
 }
 
 __global__ void k_rows_advance(StepArgs a) { // a token that needs no logits
@@ -487,63 +472,95 @@ int mlh_rows_prepare(mlh_ctx* c) {
     return 0;
 }
 
+void mlh_rows_gemm(mlh_ctx* c, int epi, const void* w, int n, RowsArgs P) {
+    P.W = (const unsigned char*)w; P.N = n; P.tiles = (n + RW_TILE - 1) / RW_TILE;
+    const bool half = c->hp.weightDtype == MLH_DTYPE_BF16;
+#define ROWS_EPI(E_) do { if (half) launch_rows<bf16_t, E_>(c->stream, P, c->numCUs); else launch_rows<float, E_>(c->stream, P, c->numCUs); } while (0)
+    if (epi == RW_PLAIN) ROWS_EPI(RW_PLAIN);
+    else if (epi == RW_RESID) ROWS_EPI(RW_RESID);
+    else if (epi == RW_SWIGLU) ROWS_EPI(RW_SWIGLU);
+    else ROWS_EPI(RW_LOGITS);
+#undef ROWS_EPI
+}
+
+// Output projection, gate / up and down projection of file block t over the rows of `base`: residual rows x -> h1 -> x.
+void mlh_rows_rest_of_layer(mlh_ctx* c, int t, const RowsArgs& base, float* x, float* h1) {
+    const mlh_hparams& hp = c->hp;
+    const LayerDev& L = c->layers[t];
+    const int d = hp.dim, F = hp.ffnDim;
+    RowsArgs P = base; // h1 = [Wo | pleUp] . [mix | e] + x (inference.cu:582-610)
+    P.K = L.ad + hp.pleDim; P.A = c->rowsMix; P.C = h1; P.ldc = d; P.R = x; P.out = c->rowsH; P.outGain = L.g2; P.ssqOut = c->rowsSsqH;
+    mlh_rows_gemm(c, RW_RESID, L.WoR, d, P);
+    P = base; // silu(gate) * up of the normalised rows (inference.cu:612-672)
+    P.K = d; P.A = c->rowsH; P.ssqIn = c->rowsSsqH; P.nparts = d / RW_TILE; P.out = c->rowsU;
+    mlh_rows_gemm(c, RW_SWIGLU, L.W13R, 2 * F, P);
+    P = base; // x = W2 . u + h1 (inference.cu:675-699), and the planes for the next layer's first product or the LM head
+    P.K = F; P.A = c->rowsU; P.C = x; P.ldc = d; P.R = h1; P.out = c->rowsX; P.outGain = t > 0 ? c->layers[t - 1].g1 : c->gF; P.ssqOut = c->rowsSsqX;
+    mlh_rows_gemm(c, RW_RESID, L.W2R, d, P);
+}
+
+void mlh_rows_embed(mlh_ctx* c, const int* tok, int n, float* x, RowsLayout lay) {
+    StepArgs a;
+    mlh_fill_args(c, a, n, tok);
+    const RowsEmbed emb = {x, c->rowsX, c->layers[c->hp.transformers - 1].g1, c->rowsSsqX, lay};
+    if (c->hp.weightDtype == MLH_DTYPE_BF16) hipLaunchKernelGGL((k_rows_embed<bf16_t>), dim3(n), dim3(256), 0, c->stream, a, emb);
+    else hipLaunchKernelGGL((k_rows_embed<float>), dim3(n), dim3(256), 0, c->stream, a, emb);
+}
+
+// Final norm and LM head of the last row of each of n <= 64 segments: logits of sequence segSeq[i], partial maxima of slot i.
+void mlh_rows_lm_head(mlh_ctx* c, int n, const float* X, const int* segStart, const int* segLen, const int* segSeq, float* amaxVal, int* amaxIdx) {
+    const mlh_hparams& hp = c->hp;
+    const RowsLayout lay = rows_layout(n);
+    const RowsEmbed emb = {nullptr, c->rowsX, c->gF, c->rowsSsqX, lay};
+    hipLaunchKernelGGL(k_rows_last, dim3(n), dim3(256), 0, c->stream, emb, X, hp.dim, hp.weightDtype == MLH_DTYPE_BF16, segStart, segLen);
+    RowsArgs P = {};
+    P.M = n; P.K = hp.dim; P.lay = lay; P.normDim = hp.dim; P.A = c->rowsX; P.ssqIn = c->rowsSsqX; P.nparts = 1; P.C = c->logits; P.ldc = hp.vocabSize;
+    P.sidx = segSeq; P.amaxVal = amaxVal; P.amaxIdx = amaxIdx; P.amaxParts = c->amaxParts;
+    mlh_rows_gemm(c, RW_LOGITS, c->ER, hp.vocabSize, P);
+}
+
 // One step of nseq sequences on the context's stream (no allocation, no synchronisation: can be captured).  embedded: the step
 // before it has already written the residual rows; embedNext: this one does that for the next.
-template <typename WT>
-static int rows_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool embedded, bool embedNext) {
+int mlh_rows_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool embedded, bool embedNext) {
+    if (!c->rowsBuf) { c->err = "row step buffers not prepared"; return -1; }
     const mlh_hparams& hp = c->hp;
     hipStream_t st = c->stream;
     const RowsLayout lay = rows_layout(nseq);
-    const int first = hp.transformers - 1, d = hp.dim, F = hp.ffnDim, cus = c->numCUs;
+    const int first = hp.transformers - 1, d = hp.dim;
     c->mixRows = c->rowsMix;
     c->mixLay = lay;
     StepArgs a;
     mlh_fill_args(c, a, nseq, tokPtr);
-    const RowsEmbed emb = {c->rowsX, c->layers[first].g1, c->rowsSsqX, lay};
-    if (!embedded) hipLaunchKernelGGL((k_rows_embed<WT>), dim3(nseq), dim3(256), 0, st, a, emb);
+    if (!embedded) mlh_rows_embed(c, tokPtr, nseq, c->x, lay);
     RowsArgs base = {};
     base.M = nseq; base.lay = lay; base.normDim = d; base.sidx = c->d_sidx;
-    auto set_w = [](RowsArgs& P, const void* w, int n) { P.W = (const unsigned char*)w; P.N = n; P.tiles = (n + RW_TILE - 1) / RW_TILE; };
     int nparts = 1; // partial sums behind rowsX: one from the embedding, one per workgroup from a down projection
     int rc = 0;
     for (int t = first; t >= 0 && rc == 0; t--) { // file block 0 is the top (inference.cu:384-385)
         const LayerDev& L = c->layers[t];
         RowsArgs P = base; // q | k | v | ... of the normalised rows (inference.cu:388-465, 487-507)
-        set_w(P, L.WaR, L.rowsA); P.K = d; P.A = c->rowsX; P.ssqIn = c->rowsSsqX; P.nparts = nparts; P.C = c->qkv; P.ldc = c->maxRowsA;
-        launch_rows<WT, RW_PLAIN>(st, P, cus);
+        P.K = d; P.A = c->rowsX; P.ssqIn = c->rowsSsqX; P.nparts = nparts; P.C = c->qkv; P.ldc = c->maxRowsA;
+        mlh_rows_gemm(c, RW_PLAIN, L.WaR, L.rowsA, P);
         rc = mlh_launch_mix(c, a, L);
         if (L.kind == MLH_KIND_ATTENTION && c->nsplit > 1) hipLaunchKernelGGL(k_rows_mix, dim3(nseq, (L.ad + hp.pleDim + 255) / 256), dim3(256), 0, st, a, L);
-        P = base; // h1 = [Wo | pleUp] . [mix | e] + x (inference.cu:582-610)
-        set_w(P, L.WoR, d); P.K = L.ad + hp.pleDim; P.A = c->rowsMix; P.C = c->h1; P.ldc = d; P.R = c->x;
-        P.out = c->rowsH; P.outGain = L.g2; P.ssqOut = c->rowsSsqH;
-        launch_rows<WT, RW_RESID>(st, P, cus);
-        P = base; // silu(gate) * up of the normalised rows (inference.cu:612-672)
-        set_w(P, L.W13R, 2 * F); P.K = d; P.A = c->rowsH; P.ssqIn = c->rowsSsqH; P.nparts = d / RW_TILE; P.out = c->rowsU;
-        launch_rows<WT, RW_SWIGLU>(st, P, cus);
-        P = base; // x = W2 . u + h1 (inference.cu:675-699), and the planes for the next layer's first product or the LM head
-        set_w(P, L.W2R, d); P.K = F; P.A = c->rowsU; P.C = c->x; P.ldc = d; P.R = c->h1;
-        P.out = c->rowsX; P.outGain = t > 0 ? c->layers[t - 1].g1 : c->gF; P.ssqOut = c->rowsSsqX;
-        launch_rows<WT, RW_RESID>(st, P, cus);
+        mlh_rows_rest_of_layer(c, t, base, c->x, c->h1);
         nparts = d / RW_TILE;
     }
     c->mixRows = nullptr;
     if (rc) return rc;
     if (lmHead) { // tied LM head of the normalised rows (inference.cu:705-743)
         RowsArgs P = base;
-        set_w(P, c->ER, hp.vocabSize); P.K = d; P.A = c->rowsX; P.ssqIn = c->rowsSsqX; P.nparts = nparts; P.C = c->logits; P.ldc = hp.vocabSize;
+        P.K = d; P.A = c->rowsX; P.ssqIn = c->rowsSsqX; P.nparts = nparts; P.C = c->logits; P.ldc = hp.vocabSize;
         P.amaxVal = c->amaxVal; P.amaxIdx = c->amaxIdx; P.amaxParts = c->amaxParts; P.stepCounter = c->d_stepCounter;
-        launch_rows<WT, RW_LOGITS>(st, P, cus);
-        hipLaunchKernelGGL((k_rows_finish<WT>), dim3(nseq), dim3(256), 0, st, a, emb, (hp.vocabSize + RW_TILE - 1) / RW_TILE, c->d_tok, embedNext ? 1 : 0);
+        mlh_rows_gemm(c, RW_LOGITS, c->ER, hp.vocabSize, P);
+        const RowsEmbed emb = {c->x, c->rowsX, c->layers[first].g1, c->rowsSsqX, lay};
+        const int np = (hp.vocabSize + RW_TILE - 1) / RW_TILE, next = embedNext ? 1 : 0;
+        if (hp.weightDtype == MLH_DTYPE_BF16) hipLaunchKernelGGL((k_rows_finish<bf16_t>), dim3(nseq), dim3(256), 0, st, a, emb, np, c->d_tok, next);
+        else hipLaunchKernelGGL((k_rows_finish<float>), dim3(nseq), dim3(256), 0, st, a, emb, np, c->d_tok, next);
     } else {
         hipLaunchKernelGGL(k_rows_advance, dim3(1), dim3(64), 0, st, a);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) { c->err = std::string("row step launch: ") + hipGetErrorString(e); return -2; }
     return 0;
-}
-
-int mlh_rows_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool embedded, bool embedNext) {
-    if (!c->rowsBuf) { c->err = "row step buffers not prepared"; return -1; }
-    return c->hp.weightDtype == MLH_DTYPE_BF16 ? rows_step<bf16_t>(c, nseq, tokPtr, lmHead, embedded, embedNext)
-                                               : rows_step<float>(c, nseq, tokPtr, lmHead, embedded, embedNext);
 }

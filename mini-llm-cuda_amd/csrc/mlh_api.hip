@@ -7,6 +7,7 @@
 #include <algorithm>
 
 #include "mlh_internal.h"
+#include "readback.h"
 
 static thread_local std::string g_create_error;
 
@@ -38,6 +39,16 @@ int mlh_dev_alloc_bytes(mlh_ctx* c, void** p, size_t bytes) {
     MLH_CHECK(c, hipMalloc(&q, bytes));
     c->allocs.push_back(q);
     *p = q;
+    return 0;
+}
+
+int mlh_pin(mlh_ctx* c, PinBuf& b, size_t bytes) {
+    if (bytes <= b.bytes) return 0;
+    MLH_CHECK(c, hipStreamSynchronize(c->stream));
+    if (b.p) (void)hipHostFree(b.p);
+    b = PinBuf();
+    MLH_CHECK(c, hipHostMalloc((void**)&b.p, bytes));
+    b.bytes = bytes;
     return 0;
 }
 
@@ -92,6 +103,8 @@ extern "C" void mlh_destroy(mlh_ctx* c) {
     for (void* p : c->mirrorAllocs) (void)hipFree(p);
     if (c->pfGdnWs) (void)hipFree(c->pfGdnWs);
     if (c->pfGdnG) (void)hipFree(c->pfGdnG);
+    if (c->fullBuf) (void)hipFree(c->fullBuf);
+    for (PinBuf* b : {&c->pinIo, &c->pinMeta, &c->pinNext, &c->pinStage}) if (b->p) (void)hipHostFree(b->p);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -240,6 +253,9 @@ extern "C" int mlh_create(const mlh_hparams* hpIn, int device, mlh_ctx** out) {
         return bail(-2);
     }
     c->h_len.assign(S, 0);
+    c->h_dirty.assign(S, 0);
+    c->h_nextKnown.assign(S, 0);
+    c->h_next.assign(S, 0);
     *out = c;
     return 0;
 }
@@ -410,18 +426,40 @@ static int check_ready(mlh_ctx* c) {
     return 0;
 }
 
+// A launch may change the lengths, GDN states and next tokens of sequences [s0, s1): called before any such launch.
+static void touch(mlh_ctx* c, int s0, int s1) {
+    for (int s = s0; s < s1; s++) { c->h_dirty[s] = 1; c->h_nextKnown[s] = 0; }
+}
+
+// grid: pieces of a sequence's states, layers, sequences
+__global__ void __launch_bounds__(256) k_reset(const LayerDev* layers, int* pos, int s0, size_t per4) {
+    const int seq = s0 + blockIdx.z;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) pos[seq] = 0;
+    float4* S = reinterpret_cast<float4*>(layers[blockIdx.y].S);
+    if (!S) return;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < per4; i += (size_t)gridDim.x * 256) S[seq * per4 + i] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// One launch per run of sequences in use, ordered on the context's stream and not waited for (64 sequences of 9 GDN layers: 9
+// fills of 25 us and their gaps before).
 extern "C" int mlh_reset(mlh_ctx* c, int seq) {
     if (!c) return -1;
     (void)hipSetDevice(c->device);
     const mlh_hparams& hp = c->hp;
     if (seq < -1 || seq >= hp.maxSeqs) { c->err = "sequence index out of range"; return -1; }
     const int s0 = seq < 0 ? 0 : seq, s1 = seq < 0 ? hp.maxSeqs : seq + 1;
-    MLH_CHECK(c, hipStreamSynchronize(c->stream));
-    MLH_CHECK(c, hipMemset(c->d_pos + s0, 0, (size_t)(s1 - s0) * 4));
-    const size_t per = (size_t)hp.gdnHeads * hp.gdnDk * hp.gdnDv;
-    for (int t = 0; t < hp.transformers; t++)
-        if (c->layers[t].S) MLH_CHECK(c, hipMemset(c->layers[t].S + s0 * per, 0, (s1 - s0) * per * 4));
-    for (int s = s0; s < s1; s++) c->h_len[s] = 0;
+    bool gdn = false;
+    for (const LayerDev& L : c->layers) gdn = gdn || L.S;
+    const size_t per4 = (size_t)hp.gdnHeads * hp.gdnDk * hp.gdnDv / 4; // (dk and dv: 64 or 128)
+    for (int s = s0; s < s1;) {
+        if (!c->h_dirty[s]) { s++; continue; }
+        int e = s;
+        while (e < s1 && c->h_dirty[e] && e - s < 65535) e++;
+        hipLaunchKernelGGL(k_reset, dim3(gdn ? (unsigned)std::min<size_t>(16, (per4 + 255) / 256) : 1, gdn ? hp.transformers : 1, e - s), dim3(256), 0, c->stream,
+                           c->d_layers, c->d_pos, s, per4);
+        MLH_CHECK(c, hipGetLastError());
+        for (; s < e; s++) { c->h_len[s] = 0; c->h_dirty[s] = 0; }
+    }
     return 0;
 }
 
@@ -436,9 +474,13 @@ extern "C" int mlh_vocab_size(const mlh_ctx* c) { return c ? c->hp.vocabSize : -
 extern "C" int mlh_greedy_token(mlh_ctx* c, int seq, int32_t* id) {
     if (!c) return -1;
     if (seq < 0 || seq >= c->hp.maxSeqs || !id) { c->err = "bad argument"; return -1; }
-    (void)hipSetDevice(c->device);
-    MLH_CHECK(c, hipStreamSynchronize(c->stream));
-    MLH_CHECK(c, hipMemcpy(id, c->d_next + seq, 4, hipMemcpyDeviceToHost));
+    if (!c->h_nextKnown[seq]) {
+        (void)hipSetDevice(c->device);
+        MLH_CHECK(c, hipStreamSynchronize(c->stream));
+        MLH_CHECK(c, hipMemcpy(&c->h_next[seq], c->d_next + seq, 4, hipMemcpyDeviceToHost));
+        c->h_nextKnown[seq] = 1;
+    }
+    *id = c->h_next[seq];
     return 0;
 }
 
@@ -473,9 +515,6 @@ static int set_identity_slots(mlh_ctx* c, int nseq) {
     return set_slots(c, id.data(), nseq);
 }
 
-// Below this many rows the GEMM tiles are mostly padding and the decode kernels are faster.
-#define MLH_PREFILL_GEMM_MIN_ROWS 16
-
 static int prefill_token_by_token(mlh_ctx* c, int seq, const int32_t* ids, int n) {
     int rc;
     if ((rc = set_slots(c, &seq, 1))) return rc;
@@ -503,7 +542,8 @@ extern "C" int mlh_prefill_batch(mlh_ctx* c, int nseg, const int32_t* seqs, cons
     }
     for (long i = 0; i < total; i++)
         if (ids[i] < 0 || ids[i] >= hp.vocabSize) { c->err = "token id out of range"; return -1; }
-    if (c->prefillMode == 0 && total >= MLH_PREFILL_GEMM_MIN_ROWS && mlh_prefill_gemm_supported(c))
+    for (int s = 0; s < nseg; s++) touch(c, seqs[s], seqs[s] + 1);
+    if (c->prefillMode == 0 && total > 1 && mlh_prefill_gemm_supported(c)) // (a single token: the decode step, which splits the keys)
         return mlh_run_prefill_gemm(c, nseg, seqs, ids, lens, nullptr);
     long off = 0;
     for (int s = 0; s < nseg; s++) {
@@ -529,40 +569,53 @@ extern "C" int mlh_forward_full(mlh_ctx* c, int seq, const int32_t* ids, int n, 
     if (c->h_len[seq] + n > hp.maxL) { c->err = "input does not fit in maxL"; return -1; }
     for (int i = 0; i < n; i++)
         if (ids[i] < 0 || ids[i] >= hp.vocabSize) { c->err = "token id out of range"; return -1; }
-    float *dLogits = nullptr, *dProbs = nullptr, *dNll = nullptr;
-    int* dTarget = nullptr;
-    std::vector<int> target(n, -1);
-    for (int i = 0; i + 1 < n; i++) target[i] = ids[i + 1];
-    std::vector<float> nll(n, 0.f);
-    hipError_t e = hipMalloc((void**)&dLogits, (size_t)n * V * 4);
-    if (e == hipSuccess && probsOut) e = hipMalloc((void**)&dProbs, (size_t)n * V * 4);
-    if (e == hipSuccess) e = hipMalloc((void**)&dNll, (size_t)n * 4);
-    if (e == hipSuccess) e = hipMalloc((void**)&dTarget, (size_t)n * 4);
-    if (e == hipSuccess) e = hipMemcpy(dTarget, target.data(), (size_t)n * 4, hipMemcpyHostToDevice);
-    if (e != hipSuccess) { c->err = std::string("forward_full buffers: ") + hipGetErrorString(e); rc = -2; }
-    if (rc == 0) {
-        if (c->prefillMode == 0 && n >= MLH_PREFILL_GEMM_MIN_ROWS && mlh_prefill_gemm_supported(c)) {
-            rc = mlh_run_prefill_gemm(c, 1, &seq, ids, &n, dLogits);
-        } else { // token by token through the decode kernels, LM head at every position
-            rc = set_slots(c, &seq, 1);
-            if (rc == 0 && hipMemcpyAsync(c->d_prompt, ids, (size_t)n * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess) rc = -2;
-            for (int i = 0; i < n && rc == 0; i++) {
-                rc = mlh_launch_step(c, 1, c->d_prompt + i, true);
-                if (rc == 0 && hipMemcpyAsync(dLogits + (size_t)i * V, c->logits + (size_t)seq * V, V * 4, hipMemcpyDeviceToDevice, c->stream) != hipSuccess) rc = -2;
-            }
-            if (rc == 0) { if (hipStreamSynchronize(c->stream) != hipSuccess) rc = -2; else c->h_len[seq] += n; }
-            if (rc == -2 && c->err.empty()) c->err = "forward_full: HIP call failed";
+    touch(c, seq, seq + 1);
+    // device results: logits, probabilities, targets, losses
+    const size_t mat = (size_t)n * V * 4, need = mat * (probsOut ? 2 : 1) + (size_t)n * 8;
+    if (need > c->fullBytes) {
+        MLH_CHECK(c, hipStreamSynchronize(c->stream));
+        if (c->fullBuf) (void)hipFree(c->fullBuf);
+        c->fullBuf = nullptr; c->fullBytes = 0;
+        MLH_CHECK(c, hipMalloc((void**)&c->fullBuf, need));
+        c->fullBytes = need;
+    }
+    if ((rc = mlh_pin(c, c->pinStage, RB_RING * RB_CHUNK)) || (rc = mlh_pin(c, c->pinIo, (size_t)n * 8))) return rc;
+    float *dLogits = c->fullBuf, *dProbs = probsOut ? dLogits + (size_t)n * V : nullptr, *dNll = dLogits + (size_t)n * V * (probsOut ? 2 : 1) + n;
+    int* dTarget = (int*)dNll - n;
+    int* target = c->pinIo.p;
+    float* nll = (float*)target + n;
+    for (int i = 0; i < n; i++) target[i] = i + 1 < n ? ids[i + 1] : -1;
+    Readback::Part parts[2];
+    int np = 0;
+    if (logitsOut) parts[np++] = {(const char*)dLogits, (char*)logitsOut, mat};
+    if (probsOut) parts[np++] = {(const char*)dProbs, (char*)probsOut, mat};
+    Readback out(parts, np); // its threads map the callers' pages from here on
+    hipError_t e = hipMemcpyAsync(dTarget, target, (size_t)n * 4, hipMemcpyHostToDevice, c->stream);
+    if (e != hipSuccess) { c->err = std::string("forward_full: ") + hipGetErrorString(e); return -2; }
+    if (c->prefillMode == 0 && n > 1 && mlh_prefill_gemm_supported(c)) {
+        rc = mlh_run_prefill_gemm(c, 1, &seq, ids, &n, dLogits);
+    } else { // token by token through the decode kernels, LM head at every position
+        rc = set_slots(c, &seq, 1);
+        if (rc == 0 && hipMemcpyAsync(c->d_prompt, ids, (size_t)n * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess) rc = -2;
+        for (int i = 0; i < n && rc == 0; i++) {
+            rc = mlh_launch_step(c, 1, c->d_prompt + i, true);
+            if (rc == 0 && hipMemcpyAsync(dLogits + (size_t)i * V, c->logits + (size_t)seq * V, V * 4, hipMemcpyDeviceToDevice, c->stream) != hipSuccess) rc = -2;
         }
+        if (rc == 0) { if (hipStreamSynchronize(c->stream) != hipSuccess) rc = -2; else c->h_len[seq] += n; }
+        if (rc == -2 && c->err.empty()) c->err = "forward_full: HIP call failed";
     }
     if (rc == 0) rc = mlh_launch_softmax_rows(c, dLogits, dProbs, dTarget, dNll, n);
     if (rc == 0) {
-        e = hipStreamSynchronize(c->stream);
-        if (e == hipSuccess && logitsOut) e = hipMemcpy(logitsOut, dLogits, (size_t)n * V * 4, hipMemcpyDeviceToHost);
-        if (e == hipSuccess && probsOut) e = hipMemcpy(probsOut, dProbs, (size_t)n * V * 4, hipMemcpyDeviceToHost);
-        if (e == hipSuccess) e = hipMemcpy(nll.data(), dNll, (size_t)n * 4, hipMemcpyDeviceToHost);
+        e = hipMemcpyAsync(nll, dNll, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = out.run(c->stream, (unsigned char*)c->pinStage.p);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) { c->err = std::string("forward_full read-back: ") + hipGetErrorString(e); rc = -2; }
     }
-    (void)hipFree(dLogits); (void)hipFree(dProbs); (void)hipFree(dNll); (void)hipFree(dTarget);
+    if (rc) (void)hipStreamSynchronize(c->stream);
+    if (need > ((size_t)512 << 20)) { // (2 048 tokens of a 32 K vocabulary with probabilities are kept)
+        (void)hipFree(c->fullBuf);
+        c->fullBuf = nullptr; c->fullBytes = 0;
+    }
     if (rc == 0 && meanNll) {
         double s = 0;
         for (int i = 0; i + 1 < n; i++) s += nll[i];
@@ -616,8 +669,7 @@ static bool use_persistent(const mlh_ctx* c, int nseq) {
 // end; the barrier kernel stores them at every step, and gets them back from the copy taken before its launch.
 static int check_persistent_abort(mlh_ctx* c) {
     if (c->d_timing) mlh_dump_persistent_timing(c);
-    unsigned flag = 0;
-    MLH_CHECK(c, hipMemcpy(&flag, c->d_sync + 64 * 20, 4, hipMemcpyDeviceToHost));
+    const int flag = c->pinIo.p[c->hp.maxSeqs]; // (end_steps)
     if (flag) {
         c->err = flag == 2 ? "XCD-rank decode kernel: the workgroups did not spread evenly over the XCDs"
                            : "persistent decode kernel abandoned a wait (were all workgroups resident?)";
@@ -631,6 +683,34 @@ static int check_persistent_abort(mlh_ctx* c) {
         MLH_CHECK(c, hipStreamSynchronize(c->stream));
         return -3;
     }
+    return 0;
+}
+
+// Before and after the steps of a call: tokens in and picks out through pinned memory that a kernel reads and writes.  A
+// launch in stream order costs 2 to 3 us, a copy from or to the caller's memory 10 to 13.
+__global__ void __launch_bounds__(256) k_steps_begin(const int* __restrict__ first, int* __restrict__ tok, int nseq, int* stepCounter) {
+    for (int i = threadIdx.x; i < nseq; i += 256) tok[i] = first[i];
+    if (threadIdx.x == 0) *stepCounter = 0;
+}
+__global__ void __launch_bounds__(256) k_steps_end(const int* __restrict__ ids, int n, const unsigned* abortFlag, int* flagOut, int* __restrict__ out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i == 0) *flagOut = (int)*abortFlag;
+    if (i < n) out[i] = ids[i];
+}
+static int begin_steps(mlh_ctx* c, const int32_t* first, int nseq, int steps) {
+    const int S = c->hp.maxSeqs; // pinned: S tokens, the flag, the picks
+    int rc = mlh_pin(c, c->pinIo, ((size_t)S + 1 + (size_t)nseq * steps) * 4);
+    if (rc) return rc;
+    memcpy(c->pinIo.p, first, (size_t)nseq * 4);
+    hipLaunchKernelGGL(k_steps_begin, dim3(1), dim3(256), 0, c->stream, c->pinIo.p, c->d_tok, nseq, c->d_stepCounter);
+    MLH_CHECK(c, hipGetLastError());
+    return 0;
+}
+static int end_steps(mlh_ctx* c, int nout) {
+    int* p = c->pinIo.p + c->hp.maxSeqs;
+    hipLaunchKernelGGL(k_steps_end, dim3((nout + 256) / 256), dim3(256), 0, c->stream, c->d_outIds, nout, c->d_sync + 64 * 20, p, p + 1);
+    MLH_CHECK(c, hipGetLastError());
+    MLH_CHECK(c, hipStreamSynchronize(c->stream));
     return 0;
 }
 
@@ -666,6 +746,7 @@ static int check_decode(mlh_ctx* c, const int32_t* ids, int nseq, int steps) {
         if (ids[s] < 0 || ids[s] >= hp.vocabSize) { c->err = "token id out of range"; return -1; }
         if (c->h_len[s] + steps > hp.maxL) { c->err = "sequence would exceed maxL"; return -1; }
     }
+    touch(c, 0, nseq);
     return set_identity_slots(c, nseq);
 }
 
@@ -684,16 +765,19 @@ extern "C" int mlh_decode_loop(mlh_ctx* c, const int32_t* first, int nseq, int s
     if (!out) { c->err = "null output"; return -1; }
     for (int attempt = 0; attempt < 2; attempt++) {
         const bool single = use_persistent(c, nseq);
-        MLH_CHECK(c, hipMemcpyAsync(c->d_tok, first, (size_t)nseq * 4, hipMemcpyHostToDevice, c->stream));
-        MLH_CHECK(c, hipMemsetAsync(c->d_stepCounter, 0, 4, c->stream));
+        if ((rc = begin_steps(c, first, nseq, steps))) return rc;
         if ((rc = run_steps(c, nseq, steps))) return rc;
-        MLH_CHECK(c, hipMemcpyAsync(out, c->d_outIds, (size_t)steps * nseq * 4, hipMemcpyDeviceToHost, c->stream));
-        MLH_CHECK(c, hipStreamSynchronize(c->stream));
+        if ((rc = end_steps(c, steps * nseq))) return rc;
         if (!single || (rc = check_persistent_abort(c)) == 0) break;
         if (rc != -3) return rc;
         fall_back_to_kernel_sequence(c); // and once more, as a sequence of kernels
     }
-    for (int s = 0; s < nseq; s++) c->h_len[s] += steps;
+    memcpy(out, c->pinIo.p + c->hp.maxSeqs + 1, (size_t)steps * nseq * 4);
+    for (int s = 0; s < nseq; s++) {
+        c->h_len[s] += steps;
+        c->h_next[s] = out[(size_t)(steps - 1) * nseq + s];
+        c->h_nextKnown[s] = 1;
+    }
     return 0;
 }
 
@@ -711,15 +795,14 @@ extern "C" int mlh_time_decode(mlh_ctx* c, const int32_t* first, int nseq, int s
     float ms = 0.f;
     for (int attempt = 0; attempt < 2; attempt++) {
         const bool single = use_persistent(c, nseq);
-        MLH_CHECK(c, hipMemcpyAsync(c->d_tok, first, (size_t)nseq * 4, hipMemcpyHostToDevice, c->stream));
-        MLH_CHECK(c, hipMemsetAsync(c->d_stepCounter, 0, 4, c->stream));
+        if ((rc = begin_steps(c, first, nseq, steps))) return rc;
         MLH_CHECK(c, hipStreamSynchronize(c->stream));
         MLH_CHECK(c, hipEventRecord(e0, c->stream));
         rc = run_steps(c, nseq, steps);
         MLH_CHECK(c, hipEventRecord(e1, c->stream));
         MLH_CHECK(c, hipEventSynchronize(e1));
         MLH_CHECK(c, hipEventElapsedTime(&ms, e0, e1));
-        if (rc) break;
+        if (rc || (rc = end_steps(c, 0))) break;
         if (!single || (rc = check_persistent_abort(c)) == 0) break;
         if (rc != -3) break;
         fall_back_to_kernel_sequence(c);
@@ -741,8 +824,7 @@ extern "C" int mlh_profile_decode(mlh_ctx* c, const int32_t* first, int nseq, in
     std::vector<int> ids;
     hipEvent_t e0;
     MLH_CHECK(c, hipEventCreate(&e0));
-    MLH_CHECK(c, hipMemcpyAsync(c->d_tok, first, (size_t)nseq * 4, hipMemcpyHostToDevice, c->stream));
-    MLH_CHECK(c, hipMemsetAsync(c->d_stepCounter, 0, 4, c->stream));
+    if ((rc = begin_steps(c, first, nseq, steps))) return rc;
     MLH_CHECK(c, hipStreamSynchronize(c->stream));
     c->profEvents = &events;
     c->profIds = &ids;
@@ -867,6 +949,7 @@ extern "C" int mlh_time_kernel(mlh_ctx* c, int kernel, int layer, int nseq, int 
     if ((rc = set_identity_slots(c, nseq))) return rc;
     for (int s = 0; s < nseq; s++)
         if (c->h_len[s] >= c->hp.maxL) { c->err = "sequence is full"; return -1; }
+    touch(c, 0, nseq);
     hipEvent_t e0, e1;
     MLH_CHECK(c, hipEventCreate(&e0));
     MLH_CHECK(c, hipEventCreate(&e1));

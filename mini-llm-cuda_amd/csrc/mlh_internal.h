@@ -91,6 +91,12 @@ struct StepArgs {
     int outCapacity;
 };
 
+// Pinned host memory of a context (the device reads and writes it directly); grows when the context's stream is idle.
+struct PinBuf {
+    int* p = nullptr;
+    size_t bytes = 0;
+};
+
 struct mlh_ctx {
     mlh_hparams hp;
     int device = 0;
@@ -164,14 +170,13 @@ struct mlh_ctx {
     std::vector<int>* profIds = nullptr;
 
     // prefill work buffers, sized on first use for the largest row count seen
-    int pfRows = 0, pfBlkCap = 0;
+    int pfRows = 0;
     int prefillMode = 0; // 0: GEMM path when the shape allows and the call is long enough; 1: token by token
     std::vector<void*> pfAllocs;
     float *pfX = nullptr, *pfQKV = nullptr, *pfH1 = nullptr;
     void *pfXn = nullptr, *pfA = nullptr, *pfU = nullptr;
     uint16_t *pfKh = nullptr, *pfVh = nullptr; // half copies of a call's K and V rows for the MFMA attention of a fresh prefill
     int* pfMeta = nullptr;
-    int pfChunkCap = 0;
     void* pfGdnWs = nullptr;   // chunk operands of the chunk-parallel GDN prefill
     float* pfGdnG = nullptr;
     size_t pfGdnChunks = 0;
@@ -184,6 +189,15 @@ struct mlh_ctx {
     void* gemmWs = nullptr;    // split-K workspace of the skinny GEMM
 
     std::vector<int> h_len; // host mirror of d_pos
+    std::vector<char> h_dirty;     // sequences that some launch may have given a length or GDN states since their last reset
+    std::vector<char> h_nextKnown; // sequences whose next token h_next holds
+    std::vector<int> h_next;
+    PinBuf pinIo;    // a decode call's first tokens, the single-launch kernels' abort flag, the picked tokens
+    PinBuf pinMeta;  // a prefill's metadata, laid out as on the device
+    PinBuf pinNext;  // a prefill's picks, by sequence
+    PinBuf pinStage; // forward_full's results on their way out
+    float* fullBuf = nullptr; // forward_full's device results, kept for the next call up to a limit
+    size_t fullBytes = 0;
     int identityNseq = 0;   // d_sidx currently holds 0..identityNseq-1 (0 = unknown)
 
     int graphSteps = 0;                 // 0: eager launches; k >= 1: one graph replay covers k decode steps
@@ -200,6 +214,7 @@ double mlh_kernel_bytes(mlh_ctx* c, int kernel, int layer, int nseq);
 void mlh_fill_args(mlh_ctx* c, StepArgs& a, int nseq, const int* tokPtr);
 int mlh_launch_copy(mlh_ctx* c);
 int mlh_dev_alloc_bytes(mlh_ctx* c, void** p, size_t bytes); // mlh_api.hip: an allocation owned by the context
+int mlh_pin(mlh_ctx* c, PinBuf& b, size_t bytes);                    // ... and its pinned memory
 int mlh_launch_probs(mlh_ctx* c, int seq);
 int mlh_init_kernels(mlh_ctx* c);
 
@@ -225,6 +240,7 @@ extern "C" int mlh_gemm_device_init(int device);
 void mlh_set_thread_error(const std::string& msg);
 
 // kernels_prefill.hip
+#define MLH_PREFILL_GEMM_MIN_ROWS 16 // bf16 models: calls of fewer tokens keep fp32 activations throughout
 bool mlh_prefill_gemm_supported(const mlh_ctx* c);
 int mlh_init_prefill_kernels(mlh_ctx* c);
 int mlh_build_gemm_operands(mlh_ctx* c); // at finalize: fp16 mirrors for bf16 models
@@ -235,6 +251,11 @@ int mlh_launch_softmax_rows(mlh_ctx* c, const float* logits, float* probs, const
 bool mlh_rows_applicable(const mlh_ctx* c, int nseq);
 int mlh_rows_prepare(mlh_ctx* c);
 int mlh_rows_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool embedded, bool embedNext);
+// its parts, for short prefills (rows: tokens) and every prefill's LM head
+void mlh_rows_gemm(mlh_ctx* c, int epi, const void* w, int n, RowsArgs P);
+void mlh_rows_embed(mlh_ctx* c, const int* tok, int n, float* x, RowsLayout lay);
+void mlh_rows_rest_of_layer(mlh_ctx* c, int t, const RowsArgs& base, float* x, float* h1);
+void mlh_rows_lm_head(mlh_ctx* c, int n, const float* X, const int* segStart, const int* segLen, const int* segSeq, float* amaxVal, int* amaxIdx);
 
 // kernels_persistent.hip
 bool mlh_persistent_supported(const mlh_ctx* c);

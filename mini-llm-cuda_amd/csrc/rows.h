@@ -41,3 +41,26 @@ __device__ __forceinline__ void rows_put(void* planes, int k, int m, RowsLayout 
 #pragma unroll
     for (int pl = 0; pl < 3; pl++) *reinterpret_cast<uint16_t*>(p + pl * l.stride()) = (uint16_t)w[pl];
 }
+
+#define RW_TILE 16 // weight rows of a tile
+enum { RW_PLAIN, RW_RESID, RW_SWIGLU, RW_LOGITS };
+
+struct RowsArgs {
+    const unsigned char* W;         // in fetch order (rows.h)
+    int M, N, K, tiles;
+    RowsLayout lay;                 // of the plane buffers
+    const unsigned char* A;         // planes of the input rows
+    const float* ssqIn;             // [nparts][64] partial sums of squares of the rows behind A, or null: no normalisation
+    int nparts, normDim;
+    float* C;                       // RW_PLAIN, RW_RESID: [M, ldc] fp32; RW_LOGITS: row sidx[m] of [*, ldc]
+    int ldc;
+    const float* R;                 // RW_RESID: added to the product, [M, ldc]
+    unsigned char* out;             // RW_RESID: planes of outGain (.) C; RW_SWIGLU: planes of silu(gate) * up
+    const float* outGain;
+    float* ssqOut;                  // RW_RESID: [workgroup][64]
+    const int* sidx;
+    float* amaxVal;                 // RW_LOGITS: [M, amaxParts] largest logit of each workgroup's rows and its index
+    int* amaxIdx;
+    int amaxParts;
+    int* stepCounter;               // RW_LOGITS: counted up once
+};
