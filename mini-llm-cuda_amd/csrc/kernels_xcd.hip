@@ -34,7 +34,9 @@
 // phases ahead, so that HBM latency is off the critical path (loads return in issue order on this ISA:
 // a wave that polled would see its poll answered only after its prefetches).  The communicator does all
 // the polling, the small reductions, q/k norm + RoPE and the softmax-partials combine, puts the result
-// in LDS and meets the workers at a workgroup barrier.  K/V tiles of a wave's first attention unit are
+// in LDS and meets the workers at a workgroup barrier.  What bounds a layer is this chain of exchanges (weights: 6 of its
+// 14 us at dim 768), so its loads go out back to back, with no test between them: 12 layers of dim 768 at 300 keys 225 -> 175 us per
+// token, 4 layers of dim 256 61 -> 41.  K/V tiles of a wave's first attention unit are
 // fetched global -> LDS directly (no registers) a whole layer ahead.
 #include <stdlib.h>
 
@@ -130,48 +132,43 @@ __device__ __forceinline__ void nap64(int n) {
     for (; n > 0; n--) __builtin_amdgcn_s_sleep(1);
 }
 
-// One wave fetches n tagged words into LDS, NB loads per lane and round, reading again until every tag is there.
-// With PIPE two rounds are in flight, a fraction of a round trip apart: the answer to a round that just missed the
-// data is followed closely by the next one instead of by a whole new round trip.  All 64 lanes take part.
-template <bool CROSS, int NB, bool PIPE>
-__device__ __forceinline__ void poll_vec(const u64* src, int n, unsigned tag, float* dst, const unsigned* abortFlag, bool& ok, int nap = 0) {
+// One wave fetches n <= 64 NB tagged words into LDS, reading again until every tag is there.  Exactly NB loads per lane and round
+// and no branch between them (indices past the end are clamped): a round of loads with a test around each one took 0.3 us longer.
+template <bool CROSS, int NB>
+__device__ __forceinline__ void poll_words(const u64* src, int n, unsigned tag, float* dst, const unsigned* abortFlag, bool& ok) {
     const int lane = threadIdx.x & 63;
+    for (unsigned spins = 0;; spins++) {
+        u64 w[NB];
+        asm volatile("" ::: "memory"); // the loads are repeated every round
+#pragma unroll
+        for (int k = 0; k < NB; k++) w[k] = ldw<CROSS>(src, (unsigned)(k == NB - 1 ? min(lane, n - 1 - 64 * k) : lane) * 8u, k * 512u);
+        bool all = true;
+#pragma unroll
+        for (int k = 0; k < NB; k++) all = all && (unsigned)(w[k] >> 32) == tag;
+        if (__all(all)) {
+#pragma unroll
+            for (int k = 0; k < NB; k++)
+                if (k < NB - 1 || k * 64 + lane < n) dst[k * 64 + lane] = __uint_as_float((unsigned)w[k]);
+            return;
+        }
+        if (!ok || spins > XSPIN || ((spins & 127) == 127 && aldu(abortFlag))) { ok = false; return; }
+    }
+}
+template <bool CROSS>
+__device__ __forceinline__ void poll_vec(const u64* src, int n, unsigned tag, float* dst, const unsigned* abortFlag, bool& ok, int nap) {
     nap64(nap);
-    for (int base = 0; base < n; base += 64 * NB) {
-        u64 wA[NB], wB[NB];
-        auto issue = [&](u64 (&w)[NB]) {
-            asm volatile("" ::: "memory"); // the loads are repeated every round
-#pragma unroll
-            for (int k = 0; k < NB; k++) {
-                const int i0 = base + k * 64; // wave-uniform
-                if (i0 < n) w[k] = ldw<CROSS>(pin_uniform(src + i0), (unsigned)min(lane, n - 1 - i0) * 8u, 0u);
-                else w[k] = (u64)tag << 32;
-            }
-        };
-        auto good = [&](const u64 (&w)[NB]) {
-            bool all = true;
-#pragma unroll
-            for (int k = 0; k < NB; k++) all = all && (unsigned)(w[k] >> 32) == tag;
-            return __all(all) != 0;
-        };
-        auto keep = [&](const u64 (&w)[NB]) {
-#pragma unroll
-            for (int k = 0; k < NB; k++) {
-                const int i = base + k * 64 + lane;
-                if (i < n) dst[i] = __uint_as_float((unsigned)w[k]);
-            }
-        };
-        issue(wA);
-        for (unsigned spins = 0;; spins++) {
-            if (PIPE) {
-                __builtin_amdgcn_s_sleep(CROSS ? 8 : 3);
-                issue(wB);
-            }
-            if (good(wA)) { keep(wA); break; }
-            if (PIPE) __builtin_amdgcn_s_sleep(CROSS ? 8 : 3);
-            issue(wA);
-            if (PIPE && good(wB)) { keep(wB); break; }
-            if (!ok || spins > XSPIN || ((spins & 127) == 127 && aldu(abortFlag))) { ok = false; break; }
+    for (int base = 0; base < n; base += 512) {
+        const u64* p = pin_uniform(src + base);
+        const int m = n - base;
+        switch ((min(m, 512) + 63) / 64) {
+            case 1: poll_words<CROSS, 1>(p, m, tag, dst + base, abortFlag, ok); break;
+            case 2: poll_words<CROSS, 2>(p, m, tag, dst + base, abortFlag, ok); break;
+            case 3: poll_words<CROSS, 3>(p, m, tag, dst + base, abortFlag, ok); break;
+            case 4: poll_words<CROSS, 4>(p, m, tag, dst + base, abortFlag, ok); break;
+            case 5: poll_words<CROSS, 5>(p, m, tag, dst + base, abortFlag, ok); break;
+            case 6: poll_words<CROSS, 6>(p, m, tag, dst + base, abortFlag, ok); break;
+            case 7: poll_words<CROSS, 7>(p, m, tag, dst + base, abortFlag, ok); break;
+            default: poll_words<CROSS, 8>(p, min(m, 512), tag, dst + base, abortFlag, ok);
         }
     }
 }
@@ -180,14 +177,15 @@ __device__ __forceinline__ void poll_vec(const u64* src, int n, unsigned tag, fl
 // eight partials of slice [rank sl, (rank + 1) sl) (sl = d / 32 <= 64) and the residual and publishes the slice inside
 // the XCD; then every workgroup fetches the whole vector from its XCD's 32 slices.  haveMask bit X' clear: that XCD
 // contributes nothing.  Reads across XCDs disturb the stores they wait for, so the first one comes late (napCross).
+template <int DW> // d / 64
 __device__ __forceinline__ void reduce_publish_fetch(const u64* part, int d, int rank, unsigned tag, unsigned haveMask,
                                                      const float* resid, u64* pub, float* dst, const unsigned* abortFlag, bool& ok,
                                                      int napCross, int napGather, int napRound, bool wide, u64* stamp = nullptr) {
     const int lane = threadIdx.x & 63;
     const int sl = wide ? 64 : d / XPER, s0 = rank * sl;
     if (s0 >= d) { // (wide slices: only d / 64 workgroups of the XCD read the other XCDs' partial sums)
-        nap64(napCross + 24);
-        poll_vec<false, 16, false>(pub, d, tag, dst, abortFlag, ok, napGather);
+        nap64(napCross + 24 + napGather);
+        poll_words<false, DW>(pub, d, tag, dst, abortFlag, ok);
         return;
     }
     const unsigned lb = (unsigned)min(lane, sl - 1) * 8u;
@@ -196,20 +194,19 @@ __device__ __forceinline__ void reduce_publish_fetch(const u64* part, int d, int
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int xc = 0; xc < XCDS; xc++) {
-            if ((haveMask >> xc) & 1u) w[xc] = ldw<true>(pin_uniform(part + (size_t)xc * d + s0), lb, 0u);
-            else w[xc] = (u64)tag << 32;
+            w[xc] = ldw<true>(pin_uniform(part + (size_t)xc * d + s0), lb, 0u);
         }
     };
     auto good = [&](const u64 (&w)[XCDS]) {
         bool all = true;
 #pragma unroll
-        for (int xc = 0; xc < XCDS; xc++) all = all && (unsigned)(w[xc] >> 32) == tag;
+        for (int xc = 0; xc < XCDS; xc++) all = all && ((unsigned)(w[xc] >> 32) == tag || !((haveMask >> xc) & 1u));
         return __all(all) != 0;
     };
     auto total = [&](const u64 (&w)[XCDS]) { // fixed order: the result does not depend on timing
         float t = 0.f;
 #pragma unroll
-        for (int xc = 0; xc < XCDS; xc++) t += __uint_as_float((unsigned)w[xc]);
+        for (int xc = 0; xc < XCDS; xc++) t += (haveMask >> xc) & 1u ? __uint_as_float((unsigned)w[xc]) : 0.f;
         return t;
     };
     float sum = 0.f;
@@ -226,7 +223,8 @@ __device__ __forceinline__ void reduce_publish_fetch(const u64* part, int d, int
     }
     if (stamp && lane == 0) stamp[0] = wall_clock64();
     if (lane < sl) lst(pub + s0 + lane, sum + resid[s0 + lane], tag);
-    poll_vec<false, 16, false>(pub, d, tag, dst, abortFlag, ok, napGather);
+    nap64(napGather);
+    poll_words<false, DW>(pub, d, tag, dst, abortFlag, ok);
 }
 
 // NCH (template parameter of the kernel): 16-byte chunks per lane of a full-width row, dim / (64 N)
@@ -374,22 +372,19 @@ __device__ __forceinline__ int rowA_hyb(const LayerDev& L, int X, int nh, int np
     return uni(L.offPle) + X * pleX + e;
 }
 
-// Wo columns of the XCD's heads: a pass covers N rows per wave (64/N lanes per 64-column head segment).  Rows
-// and heads beyond the end are clamped to the last valid one (loaded, never used).
-template <typename WT, int G = 1>
-__device__ __forceinline__ void issue_wo(XPf<WT>& pf, const WT* Wo, int ad, int X, int nh, int heads, int lw, int d) {
+// Wo columns of the XCD's heads: a pass covers N rows per wave (64/N lanes per 64-column head segment).  Load i of two
+// passes: head segment i % XNH of pass i / XNH; rows and heads beyond the end are clamped to the last valid one (loaded, never used).
+template <typename WT, int G>
+__device__ __forceinline__ const WT* wo_base(const WT* Wo, int ad, int X, int nh, int heads, int lw, int d, int i) {
+    constexpr int N = PVec<WT>::N;
+    const int rb = min((i / XNH * XLW + lw) * N, d - N);
+    const int h = min(slice_of<G>(X, min(i % XNH, max(nh, 1) - 1)), G * heads - 1); // slice, clamped to the last one
+    return Wo + (size_t)rb * ad + h * XHD;
+}
+template <typename WT> __device__ __forceinline__ unsigned wo_lane(int ad) { // bytes: row within the pass, chunk within the head segment
     constexpr int N = PVec<WT>::N, CPS = XHD / N;
     const unsigned lane = threadIdx.x & 63u;
-    const unsigned lb = ((lane / CPS) * (unsigned)ad + (lane % CPS) * N) * (unsigned)sizeof(WT); // row within the pass, chunk within the head segment
-#pragma unroll
-    for (int p = 0; p < 2; p++) {
-        const int rb = min((p * XLW + lw) * N, d - N);
-#pragma unroll
-        for (int j = 0; j < XNH; j++) {
-            const int h = min(slice_of<G>(X, min(j, max(nh, 1) - 1)), G * heads - 1); // slice, clamped to the last one
-            pf.r[p * XNH + j] = load16<WT>(pin_uniform(Wo + (size_t)rb * ad + h * XHD), lb, 0u);
-        }
-    }
+    return ((lane / CPS) * (unsigned)ad + (lane % CPS) * N) * (unsigned)sizeof(WT);
 }
 // W2 columns [X fs, (X+1) fs): a wave takes blocks of four consecutive rows (block wb first); the first block, two
 // chunks per lane, is prefetched (clamped likewise).
@@ -428,6 +423,39 @@ __device__ __forceinline__ void issue_kv_tile(const float* Kh, const float* Vh, 
     }
 }
 
+// One round of the softmax-partials combine: nb <= NB tiles at ub (lane = dimension) into the running maximum M, weighted sum num and
+// weight sum den.  NB loads with nothing between them (those past tile nb - 1 are dropped: they lie inside the exchange words).
+template <int NB>
+__device__ __forceinline__ void combine_tiles(const u64* ub, int nb, unsigned lt, const unsigned* abortFlag, bool& ok, float& M, float& num, float& den) {
+    const int lane = threadIdx.x & 63;
+    u64 wa[NB], wm, wl;
+    const unsigned uOff = (unsigned)min(lane & 31, nb - 1) * ((XHD + 2) * 8u);
+    for (unsigned spins = 0;; spins++) {
+        asm volatile("" ::: "memory");
+        bool all = true;
+#pragma unroll
+        for (int k = 0; k < NB; k++) wa[k] = ldw<false>(ub + (k & ~3) * (XHD + 2), (unsigned)lane * 8u, (k & 3) * ((XHD + 2) * 8u));
+        wm = ldw<false>(ub, uOff, XHD * 8u);       // lane k < 32: running maximum of tile k
+        wl = ldw<false>(ub, uOff, (XHD + 1) * 8u); //              and its sum of exponentials
+#pragma unroll
+        for (int k = 0; k < NB; k++) all = all && ((unsigned)(wa[k] >> 32) == lt || k >= nb);
+        all = all && (unsigned)(wm >> 32) == lt && (unsigned)(wl >> 32) == lt;
+        if (__all(all)) break;
+        if (!ok || spins > XSPIN || ((spins & 255) == 255 && aldu(abortFlag))) { ok = false; break; }
+    }
+    const float mk = __uint_as_float((unsigned)wm), lk = __uint_as_float((unsigned)wl);
+    const bool mine = lane < nb;
+    const float Mn = fmaxf(M, pwave_max(mine ? mk : -1.0e30f));
+    const float corr = __expf(M - Mn);
+    const float w = mine ? __expf(mk - Mn) : 0.f;
+    den = fmaf(den, corr, pwave_sum(w * lk));
+    num *= corr;
+#pragma unroll
+    for (int k = 0; k < NB; k++)
+        num = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), k)), k < nb ? __uint_as_float((unsigned)wa[k]) : 0.f, num);
+    M = Mn;
+}
+
 struct XShared {
     float *xs, *h1s, *qkvs, *as, *us, *scratch, *bestv, *tiles;
     float *es, *gst; // hybrid models: the XCD's PLE values of the layer; this workgroup's GDN state rows [layer][4][64]
@@ -446,7 +474,7 @@ struct XShared {
     } while (0)
 
 // ------------------------------------------------------------------------------------------------ communicator
-template <typename WT, bool HYB, int G>
+template <typename WT, int NCH, bool HYB, int G>
 __device__ __forceinline__ void xcd_communicator(const XcdArgs& P, const XShared& S, int tok, int pos, unsigned tagBase, int X, int r) {
     const StepArgs& a = P.a;
     const int d = a.dim, V = a.vocab;
@@ -471,7 +499,7 @@ __device__ __forceinline__ void xcd_communicator(const XcdArgs& P, const XShared
             const int ts = (P.NL - 1 - t) * 16;
             X_STAMP(ts + 0);
             if (t != P.NL - 1) // partial x of the layer below, all XCDs, + its residual h1
-                reduce_publish_fetch(P.xP, d, r, lt - 1, 0xffu, S.h1s, P.xL + (size_t)X * d, S.xs, P.abortFlag, ok, P.nap[0], P.nap[1], P.napRound, P.wide != 0,
+                reduce_publish_fetch<NCH * PVec<WT>::N>(P.xP, d, r, lt - 1, 0xffu, S.h1s, P.xL + (size_t)X * d, S.xs, P.abortFlag, ok, P.nap[0], P.nap[1], P.napRound, P.wide != 0,
                                      (P.timing && wg == 0 && step == P.steps - 1) ? P.timing + ts + 6 : nullptr);
             if (!ok) { S.ctl[0] = 1; astu(P.abortFlag, 1u); }
             X_STAMP(ts + 1);
@@ -483,7 +511,7 @@ __device__ __forceinline__ void xcd_communicator(const XcdArgs& P, const XShared
                 const bool gdnL = uni(L.kind) != MLH_KIND_ATTENTION;
                 RAL = (gdnL ? 3 : np) * nh * XHD + (gdnL ? 2 * nh : 0) + a.ple / XCDS;
             }
-            poll_vec<false, 8, false>(qkvL, RAL, lt, S.qkvs, P.abortFlag, ok, P.nap[2]);
+            poll_vec<false>(qkvL, RAL, lt, S.qkvs, P.abortFlag, ok, P.nap[2]);
             if (!ok) { S.ctl[0] = 1; astu(P.abortFlag, 1u); }
             X_STAMP(ts + 2);
             X_BARRIER(); // 2: q, k, v, gate in LDS
@@ -493,13 +521,13 @@ __device__ __forceinline__ void xcd_communicator(const XcdArgs& P, const XShared
             X_BARRIER(); // 3: mixing output of the XCD's heads in LDS
 
             // h1 = x + sum of the XCDs' Wo partials (inference.cu:252-260)
-            reduce_publish_fetch(P.h1P, d, r, lt, headMask, S.xs, P.h1L + (size_t)X * d, S.h1s, P.abortFlag, ok, P.nap[0], P.nap[1], P.napRound, P.wide != 0,
+            reduce_publish_fetch<NCH * PVec<WT>::N>(P.h1P, d, r, lt, headMask, S.xs, P.h1L + (size_t)X * d, S.h1s, P.abortFlag, ok, P.nap[0], P.nap[1], P.napRound, P.wide != 0,
                                  (P.timing && wg == 0 && step == P.steps - 1) ? P.timing + ts + 8 : nullptr);
             if (!ok) { S.ctl[0] = 1; astu(P.abortFlag, 1u); }
             X_STAMP(ts + 4);
             X_BARRIER(); // 4: h1 in LDS
 
-            poll_vec<false, 8, false>(P.uL + (size_t)X * P.fs, P.fs, lt, S.us, P.abortFlag, ok, P.nap[3]);
+            poll_vec<false>(P.uL + (size_t)X * P.fs, P.fs, lt, S.us, P.abortFlag, ok, P.nap[3]);
             if (!ok) { S.ctl[0] = 1; astu(P.abortFlag, 1u); }
             X_STAMP(ts + 5);
             X_BARRIER(); // 5: the XCD's FFN activations in LDS
@@ -507,7 +535,7 @@ __device__ __forceinline__ void xcd_communicator(const XcdArgs& P, const XShared
 
         // ---------------------------------------------------------------------- LM head + argmax
         const unsigned ltLast = tagBase + (unsigned)(step * P.NL + P.NL);
-        reduce_publish_fetch(P.xP, d, r, ltLast, 0xffu, S.h1s, P.xL + (size_t)X * d, S.xs, P.abortFlag, ok, P.nap[0], P.nap[1], P.napRound, P.wide != 0);
+        reduce_publish_fetch<NCH * PVec<WT>::N>(P.xP, d, r, ltLast, 0xffu, S.h1s, P.xL + (size_t)X * d, S.xs, P.abortFlag, ok, P.nap[0], P.nap[1], P.napRound, P.wide != 0);
         if (!ok) { S.ctl[0] = 1; astu(P.abortFlag, 1u); }
         X_BARRIER(); // final x in LDS
         X_BARRIER(); // the workers' best logits in LDS
@@ -524,7 +552,7 @@ __device__ __forceinline__ void xcd_communicator(const XcdArgs& P, const XShared
                 xst(P.amax + 2 * wg, v, tagBase + (unsigned)step + 1);
                 xst(P.amax + 2 * wg + 1, __uint_as_float((unsigned)i), tagBase + (unsigned)step + 1);
             }
-            poll_vec<true, 8, true>(P.amax, 2 * (int)gridDim.x, tagBase + (unsigned)step + 1, S.scratch, P.abortFlag, ok, P.nap[0] / 2);
+            poll_vec<true>(P.amax, 2 * (int)gridDim.x, tagBase + (unsigned)step + 1, S.scratch, P.abortFlag, ok, P.nap[0] / 2);
             v = -3.0e38f; i = 0x7fffffff;
             for (int k = lane; k < (int)gridDim.x; k += 64) {
                 const float v2 = S.scratch[2 * k];
@@ -601,14 +629,28 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
     XRows<WT, XS1, NCH> s1; // rows of phases A / D / LM head
     XPf<WT> s2;      // rows of phases C / E / LM head
     XGain<WT, NCH> gn;
-    // first-phase rows lw, lw + XLW, ... of layer Lx and its first gain vector
-    auto issueA = [&](const LayerDev& Lx) {
+    // What a wave works on after the FFN of a layer: the first-phase rows lw, lw + XLW, ... and the first gain vector of layer Lx,
+    // or, behind the last layer, its LM-head rows gwl, gwl + TWL, ... and the final gain.  One set of loads with selected
+    // addresses: loads in two branches meet in register copies, and a copy waits for its load (2 us per layer).
+    auto issueA = [&](const LayerDev& Lx, bool lm) {
         const int ra = rowsA(Lx);
         int rows[XS1];
 #pragma unroll
-        for (int k = 0; k < XS1; k++) rows[k] = nh > 0 ? rowA(Lx, min(lw + XLW * k, ra - 1)) : 0;
-        issue_rows<WT, XS1, NCH>(s1.r, uni_ptr((const WT*)Lx.Wa), d, rows);
-        issue_gain<WT, NCH>(gn, uni_ptr(Lx.g1));
+        for (int k = 0; k < XS1; k++) rows[k] = lm ? min(gwl + TWL * k, V - 1) : nh > 0 ? rowA(Lx, min(lw + XLW * k, ra - 1)) : 0;
+        issue_rows<WT, XS1, NCH>(s1.r, lm ? E : uni_ptr((const WT*)Lx.Wa), d, rows);
+        issue_gain<WT, NCH>(gn, lm ? a.gF : uni_ptr(Lx.g1));
+    };
+    // The same for the second register set: Wo of layer Lx, or two more LM-head rows (a row has at most 4 chunks)
+    auto issueWo = [&](const LayerDev& Lx, bool lm) {
+        const int rows[2] = {min(gwl + XS1 * TWL, V - 1), min(gwl + (XS1 + 1) * TWL, V - 1)};
+        const WT* Wo = uni_ptr((const WT*)Lx.Wo);
+        const int ad = uni(Lx.ad);
+        const unsigned lb = lm ? lane * 16u : wo_lane<WT>(ad);
+#pragma unroll
+        for (int i = 0; i < 2 * XNH; i++) {
+            const WT *w = wo_base<WT, G>(Wo, ad, X, nh, a.heads, lw, d, i), *e = E + (size_t)rows[i < NCH ? 0 : 1] * d + (i < NCH ? i : min(i - NCH, NCH - 1)) * (64 * N);
+            s2.r[i] = load16<WT>(pin_uniform(lm ? e : w), lb, 0u);
+        }
     };
     // first K/V tile of this wave in layer Lx when the sequence holds npos rows, and the q/k gains of its head
     float gqv[G], gkv[G];
@@ -675,8 +717,8 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
     }
     {
         const LayerDev& L0 = S.Ls[P.NL - 1];
-        issueA(L0);
-        issue_wo<WT, G>(s2, uni_ptr((const WT*)L0.Wo), uni(L0.ad), X, nh, a.heads, lw, d);
+        issueA(L0, false);
+        issueWo(L0, false);
         issuePlw(L0);
         if (wave < XAW && (!HYB || uni(L0.kind) == MLH_KIND_ATTENTION)) issueKV(L0, pos);
     }
@@ -707,6 +749,9 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
             const int RAL = rowsA(L);                       // rows of the first phase in this layer
             const int RAq = (gdnL ? 3 : np) * nh * XHD;     // of which q | k | v | gate
             const LayerDev& Ln = S.Ls[lastLayer ? P.NL - 1 : t - 1];
+            int laneNow = threadIdx.x & 63; // opaque in every pass: addresses formed from it are not kept in registers from layer to layer
+            asm volatile("" : "+v"(laneNow));
+            const int lane = laneNow;
             X_BARRIER(); // 1
             const int ts = (P.NL - 1 - t) * 16;
             const bool stampW = P.timing && wg == 0 && wave == 0 && lane == 0 && step == P.steps - 1;
@@ -775,8 +820,6 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
                         S.as[j * XHD + lane] = __uint_as_float((unsigned)w);
                     }
                     if (!ok) { S.ctl[0] = 1; astu(P.abortFlag, 1u); }
-                    if (wave < XAW && !(lastLayer && step == P.steps - 1) && uni(Ln.kind) == MLH_KIND_ATTENTION)
-                        issueKV(Ln, lastLayer ? pos + 1 : pos);
                 }
             }
             if (wave < XAW && !gdnL) {
@@ -899,39 +942,48 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
                     float M = -1.0e30f, num = 0.f, den = 0.f;
                     for (int t0 = 0; t0 < ntiles; t0 += XCB) {
                         const int nb = ntiles - t0 < XCB ? ntiles - t0 : XCB;
-                        u64 wa[XCB], wm, wl;
                         const u64* ub = pin_uniform(partL + ((size_t)j * ntiles + t0) * (XHD + 2));
-                        const unsigned uOff = (unsigned)min(lane & 31, nb - 1) * ((XHD + 2) * 8u);
-                        for (unsigned spins = 0;; spins++) {
-                            asm volatile("" ::: "memory");
-                            bool all = true;
+                        // The form that tests before every load takes 0.5 us per layer more and fewer registers: for the widest models,
+                        // where the other one spills (dim 2048 bf16, 6 layers: 271 us per token instead of 342).
+                        if constexpr (NCH <= (N == 4 ? 3 : 2)) {
+                            if (nb <= 4) combine_tiles<4>(ub, nb, lt, P.abortFlag, ok, M, num, den);
+                            else if (nb <= 8) combine_tiles<8>(ub, nb, lt, P.abortFlag, ok, M, num, den);
+                            else if (nb <= 12) combine_tiles<12>(ub, nb, lt, P.abortFlag, ok, M, num, den);
+                            else combine_tiles<XCB>(ub, nb, lt, P.abortFlag, ok, M, num, den);
+                        } else {
+                            u64 wa[XCB], wm, wl;
+                            const unsigned uOff = (unsigned)min(lane & 31, nb - 1) * ((XHD + 2) * 8u);
+                            for (unsigned spins = 0;; spins++) {
+                                asm volatile("" ::: "memory");
+                                bool all = true;
 #pragma unroll
-                            for (int k = 0; k < XCB; k++) {
-                                if (k < nb) wa[k] = ldw<false>(ub, (unsigned)lane * 8u, k * ((XHD + 2) * 8u));
-                                else wa[k] = (u64)lt << 32;
-                                all = all && (unsigned)(wa[k] >> 32) == lt;
+                                for (int k = 0; k < XCB; k++) {
+                                    if (k < nb) wa[k] = ldw<false>(ub, (unsigned)lane * 8u, k * ((XHD + 2) * 8u));
+                                    else wa[k] = (u64)lt << 32;
+                                    all = all && (unsigned)(wa[k] >> 32) == lt;
+                                }
+                                wm = ldw<false>(ub, uOff, XHD * 8u);       // lane k < 32: running maximum of tile t0 + k
+                                wl = ldw<false>(ub, uOff, (XHD + 1) * 8u); //              and its sum of exponentials
+                                all = all && (unsigned)(wm >> 32) == lt && (unsigned)(wl >> 32) == lt;
+                                if (__all(all)) break;
+                                if (!ok || spins > XSPIN || ((spins & 255) == 255 && aldu(P.abortFlag))) { ok = false; break; }
                             }
-                            wm = ldw<false>(ub, uOff, XHD * 8u);       // lane k < 32: running maximum of tile t0 + k
-                            wl = ldw<false>(ub, uOff, (XHD + 1) * 8u); //              and its sum of exponentials
-                            all = all && (unsigned)(wm >> 32) == lt && (unsigned)(wl >> 32) == lt;
-                            if (__all(all)) break;
-                            if (!ok || spins > XSPIN || ((spins & 255) == 255 && aldu(P.abortFlag))) { ok = false; break; }
+                            const float mk = __uint_as_float((unsigned)wm), lk = __uint_as_float((unsigned)wl);
+                            const bool mine = lane < nb;
+                            const float Mn = fmaxf(M, pwave_max(mine ? mk : -1.0e30f));
+                            const float corr = __expf(M - Mn);
+                            const float w = mine ? __expf(mk - Mn) : 0.f;
+                            den = fmaf(den, corr, pwave_sum(w * lk));
+                            num *= corr;
+#pragma unroll
+                            for (int k8 = 0; k8 < XCB; k8 += 8)
+                                if (k8 < nb) {
+#pragma unroll
+                                    for (int k = k8; k < k8 + 8; k++)
+                                        num = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), k)), __uint_as_float((unsigned)wa[k]), num);
+                                }
+                            M = Mn;
                         }
-                        const float mk = __uint_as_float((unsigned)wm), lk = __uint_as_float((unsigned)wl);
-                        const bool mine = lane < nb;
-                        const float Mn = fmaxf(M, pwave_max(mine ? mk : -1.0e30f));
-                        const float corr = __expf(M - Mn);
-                        const float w = mine ? __expf(mk - Mn) : 0.f;
-                        den = fmaf(den, corr, pwave_sum(w * lk));
-                        num *= corr;
-#pragma unroll
-                        for (int k8 = 0; k8 < XCB; k8 += 8)
-                            if (k8 < nb) {
-#pragma unroll
-                                for (int k = k8; k < k8 + 8; k++)
-                                    num = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), k)), __uint_as_float((unsigned)wa[k]), num);
-                            }
-                        M = Mn;
                     }
                     float v = num * __builtin_amdgcn_rcpf(den);
                     if (a.gating) v = v * __builtin_amdgcn_rcpf(1.0f + __expf(-gsAll[j * XHD + lane])); // inference.cu:248
@@ -940,8 +992,6 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
                 if (dbg) P.timing[16 * (P.NL + 1) + 4 * wg + 2] = wave < nh ? wall_clock64() : 0;
                 W_STAMP(15);
                 if (!ok) { S.ctl[0] = 1; astu(P.abortFlag, 1u); }
-                // first tile of this wave for the next layer pass (the next step's first layer sees one more row)
-                if (!(lastLayer && step == P.steps - 1) && (!HYB || uni(Ln.kind) == MLH_KIND_ATTENTION)) issueKV(Ln, lastLayer ? pos + 1 : pos);
             }
             // gate/up rows of this wave's first two FFN units, and the second gain vector
             {
@@ -961,28 +1011,34 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
             if (nh > 0) {
                 const int rs = lane / CPS, c = lane % CPS;
                 const int ad = uni(L.ad);
-                for (int p = 0; (p * XLW + lw) * N < d; p++) {
+                auto pass = [&](int p, const typename PVec<WT>::Raw* w, float plwv) __attribute__((always_inline)) { // N rows; w: this lane's chunk of every head segment
                     const int row = (p * XLW + lw) * N + rs;
                     float acc = 0.f;
 #pragma unroll
                     for (int j = 0; j < XNH; j++)
-                        if (j < nh) {
-                            const typename PVec<WT>::Raw w = p == 0 ? s2.r[j] : p == 1 ? s2.r[XNH + j]
-                                : PVec<WT>::load(uni_ptr((const WT*)L.Wo) + (size_t)row * ad + slice_of<G>(X, j) * XHD + c * N);
-                            acc = chunk_dot_lds<WT>(w, S.as + j * XHD + c * N, acc);
-                        }
-                    if constexpr (HYB) { // + pleUp . e over the XCD's PLE columns (one column per lane of the row group)
-                        if (pleX > 0) {
-                            const float w = p == 0 ? plw[0] : p == 1 ? plw[1]
-                                                  : PVec<WT>::one(uni_ptr((const WT*)L.pleUp) + (size_t)row * a.ple + X * pleX + min(c, pleX - 1));
-                            if (c < pleX) acc = fmaf(w, S.es[c], acc);
-                        }
-                    }
+                        if (j < nh) acc = chunk_dot_lds<WT>(w[j], S.as + j * XHD + c * N, acc);
+                    if constexpr (HYB) // + pleUp . e over the XCD's PLE columns (one column per lane of the row group)
+                        if (pleX > 0 && c < pleX) acc = fmaf(plwv, S.es[c], acc);
                     acc = pgroup_sum<CPS>(acc);
                     if (c == 0) xst(P.h1P + (size_t)X * d + row, acc, lt);
+                };
+                // The prefetched passes stand alone: a path with loads of its own joining theirs would make every use wait for
+                // all that is in flight, the weights of the next phase included (0.9 us instead of 0.1).
+                if (lw * N < d) pass(0, s2.r, plw[0]);
+                if ((XLW + lw) * N < d) pass(1, s2.r + XNH, plw[1]);
+                for (int p = 2; (p * XLW + lw) * N < d; p++) {
+                    const int row = (p * XLW + lw) * N + rs;
+                    typename PVec<WT>::Raw w[XNH];
+#pragma unroll
+                    for (int j = 0; j < XNH; j++) w[j] = PVec<WT>::load(uni_ptr((const WT*)L.Wo) + (size_t)row * ad + slice_of<G>(X, min(j, nh - 1)) * XHD + c * N);
+                    float pw = 0.f;
+                    if constexpr (HYB) if (pleX > 0) pw = PVec<WT>::one(uni_ptr((const WT*)L.pleUp) + (size_t)row * a.ple + X * pleX + min(c, pleX - 1));
+                    pass(p, w, pw);
                 }
             }
             W_STAMP(14);
+            // first tile of this wave for the next layer pass (the next step's first layer sees one more row)
+            if (wave < XAW && !(lastLayer && step == P.steps - 1) && (!HYB || uni(Ln.kind) == MLH_KIND_ATTENTION)) issueKV(Ln, lastLayer ? pos + 1 : pos);
             issue_w2<WT>(s2, uni_ptr((const WT*)L.W2), X, fs, F, wbE, d);
             X_BARRIER(); // 4
             // ------------------------------------------------------------------ phase D
@@ -1008,15 +1064,7 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
                 }
             }
             W_STAMP(7);
-            if (!lastLayer) {
-                issueA(Ln);
-            } else { // LM-head rows gwl, gwl + TWL, ... and the final gain
-                int rows[XS1];
-#pragma unroll
-                for (int k = 0; k < XS1; k++) rows[k] = min(gwl + TWL * k, V - 1);
-                issue_rows<WT, XS1, NCH>(s1.r, E, d, rows);
-                issue_gain<WT, NCH>(gn, a.gF);
-            }
+            issueA(Ln, lastLayer);
             X_BARRIER(); // 5
             // ------------------------------------------------------------------ phase E
             {
@@ -1025,20 +1073,25 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
                 const int CR = fs / N;
                 const WT* W2x = uni_ptr((const WT*)L.W2) + (size_t)X * fs;
                 if (wbE * 4 < d) {
-                    float val = 0.f;
+                    float acc[4], val = 0.f;
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
-                        const int row = min(wbE * 4 + k, d - 1);
-                        float acc = 0.f;
+                        acc[k] = 0.f;
 #pragma unroll
                         for (int c0 = 0; c0 < 2; c0++) {
                             const int cc = lane + 64 * c0;
-                            if (cc < CR) acc = chunk_dot_lds<WT>(s2.r[k * 2 + c0], S.us + cc * N, acc);
+                            if (cc < CR) acc[k] = chunk_dot_lds<WT>(s2.r[k * 2 + c0], S.us + cc * N, acc[k]);
                         }
+                    }
+                    if (CR > 128) // (apart from the prefetched columns: see the output projection)
                         for (int cc = lane + 128; cc < CR; cc += 64)
-                            acc = chunk_dot_lds<WT>(PVec<WT>::load(W2x + (size_t)row * F + cc * N), S.us + cc * N, acc);
-                        acc = pwave_sum(acc);
-                        val = lane == k ? acc : val;
+#pragma unroll
+                            for (int k = 0; k < 4; k++)
+                                acc[k] = chunk_dot_lds<WT>(PVec<WT>::load(W2x + (size_t)min(wbE * 4 + k, d - 1) * F + cc * N), S.us + cc * N, acc[k]);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const float t4 = pwave_sum(acc[k]);
+                        val = lane == k ? t4 : val;
                     }
                     if (lane < 4 && wbE * 4 + lane < d) xst(P.xP + (size_t)X * d + wbE * 4 + lane, val, lt); // inference.cu:283-291 (the readers add the residual)
                 }
@@ -1056,15 +1109,8 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
                 }
             }
             W_STAMP(9);
-            if (!lastLayer) {
-                issue_wo<WT, G>(s2, uni_ptr((const WT*)Ln.Wo), uni(Ln.ad), X, nh, a.heads, lw, d);
-                issuePlw(Ln);
-            } else {
-                // two more LM-head rows; the second register set has room for them when a row has at most 4 chunks
-                const int rows[2] = {min(gwl + XS1 * TWL, V - 1), min(gwl + (XS1 + 1) * TWL, V - 1)};
-                typename PVec<WT>::Raw (&lm)[2 * NCH] = reinterpret_cast<typename PVec<WT>::Raw (&)[2 * NCH]>(s2.r);
-                issue_rows<WT, 2, NCH>(lm, E, d, rows);
-            }
+            issueWo(Ln, lastLayer);
+            issuePlw(Ln);
         }
 
         // ---------------------------------------------------------------------- LM head + argmax
@@ -1100,9 +1146,8 @@ __device__ __forceinline__ void xcd_worker(const XcdArgs& P, const XShared& S, i
         }
         if (step + 1 < P.steps) { // first layer of the next step
             const LayerDev& L0 = S.Ls[P.NL - 1];
-            issueA(L0);
-            issue_wo<WT, G>(s2, uni_ptr((const WT*)L0.Wo), uni(L0.ad), X, nh, a.heads, lw, d);
-            issuePlw(L0);
+            issueA(L0, false);
+            issueWo(L0, false); // (its PLE columns are there: the last layer fetched them)
         }
         X_BARRIER(); // best logits in LDS
         X_BARRIER(); // next token in LDS
@@ -1159,7 +1204,8 @@ __global__ void __launch_bounds__(XWG) k_decode_xcd(XcdArgs P) {
     const int X = uni(S.ctl[2]), r = uni(S.ctl[3]);
     const int tok = uni(a.tok[0]), pos = uni(a.pos[P.seq]);
     const unsigned tagBase = *P.tagCounter; // tags do not repeat from launch to launch (the host clears everything before the count wraps)
-    if (wave == XWORK) xcd_communicator<WT, HYB, G>(P, S, tok, pos, tagBase, X, r);
+    if (wave == XWORK) __builtin_amdgcn_s_setprio(3); // the communicator's few instructions are the critical path, the prefetches of the others are not (2 %)
+    if (wave == XWORK) xcd_communicator<WT, NCH, HYB, G>(P, S, tok, pos, tagBase, X, r);
     else xcd_worker<WT, NCH, HYB, G>(P, S, tok, pos, tagBase, X, r);
 }
 

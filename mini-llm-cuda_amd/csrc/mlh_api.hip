@@ -242,7 +242,7 @@ extern "C" int mlh_create(const mlh_hparams* hpIn, int device, mlh_ctx** out) {
         // Measured one at a time and in combination on the benchmark shapes: a short stay away from the FFN activations
         // and the softmax partials pays from dim 768 on (+0.6 %), and costs 2 % on the 256-wide model.
         const bool wideModel = hp.dim >= 512;
-        const int dflt[5] = {44, 0, 0, wideModel ? 6 : 0, wideModel ? 16 : 0};
+        const int dflt[5] = {wideModel ? 37 : 28, 0, 0, wideModel ? 6 : 0, wideModel ? 16 : 0};
         for (int k = 0; k < 5; k++) c->xcdNap[k] = knob(names[k], dflt[k], 0, 400);
     }
 
