@@ -1385,8 +1385,7 @@ static int ensure_prefill_buffers(mlh_ctx* c, int rows) {
     for (void* p : c->pfAllocs) (void)hipFree(p);
     c->pfAllocs.clear();
     c->pfRows = 0;
-    for (int g = 0; g < 2; g++) // captured batched steps hold the old buffer addresses
-        if (c->graphExec[g]) { (void)hipGraphExecDestroy(c->graphExec[g]); c->graphExec[g] = nullptr; }
+    mlh_drop_graphs(c); // captured batched steps hold the old buffer addresses
     const size_t n = (size_t)rows, wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 6; // GEMM input elements: halves, or three bf16 planes
     auto alloc = [&](void** p, size_t bytes) -> int {
         MLH_CHECK(c, hipMalloc(p, std::max<size_t>(bytes, 16)));

@@ -52,6 +52,11 @@ int mlh_pin(mlh_ctx* c, PinBuf& b, size_t bytes) {
     return 0;
 }
 
+void mlh_drop_graphs(mlh_ctx* c) {
+    for (hipGraphExec_t& g : c->graphExec)
+        if (g) { (void)hipGraphExecDestroy(g); g = nullptr; }
+}
+
 static int fail_create(const std::string& msg) {
     g_create_error = msg;
     return -1;
@@ -97,7 +102,7 @@ extern "C" void mlh_destroy(mlh_ctx* c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    for (int i = 0; i < 2; i++) if (c->graphExec[i]) (void)hipGraphExecDestroy(c->graphExec[i]);
+    mlh_drop_graphs(c);
     for (void* p : c->allocs) (void)hipFree(p);
     for (void* p : c->pfAllocs) (void)hipFree(p);
     for (void* p : c->mirrorAllocs) (void)hipFree(p);
@@ -404,6 +409,7 @@ extern "C" int mlh_finalize(mlh_ctx* c) {
             }
     }
     (void)hipSetDevice(c->device);
+    mlh_drop_graphs(c); // recorded launches hold the addresses of the operands that are rebuilt below
     int rc = mlh_init_kernels(c);
     if (rc == 0) rc = mlh_init_prefill_kernels(c);
     if (rc == 0) rc = mlh_build_gemm_operands(c);
@@ -627,9 +633,7 @@ extern "C" int mlh_forward_full(mlh_ctx* c, int seq, const int32_t* ids, int n, 
 extern "C" int mlh_set_prefill_mode(mlh_ctx* c, int mode) {
     if (!c) return -1;
     if (mode != 0 && mode != 1) { c->err = "prefill mode must be 0 (auto) or 1 (token by token)"; return -1; }
-    if (mode != c->prefillMode)
-        for (int g = 0; g < 2; g++) // a captured step follows the mode it was captured under
-            if (c->graphExec[g]) { (void)hipGraphExecDestroy(c->graphExec[g]); c->graphExec[g] = nullptr; }
+    if (mode != c->prefillMode) mlh_drop_graphs(c); // a captured step follows the mode it was captured under
     c->prefillMode = mode;
     return 0;
 }
@@ -885,9 +889,7 @@ extern "C" int mlh_read_probs(mlh_ctx* c, int seq, float* out) {
 extern "C" int mlh_set_sampling(mlh_ctx* c, float temperature, unsigned long long seed) {
     if (!c) return -1;
     if (!(temperature >= 0.f) || temperature > 1.0e4f) { c->err = "sampling temperature must be in [0, 1e4]"; return -1; }
-    if (c->temperature != temperature || c->sampleSeed != seed)
-        for (int g = 0; g < 2; g++) // recorded launches carry the old values in their kernel arguments
-            if (c->graphExec[g]) { (void)hipGraphExecDestroy(c->graphExec[g]); c->graphExec[g] = nullptr; }
+    if (c->temperature != temperature || c->sampleSeed != seed) mlh_drop_graphs(c); // recorded launches carry the old values in their kernel arguments
     c->temperature = temperature;
     c->sampleSeed = seed;
     return 0;

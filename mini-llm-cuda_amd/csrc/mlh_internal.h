@@ -215,6 +215,7 @@ void mlh_fill_args(mlh_ctx* c, StepArgs& a, int nseq, const int* tokPtr);
 int mlh_launch_copy(mlh_ctx* c);
 int mlh_dev_alloc_bytes(mlh_ctx* c, void** p, size_t bytes); // mlh_api.hip: an allocation owned by the context
 int mlh_pin(mlh_ctx* c, PinBuf& b, size_t bytes);                    // ... and its pinned memory
+void mlh_drop_graphs(mlh_ctx* c);                                    // ... and its captured steps, before anything they hold the address of goes
 int mlh_launch_probs(mlh_ctx* c, int seq);
 int mlh_init_kernels(mlh_ctx* c);
 

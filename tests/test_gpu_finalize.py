@@ -1,0 +1,49 @@
+"""A context whose tensors are uploaded and finalized again (include/mlh.h) against a context that only ever had the new ones."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def config(pkg, bf16=0, **kw):
+    hp = pkg.config(3, dim=256, attnHeads=4, headDim=64, ffnDim=704, transformers=4, vocabSize=1000, gdnHeads=4, pleDim=64, maxL=160,
+                    weightDtype=bf16, **kw)
+    pkg.set_layer_pattern(hp, 1)
+    return hp
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("nseq,graph", [(1, 1), (3, 1), (3, 4), (9, 2)])
+def test_graphs_follow_a_repeated_finalize(pkg, bf16, nseq, graph):
+    """A finalize replaces the operands whose addresses a captured step holds: the next decode must not replay the old capture."""
+    hp = config(pkg, bf16, maxSeqs=nseq)
+    old, new = (pkg.Model.generate(hp, seed).randomize_gains(seed) for seed in (5, 6))
+    prompts = [pkg.random_tokens(5, s, hp.vocabSize, 20 + 3 * s) for s in range(nseq)]
+
+    def decode(dev):
+        dev.reset()
+        dev.prefill_batch(list(range(nseq)), prompts)
+        firsts = [dev.greedy_token(s) for s in range(nseq)]
+        runs = [dev.decode_loop(firsts, 9)]  # whole replays and a remainder
+        for _ in range(2):
+            dev.synchronize()
+            runs.append(dev.decode_loop(runs[-1][-1], 9))
+        return np.concatenate(runs), np.stack([dev.logits(s) for s in range(nseq)])
+
+    def device(model):
+        dev = pkg.Device(hp, 0)
+        dev.set_persistent(0)
+        dev.set_graph(graph)
+        dev.upload(model)
+        return dev
+
+    dev = device(old)
+    before = decode(dev)
+    dev.upload(new)
+    got = decode(dev)
+    dev.close()
+    dev = device(new)
+    want = decode(dev)
+    dev.close()
+    assert not np.array_equal(before[1], want[1])
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
