@@ -100,7 +100,12 @@ int mlh_upload_tensor(mlh_ctx* ctx, int layer, int tensor_id, const float* host,
 int mlh_upload_rope_table(mlh_ctx* ctx, const float* tab, int n);
 
 /* Must be called once after the uploads and before any forward call: checks
- * that every tensor the hyper-parameters require has arrived. */
+ * that every tensor the hyper-parameters require has arrived.
+ * Infinities and NaN go through the products as fp32 arithmetic has them.  The MFMA kernels multiply sums of planes, where an
+ * infinity would become NaN: a model with a matrix element that is infinite, NaN or (fp32) 3.3962e38 or more, or a gain of 2^60
+ * or more, runs without them, its prompts token by token.  Two limits remain: an activation of 3.3962e38 or more counts as
+ * NaN (the next norm's sum of squares has overflowed by then), and a sum with terms of 0.99 of the largest float may
+ * be infinite. */
 int mlh_finalize(mlh_ctx* ctx);
 
 /* Empties a sequence (length 0, GDN states zero).  seq = -1: all sequences.

@@ -1259,7 +1259,10 @@ int mlh_launch_softmax_rows(mlh_ctx* c, const float* logits, float* probs, const
 // ----------------------------------------------------------------------------
 static int cdiv(int a, int b) { return (a + b - 1) / b; }
 
-bool mlh_prefill_gemm_supported(const mlh_ctx* c) {
+bool mlh_prefill_gemm_supported(const mlh_ctx* c) { return c->operands; }
+
+// widths that the MFMA kernels take: whole chunks of 128 bytes
+static bool operand_widths(const mlh_ctx* c) {
     const mlh_hparams& hp = c->hp;
     const int esz = c->wbytes, kmul = 128 / esz;
     if (hp.dim % kmul || hp.ffnDim % kmul || (hp.pleDim && hp.pleDim % kmul)) return false;
@@ -1312,6 +1315,55 @@ static int build_mirror(mlh_ctx* c, const void* src, size_t n, const void** dst,
     return 0;
 }
 
+// Sets *found when the magnitude of an element (as bits: infinities and NaN are the largest) reaches `limit`.
+template <typename WT>
+__global__ void __launch_bounds__(256) k_find_beyond(const uint4* __restrict__ w, size_t n16, uint32_t limit, unsigned* found) {
+    bool any = false;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) {
+        const uint4 v = w[i];
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            if (sizeof(WT) == 4) any = any || (x[e] & 0x7fffffffu) >= limit;
+            else any = any || (x[e] & 0x7fffu) >= limit || (x[e] >> 16 & 0x7fffu) >= limit;
+        }
+    }
+    if (any) *found = 1;
+}
+
+// Whether the MFMA kernels may multiply this model's matrices.  Their products are sums over planes (of the activations, and of fp32
+// weights) or of scaled halves, which an infinite operand turns into NaN where inf * x is infinite; the GEMV and
+// single-launch kernels multiply in fp32 and keep it.  So no weight may lie beyond the planes, and no gain above 2^60: rows
+// are multiplied by it before they are normalised, and their squares overflow from 2^64 on.  One pass over the weights per finalize.
+static int operand_values(mlh_ctx* c, bool* within) {
+    const mlh_hparams& hp = c->hp;
+    const size_t d = hp.dim, F = hp.ffnDim, pl = hp.pleDim;
+    unsigned* found = nullptr;
+    unsigned h = 0;
+    MLH_CHECK(c, hipMalloc((void**)&found, 4));
+    hipError_t e = hipMemsetAsync(found, 0, 4, c->stream);
+    auto matrix = [&](const void* w, size_t n) { // (rows are multiples of 128 bytes)
+        if (c->wbytes == 4) hipLaunchKernelGGL((k_find_beyond<float>), dim3(2048), dim3(256), 0, c->stream, (const uint4*)w, n / 4, P3_BEYOND, found);
+        else hipLaunchKernelGGL((k_find_beyond<bf16_t>), dim3(2048), dim3(256), 0, c->stream, (const uint4*)w, n / 8, 0x7f80u, found);
+    };
+    auto gain = [&](const float* g) { hipLaunchKernelGGL((k_find_beyond<float>), dim3(4), dim3(256), 0, c->stream, (const uint4*)g, d / 4, 0x5d800000u, found); };
+    matrix(c->E, (size_t)hp.vocabSize * d);
+    gain(c->gF);
+    for (const LayerDev& L : c->layers) {
+        matrix(L.Wa, L.rowsA * d); matrix(L.Wo, d * L.ad); matrix(L.W13, 2 * F * d); matrix(L.W2, d * F);
+        if (pl) matrix(L.pleUp, d * pl);
+        gain(L.g1); gain(L.g2);
+    }
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(&h, found, 4, hipMemcpyDeviceToHost, c->stream);
+    const hipError_t e2 = hipStreamSynchronize(c->stream);
+    (void)hipFree(found);
+    MLH_CHECK(c, e);
+    MLH_CHECK(c, e2);
+    *within = h == 0;
+    return 0;
+}
+
 // An fp32 matrix as three bf16 planes, what the tiled products of the prefill multiply.
 static int build_planes(mlh_ctx* c, const void* src, int rows, int cols, const void** dst) {
     void* buf = nullptr;
@@ -1324,18 +1376,22 @@ static int build_planes(mlh_ctx* c, const void* src, int rows, int cols, const v
 
 int mlh_build_gemm_operands(mlh_ctx* c) {
     const mlh_hparams& hp = c->hp;
-    const bool supported = mlh_prefill_gemm_supported(c), mirror = hp.weightDtype == MLH_DTYPE_BF16 && supported;
-    const bool planes = hp.weightDtype == MLH_DTYPE_F32 && supported;
-    c->pfDtype = planes ? MLH_GEMM_P3 : mirror ? MLH_GEMM_F16 : hp.weightDtype;
+    c->operands = false;
     c->f16Inexact = 0;
     for (void* p : c->mirrorAllocs) (void)hipFree(p); // a repeated finalize rebuilds them
     c->mirrorAllocs.clear();
+    for (LayerDev& L : c->layers) L.WaP = L.WoP = L.W13P = L.W2P = L.WaR = L.WoR = L.W13R = L.W2R = nullptr;
+    c->EP = c->ER = nullptr;
+    if (!operand_widths(c)) return 0;
+    int rc = 0;
+    bool within = false;
+    if ((rc = operand_values(c, &within)) || !within) return rc;
+    const bool mirror = hp.weightDtype == MLH_DTYPE_BF16, planes = !mirror;
+    c->pfDtype = planes ? MLH_GEMM_P3 : MLH_GEMM_F16;
     unsigned* d_scratch = nullptr;
     if (mirror) { MLH_CHECK(c, hipMalloc((void**)&d_scratch, 8)); }
-    int rc = 0;
     const size_t d = hp.dim, F = hp.ffnDim, pl = hp.pleDim, wb = c->wbytes;
     for (LayerDev& L : c->layers) {
-        L.WaP = L.Wa; L.WoP = L.Wo; L.W13P = L.W13; L.W2P = L.W2;
         L.sWa = L.sWo = L.sW13 = L.sW2 = 1.0f;
         const void* wo = L.Wo;
         if (pl > 0) { // [Wo | pleUp] along K, in the storage type
@@ -1357,10 +1413,11 @@ int mlh_build_gemm_operands(mlh_ctx* c) {
             (rc = build_mirror(c, L.W2, d * F, &L.W2P, &L.sW2, d_scratch)))
             break;
     }
-    c->EP = c->E; c->sE = 1.0f;
+    c->sE = 1.0f;
     if (rc == 0 && mirror) rc = build_mirror(c, c->E, (size_t)hp.vocabSize * hp.dim, &c->EP, &c->sE, d_scratch);
     if (rc == 0 && planes) rc = build_planes(c, c->E, hp.vocabSize, hp.dim, &c->EP);
     if (d_scratch) (void)hipFree(d_scratch);
+    c->operands = rc == 0;
     return rc;
 }
 

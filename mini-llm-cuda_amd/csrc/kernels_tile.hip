@@ -375,7 +375,16 @@ __global__ void __launch_bounds__(256) k_split_p3(const float* __restrict__ src,
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = c + e < cols ? src[(size_t)r * lds_ + c + e] : 0.f;
-        p3_put4((unsigned char*)dst + (size_t)r * ldd * 6, c, v[0], v[1], v[2], v[3]);
+        unsigned char* row = (unsigned char*)dst + (size_t)r * ldd * 6;
+        p3_put4(row, c, v[0], v[1], v[2], v[3]);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (p3_beyond(v[e])) {
+                uint32_t h[3];
+                p3_split_beyond(v[e], h);
+#pragma unroll
+                for (int k = 0; k < 3; k++) *reinterpret_cast<uint16_t*>(row + p3_offset(c + e) + k * P3_PLANE) = (uint16_t)h[k];
+            }
     }
 }
 hipError_t mlh_split_p3(hipStream_t stream, const float* src, int lds_, void* dst, int ldd, int rows, int cols) {

@@ -20,7 +20,13 @@ struct p3_t { uint16_t bits[3]; }; // only its size (6 bytes per element) is use
 typedef float p3_f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 p3_bf16x2 __attribute__((ext_vector_type(2)));
 
-// the planes of two neighbouring elements, packed two to a word
+// Magnitudes from here on (as bits: infinities and NaN too) have no finite bf16 nearest to them.
+#define P3_BEYOND 0x7f7f8000u
+__device__ __forceinline__ bool p3_beyond(float v) { return (__float_as_uint(v) & 0x7fffffffu) >= P3_BEYOND; }
+
+// The planes of two neighbouring elements, packed two to a word.  Beyond P3_BEYOND they make NaN of every product: weights and gains
+// that reach it keep a model off this path (mlh_build_gemm_operands).  An activation that does has overflowed: its row's sum of
+// squares is infinite or NaN at the next norm, whatever this product gives.
 __device__ __forceinline__ void p3_split2(float a, float b, uint32_t (&w)[3]) {
 #pragma unroll
     for (int p = 0; p < 3; p++) {
@@ -31,6 +37,25 @@ __device__ __forceinline__ void p3_split2(float a, float b, uint32_t (&w)[3]) {
     }
 }
 __device__ __forceinline__ size_t p3_offset(int col) { return (size_t)(col >> 5) * P3_BYTES + (size_t)(col & 31) * 2; }
+// The planes of an element beyond.  An infinity goes into the plane that meets the other operand's hi plane alone, with
+// +-1 in front of it: its plane products with a finite b are +-b, 0 and the infinity times hi(b), so their sum is what inf * b
+// is (NaN for b = 0), and with another infinity it is that infinity.  The largest finite values are cut instead of rounded (no
+// plane exceeds the value; exact as well).
+__device__ __forceinline__ void p3_split_beyond(float a, uint32_t (&h)[3]) {
+    const uint32_t u = __float_as_uint(a);
+    if ((u & 0x7fffffffu) >= 0x7f800000u) {
+        const bool nan = (u & 0x7fffffu) != 0;
+        h[0] = nan ? 0x7fc0u : 0x3f80u | (u >> 31 << 15);
+        h[1] = 0;
+        h[2] = nan ? 0u : u >> 16;
+        return;
+    }
+    h[0] = u >> 16;
+    a -= __uint_as_float(u & 0xffff0000u);
+    h[1] = __float_as_uint(a) >> 16;
+    a -= __uint_as_float(h[1] << 16);
+    h[2] = __float_as_uint(a) >> 16;
+}
 // one element / four neighbouring elements (col a multiple of 4) of the row that starts at `row`
 __device__ __forceinline__ void p3_put(void* row, int col, float v) {
     uint32_t w[3];
