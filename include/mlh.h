@@ -108,6 +108,17 @@ int mlh_upload_rope_table(mlh_ctx* ctx, const float* tab, int n);
  * be infinite. */
 int mlh_finalize(mlh_ctx* ctx);
 
+/* Device memory: mlh_create allocates the matrices as uploaded (4 or 2 bytes an element).  mlh_finalize adds what the MFMA kernels
+ * read, where the widths allow them (mlh_set_prefill_mode): in fp32 10 bytes an element (three bf16 planes; the matrix in
+ * the decode step's order), with bf16 weights 4 (halves; that order), and [output projection | PLE up] once more.  So a context
+ * holds its matrices 3.5 times in fp32, 3 times in bf16.  The copies are made only if a prefill call over all
+ * maxSeqs * maxL positions (or a sixteenth of the device's memory, if that is less) still has room beside them; without
+ * them the context runs as with mlh_set_prefill_mode(ctx, 1), prompts token by token and decode steps through the GEMV or
+ * single-launch kernels.  mlh_limit_operands sets the most bytes they may take (0: none) from the next mlh_finalize on;
+ * mlh_operand_bytes is what they take now. */
+int mlh_limit_operands(mlh_ctx* ctx, uint64_t bytes);
+uint64_t mlh_operand_bytes(const mlh_ctx* ctx);
+
 /* Empties a sequence (length 0, GDN states zero).  seq = -1: all sequences.
  * The reference has one implicit sequence in seqTokenIndices (network_globals.h:147-148). */
 int mlh_reset(mlh_ctx* ctx, int seq);

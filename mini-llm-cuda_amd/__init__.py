@@ -72,6 +72,8 @@ _sigs_dev = {
     "mlh_upload_tensor": (c_int, [c_void_p, c_int, c_int, c_void_p, c_int, c_int]),
     "mlh_upload_rope_table": (c_int, [c_void_p, c_void_p, c_int]),
     "mlh_finalize": (c_int, [c_void_p]),
+    "mlh_limit_operands": (c_int, [c_void_p, c_uint64]),
+    "mlh_operand_bytes": (c_uint64, [c_void_p]),
     "mlh_reset": (c_int, [c_void_p, c_int]),
     "mlh_seq_len": (c_int, [c_void_p, c_int]),
     "mlh_max_len": (c_int, [c_void_p]),
@@ -287,6 +289,13 @@ class Device:
 
     def finalize(self):
         self._check(dev.mlh_finalize(self._h))
+
+    def limit_operands(self, nbytes):
+        """Most device bytes that the next finalize may spend on the copies of the matrices that the MFMA kernels read (0: none)."""
+        self._check(dev.mlh_limit_operands(self._h, int(nbytes)))
+
+    def operand_bytes(self):
+        return dev.mlh_operand_bytes(self._h)
 
     def reset(self, seq=-1):
         self._check(dev.mlh_reset(self._h, seq))

@@ -1293,10 +1293,18 @@ __global__ void k_bf16_to_f16(const bf16_t* __restrict__ w, f16_t* __restrict__ 
     if (bad) atomicAdd(inexact, bad);
 }
 
+int mlh_operand_alloc(mlh_ctx* c, void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) { (void)hipGetLastError(); return MLH_NO_ROOM; }
+    MLH_CHECK(c, e);
+    c->mirrorAllocs.push_back(*p);
+    c->operandBytes += bytes;
+    return 0;
+}
+
 static int build_mirror(mlh_ctx* c, const void* src, size_t n, const void** dst, float* alpha, unsigned* d_scratch) {
     void* buf = nullptr;
-    MLH_CHECK(c, hipMalloc(&buf, n * 2));
-    c->mirrorAllocs.push_back(buf);
+    if (const int rc = mlh_operand_alloc(c, &buf, n * 2)) return rc;
     MLH_CHECK(c, hipMemsetAsync(d_scratch, 0, 8, c->stream));
     hipLaunchKernelGGL(k_absmax_bf16, dim3(1024), dim3(256), 0, c->stream, (const bf16_t*)src, n, d_scratch);
     unsigned h[2] = {0, 0};
@@ -1367,58 +1375,94 @@ static int operand_values(mlh_ctx* c, bool* within) {
 // An fp32 matrix as three bf16 planes, what the tiled products of the prefill multiply.
 static int build_planes(mlh_ctx* c, const void* src, int rows, int cols, const void** dst) {
     void* buf = nullptr;
-    MLH_CHECK(c, hipMalloc(&buf, (size_t)rows * cols * 6));
-    c->mirrorAllocs.push_back(buf);
+    if (const int rc = mlh_operand_alloc(c, &buf, (size_t)rows * cols * 6)) return rc;
     MLH_CHECK(c, mlh_split_p3(c->stream, (const float*)src, cols, buf, cols, rows, cols));
     *dst = buf;
     return 0;
 }
 
-int mlh_build_gemm_operands(mlh_ctx* c) {
+// Work buffers of a prefill call of that many rows (ensure_prefill_buffers), within a few percent.
+static size_t prefill_row_bytes(const mlh_ctx* c) {
     const mlh_hparams& hp = c->hp;
+    const size_t wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 6, d = hp.dim;
+    return d * (8 + wb + (wb == 2 ? 4 : 0)) + (size_t)c->maxRowsA * 4 + ((size_t)c->maxAd + hp.pleDim + hp.ffnDim) * wb + 64;
+}
+
+// Whether the copies fit: into the caller's limit, and onto the device with room left for a prefill call over every position of the
+// context or, if that is less, a sixteenth of the device's memory.  Without them a model of which only the matrices
+// fit still runs (they take 2.5 times the matrices' bytes in fp32, twice in bf16, [Wo | pleUp] once more).
+static int operand_room(mlh_ctx* c, bool* fits) {
+    const mlh_hparams& hp = c->hp;
+    const size_t d = hp.dim, F = hp.ffnDim, pl = hp.pleDim, wb = c->wbytes, per = wb == 4 ? 10 : 4;
+    auto rows16 = [](size_t n) { return (n + 15) / 16 * 16; };
+    size_t need = rows16(hp.vocabSize) * d * per;
+    for (const LayerDev& L : c->layers)
+        need += (rows16(L.rowsA) * d + rows16(d) * (L.ad + pl) + rows16(2 * F) * d + rows16(d) * F) * per + (pl ? d * (L.ad + pl) * wb : 0);
+    size_t free = 0, total = 0;
+    MLH_CHECK(c, hipMemGetInfo(&free, &total));
+    const size_t row = prefill_row_bytes(c), work = std::min((size_t)hp.maxSeqs * hp.maxL * row, total / 16), have = c->pfRows * row; // (of earlier calls)
+    *fits = need <= c->operandLimit && need + (work > have ? work - have : 0) <= free;
+    return 0;
+}
+
+void mlh_drop_operands(mlh_ctx* c) {
     c->operands = false;
-    c->f16Inexact = 0;
-    for (void* p : c->mirrorAllocs) (void)hipFree(p); // a repeated finalize rebuilds them
+    for (void* p : c->mirrorAllocs) (void)hipFree(p);
     c->mirrorAllocs.clear();
+    c->operandBytes = 0;
     for (LayerDev& L : c->layers) L.WaP = L.WoP = L.W13P = L.W2P = L.WaR = L.WoR = L.W13R = L.W2R = nullptr;
     c->EP = c->ER = nullptr;
-    if (!operand_widths(c)) return 0;
-    int rc = 0;
-    bool within = false;
-    if ((rc = operand_values(c, &within)) || !within) return rc;
-    const bool mirror = hp.weightDtype == MLH_DTYPE_BF16, planes = !mirror;
-    c->pfDtype = planes ? MLH_GEMM_P3 : MLH_GEMM_F16;
-    unsigned* d_scratch = nullptr;
-    if (mirror) { MLH_CHECK(c, hipMalloc((void**)&d_scratch, 8)); }
+}
+
+// The planes or halves; on MLH_NO_ROOM what has been allocated so far is still there.
+static int build_operands(mlh_ctx* c, unsigned* d_scratch) {
+    const mlh_hparams& hp = c->hp;
+    const bool mirror = hp.weightDtype == MLH_DTYPE_BF16;
     const size_t d = hp.dim, F = hp.ffnDim, pl = hp.pleDim, wb = c->wbytes;
+    int rc = 0;
     for (LayerDev& L : c->layers) {
         L.sWa = L.sWo = L.sW13 = L.sW2 = 1.0f;
         const void* wo = L.Wo;
         if (pl > 0) { // [Wo | pleUp] along K, in the storage type
             void* cat = nullptr;
-            MLH_CHECK(c, hipMalloc(&cat, d * (L.ad + pl) * wb));
-            c->mirrorAllocs.push_back(cat);
+            if ((rc = mlh_operand_alloc(c, &cat, d * (L.ad + pl) * wb))) return rc;
             MLH_CHECK(c, hipMemcpy2D(cat, (L.ad + pl) * wb, L.Wo, L.ad * wb, L.ad * wb, d, hipMemcpyDeviceToDevice));
             MLH_CHECK(c, hipMemcpy2D((char*)cat + L.ad * wb, (L.ad + pl) * wb, L.pleUp, pl * wb, pl * wb, d, hipMemcpyDeviceToDevice));
             wo = cat;
         }
         L.WoR = wo;
-        if (planes && ((rc = build_planes(c, L.Wa, L.rowsA, (int)d, &L.WaP)) || (rc = build_planes(c, wo, (int)d, L.ad + (int)pl, &L.WoP)) ||
-                       (rc = build_planes(c, L.W13, 2 * (int)F, (int)d, &L.W13P)) || (rc = build_planes(c, L.W2, (int)d, (int)F, &L.W2P))))
-            break;
-        if (!mirror) continue;
-        if ((rc = build_mirror(c, L.Wa, (size_t)L.rowsA * d, &L.WaP, &L.sWa, d_scratch)) ||
-            (rc = build_mirror(c, wo, d * (L.ad + pl), &L.WoP, &L.sWo, d_scratch)) ||
-            (rc = build_mirror(c, L.W13, 2 * F * d, &L.W13P, &L.sW13, d_scratch)) ||
-            (rc = build_mirror(c, L.W2, d * F, &L.W2P, &L.sW2, d_scratch)))
-            break;
+        if (mirror) {
+            if ((rc = build_mirror(c, L.Wa, (size_t)L.rowsA * d, &L.WaP, &L.sWa, d_scratch)) ||
+                (rc = build_mirror(c, wo, d * (L.ad + pl), &L.WoP, &L.sWo, d_scratch)) ||
+                (rc = build_mirror(c, L.W13, 2 * F * d, &L.W13P, &L.sW13, d_scratch)) ||
+                (rc = build_mirror(c, L.W2, d * F, &L.W2P, &L.sW2, d_scratch)))
+                return rc;
+        } else {
+            if ((rc = build_planes(c, L.Wa, L.rowsA, (int)d, &L.WaP)) || (rc = build_planes(c, wo, (int)d, L.ad + (int)pl, &L.WoP)) ||
+                (rc = build_planes(c, L.W13, 2 * (int)F, (int)d, &L.W13P)) || (rc = build_planes(c, L.W2, (int)d, (int)F, &L.W2P)))
+                return rc;
+        }
     }
     c->sE = 1.0f;
-    if (rc == 0 && mirror) rc = build_mirror(c, c->E, (size_t)hp.vocabSize * hp.dim, &c->EP, &c->sE, d_scratch);
-    if (rc == 0 && planes) rc = build_planes(c, c->E, hp.vocabSize, hp.dim, &c->EP);
-    if (d_scratch) (void)hipFree(d_scratch);
+    return mirror ? build_mirror(c, c->E, (size_t)hp.vocabSize * hp.dim, &c->EP, &c->sE, d_scratch) : build_planes(c, c->E, hp.vocabSize, hp.dim, &c->EP);
+}
+
+int mlh_build_gemm_operands(mlh_ctx* c) {
+    mlh_drop_operands(c); // a repeated finalize rebuilds them
+    c->f16Inexact = 0;
+    if (!operand_widths(c)) return 0;
+    int rc = 0;
+    bool ok = false;
+    if ((rc = operand_values(c, &ok)) || !ok || (rc = operand_room(c, &ok)) || !ok) return rc;
+    c->pfDtype = c->hp.weightDtype == MLH_DTYPE_BF16 ? MLH_GEMM_F16 : MLH_GEMM_P3;
+    unsigned* d_scratch = nullptr;
+    MLH_CHECK(c, hipMalloc((void**)&d_scratch, 8));
+    rc = build_operands(c, d_scratch);
+    (void)hipFree(d_scratch);
+    if (rc == 0) rc = mlh_rows_prepare(c);
+    if (rc) mlh_drop_operands(c);
     c->operands = rc == 0;
-    return rc;
+    return rc == MLH_NO_ROOM ? 0 : rc; // (another context or process took the room in between)
 }
 
 // The headDim-128 attention tiles exceed the 64 KB a launch may use without opting in.

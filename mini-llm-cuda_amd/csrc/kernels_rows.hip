@@ -444,8 +444,7 @@ static int pack(mlh_ctx* c, const void* src, int rows, int cols, const void** ds
     const int rowBytes = cols * c->wbytes;
     const size_t pieces = (size_t)((rows + RW_TILE - 1) / RW_TILE) * RW_TILE * rowBytes / 16;
     void* buf = nullptr;
-    MLH_CHECK(c, hipMalloc(&buf, pieces * 16));
-    c->mirrorAllocs.push_back(buf);
+    if (const int rc = mlh_operand_alloc(c, &buf, pieces * 16)) return rc;
     hipLaunchKernelGGL(k_rows_pack, dim3(4096), dim3(256), 0, c->stream, (const unsigned char*)src, (unsigned char*)buf, rows, rowBytes, pieces);
     MLH_CHECK(c, hipGetLastError());
     *dst = buf;

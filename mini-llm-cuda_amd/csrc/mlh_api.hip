@@ -409,11 +409,11 @@ extern "C" int mlh_finalize(mlh_ctx* c) {
             }
     }
     (void)hipSetDevice(c->device);
-    mlh_drop_graphs(c); // recorded launches hold the addresses of the operands that are rebuilt below
+    c->finalized = false; // until everything below has been rebuilt
+    mlh_drop_graphs(c);   // recorded launches hold the addresses of the operands
     int rc = mlh_init_kernels(c);
     if (rc == 0) rc = mlh_init_prefill_kernels(c);
     if (rc == 0) rc = mlh_build_gemm_operands(c);
-    if (rc == 0 && mlh_prefill_gemm_supported(c)) rc = mlh_rows_prepare(c);
     if (rc) return rc;
     MLH_CHECK(c, hipMemcpy(c->d_layers, c->layers.data(), c->layers.size() * sizeof(LayerDev), hipMemcpyHostToDevice));
     // function attributes and occupancy of the single-launch decode kernels, here and not on every launch
@@ -424,6 +424,14 @@ extern "C" int mlh_finalize(mlh_ctx* c) {
     c->finalized = true;
     return 0;
 }
+
+extern "C" int mlh_limit_operands(mlh_ctx* c, uint64_t bytes) {
+    if (!c) return -1;
+    c->operandLimit = (size_t)bytes;
+    return 0;
+}
+
+extern "C" uint64_t mlh_operand_bytes(const mlh_ctx* c) { return c ? c->operandBytes : 0; }
 
 static int check_ready(mlh_ctx* c) {
     if (!c) return -1;

@@ -186,6 +186,7 @@ struct mlh_ctx {
     int pfDtype = MLH_DTYPE_F32; // operand type of those: MLH_GEMM_P3 or MLH_GEMM_F16
     bool operands = false;     // the copies of the matrices that the MFMA kernels read (LayerDev::WaP .. W2R) exist
     std::vector<void*> mirrorAllocs;
+    size_t operandBytes = 0, operandLimit = SIZE_MAX; // what they take and may take
     long f16Inexact = 0;       // bf16 weights that had no exact scaled-half representation (reported at finalize)
     void* gemmWs = nullptr;    // split-K workspace of the skinny GEMM
 
@@ -245,7 +246,10 @@ void mlh_set_thread_error(const std::string& msg);
 #define MLH_PREFILL_GEMM_MIN_ROWS 16 // bf16 models: calls of fewer tokens keep fp32 activations throughout
 bool mlh_prefill_gemm_supported(const mlh_ctx* c);
 int mlh_init_prefill_kernels(mlh_ctx* c);
-int mlh_build_gemm_operands(mlh_ctx* c); // at finalize: planes or halves of every matrix, where the model's widths and weights allow
+#define MLH_NO_ROOM (-4) // inside a finalize only: a copy does not fit on the device
+int mlh_operand_alloc(mlh_ctx* c, void** p, size_t bytes); // memory of the copies: 0, MLH_NO_ROOM or an error
+void mlh_drop_operands(mlh_ctx* c);
+int mlh_build_gemm_operands(mlh_ctx* c); // at finalize: planes or halves and packed rows of every matrix, where the model's widths, its weights and memory allow
 int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_t* ids, const int32_t* lens, float* allLogits);
 int mlh_launch_softmax_rows(mlh_ctx* c, const float* logits, float* probs, const int* target, float* nll, int rows);
 

@@ -47,3 +47,49 @@ def test_graphs_follow_a_repeated_finalize(pkg, bf16, nseq, graph):
     dev.close()
     assert not np.array_equal(before[1], want[1])
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+def test_without_copies_of_the_matrices(pkg, bf16):
+    """A context that may not spend memory on them (or has none left for them) answers as the token-by-token path does."""
+    hp = config(pkg, bf16, maxSeqs=3)
+    model = pkg.Model.generate(hp, 5).randomize_gains(5)
+    prompts = [pkg.random_tokens(5, s, hp.vocabSize, n) for s, n in enumerate((20, 70, 1))]
+
+    def answers(dev):
+        out = []
+        dev.reset()
+        out.extend(dev.forward_full(0, prompts[1]))
+        dev.reset()
+        dev.prefill_batch([0, 1, 2], prompts)
+        out.append(dev.decode_loop([dev.greedy_token(s) for s in range(3)], 6))
+        out.append(np.stack([dev.logits(s) for s in range(3)]))
+        dev.reset()
+        dev.prefill(0, prompts[0])
+        out.append(dev.decode_loop([3], 6))
+        out.append(dev.logits(0))
+        return out
+
+    dev = pkg.Device(hp, 0)
+    dev.upload(model)
+    d, per = hp.dim, 4 if bf16 else 10
+    rows = sum((d * 3 if hp.layerKinds[t] == 0 else d * 3 + 8) + hp.pleDim for t in range(4))
+    exact = ((1000 + rows + 4 * 2 * hp.ffnDim) * d + 4 * d * (d + hp.pleDim + hp.ffnDim)) * per + 4 * d * (d + hp.pleDim) * (2 if bf16 else 4)
+    full = dev.operand_bytes()
+    assert exact <= full <= exact * 1.02  # (packed rows are padded to 16)
+    fast = answers(dev)
+    dev.set_prefill_mode(1)
+    want = answers(dev)
+    dev.set_prefill_mode(0)
+    for limit in (0, full - full // 16):
+        dev.limit_operands(limit)
+        dev.finalize()
+        assert dev.operand_bytes() == 0
+        for a, b in zip(answers(dev), want):
+            assert np.array_equal(a, b)
+    dev.limit_operands(2 * full)
+    dev.finalize()
+    assert dev.operand_bytes() == full
+    for a, b in zip(answers(dev), fast):
+        assert np.array_equal(a, b)
+    dev.close()
