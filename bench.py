@@ -224,12 +224,12 @@ def matrix_params(hp):
     return total
 
 
-def batched_decode_leg(m, steps=48):
-    """Configuration 4: 64 concurrent sequences of the hybrid architecture, prompt lengths uniform in
+def batched_decode_leg(m, steps=48, nseq=0):
+    """Configuration 4: 64 concurrent sequences (nseq: another number) of the hybrid architecture, prompt lengths uniform in
     [32, 512] (seeded), greedy decode.  Returns tok/s and the fraction of the bytes-per-step roofline
     (weights once per step + every sequence's K/V rows and GDN states)."""
     hp = m.config(4)
-    nseq = hp.maxSeqs
+    nseq = nseq or hp.maxSeqs
     model = m.Model.generate(hp, seed=4)
     dev = m.Device(hp, 0)
     dev.upload(model)
@@ -252,7 +252,7 @@ def batched_decode_leg(m, steps=48):
     per_seq = [decode_bytes_per_token(hp, int(n) + 8 + (REPS * steps) // 2, wb) - weights for n in lens]
     step_bytes = weights + float(np.sum(per_seq))
     dev.close()
-    return {"workload": "config 4: 64 sequences, prompts uniform in [32, 512], hybrid 3 GDN : 1 attention + PLE, fp32",
+    return {"workload": f"config 4: {nseq} sequences, prompts uniform in [32, 512], hybrid 3 GDN : 1 attention + PLE, fp32",
             "steps": steps, "ms_per_step": wall / steps * 1e3, "tok_s": nseq * steps / wall,
             "ms_per_step_stats": stats([w / steps * 1e3 for w in walls]),
             "bytes_per_step": step_bytes, "achieved_GBps": step_bytes / (wall / steps) / 1e9,
@@ -414,6 +414,21 @@ def vendor_gemm(a, b, iters, reps, flop):
             "zero_operands": res["zero_operands"]}
 
 
+def products_leg(m, iters=20):
+    """The products of the prefill passes alone, at the row counts of ordinary prompts: us per launch (HIP events, back to
+    back), planes for fp32 models and halves for bf16 ones."""
+    out = {}
+    rng = np.random.default_rng(7)
+    for rows in (128, 256, 517, 777, 1024, 2048):
+        for what, f16, shapes in (("fp32 d768", False, ((2304, 768), (768, 768), (6144, 768), (768, 3072))),
+                                  ("half d2048", True, ((6240, 2048), (2048, 2112), (11264, 2048), (2048, 5632)))):
+            for n, k in shapes:
+                a, b = rng.standard_normal((rows, k), dtype=np.float32), rng.standard_normal((n, k), dtype=np.float32)
+                us = stats([m.selftest_gemm(a, b, None, f16=f16, iters=iters)[1] for _ in range(3)])["median"]
+                out[f"{what} {rows} x {n} x {k}"] = {"us": round(us, 2), "TFLOPs": round(2e-6 * rows * n * k / us, 1)}
+    return out
+
+
 def timed_decode(dev, prompt, K, W, persistent, maxL):
     """W untimed warm-up steps, then REPS repetitions of exactly K timed steps from the same starting state (prompt
     prefilled anew each time), the device idle on both sides of each.  Returns (wall seconds per repetition, HIP-event
@@ -450,10 +465,11 @@ def main():
     ap.add_argument("--path", choices=["xcd", "persistent", "kernels"], default="xcd",
                     help="decode path reported as `value`")
     ap.add_argument("--no-extras", action="store_true", help="skip the batched-decode (config 4) and prefill (config 5) legs")
-    ap.add_argument("--leg", choices=["all", "batched", "prefill", "gemm", "hybrid", "config1", "refdefault"], default="all",
-                    help="profiler runs: run only the batched-decode leg, the prefill leg, the big GEMM alone, the "
+    ap.add_argument("--leg", choices=["all", "batched", "prefill", "gemm", "products", "hybrid", "config1", "refdefault"], default="all",
+                    help="profiler runs: run only the batched-decode leg, the prefill leg, the big GEMM alone, the passes' products, the "
                          "batch-1 hybrid decode leg, configuration 1 or the reference-default shape and print its JSON object")
     ap.add_argument("--passes", type=int, default=2, help="--leg prefill: timed passes over the 8 x 2048-token batch")
+    ap.add_argument("--seqs", type=int, default=0, help="--leg batched: sequences (0: the 64 of the configuration)")
     ap.add_argument("--only-path", action="store_true", help="time only the chosen path (for profiler runs)")
     ap.add_argument("--graph-steps", type=int, default=0,
                     help="kernels path: decode steps per hipGraph replay; 0 = plain launches (use 0 under rocprofv3)")
@@ -465,7 +481,7 @@ def main():
 
     m = entry.load_package()
     if args.leg != "all":
-        leg = {"batched": batched_decode_leg, "prefill": lambda mm: prefill_leg(mm, reps=max(1, args.passes), with_gemm=False),
+        leg = {"batched": lambda mm: batched_decode_leg(mm, nseq=args.seqs), "products": products_leg, "prefill": lambda mm: prefill_leg(mm, reps=max(1, args.passes), with_gemm=False),
                "gemm": gemm_leg, "hybrid": hybrid_decode_leg, "config1": lambda mm: config1_decode_leg(mm)[0],
                "refdefault": reference_default_decode_leg}[args.leg]
         print(json.dumps({args.leg: leg(m)}))
@@ -506,8 +522,8 @@ def main():
     mean_bytes = float(np.mean([decode_bytes_per_token(hp, PROMPT_LEN + 1 + i) for i in range(K)]))
     step_gbps = mean_bytes / wall_per_step / 1e9
 
-    # per-kernel times inside the decode sequence: a HIP event after every launch on the context's
-    # stream, over 64 further steps from the middle of the run (run time plus the launch gap before it)
+    # per-kernel times inside the kernel sequence (the row step of csrc/kernels_rows.hip): a HIP event after every part of
+    # the step on the context's stream, over 64 further steps from the middle of the run (run time plus the launch gap before it)
     dev.set_persistent(0)
     dev.reset()
     dev.prefill(0, prompt)
@@ -518,11 +534,14 @@ def main():
     nprof = min(64, hp.maxL - PROMPT_LEN - mid)
     prof = dev.profile_decode([tok], nprof)
     T_mid = PROMPT_LEN + mid + nprof // 2
-    algo = {"k_phaseA": 4.0 * 3 * hp.dim * hp.dim, "k_attn": 2.0 * 4 * hp.dim * (T_mid + 1) + 2.0 * 4 * hp.dim,
-            "k_oproj": 4.0 * hp.dim * hp.dim, "k_ffn13": 4.0 * 2 * hp.ffnDim * hp.dim,
-            "k_down": 4.0 * hp.dim * hp.ffnDim, "k_lmhead": 4.0 * hp.vocabSize * hp.dim}
+    part = {"k_phaseA": "k_rows qkv", "k_attn": "k_attn + k_rows_mix", "k_oproj": "k_rows output projection", "k_ffn13": "k_rows gate/up",
+            "k_down": "k_rows down projection", "k_lmhead": "k_rows LM head", "k_embed": "k_rows_embed", "k_finish": "k_rows_finish"}
+    algo = {part["k_phaseA"]: 4.0 * 3 * hp.dim * hp.dim, part["k_attn"]: 2.0 * 4 * hp.dim * (T_mid + 1) + 2.0 * 4 * hp.dim,
+            part["k_oproj"]: 4.0 * hp.dim * hp.dim, part["k_ffn13"]: 4.0 * 2 * hp.ffnDim * hp.dim,
+            part["k_down"]: 4.0 * hp.dim * hp.ffnDim, part["k_lmhead"]: 4.0 * hp.vocabSize * hp.dim}
     kernels = {}
     for name, (us, n) in prof.items():
+        name = part.get(name, name)
         if us <= 0:
             continue
         kernels[name] = {"avg_us_in_sequence": round(us, 3), "launches_per_token": n,
@@ -572,13 +591,8 @@ def main():
         dom = max(kernels, key=lambda k: kernels[k]["avg_us_in_sequence"] * kernels[k]["launches_per_token"])
         kd = kernels[dom]
         gbps = kd["algo_bytes"] / kd["avg_us_in_sequence"] / 1e3
-        # HBM bytes per launch from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, scaled by what the same counters
-        # read for a plain copy of known size (see profiles/); only known for the kernels measured there
-        traffic_ratio = {"k_attn": 1.46, "k_ffn13": 1.01, "k_phaseA": 1.02, "k_down": 1.02, "k_oproj": 1.08,
-                         "k_lmhead": 1.01}.get(dom)
-        traffic = traffic_ratio * kd["algo_bytes"] if traffic_ratio else None
         roofline = {"kernel": dom, "bound": "hbm", "achieved": gbps, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
-                    "frac": gbps / HBM_PEAK_GBPS, "traffic": traffic, "avg_launch_us": kd["avg_us_in_sequence"],
+                    "frac": gbps / HBM_PEAK_GBPS, "traffic": None, "avg_launch_us": kd["avg_us_in_sequence"],
                     "algo_bytes_per_launch": kd["algo_bytes"], "share_of_step_time":
                         kd["avg_us_in_sequence"] * kd["launches_per_token"] / sum(
                             v["avg_us_in_sequence"] * v["launches_per_token"] for v in kernels.values())}

@@ -245,7 +245,8 @@ int mlh_synchronize(mlh_ctx* ctx);
 
 /* Measurement support.  Times `iters` back-to-back launches of one kernel of
  * the decode step with HIP events on the context's stream and returns the
- * average duration in microseconds plus the algorithmic bytes one launch moves. */
+ * average duration in microseconds plus the algorithmic bytes one launch moves.
+ * The products are timed in their GEMV form, which mlh_kernel_name names. */
 enum {
     MLH_K_QKV = 0,
     MLH_K_ATTN = 1,
@@ -263,10 +264,11 @@ int mlh_time_kernel(mlh_ctx* ctx, int kernel, int layer, int nseq, int iters, do
                     double* algo_bytes);
 const char* mlh_kernel_name(int kernel);
 
-/* In-sequence kernel times: runs `steps` decode steps as plain launches with a HIP event after
- * every kernel on the context's stream and returns, per kernel id, the mean time from the previous
- * event to its own (its run time plus the launch gap before it) in us_per_launch[MLH_K_COUNT] and
- * the launches per step in launches_per_step[MLH_K_COUNT].  The sequences advance by `steps`. */
+/* In-sequence kernel times: runs `steps` decode steps as the kernel sequence that nseq sequences take in the prefill mode in effect
+ * (row kernels; mode 1: GEMVs), as plain launches with a HIP event after every part of the step on the context's stream, and
+ * returns, per kernel id, the mean time from the previous event to its own (run time plus the launch gap before it; the row
+ * step's attention together with the combination of its partial results) in us_per_launch[MLH_K_COUNT] and the number of such
+ * parts per step in launches_per_step[MLH_K_COUNT].  The sequences advance by `steps`. */
 int mlh_profile_decode(mlh_ctx* ctx, const int32_t* first_ids, int nseq, int steps, double* us_per_launch,
                        int32_t* launches_per_step);
 

@@ -490,12 +490,15 @@ void mlh_rows_rest_of_layer(mlh_ctx* c, int t, const RowsArgs& base, float* x, f
     RowsArgs P = base; // h1 = [Wo | pleUp] . [mix | e] + x (inference.cu:582-610)
     P.K = L.ad + hp.pleDim; P.A = c->rowsMix; P.C = h1; P.ldc = d; P.R = x; P.out = c->rowsH; P.outGain = L.g2; P.ssqOut = c->rowsSsqH;
     mlh_rows_gemm(c, RW_RESID, L.WoR, d, P);
+    mlh_mark(c, MLH_K_OPROJ);
     P = base; // silu(gate) * up of the normalised rows (inference.cu:612-672)
     P.K = d; P.A = c->rowsH; P.ssqIn = c->rowsSsqH; P.nparts = d / RW_TILE; P.out = c->rowsU;
     mlh_rows_gemm(c, RW_SWIGLU, L.W13R, 2 * F, P);
+    mlh_mark(c, MLH_K_FFN_GATEUP);
     P = base; // x = W2 . u + h1 (inference.cu:675-699), and the planes for the next layer's first product or the LM head
     P.K = F; P.A = c->rowsU; P.C = x; P.ldc = d; P.R = h1; P.out = c->rowsX; P.outGain = t > 0 ? c->layers[t - 1].g1 : c->gF; P.ssqOut = c->rowsSsqX;
     mlh_rows_gemm(c, RW_RESID, L.W2R, d, P);
+    mlh_mark(c, MLH_K_FFN_DOWN);
 }
 
 void mlh_rows_embed(mlh_ctx* c, const int* tok, int n, float* x, RowsLayout lay) {
@@ -531,6 +534,7 @@ int mlh_rows_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool emb
     StepArgs a;
     mlh_fill_args(c, a, nseq, tokPtr);
     if (!embedded) mlh_rows_embed(c, tokPtr, nseq, c->x, lay);
+    if (!embedded) mlh_mark(c, MLH_K_EMBED);
     RowsArgs base = {};
     base.M = nseq; base.lay = lay; base.normDim = d; base.sidx = c->d_sidx;
     int nparts = 1; // partial sums behind rowsX: one from the embedding, one per workgroup from a down projection
@@ -540,8 +544,10 @@ int mlh_rows_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool emb
         RowsArgs P = base; // q | k | v | ... of the normalised rows (inference.cu:388-465, 487-507)
         P.K = d; P.A = c->rowsX; P.ssqIn = c->rowsSsqX; P.nparts = nparts; P.C = c->qkv; P.ldc = c->maxRowsA;
         mlh_rows_gemm(c, RW_PLAIN, L.WaR, L.rowsA, P);
+        mlh_mark(c, MLH_K_QKV);
         rc = mlh_launch_mix(c, a, L);
         if (L.kind == MLH_KIND_ATTENTION && c->nsplit > 1) hipLaunchKernelGGL(k_rows_mix, dim3(nseq, (L.ad + hp.pleDim + 255) / 256), dim3(256), 0, st, a, L);
+        mlh_mark(c, L.kind == MLH_KIND_ATTENTION ? MLH_K_ATTN : MLH_K_GDN); // (the combination of the partial results with it)
         mlh_rows_rest_of_layer(c, t, base, c->x, c->h1);
         nparts = d / RW_TILE;
     }
@@ -552,10 +558,12 @@ int mlh_rows_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool emb
         P.K = d; P.A = c->rowsX; P.ssqIn = c->rowsSsqX; P.nparts = nparts; P.C = c->logits; P.ldc = hp.vocabSize;
         P.amaxVal = c->amaxVal; P.amaxIdx = c->amaxIdx; P.amaxParts = c->amaxParts; P.stepCounter = c->d_stepCounter;
         mlh_rows_gemm(c, RW_LOGITS, c->ER, hp.vocabSize, P);
+        mlh_mark(c, MLH_K_LMHEAD);
         const RowsEmbed emb = {c->x, c->rowsX, c->layers[first].g1, c->rowsSsqX, lay};
         const int np = (hp.vocabSize + RW_TILE - 1) / RW_TILE, next = embedNext ? 1 : 0;
         if (hp.weightDtype == MLH_DTYPE_BF16) hipLaunchKernelGGL((k_rows_finish<bf16_t>), dim3(nseq), dim3(256), 0, st, a, emb, np, c->d_tok, next);
         else hipLaunchKernelGGL((k_rows_finish<float>), dim3(nseq), dim3(256), 0, st, a, emb, np, c->d_tok, next);
+        mlh_mark(c, MLH_K_FINISH);
     } else {
         hipLaunchKernelGGL(k_rows_advance, dim3(1), dim3(64), 0, st, a);
     }

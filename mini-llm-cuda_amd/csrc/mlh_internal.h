@@ -210,6 +210,7 @@ struct mlh_ctx {
 
 // kernels_decode.hip
 int mlh_launch_step(mlh_ctx* c, int nseq, const int* tokPtr, bool lmHead, bool embedded = false, bool embedNext = false);
+void mlh_mark(mlh_ctx* c, int id);
 int mlh_launch_mix(mlh_ctx* c, const StepArgs& a, const LayerDev& L);
 int mlh_launch_one(mlh_ctx* c, int kernel, int layer, int nseq);
 double mlh_kernel_bytes(mlh_ctx* c, int kernel, int layer, int nseq);
