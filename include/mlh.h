@@ -140,10 +140,10 @@ int mlh_set_page_table(mlh_ctx* ctx, const int32_t* table, int n);
 int mlh_prefill(mlh_ctx* ctx, int seq, const int32_t* ids, int n);
 
 /* The same for nseg distinct sequences in one pass: segment s appends lens[s]
- * tokens (ids holds the segments back to back) to sequence seqs[s].  With 16
- * or more tokens in the call, every projection is one MFMA GEMM over all
+ * tokens (ids holds the segments back to back) to sequence seqs[s].  With two
+ * or more tokens in the call, every projection is one MFMA product over all
  * tokens (cuBLAS SGEMM over the L columns in the reference, inference.cu:409-449,
- * 575-596, 634-699), attention is tiled and causal over the pages
+ * 575-596, 634-699; up to 64 of them, 32 with bf16 weights, go through the decode step's row kernels), attention is tiled and causal over the pages
  * (inference.cu:511-573), GDN layers run their recurrence over the segment. */
 int mlh_prefill_batch(mlh_ctx* ctx, int nseg, const int32_t* seqs, const int32_t* ids, const int32_t* lens);
 
@@ -158,8 +158,8 @@ int mlh_prefill_batch(mlh_ctx* ctx, int nseg, const int32_t* seqs, const int32_t
 int mlh_forward_full(mlh_ctx* ctx, int seq, const int32_t* ids, int n, float* logits_out, float* probs_out, float* mean_nll);
 
 /* 0 (default): MFMA products when the call has two or more tokens and dim, ffnDim,
- * pleDim and the mixing widths are multiples of 32 (fp32) / 64 (bf16);
- * 1: always token by token through the decode kernels. */
+ * pleDim and the mixing widths are multiples of 32 (fp32) / 64 (bf16), and in decode steps of up to 64 sequences;
+ * 1: always token by token, and decode steps through the GEMV kernels. */
 int mlh_set_prefill_mode(mlh_ctx* ctx, int mode);
 
 /* One greedy decode step for sequences 0..nseq-1: feeds last_ids[s] at each
@@ -295,7 +295,7 @@ int mlh_probe_lds_loads(mlh_ctx* ctx, int slices, double* tb_per_s);
  * with HIP events on the context's stream: total milliseconds. */
 int mlh_time_decode(mlh_ctx* ctx, const int32_t* first_ids, int nseq, int steps, double* total_ms);
 
-/* Stand-alone run of the MFMA GEMM used by prefill and batched decode (no context needed):
+/* Stand-alone run of the prefill's MFMA GEMM (no context needed):
  * C[M,N] = A[M,K] . B[N,K]^T (+ R[M,N]), host fp32 arrays in and out; with MLH_DTYPE_BF16 (or 2 = IEEE half) both
  * operands are rounded to that type first; 3 takes fp32 through the three-bf16-plane products of the prefill (at fp32
  * precision; so does MLH_DTYPE_F32 from 65 rows on).  K*4 (fp32) or K*2 (bf16, half) must be a multiple of 128.

@@ -1,16 +1,17 @@
-// MFMA GEMM for prefill and batched decode on gfx950:
+// MFMA GEMM for prefill on gfx950, and its dispatch:
 //
 //     C[M, N] = A[M, K] . B[N, K]^T  (+ R[M, N])        C, R fp32;  A and B both fp32, bf16 or IEEE half
 //
-// A holds activations (one token per row), B a weight matrix in the checkpoint's row-major [out, in]
-// order -- both operands are K-contiguous, which is what the MFMA operand layout wants: for the
+// (MFMA products of decode steps: kernels_rows.hip.)  A holds activations (one token per row), B a weight matrix in the
+// checkpoint's row-major [out, in] order -- both operands are K-contiguous, which is what the MFMA operand layout wants: for the
 // 32x32 tiles used here lane l supplies row (l % 32) and the K elements of half (l / 32), so a
 // 16-byte piece of a row is one operand (eight bf16 for v_mfma_f32_32x32x16_bf16, or four floats
 // feeding four v_mfma_f32_32x32x2_f32 steps).  This replaces the cublasGemmEx calls of
 // inference.cu:401-465, 487-507, 582-602, 624-695 and 723-743 for L > 1 columns.
 //
 // Here: the 256 x 256-tile kernel of the long two-byte products (k_gemm_tn_w4), the weight-streaming kernels for up to
-// 64 rows (k_gemm_skinny*) and the dispatch; kernels_tile.hip has what lies between, and every longer fp32 product.
+// 64 rows (k_gemm_skinny*: bf16 models' prompts of 33 to 64 tokens as halves; every type through mlh_gemm_device and the self-test,
+// which alone uses k_gemm_tn_w4 with bf16) and the dispatch; kernels_tile.hip has what lies between, and every longer fp32 product.
 #include <string.h>
 
 #include <algorithm>

@@ -1,7 +1,8 @@
 // Prefill: many tokens of one or more sequences through the stack at once.
 //
 // Rows of the activation matrices are tokens (all segments concatenated); the projections are MFMA
-// GEMMs (kernels_gemm.hip) against the same weight buffers the decode path streams; per layer
+// GEMMs (kernels_gemm.hip, kernels_tile.hip) against copies of the weights as planes or halves, or, in short calls, the row
+// kernels of the decode step (kernels_rows.hip); per layer
 //
 //   rmsnorm rows -> GEMM Wa -> attention: per-head QK-norm + RoPE + KV-page write, tiled causal attention
 //                              GDN:       chunked recurrence, one head of one sequence per workgroup
@@ -19,7 +20,6 @@
 #include <algorithm>
 
 #include "mlh_internal.h"
-#include "sample.h"
 #include "p3.h"
 #include "sample.h"
 
@@ -40,7 +40,7 @@ struct PfArgs {
     const int* blkSeg; // attention query blocks: segment and first query of the block
     const int* blkQ0;
     float* X;          // [n, dim] residual stream
-    void* Xn;          // [n, dim] GEMM input (weight dtype)
+    void* Xn;          // [n, dim] GEMM input (planes or halves)
     float* QKV;        // [n, qkvLd]
     int qkvLd;
     void* Amix;        // [n, aLd] GEMM input of the output projection: mixing output, then (at column L.ad) the PLE row
@@ -67,15 +67,8 @@ __device__ __forceinline__ float pf_wave_max(float v) {
 __device__ __forceinline__ float pf_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); } // inference.cu:248
 __device__ __forceinline__ float pf_silu(float v) { return v / (1.0f + expf(-v)); }       // inference.cu:270
 
-// store a float as the GEMM input type (fp32; IEEE half for bf16 models, whose MFMA path runs in fp16; bf16)
+// store a float as the GEMM input type (IEEE half for bf16 models, whose MFMA path runs in fp16)
 template <typename AT> __device__ __forceinline__ void put(AT* p, float v);
-template <> __device__ __forceinline__ void put<float>(float* p, float v) { *p = v; }
-template <> __device__ __forceinline__ void put<bf16_t>(bf16_t* p, float v) {
-    uint32_t u = __float_as_uint(v);
-    if ((u & 0x7fffffffu) > 0x7f800000u) u |= 0x00400000u;
-    else u += 0x7fffu + ((u >> 16) & 1u);
-    *p = (bf16_t)(u >> 16);
-}
 template <> __device__ __forceinline__ void put<f16_t>(f16_t* p, float v) { // saturating: an overflow must not become inf
     const _Float16 h = (_Float16)fminf(fmaxf(v, -65504.0f), 65504.0f);
     p->bits = __builtin_bit_cast(uint16_t, h);
@@ -104,13 +97,6 @@ __global__ void k_pf_embed(PfArgs P) {
 // 4096 elements stay in registers between the sum of squares and the scaling (one pass over memory), and a lane's
 // four results leave as one store.
 template <typename AT> __device__ __forceinline__ void put4(AT* o, float a, float b, float c, float d);
-template <> __device__ __forceinline__ void put4<float>(float* o, float a, float b, float c, float d) {
-    f32x4 v; v.x = a; v.y = b; v.z = c; v.w = d;
-    *reinterpret_cast<f32x4*>(o) = v;
-}
-template <> __device__ __forceinline__ void put4<bf16_t>(bf16_t* o, float a, float b, float c, float d) {
-    put<bf16_t>(o, a); put<bf16_t>(o + 1, b); put<bf16_t>(o + 2, c); put<bf16_t>(o + 3, d);
-}
 template <> __device__ __forceinline__ void put4<f16_t>(f16_t* o, float a, float b, float c, float d) { // saturating like put<f16_t>
     auto h = [](float v) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)fminf(fmaxf(v, -65504.0f), 65504.0f)); };
     uint2 w;
@@ -1486,7 +1472,6 @@ static int ensure_prefill_buffers(mlh_ctx* c, int rows) {
     for (void* p : c->pfAllocs) (void)hipFree(p);
     c->pfAllocs.clear();
     c->pfRows = 0;
-    mlh_drop_graphs(c); // captured batched steps hold the old buffer addresses
     const size_t n = (size_t)rows, wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 6; // GEMM input elements: halves, or three bf16 planes
     auto alloc = [&](void** p, size_t bytes) -> int {
         MLH_CHECK(c, hipMalloc(p, std::max<size_t>(bytes, 16)));

@@ -1,5 +1,5 @@
-// The products of a batched decode step: C[M, N] = A[M, K] . W[N, K]^T for at most 64 rows of A, fp32 or bf16 weights in the
-// checkpoint's row order, at fp32 precision.
+// The products of a decode step and of short prefills: C[M, N] = A[M, K] . W[N, K]^T for at most 64 rows of A, fp32 or bf16
+// weights packed once into the order the waves fetch them in (rows.h), at fp32 precision.
 //
 // Every weight is read once and the activations once per workgroup, so a product is a launch, a memory latency and the bytes
 // behind it; the arithmetic must not add to that.  A workgroup of eight waves owns 16 weight rows at a time and MB blocks of
@@ -285,7 +285,12 @@ static void launch_rows(hipStream_t st, const RowsArgs& P, int cus) {
     const dim3 walk((P.tiles + rounds - 1) / rounds, gy), each(P.tiles, gy);
 #define ROWS(MB_, CNT_) do { hipLaunchKernelGGL((k_rows<WT, MB_, CNT_, EPI>), walk, dim3(RW_THREADS), 0, st, P); return; } while (0)
 #define ROWS_LONG(MB_, D_, AD_) do { hipLaunchKernelGGL((k_rows_long<WT, MB_, D_, AD_, EPI>), each, dim3(RW_THREADS), 0, st, P); return; } while (0)
-    // (CNT: what the registers hold, 12 MB per fp32 chunk and 24 MB per bf16 chunk beside two tiles' weights)
+    // CNT, the chunks per wave whose activations stay in registers (12 MB registers per fp32 chunk, 24 MB per bf16 chunk, beside two
+    // tiles' weights): the steps are those that widths of 256, 768, 1024 and 2048 need, alone and beside 64 PLE columns (fp32 K up to
+    // 256, 768, 1024; bf16 up to 1024, 2048, 2560), where the form was timed, and not every depth there could be.  K in between takes the next deeper form: a wave that is a chunk
+    // short fetches its row's last chunk once more, from the cache, and does not multiply it.  The deepest are bounded by the 256
+    // registers of two waves per SIMD (250 with one block of bf16, 248 with four blocks of fp32); beyond them, and where four blocks
+    // of bf16 would not fit at all, both operands are streamed.
     if constexpr (sizeof(WT) == 4) {
         if (mb == 1) { if (cnt <= 1) ROWS(1, 1); if (cnt <= 3) ROWS(1, 3); if (cnt <= 4) ROWS(1, 4); ROWS_LONG(1, 8, 4); }
         if (mb == 2) { if (cnt <= 1) ROWS(2, 1); if (cnt <= 3) ROWS(2, 3); ROWS_LONG(2, 4, 2); }

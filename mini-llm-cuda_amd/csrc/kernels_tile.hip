@@ -1,7 +1,9 @@
-// Tiled MFMA GEMM for row counts between the decode batches and the long prefills, and for every product of fp32
-// models over more than a few rows:
+// Tiled MFMA GEMM for the prefill's products: those of fp32 models (prompts of more than 64 tokens in a call; fewer run through
+// kernels_rows.hip), and those of bf16 models that are too small for the 256 x 256 tiles of kernels_gemm.hip:
 //
-//     C[M, N] = A[M, K] . B[N, K]^T  (+ R[M, N])        A, B: IEEE half, bf16, or fp32 as three bf16 planes (p3.h)
+//     C[M, N] = A[M, K] . B[N, K]^T  (+ R[M, N])        A, B: IEEE half, fp32 as three bf16 planes (p3.h), or bf16
+//
+// (bf16 operands: the GEMM self-test only; models with bf16 weights multiply halves.)
 //
 // A workgroup of 2 x NW waves owns one TM x TN tile, 128 x 128 or 64 x 64, every wave WM x WN blocks of 16 x 16.  K goes by in slices of RB bytes per row: 64
 // two-byte elements (128 bytes) or 32 elements of three planes (192 bytes).  Slices go global -> LDS directly into a ring
@@ -20,7 +22,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
 
 template <typename T> struct TileTraits;
 template <> struct TileTraits<f16_t> {

@@ -188,7 +188,7 @@ struct mlh_ctx {
     std::vector<void*> mirrorAllocs;
     size_t operandBytes = 0, operandLimit = SIZE_MAX; // what they take and may take
     long f16Inexact = 0;       // bf16 weights that had no exact scaled-half representation (reported at finalize)
-    void* gemmWs = nullptr;    // split-K workspace of the skinny GEMM
+    void* gemmWs = nullptr;    // split-K workspace of the prefill's products
 
     std::vector<int> h_len; // host mirror of d_pos
     std::vector<char> h_dirty;     // sequences that some launch may have given a length or GDN states since their last reset

@@ -3,7 +3,9 @@
 // x = hi + mid + lo with hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid), each rounded to nearest even: three
 // times eight significand bits hold the 24 of x, so the sum is exact (down to the bf16 denormals).  A product a.b is formed from
 // the six plane products hi.hi, hi.mid, mid.hi, mid.mid, hi.lo, lo.hi, every one exact in the fp32 accumulator; what
-// is left out (mid.lo, lo.mid, lo.lo) is below 2^-25 of |a||b|, less than one fp32 rounding of it.
+// is left out (mid.lo, lo.mid, lo.lo) is below 2^-24 of |a||b|: over all significands |mid| <= 2^-8.006 |a| and |lo| <= 2^-17.003 |a|,
+// at worst 0.995 2^-24 together, which is what rounding the product to fp32 may cost.  In sums it is far less: of 768 normal terms it
+// moves the result by 5.7e-9 (rms, of |a||b| / sqrt(768)), a sequential fp32 sum by 5.1e-7; of 3072, 5.6e-9 against 1.0e-6.
 //
 // Storage: 32 elements of a row take 192 bytes, their hi, mid and lo halves in turn (64 bytes each); a row of K elements
 // (K a multiple of 32) is K * 6 bytes.  Leading dimensions are counted in elements.
