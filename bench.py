@@ -290,13 +290,13 @@ def hybrid_decode_leg(m, steps=192):
             "frac_of_hbm_peak": nbytes / (wall / steps) / 1e9 / HBM_PEAK_GBPS, "last_ids": [int(x) for x in out[-4:, 0]]}
 
 
-def prefill_leg(m, reps=REPS, with_gemm=True):
-    """Configuration 5: 8 prompts of 2048 uniform-random tokens through the bf16 model in one pass.
+def prefill_leg(m, reps=REPS, with_gemm=True, nseq=0):
+    """Configuration 5: 8 prompts (nseq: another number) of 2048 uniform-random tokens through the bf16 model in one pass.
     MFMA utilisation = algorithmic flops (projections + causal attention, LM head on the last position
     only) / time / the published dense bf16 peak; the GEMM kernel alone is also timed on the pass's own
     gate/up shape (M = 16384 rows)."""
     hp = m.config(5)
-    nseq, plen = hp.maxSeqs, 2048
+    nseq, plen = nseq or hp.maxSeqs, 2048
     model = m.Model.generate(hp, seed=5)
     dev = m.Device(hp, 0)
     dev.upload(model)
@@ -324,7 +324,7 @@ def prefill_leg(m, reps=REPS, with_gemm=True):
     dec = stats(decs)["median"]
     dev.close()
     gemm = gemm_leg(m, iters=10, reps=REPS) if with_gemm else None
-    return {"workload": "config 5: 8 x 2048-token prompts, d2048 x 24 layers (3 GDN : 1 attention), 16 heads x 128, "
+    return {"workload": f"config 5: {nseq} x 2048-token prompts, d2048 x 24 layers (3 GDN : 1 attention), 16 heads x 128, "
                         "ffn 5632, vocab 32000, PLE 64, bf16 weights, fp32 accumulation",
             "tokens": tokens, "ms": med * 1e3, "ms_stats": stats([t * 1e3 for t in times]), "tok_s": tokens / med,
             "algo_tflop": flops / 1e12,
@@ -469,7 +469,7 @@ def main():
                     help="profiler runs: run only the batched-decode leg, the prefill leg, the big GEMM alone, the passes' products, the "
                          "batch-1 hybrid decode leg, configuration 1 or the reference-default shape and print its JSON object")
     ap.add_argument("--passes", type=int, default=2, help="--leg prefill: timed passes over the 8 x 2048-token batch")
-    ap.add_argument("--seqs", type=int, default=0, help="--leg batched: sequences (0: the 64 of the configuration)")
+    ap.add_argument("--seqs", type=int, default=0, help="--leg batched, prefill: sequences (0: those of the configuration)")
     ap.add_argument("--only-path", action="store_true", help="time only the chosen path (for profiler runs)")
     ap.add_argument("--graph-steps", type=int, default=0,
                     help="kernels path: decode steps per hipGraph replay; 0 = plain launches (use 0 under rocprofv3)")
@@ -481,7 +481,7 @@ def main():
 
     m = entry.load_package()
     if args.leg != "all":
-        leg = {"batched": lambda mm: batched_decode_leg(mm, nseq=args.seqs), "products": products_leg, "prefill": lambda mm: prefill_leg(mm, reps=max(1, args.passes), with_gemm=False),
+        leg = {"batched": lambda mm: batched_decode_leg(mm, nseq=args.seqs), "products": products_leg, "prefill": lambda mm: prefill_leg(mm, reps=max(1, args.passes), with_gemm=False, nseq=args.seqs),
                "gemm": gemm_leg, "hybrid": hybrid_decode_leg, "config1": lambda mm: config1_decode_leg(mm)[0],
                "refdefault": reference_default_decode_leg}[args.leg]
         print(json.dumps({args.leg: leg(m)}))

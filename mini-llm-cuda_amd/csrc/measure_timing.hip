@@ -19,10 +19,7 @@ void mlh_dump_persistent_timing(mlh_ctx* c) {
     const bool xcd = c->usePersistent == 3 && mlh_xcd_supported(c);
     for (int l = 0; l < c->hp.transformers; l++)
         for (int k = 0; k < (xcd ? 5 : 15); k++) tot[k] += (double)(t[l * 16 + k + 1] - t[l * 16 + k]) / 100.0; // 100 MHz clock
-    static const char* tnames[15] = {"x.wait", "A.norm", "A.rows", "B.mix", "C.wait", "C.rows", "h1.wait", "D.norm", "D.rows",
-                                     "u.wait", "E.rows", "-", "-", "-", "-"};
     static const char* xnames[15] = {"x.exchange", "A+hop", "B+hop", "C+2hops", "D+hop", "-", "-", "-", "-", "-", "-", "-", "-", "-", "-"};
-    if (c->usePersistent == 2) for (int k = 0; k < 15; k++) names[k] = tnames[k];
     if (xcd) for (int k = 0; k < 15; k++) names[k] = xnames[k];
     if (xcd) { // skew between workgroups at four points of the last layer pass
         std::vector<unsigned long long> sk(4 * 256);
@@ -56,10 +53,16 @@ void mlh_dump_persistent_timing(mlh_ctx* c) {
             }
         }
     }
-    if (xcd) { // raw stamps relative to the start of the layer pass: communicator 0-9, worker wave 0 10-14
-        double rel[16] = {0};
-        for (int l = 0; l < c->hp.transformers; l++)
-            for (int k = 0; k < 16; k++) rel[k] += ((double)t[l * 16 + k] - (double)t[l * 16]) / 100.0 / c->hp.transformers;
+    if (xcd) { // raw stamps relative to the start of the layer pass: communicator 0-6 and 8, worker wave 0 the others
+        // (a workgroup without a slice of its own leaves 6 and 8 at 0, and every one 6 of the first layer: means over the rest, -1 for none)
+        double rel[16];
+        for (int k = 0; k < 16; k++) {
+            double sum = 0;
+            int n = 0;
+            for (int l = 0; l < c->hp.transformers; l++)
+                if (t[l * 16 + k]) { sum += ((double)t[l * 16 + k] - (double)t[l * 16]) / 100.0; n++; }
+            rel[k] = n ? sum / n : -1.0;
+        }
         for (int l = 0; l < c->hp.transformers; l++) {
             fprintf(stderr, "[xcd layer %2d]", l);
             for (int k = 0; k < 16; k++) fprintf(stderr, " %d:%.2f", k, t[l * 16 + k] ? ((double)t[l * 16 + k] - (double)t[l * 16]) / 100.0 : -1.0);
@@ -69,7 +72,6 @@ void mlh_dump_persistent_timing(mlh_ctx* c) {
                         "wave 0: units done %.2f combine done %.2f | worker C %.2f..%.2f | h1: partials seen %.2f gathered %.2f | worker D end %.2f | "
                         "u in LDS %.2f | worker E end %.2f\n",
                 rel[6], rel[1], rel[10], rel[11], rel[2], rel[12], rel[15], rel[13], rel[14], rel[8], rel[4], rel[7], rel[5], rel[9]);
-
     }
     fprintf(stderr, "[persistent decode, workgroup 0, last step] mean us per layer:");
     double sum = 0;
