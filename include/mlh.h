@@ -206,7 +206,12 @@ int mlh_set_graph(mlh_ctx* ctx, int stepsPerGraph);
  * normal end only; the XCD-rank kernel keeps gated-delta-net states in LDS until then, the barrier kernel's are put
  * back from a copy taken before its launch), and the call redoes its steps as the kernel sequence and
  * leaves the context at mode 0 (mlh_get_persistent, mlh_persistent_fallbacks).
- * Mode 0, unsupported shapes and nseq > 1: a sequence of kernels issued as mlh_set_graph says. */
+ * In mode 3 a call of up to 16 sequences (mlh_single_launch_sequences; without graph replays) runs its steps in one launch as
+ * well: models with 8 to 16 heads of 64 or 128, gated-delta-net heads of the same size and number, per-layer embeddings of width
+ * 32 (fp32), 64 or 128, dim up to 768 (fp32) / 2048 (bf16), ffnDim up to 2048 / 6144 in multiples of 256 / 512.  Its workgroups
+ * meet before anything is written; when they do not, the call falls back in the same way.  A wait that expires behind the
+ * meeting is an error (-2): the sequences of the call have to be reset.
+ * Mode 0, unsupported shapes and more sequences: a sequence of kernels issued as mlh_set_graph says. */
 int mlh_set_persistent(mlh_ctx* ctx, int mode);
 
 /* The mode in effect (it differs from what mlh_set_persistent was given after a fallback), and how many decode
@@ -216,12 +221,12 @@ int mlh_get_persistent(mlh_ctx* ctx);
 int mlh_persistent_fallbacks(mlh_ctx* ctx);
 
 /* Test hooks (no counterpart in the reference).  mlh_debug_inject_abort: the next `launches` single-launch decode
- * launches find their bounded wait already given up (XCD-rank kernel: arrival counters that start full; barrier
+ * launches find their bounded wait already given up (XCD-rank kernels: arrival counters that start full; barrier
  * kernel: an abort flag that starts raised), so every workgroup leaves at once and the fallback path runs without
  * any wait having to expire.  mlh_debug_set_xcd_tag: sets the XCD-rank kernel's running tag count (device word and
  * host mirror), to exercise the reset that precedes a wrap of the 32-bit tags. */
 int mlh_debug_inject_abort(mlh_ctx* ctx, int launches);
-/* mlh_debug_inject_abort_at_step: the next single-launch decode launch gives up by itself when workgroup 0 reaches
+/* mlh_debug_inject_abort_at_step: the next single-launch decode launch of one sequence gives up by itself when workgroup 0 reaches
  * decode step `step` (> 0; counted from 0 inside the launch) -- after the earlier steps have run and written what
  * they write -- so the test can see that the redo starts from the state before the launch.  0 switches it off. */
 int mlh_debug_inject_abort_at_step(mlh_ctx* ctx, int step);
@@ -233,13 +238,15 @@ int mlh_debug_set_xcd_tag(mlh_ctx* ctx, unsigned tagsUsed);
  * softmax(logits / temperature) -- the smallest index whose cumulative probability exceeds u, with u a 53-bit
  * uniform from a counter-based generator (SplitMix64) keyed by (seed, sequence id, position of the drawn token), so
  * a sequence draws the same tokens alone, in a batch or from a graph.  Sampling has no counterpart in the
- * reference.  While it is on, batch-1 decode runs as the kernel sequence (the single-launch modes fuse the argmax
+ * reference.  While it is on, decode runs as the kernel sequence (the single-launch modes fuse the argmax
  * only).  Returns 0, or -1 for a temperature outside [0, 1e4]. */
 int mlh_set_sampling(mlh_ctx* ctx, float temperature, unsigned long long seed);
 
 /* 1 when mode 3 of mlh_set_persistent applies to this context's model and device, else 0
  * (no counterpart in the reference: its decode loop is one kernel sequence, inference_orchestrator.cu:120-165). */
 int mlh_xcd_decode_supported(mlh_ctx* ctx);
+/* The largest nseq whose decode calls run as a single launch in mode 3 (0: none; no counterpart in the reference). */
+int mlh_single_launch_sequences(mlh_ctx* ctx);
 
 int mlh_synchronize(mlh_ctx* ctx);
 

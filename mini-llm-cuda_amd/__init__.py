@@ -98,6 +98,7 @@ _sigs_dev = {
     "mlh_debug_inject_abort_at_step": (c_int, [c_void_p, c_int]),
     "mlh_debug_set_xcd_tag": (c_int, [c_void_p, ctypes.c_uint]),
     "mlh_xcd_decode_supported": (c_int, [c_void_p]),
+    "mlh_single_launch_sequences": (c_int, [c_void_p]),
     "mlh_synchronize": (c_int, [c_void_p]),
     "mlh_time_kernel": (c_int, [c_void_p, c_int, c_int, c_int, c_int, _P(c_double), _P(c_double)]),
     "mlh_kernel_name": (c_char_p, [c_int]),
@@ -391,6 +392,9 @@ class Device:
 
     def xcd_decode_supported(self):
         return bool(dev.mlh_xcd_decode_supported(self._h))
+
+    def single_launch_sequences(self):
+        return dev.mlh_single_launch_sequences(self._h)
 
     def synchronize(self):
         self._check(dev.mlh_synchronize(self._h))

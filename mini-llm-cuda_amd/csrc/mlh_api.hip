@@ -420,6 +420,7 @@ extern "C" int mlh_finalize(mlh_ctx* c) {
     c->xcdPrepared = c->persistentPrepared = false;
     if (mlh_xcd_supported(c) && (rc = mlh_launch_xcd(c, 0))) return rc;
     if (mlh_persistent_supported(c) && mlh_launch_persistent(c, 0)) c->err.clear(); // a model too wide for it simply does not use it
+    if ((rc = mlh_ranks_prepare(c))) return rc;
     MLH_CHECK(c, hipDeviceSynchronize());
     c->finalized = true;
     return 0;
@@ -665,7 +666,15 @@ static int ensure_graph(mlh_ctx* c, int slot, int nseq, int k) {
     return 0;
 }
 
+// Up to 16 sequences, and one of a model that the XCD-rank kernel does not cover, in one launch of kernels_ranks.hip.  (A caller who
+// asked for graph replays gets those.)
+static bool use_ranks(const mlh_ctx* c, int nseq) {
+    if (c->usePersistent != 3 || c->temperature > 0.f || c->graphSteps > 0 || !mlh_ranks_applicable(c, nseq)) return false;
+    return nseq > 1 || !mlh_xcd_supported(c);
+}
+
 static bool use_persistent(const mlh_ctx* c, int nseq) {
+    if (use_ranks(c, nseq)) return true;
     // (the single-launch kernels fuse the argmax only: sampling runs through the kernel sequence)
     if (nseq != 1 || !c->usePersistent || c->temperature > 0.f) return false;
     // mode 3 on a model the XCD-rank kernel does not cover: the row step where it applies (its launches cost less than the
@@ -679,9 +688,16 @@ static bool use_persistent(const mlh_ctx* c, int nseq) {
 // position, token and the tag counter are written at a kernel's normal end only; K/V rows of the steps that did run
 // are written again with the same values; the XCD-rank kernel keeps gated-delta-net states in LDS until its normal
 // end; the barrier kernel stores them at every step, and gets them back from the copy taken before its launch.
-static int check_persistent_abort(mlh_ctx* c) {
-    if (c->d_timing) mlh_dump_persistent_timing(c);
+static int check_persistent_abort(mlh_ctx* c, int nseq) {
+    if (c->d_timing && !use_ranks(c, nseq)) mlh_dump_persistent_timing(c);
     const int flag = c->pinIo.p[c->hp.maxSeqs]; // (end_steps)
+    if (flag && use_ranks(c, nseq)) { // 1, 2: not all workgroups found a place, nothing was written; 3: a wait expired behind that
+        const int rc = mlh_ranks_reset(c);
+        if (rc) return rc;
+        MLH_CHECK(c, hipStreamSynchronize(c->stream));
+        c->err = flag == 3 ? "decode kernel of several sequences abandoned a wait in mid-run: its sequences have to be reset" : "decode kernel of several sequences: not all workgroups were resident";
+        return flag == 3 ? -2 : -3;
+    }
     if (flag) {
         c->err = flag == 2 ? "XCD-rank decode kernel: the workgroups did not spread evenly over the XCDs"
                            : "persistent decode kernel abandoned a wait (were all workgroups resident?)";
@@ -728,6 +744,7 @@ static int end_steps(mlh_ctx* c, int nout) {
 
 static int run_steps(mlh_ctx* c, int nseq, int steps) {
     int rc;
+    if (use_ranks(c, nseq)) return mlh_launch_ranks(c, nseq, steps);
     if (use_persistent(c, nseq)) return (c->usePersistent == 3 && mlh_xcd_supported(c)) ? mlh_launch_xcd(c, steps) : mlh_launch_persistent(c, steps);
     if (c->graphSteps >= 1) {
         const int k = c->graphSteps;
@@ -780,7 +797,7 @@ extern "C" int mlh_decode_loop(mlh_ctx* c, const int32_t* first, int nseq, int s
         if ((rc = begin_steps(c, first, nseq, steps))) return rc;
         if ((rc = run_steps(c, nseq, steps))) return rc;
         if ((rc = end_steps(c, steps * nseq))) return rc;
-        if (!single || (rc = check_persistent_abort(c)) == 0) break;
+        if (!single || (rc = check_persistent_abort(c, nseq)) == 0) break;
         if (rc != -3) return rc;
         fall_back_to_kernel_sequence(c); // and once more, as a sequence of kernels
     }
@@ -815,7 +832,7 @@ extern "C" int mlh_time_decode(mlh_ctx* c, const int32_t* first, int nseq, int s
         MLH_CHECK(c, hipEventSynchronize(e1));
         MLH_CHECK(c, hipEventElapsedTime(&ms, e0, e1));
         if (rc || (rc = end_steps(c, 0))) break;
-        if (!single || (rc = check_persistent_abort(c)) == 0) break;
+        if (!single || (rc = check_persistent_abort(c, nseq)) == 0) break;
         if (rc != -3) break;
         fall_back_to_kernel_sequence(c);
     }
@@ -939,6 +956,11 @@ extern "C" int mlh_debug_set_xcd_tag(mlh_ctx* c, unsigned tagsUsed) {
     MLH_CHECK(c, hipMemcpy(c->d_sync + 64 * 21, &tagsUsed, 4, hipMemcpyHostToDevice));
     c->xcdTagNext = tagsUsed;
     return 0;
+}
+
+extern "C" int mlh_single_launch_sequences(mlh_ctx* c) {
+    if (!c) return 0;
+    return std::max(c->ranksMax, mlh_xcd_supported(c) ? 1 : 0);
 }
 
 extern "C" int mlh_xcd_decode_supported(mlh_ctx* c) { return c && mlh_xcd_supported(c) ? 1 : 0; }

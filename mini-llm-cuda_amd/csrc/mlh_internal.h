@@ -159,6 +159,10 @@ struct mlh_ctx {
     int xcdWide = 1, xcdNapRound = 0, xcdNap[5] = {44, 0, 0, 0, 0}; // tuning knobs, read from the environment once at creation
     unsigned long long* xcdBuf = nullptr; // (value, tag) exchange words of mode 3
     size_t xcdWords = 0;
+    int ranksMax = 0;              // sequences the kernel of several sequences takes (kernels_ranks.hip); 0: not this model
+    void* ranksBuf = nullptr;      // its exchange words
+    size_t ranksBytes = 0;
+    unsigned long long ranksTag = 0; // tags its launches have used
     LayerDev* d_layers = nullptr;  // device copy of `layers`
     unsigned* d_sync = nullptr;    // barrier words + abort flag
     float* pamaxVal = nullptr;     // [numCUs]
@@ -263,6 +267,12 @@ void mlh_rows_gemm(mlh_ctx* c, int epi, const void* w, int n, RowsArgs P);
 void mlh_rows_embed(mlh_ctx* c, const int* tok, int n, float* x, RowsLayout lay);
 void mlh_rows_rest_of_layer(mlh_ctx* c, int t, const RowsArgs& base, float* x, float* h1);
 void mlh_rows_lm_head(mlh_ctx* c, int n, const float* X, const int* segStart, const int* segLen, const int* segSeq, float* amaxVal, int* amaxIdx);
+
+// kernels_ranks.hip: decode steps of several sequences in one launch
+bool mlh_ranks_applicable(const mlh_ctx* c, int nseq);
+int mlh_ranks_prepare(mlh_ctx* c);
+int mlh_ranks_reset(mlh_ctx* c);
+int mlh_launch_ranks(mlh_ctx* c, int nseq, int steps);
 
 // kernels_persistent.hip
 bool mlh_persistent_supported(const mlh_ctx* c);
