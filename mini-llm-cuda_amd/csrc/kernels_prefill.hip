@@ -81,6 +81,13 @@ template <typename AT> __device__ __forceinline__ void put_mix(const PfArgs& P, 
     if (P.rows) rows_put(P.rows, col, (int)row, P.lay, P.half != 0, v);
     else put_at<AT>(P.Amix, row, P.aLd, col, v);
 }
+// ... four of them
+template <typename AT> __device__ __forceinline__ void put_mix4(const PfArgs& P, size_t row, int col, const f32x4& v) {
+    if (P.rows) rows_put4(P.rows, col, (int)row, P.lay, P.half != 0, v.x, v.y, v.z, v.w);
+    else if constexpr (sizeof(AT) == 6) p3_put4((unsigned char*)P.Amix + row * P.aLd * 6, col, v.x, v.y, v.z, v.w);
+    else
+        for (int e = 0; e < 4; e++) put_at<AT>(P.Amix, row, P.aLd, col + e, v[e]);
+}
 template <typename WT> __device__ __forceinline__ float getw(const WT* p);
 template <> __device__ __forceinline__ float getw<float>(const float* p) { return *p; }
 template <> __device__ __forceinline__ float getw<bf16_t>(const bf16_t* p) { return __uint_as_float(((uint32_t)*p) << 16); }
@@ -208,94 +215,128 @@ __global__ void __launch_bounds__(64) k_pf_qk_rope_kv(PfArgs P, LayerDev L) {
     }
 }
 
-// Tiled causal attention for 16 queries of one head: K and V of 64 positions at a time in LDS, online
-// softmax per query (inference.cu:136-239, 511-573 for these columns), optional sigmoid gate (:241-250).
+// Causal attention for 16 queries of one head at fp32 precision (inference.cu:136-239, 511-573 for these columns), optional sigmoid gate
+// (:241-250), on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: every product and sum fp32).
+//
+// The four waves of a workgroup take key tiles of 16 in turn, each with an online softmax of its own, and meet once at the end; nothing goes through
+// LDS on the way.  S^T[key, query] = K . Q^T: lane 16 g + n holds a key's (a query's) columns [g HD/4, (g + 1) HD/4), the order of the contraction being
+// free.  The accumulator leaves the lane the scores of keys 4 g .. 4 g + 3 of query n, which is the operand P of O^T += V^T . P^T as it stands; row m of the
+// V operand of block b is dimension m HD/16 + b, so V comes in 16-byte pieces as well.  Loads of the wave's next tile go out before this one's products.
+// Bound by the matrix cores' fp32 rate and, for few rows, by the longest chain of tiles.  Measured: 517 rows, 6 heads of 128: 30 us (107 on the
+// vector ALU through LDS tiles of 64 keys); 17 376 rows of 64 sequences, 12 heads of 64: 178 us (899).
 #define PF_QB 16
 template <int HD, typename AT>
 __global__ void __launch_bounds__(PWG) k_pf_attn(PfArgs P, LayerDev L) {
-    constexpr int LDK = HD + 4, EPL = HD / 64, QPW = PF_QB / 4;
-    extern __shared__ float lds[];
-    float* Kt = lds;              // [64][LDK]
-    float* Vt = Kt + 64 * LDK;    // [64][LDK]
-    float* qs = Vt + 64 * LDK;    // [PF_QB][HD]
+    constexpr int NW = PWG / 64, KC = HD / 4, VB = HD / 16, LDO = HD + 4;
+    __shared__ float part[NW][PF_QB][LDO], stat[NW][2][PF_QB];
     const StepArgs& a = P.a;
-    const int h = blockIdx.x, blk = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int h = blockIdx.x, blk = blockIdx.y, tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = lane & 15, g = lane >> 4;
     const int seg = P.blkSeg[blk], q0 = P.blkQ0[blk];
     const int seq = P.segSeq[seg], pos0 = P.segPos0[seg], len = P.segLen[seg], row0 = P.segStart[seg] + q0;
-    const int nq = min(PF_QB, len - q0);
-    const int maxPos = pos0 + q0 + nq - 1;
-    for (int i = tid; i < PF_QB * HD; i += PWG) {
-        const int q = i / HD, e = i - q * HD;
-        qs[i] = q < nq ? P.QKV[(size_t)(row0 + q) * P.qkvLd + h * HD + e] : 0.f;
+    const int nq = min(PF_QB, len - q0), maxPos = pos0 + q0 + nq - 1, qpos = pos0 + q0 + n;
+    f32x4 q[KC / 4];
+    {
+        const float* qr = P.QKV + (size_t)(row0 + min(n, nq - 1)) * P.qkvLd + h * HD + g * KC;
+#pragma unroll
+        for (int c = 0; c < KC / 4; c++) q[c] = *reinterpret_cast<const f32x4*>(qr + 4 * c);
     }
-    float m[QPW], l[QPW], acc[QPW][EPL];
+    const float scale = 1.0f / sqrtf((float)HD);
+    f32x4 k[2][KC / 4], v[2][4][VB / 4], acc[VB];
 #pragma unroll
-    for (int q = 0; q < QPW; q++) {
-        m[q] = -1.0e30f; l[q] = 0.f;
+    for (int b = 0; b < VB; b++) acc[b] = (f32x4)(0.f);
+    float m = -1.0e30f, l = 0.f; // of query n; l: over this lane's keys
+    const int ntiles = (maxPos >> 4) + 1;
+    auto fetch = [&](int t, int set) __attribute__((always_inline)) { // (rows behind the last position that a query here sees: that row again, with weight zero)
+        const int j0 = t * 16, last = maxPos - j0;
+        const size_t base = ((size_t)a.pageTable[seq * a.pagesPerSeq + (j0 >> 6)] * MLH_KV_PAGE + (j0 & 63)) * a.dim + h * HD;
+        const float* kr = L.K + base + (size_t)min(n, last) * a.dim + g * KC;
 #pragma unroll
-        for (int e = 0; e < EPL; e++) acc[q][e] = 0.f;
+        for (int c = 0; c < KC / 4; c++) k[set][c] = *reinterpret_cast<const f32x4*>(kr + 4 * c);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float* vr = L.V + base + (size_t)min(4 * g + i, last) * a.dim + n * VB;
+#pragma unroll
+            for (int c = 0; c < VB / 4; c++) v[set][i][c] = *reinterpret_cast<const f32x4*>(vr + 4 * c);
+        }
+    };
+    auto tile = [&](int t, int set) __attribute__((always_inline)) {
+        f32x4 s0 = (f32x4)(0.f), s1 = (f32x4)(0.f); // two chains
+#pragma unroll
+        for (int c = 0; c < KC / 4; c++) {
+            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[set][c].x, q[c].x, s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[set][c].y, q[c].y, s1, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[set][c].z, q[c].z, s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[set][c].w, q[c].w, s1, 0, 0, 0);
+        }
+        const int key = t * 16 + 4 * g;
+        float s[4], mt = m;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            s[i] = key + i <= qpos ? (s0[i] + s1[i]) * scale : -1.0e30f;
+            mt = fmaxf(mt, s[i]);
+        }
+        mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+        const float corr = expf(m - mt);
+        l *= corr;
+        m = mt;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            s[i] = key + i <= qpos ? expf(s[i] - mt) : 0.f;
+            l += s[i];
+        }
+#pragma unroll
+        for (int b = 0; b < VB; b++) acc[b] *= corr;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int b = 0; b < VB; b++) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[set][i][b / 4][b % 4], s[i], acc[b], 0, 0, 0);
+    };
+    int t = wave;
+    if (t < ntiles) fetch(t, 0);
+    while (t < ntiles) { // (no further tile: the same loads again, dropped)
+        fetch(min(t + NW, ntiles - 1), 1);
+        tile(t, 0);
+        t += NW;
+        if (t >= ntiles) break;
+        fetch(min(t + NW, ntiles - 1), 0);
+        tile(t, 1);
+        t += NW;
     }
-    const float scale = sqrtf((float)HD);
-    const int ntiles = (maxPos >> 6) + 1;
-    for (int t = 0; t < ntiles; t++) {
-        const int j0 = t << 6;
-        const int page = a.pageTable[seq * a.pagesPerSeq + t];
-        const size_t base = ((size_t)page * MLH_KV_PAGE) * a.dim + h * HD;
-        __syncthreads();
-        for (int i = tid; i < 64 * (HD / 4); i += PWG) {
-            const int r = i / (HD / 4), c4 = (i % (HD / 4)) * 4;
-            f32x4 kk = (f32x4)(0.f), vv = (f32x4)(0.f);
-            if (j0 + r <= maxPos) {
-                kk = *reinterpret_cast<const f32x4*>(L.K + base + (size_t)r * a.dim + c4);
-                vv = *reinterpret_cast<const f32x4*>(L.V + base + (size_t)r * a.dim + c4);
-            }
-            *reinterpret_cast<f32x4*>(Kt + r * LDK + c4) = kk;
-            *reinterpret_cast<f32x4*>(Vt + r * LDK + c4) = vv;
-        }
-        __syncthreads();
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (g == 0) { stat[wave][0][n] = m; stat[wave][1][n] = l; }
+    __syncthreads();
+    { // this wave's share, at the common maximum
+        float M = stat[0][0][n];
 #pragma unroll
-        for (int qq = 0; qq < QPW; qq++) {
-            const int q = wave * QPW + qq;
-            const int qpos = pos0 + q0 + q;
-            if (q >= nq || j0 > qpos) continue; // wave-uniform
-            float s = 0.f;
-            const float* kr = Kt + lane * LDK;
-            const float* qr = qs + q * HD;
+        for (int w = 1; w < NW; w++) M = fmaxf(M, stat[w][0][n]);
+        const float f = expf(m - M);
 #pragma unroll
-            for (int i = 0; i < HD; i += 4) {
-                const f32x4 kk = *reinterpret_cast<const f32x4*>(kr + i);
-                const f32x4 qv = *reinterpret_cast<const f32x4*>(qr + i);
-                s = fmaf(kk.x, qv.x, s); s = fmaf(kk.y, qv.y, s); s = fmaf(kk.z, qv.z, s); s = fmaf(kk.w, qv.w, s);
-            }
-            const bool valid = j0 + lane <= qpos;
-            s = valid ? s / scale : -1.0e30f;
-            const float mn = fmaxf(m[qq], pf_wave_max(s));
-            const float e = valid ? expf(s - mn) : 0.f;
-            const float corr = expf(m[qq] - mn);
-            l[qq] = l[qq] * corr + pf_wave_sum(e);
-            m[qq] = mn;
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int ee = 0; ee < EPL; ee++) acc[qq][ee] *= corr;
-#pragma unroll 16
-            for (int j = 0; j < 64; j++) {
-                const float pj = __shfl(e, j, 64);
-#pragma unroll
-                for (int ee = 0; ee < EPL; ee++) acc[qq][ee] = fmaf(pj, Vt[j * LDK + lane + 64 * ee], acc[qq][ee]);
-            }
-        }
+            for (int b = 0; b < VB; b += 4)
+                *reinterpret_cast<f32x4*>(&part[wave][n][(4 * g + i) * VB + b]) = f32x4{acc[b][i], acc[b + 1][i], acc[b + 2][i], acc[b + 3][i]} * f;
     }
+    __syncthreads();
+    for (int i = tid; i < nq * (HD / 4); i += PWG) {
+        const int qi = i / (HD / 4), c4 = (i % (HD / 4)) * 4;
+        float M = stat[0][0][qi], den = 0.f;
 #pragma unroll
-    for (int qq = 0; qq < QPW; qq++) {
-        const int q = wave * QPW + qq;
-        if (q >= nq) continue;
-        const size_t row = (size_t)(row0 + q);
+        for (int w = 1; w < NW; w++) M = fmaxf(M, stat[w][0][qi]);
+        f32x4 o = (f32x4)(0.f);
 #pragma unroll
-        for (int ee = 0; ee < EPL; ee++) {
-            const int dcol = h * HD + lane + 64 * ee;
-            float v = acc[qq][ee] / l[qq];
-            if (a.gating) v = v * pf_sigmoid(P.QKV[row * P.qkvLd + L.offG + dcol]);
-            put_mix<AT>(P, row, dcol, v);
+        for (int w = 0; w < NW; w++) {
+            den = fmaf(stat[w][1][qi], expf(stat[w][0][qi] - M), den);
+            o += *reinterpret_cast<const f32x4*>(&part[w][qi][c4]);
         }
+        const size_t row = (size_t)(row0 + qi);
+        o.x /= den; o.y /= den; o.z /= den; o.w /= den;
+        if (a.gating) {
+            const f32x4 z = *reinterpret_cast<const f32x4*>(P.QKV + row * P.qkvLd + L.offG + h * HD + c4);
+            o.x *= pf_sigmoid(z.x); o.y *= pf_sigmoid(z.y); o.z *= pf_sigmoid(z.z); o.w *= pf_sigmoid(z.w);
+        }
+        put_mix4<AT>(P, row, h * HD + c4, o);
     }
 }
 
@@ -1459,9 +1500,6 @@ int mlh_init_prefill_kernels(mlh_ctx* c) {
     MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gdn_prep<128>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_prep_lds(128)));
     MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gdn_scan<64>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * GdLayout<64>::image));
     MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gdn_scan<128>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * GdLayout<128>::image));
-    const int lds = (2 * 64 * 132 + PF_QB * 128) * 4;
-    MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_attn<128, p3_t>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_attn<128, f16_t>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     return 0;
 }
 
@@ -1601,14 +1639,14 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
                 hipLaunchKernelGGL((k_pf_qk_rope_kv<64>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<64, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<64, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
-                else if (P.half) hipLaunchKernelGGL((k_pf_attn<64, f16_t>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 68 + PF_QB * 64) * 4, st, P, L);
-                else hipLaunchKernelGGL((k_pf_attn<64, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 68 + PF_QB * 64) * 4, st, P, L);
+                else if (P.half) hipLaunchKernelGGL((k_pf_attn<64, f16_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
+                else hipLaunchKernelGGL((k_pf_attn<64, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
             } else {
                 hipLaunchKernelGGL((k_pf_qk_rope_kv<128>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<128, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<128, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
-                else if (P.half) hipLaunchKernelGGL((k_pf_attn<128, f16_t>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 132 + PF_QB * 128) * 4, st, P, L);
-                else hipLaunchKernelGGL((k_pf_attn<128, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), (size_t)(2 * 64 * 132 + PF_QB * 128) * 4, st, P, L);
+                else if (P.half) hipLaunchKernelGGL((k_pf_attn<128, f16_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
+                else hipLaunchKernelGGL((k_pf_attn<128, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
             }
         } else {
             const int skipFrom = nchunk > 0 ? GD_C : 0x7fffffff;

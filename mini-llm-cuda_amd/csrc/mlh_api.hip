@@ -174,7 +174,7 @@ extern "C" int mlh_create(const mlh_hparams* hpIn, int device, mlh_ctx** out) {
         if (pl > 0) { L.offPle = r; r += pl; }
         if (L.kind == MLH_KIND_GDN) { L.offGa = r; r += hp.gdnHeads; L.offGb = r; r += hp.gdnHeads; }
         L.rowsA = r;
-        c->maxRowsA = std::max(c->maxRowsA, r);
+        c->maxRowsA = std::max(c->maxRowsA, (r + 3) & ~3); // (rows of it start 16-byte aligned)
         c->maxAd = std::max(c->maxAd, L.ad);
         if (L.ad % 8) { c->err = "mixing width must be a multiple of 8"; return bail(-1); }
         char *wa, *wo, *w13, *w2, *pu = nullptr, *pt = nullptr;

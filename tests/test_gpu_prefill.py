@@ -363,3 +363,26 @@ def test_reference_default_architecture(pkg, orc):
     exact, tol = check_greedy_against_oracle(dec, prompt, ids, GAP_TOL, logits, FP32_RTOL, "reference defaults")
     assert exact + tol == len(ids)
     dev.close()
+
+
+@pytest.mark.parametrize("kind", ["attn_flags", "hd128"])
+def test_prefill_fp32_attention_edges(pkg, orc, kind):
+    """The fp32 attention walks key tiles of 16 for blocks of 16 queries, four tiles at a time: lengths on both sides of one tile, of four and of a
+    page, in one ragged call and appended to a cache (blocks that start in the middle of a tile), against the float64 oracle.  Tolerance: every logit is
+    the end of some ten fp32 contractions a layer, each off by at most 2^-24 sqrt(K) of its largest term, K up to the feed-forward width."""
+    hp = small_cfg(pkg, kind, maxSeqs=6, **({"maxL": 200} if kind == "attn_flags" else {}))
+    model, dev, w = make(pkg, orc, hp, seed=43)
+    tol = 10 * hp.transformers * np.sqrt(hp.ffnDim) * 2.0 ** -24
+    for lens in ([15, 16, 17, 63, 64, 65], [1, 2, 49, 127, 129, 197]):
+        prompts = [pkg.random_tokens(400 + n, 0, hp.vocabSize, n) for n in lens]
+        wants = [orc.forward_full(w, p, "f64", last_only=True)["logits"][-1] for p in prompts]
+        for cut in (0, 7, 33):  # of the prompt in an earlier call
+            dev.reset()
+            seqs = [s for s, n in enumerate(lens) if n > cut]
+            if cut:
+                dev.prefill_batch(seqs, [prompts[s][:cut] for s in seqs])
+            dev.prefill_batch(seqs, [prompts[s][cut:] for s in seqs])
+            for s in seqs:
+                err = np.max(np.abs(dev.logits(s) - wants[s])) / np.max(np.abs(wants[s]))
+                assert err <= tol, (lens[s], cut, err, tol)
+    dev.close()
