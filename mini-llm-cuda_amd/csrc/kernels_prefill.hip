@@ -151,7 +151,8 @@ __global__ void __launch_bounds__(PWG) k_pf_rmsnorm(const float* __restrict__ X,
 // Per (head, row): per-head RMSNorm of q and k (inference.cu:52-81, 97-111), RoPE on adjacent pairs at the
 // row's position (inference.cu:113-134), q written back in place, k and v written to the KV pages.
 __device__ __forceinline__ uint32_t pack_f16(float lo, float hi) { // two floats -> two IEEE halves (round to nearest even)
-    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16);
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, f16x2{(_Float16)lo, (_Float16)hi}); // (one instruction; put together from two halves it is three)
 }
 
 template <int HD>
@@ -773,19 +774,18 @@ __host__ __device__ __forceinline__ int slot_of(int x) {
     const int i = 4 * (x32 >> 3) + (x32 & 3), hh = (x32 >> 2) & 1;
     return (x & ~31) + 16 * (i >> 3) + 8 * hh + (i & 7);
 }
-template <int DK> struct GdLayout { // one chunk's operand image (bytes), rows padded by 16 bytes against LDS bank conflicts
-    static constexpr int KP = (DK + 8) * 2, TP = (GD_C + 8) * 2; // row pitches of [*, DK] and [*, 64] half matrices
-    static constexpr int oKt = 0, oQh = oKt + GD_C * KP, oM = oQh + GD_C * KP, oKhT = oM + GD_C * TP;
-    static constexpr int oVt = oKhT + DK * TP;                    // half [DV, 64]: a column's 64 tokens contiguous
-    static constexpr int image = oVt + DK * TP;                   // 80896 (DK 128), 46080 (DK 64): multiples of 1024
-    static constexpr int total = image;
+// One chunk's operands as fragments of 1 KB: what a wave's lanes take of a 32-row, 16-step operand, 16 bytes each.
+template <int DK> struct GdLayout {
+    static constexpr int JT = DK / 32;
+    static constexpr int fKt = 0, fQh = fKt + 4 * JT, fM = fQh + 4 * JT, fKhT = fM + 6, fVt = fKhT + 4 * JT; // [token tile][dk step]; M's three tiles; [dk tile][token step]; [dv tile][token step]
+    static constexpr int frags = fVt + 4 * JT, total = frags * 1024;
 };
 __device__ __forceinline__ uint16_t f16_bits(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
 
 template <int DK>
 __global__ void __launch_bounds__(2 * DK, 2) k_gdn_prep(PfArgs P, LayerDev L, const int* __restrict__ chunkSeg, const int* __restrict__ chunkT0,
                                                       unsigned char* __restrict__ ws, float* __restrict__ gCexp) {
-    constexpr int DV = DK, NT = 2 * DK;
+    constexpr int DV = DK, NT = 2 * DK, JT = DK / 32;
     typedef GdLayout<DK> Lay;
     extern __shared__ __attribute__((aligned(16))) unsigned char pls[];
     float* Am = reinterpret_cast<float*>(pls);            // [64][64]
@@ -884,7 +884,9 @@ __global__ void __launch_bounds__(2 * DK, 2) k_gdn_prep(PfArgs P, LayerDev L, co
                 const int t = 32 * tt + 8 * (e >> 2) + 4 * half + (e & 3);
                 const float dec = expf(g[t] - g[i_]); // <= 1 where it is used (i <= t)
                 if (which == 0) Am[t * GD_C + i_] = i_ < t ? beta[t] * dec * acc[e] : 0.f;
-                else *reinterpret_cast<uint16_t*>(img + Lay::oM + t * Lay::TP + 2 * slot_of(i_)) = f16_bits(i_ <= t ? dec * acc[e] : 0.f);
+                else if (ti <= tt) // (the tile above the diagonal is zero and not stored)
+                    *reinterpret_cast<uint16_t*>(img + (Lay::fM + (tt + ti) * 2 + ((slot_of(i_) >> 4) & 1)) * 1024 + (((slot_of(i_) >> 3) & 1) * 32 + (t & 31)) * 16 + 2 * (slot_of(i_) & 7)) =
+                        f16_bits(i_ <= t ? dec * acc[e] : 0.f);
             }
         }
     }
@@ -993,17 +995,18 @@ __global__ void __launch_bounds__(2 * DK, 2) k_gdn_prep(PfArgs P, LayerDev L, co
     const float gC = g[GD_C - 1];
     const int sl = slot_of(col);
     // Kt, diag(e^g) Q and Kh^T are assembled in LDS in the image layout (the half copies of k and q are no longer
-    // needed: the MFMAs are done) and leave as 16-byte rows; element-wise 2-byte stores to global would touch a
-    // different cache line per lane.
+    // needed: the MFMAs are done), Vt in slot order as well, and leave in fragment order, 16 bytes a lane; element-wise
+    // 2-byte stores to global would touch a different cache line per lane.
     uint16_t* khs = q16 + GD_C * (DK + 8); // [DK][64 + 8]
     __syncthreads();                       // every column is solved: the triangular matrix has been read for the last time
     uint16_t* vts = reinterpret_cast<uint16_t*>(Am); // V^T [DV][64] takes its place (the same 64 * DV * 2 bytes)
     if (tid < DV) { // holds the q column
 #pragma unroll
-        for (int t = 0; t < GD_C; t += 8) { // this column's 64 tokens in a row: the scan reads four at a time
+        for (int q = 0; q < 8; q++) { // piece q: step q / 2, half q % 2; at a place of the row that spreads the rows over the banks
+            const int t = 16 * (q >> 1) + 4 * (q & 1);
             u32x4 w;
-            w.x = pack_f16(X[t], X[t + 1]); w.y = pack_f16(X[t + 2], X[t + 3]); w.z = pack_f16(X[t + 4], X[t + 5]); w.w = pack_f16(X[t + 6], X[t + 7]);
-            *reinterpret_cast<u32x4*>(vts + col * GD_C + t) = w;
+            w.x = pack_f16(X[t], X[t + 1]); w.y = pack_f16(X[t + 2], X[t + 3]); w.z = pack_f16(X[t + 8], X[t + 9]); w.w = pack_f16(X[t + 10], X[t + 11]);
+            *reinterpret_cast<u32x4*>(vts + col * GD_C + (q ^ (col & 7)) * 8) = w;
         }
 #pragma unroll
         for (int t = 0; t < GD_C; t++) q16[t * (DK + 8) + sl] = f16_bits(eg[t] * colv[t]);
@@ -1016,74 +1019,63 @@ __global__ void __launch_bounds__(2 * DK, 2) k_gdn_prep(PfArgs P, LayerDev L, co
     }
     __syncthreads();
     {
-        const u32x4* s1 = reinterpret_cast<const u32x4*>(k16);
-        u32x4* d1 = reinterpret_cast<u32x4*>(img + Lay::oKt);
-        for (int i = tid; i < 2 * GD_C * Lay::KP / 16; i += NT) d1[i] = s1[i];
-        const u32x4* s2 = reinterpret_cast<const u32x4*>(khs);
-        u32x4* d2 = reinterpret_cast<u32x4*>(img + Lay::oKhT);
-        for (int i = tid; i < DK * Lay::TP / 16; i += NT) d2[i] = s2[i];
-        const u32x4* s3 = reinterpret_cast<const u32x4*>(vts); // rows of eight 16-byte pieces to rows of pitch TP
-        for (int i = tid; i < DV * 8; i += NT) *reinterpret_cast<u32x4*>(img + Lay::oVt + (i >> 3) * Lay::TP + (i & 7) * 16) = s3[i];
+        u32x4* d1 = reinterpret_cast<u32x4*>(img);
+        for (int i = tid; i < 2 * 4 * JT * 64; i += NT) { // Kt and Qh: the rows of k16 and q16 follow one another
+            const int f = i >> 6, l32 = i & 31, hh = (i >> 5) & 1, f1 = f % (4 * JT);
+            d1[i] = *reinterpret_cast<const u32x4*>((f < 4 * JT ? k16 : q16) + (32 * (f1 / (2 * JT)) + l32) * (DK + 8) + 16 * (f1 % (2 * JT)) + 8 * hh);
+        }
+        for (int i = tid; i < 4 * JT * 64; i += NT) { // Kh^T and Vt^T
+            const int f = i >> 6, l32 = i & 31, hh = (i >> 5) & 1, row = 32 * (f >> 2) + l32;
+            d1[Lay::fKhT * 64 + i] = *reinterpret_cast<const u32x4*>(khs + row * (GD_C + 8) + 16 * (f & 3) + 8 * hh);
+            d1[Lay::fVt * 64 + i] = *reinterpret_cast<const u32x4*>(vts + row * GD_C + ((2 * (f & 3) + hh) ^ (row & 7)) * 8);
+        }
     }
     if (tid == 0) gCexp[(size_t)chunk * a.gdnHeads + h] = expf(gC);
 }
 
-// Copies one chunk's operand image (IMG bytes, a multiple of 1 KB) from global memory straight into LDS, 1 KB per
-// instruction, the NW waves of the workgroup taking instructions in turn.
-template <int IMG, int NW>
-__device__ __forceinline__ void gd_issue_image(const unsigned char* src, unsigned char* dst, int wave, int lane) {
-    for (int q = wave; q < IMG / 1024; q += NW) __builtin_amdgcn_global_load_lds(src + q * 1024 + lane * 16, dst + q * 1024, 16, 0, 0);
-}
-
-// The same, one instruction at a time: load k of this wave (k < ceil(IMG / 1024 / NW)), to be spread over other work.
-template <int IMG, int NW>
-__device__ __forceinline__ void gd_issue_image_one(const unsigned char* src, unsigned char* dst, int wave, int lane, int k) {
-    const int q = wave + k * NW;
-    if (q < IMG / 1024) __builtin_amdgcn_global_load_lds(src + q * 1024 + lane * 16, dst + q * 1024, 16, 0, 0);
-}
-
+// One wave per 32 state columns dv of a head: nothing of a chunk's products crosses columns, so the waves of a head are workgroups of their own, on
+// different compute units.  An operand is used once by a wave: it comes from memory straight into registers, and the load of the next chunk's same
+// operand goes out behind its use, a whole chunk ahead.  Bound by the MFMA chain of a chunk (56 a wave) where few heads times segments run, by the
+// operands' way through the caches where many do.  Measured (head size 128): 13 chunks, 16 heads: 26 us (51 with the four waves of a head in one
+// workgroup and the operands through LDS); 32 chunks, 8 x 16 heads: 95 us (122).
 template <int DK>
-__global__ void __launch_bounds__(2 * DK) k_gdn_scan(PfArgs P, LayerDev L, const int* __restrict__ chunkBase, const unsigned char* __restrict__ ws,
+__global__ void __launch_bounds__(64, 1) k_gdn_scan(PfArgs P, LayerDev L, const int* __restrict__ chunkBase, const unsigned char* __restrict__ ws,
                                                       const float* __restrict__ gCexp) {
-    constexpr int DV = DK, NW = DV / 32, JT = DK / 32; // waves (one per 32 state columns dv), dk tiles
+    constexpr int DV = DK, JT = DK / 32; // dk tiles
     typedef GdLayout<DK> Lay;
-    extern __shared__ __attribute__((aligned(16))) unsigned char sls[]; // two operand images
     const StepArgs& a = P.a;
-    const int h = blockIdx.x, seg = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int h = blockIdx.x, seg = blockIdx.y, dt = blockIdx.z, lane = threadIdx.x;
     const int len = P.segLen[seg];
     if (len < GD_C) return; // short segments take the recurrent kernel
     const int seq = P.segSeq[seg], row0 = P.segStart[seg], nch = (len + GD_C - 1) / GD_C, cb = chunkBase[seg];
-    const int n32 = lane & 31, half = lane >> 5, dv = 32 * wave + n32;
+    const int n32 = lane & 31, half = lane >> 5, dv = 32 * dt + n32;
     float* Sg = L.S + ((size_t)seq * a.gdnHeads + h) * DV * DK;
     f32x16 St[JT]; // S^T tile j: rows dk = 32 j + 8(i/4) + 4 half + i%4, column dv
 #pragma unroll
     for (int j = 0; j < JT; j++)
 #pragma unroll
         for (int i = 0; i < 16; i++) St[j][i] = Sg[(size_t)dv * DK + 32 * j + 8 * (i >> 2) + 4 * half + (i & 3)];
-    auto image_of = [&](int c) { return ws + ((size_t)(cb + c) * a.gdnHeads + h) * Lay::total; };
-    auto issue = [&](int c, int stage) { gd_issue_image<Lay::image, NW>(image_of(c), sls + stage * Lay::image, wave, lane); };
-    constexpr int NIMG = (Lay::image / 1024 + NW - 1) / NW; // loads per wave and image
-    auto issue_one = [&](int c, int stage, int k) { gd_issue_image_one<Lay::image, NW>(image_of(c), sls + stage * Lay::image, wave, lane, k); };
-    // V^T - (what the state predicts) needs tokens 8 g + 4 half + e, e = 0..3, of column dv: eight bytes of the image
-    auto vt_of = [&](const unsigned char* im, int tt, int st, float (&v)[8]) { // elements 8 st .. 8 st + 7 of tile tt
-        const unsigned char* p = im + Lay::oVt + dv * Lay::TP + (32 * tt + 16 * st + 4 * half) * 2;
-#pragma unroll
-        for (int g = 0; g < 2; g++) {
-            const u32x2 w = *reinterpret_cast<const u32x2*>(p + 16 * g);
-            v[4 * g + 0] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.x & 0xffff));
-            v[4 * g + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.x >> 16));
-            v[4 * g + 2] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.y & 0xffff));
-            v[4 * g + 3] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w.y >> 16));
-        }
+    u32x4 kt[4 * JT], qh[4 * JT], mm[6], kh[4 * JT], vt[4]; // this chunk's fragments, each the next chunk's once it has been used
+    auto frag = [&](int c, int f) __attribute__((always_inline)) {
+        return reinterpret_cast<const u32x4*>(ws + ((size_t)(cb + c) * a.gdnHeads + h) * Lay::total + f * 1024)[lane];
     };
-    issue(0, 0);
-    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
-    asm volatile("" ::: "memory");
-    __syncthreads();
+#pragma unroll
+    for (int f = 0; f < 4 * JT; f++) { kt[f] = frag(0, Lay::fKt + f); qh[f] = frag(0, Lay::fQh + f); }
+#pragma unroll
+    for (int f = 0; f < 4; f++) vt[f] = frag(0, Lay::fVt + 4 * dt + f);
+#pragma unroll
+    for (int f = 0; f < 6; f++) mm[f] = frag(0, Lay::fM + f);
+#pragma unroll
+    for (int f = 0; f < 4 * JT; f++) kh[f] = frag(0, Lay::fKhT + f);
+    auto mfma = [](const u32x4& x, const u32x4& y, const f32x16& z) __attribute__((always_inline)) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, x), __builtin_bit_cast(f16x8, y), z, 0, 0, 0);
+    };
+    float gC = gCexp[(size_t)cb * a.gdnHeads + h];
+    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0), as a builtin: the compiler then knows that no load from before the loop is open in it, and does not
+    asm volatile("" ::: "memory");      // wait for the state at the head of every trip
     for (int c = 0; c < nch; c++) {
-        const unsigned char* im = sls + (c & 1) * Lay::image;
-        const bool more = c + 1 < nch;
-        const float gC = gCexp[(size_t)(cb + c) * a.gdnHeads + h];
+        const int cn = min(c + 1, nch - 1); // (behind the last chunk: that one again, dropped)
+        const float gN = gCexp[(size_t)(cb + cn) * a.gdnHeads + h];
         // S0^T as B operands: step (j, st) = elements 8 st .. 8 st + 7 of tile j, rounded to half
         u32x4 sop[JT][2];
 #pragma unroll
@@ -1094,103 +1086,95 @@ __global__ void __launch_bounds__(2 * DK) k_gdn_scan(PfArgs P, LayerDev L, const
                 sop[j][st].z = pack_f16(St[j][8 * st + 4], St[j][8 * st + 5]); sop[j][st].w = pack_f16(St[j][8 * st + 6], St[j][8 * st + 7]);
             }
         // X = Kt S0^T : [64 tokens, 32 dv] (lane = dv), Y^T = S0 (diag(e^g) Q)^T : [32 dv, 64 tokens] (lane = token: the
-        // operands swapped), so that an output row leaves as four neighbouring columns per store.  The next image's
-        // loads go out between the MFMAs, one per pair: issued in one go they hold the wave for a microsecond.
+        // operands swapped), so that an output row leaves as four neighbouring columns per store.
         f32x16 X[2], Y[2];
 #pragma unroll
         for (int tt = 0; tt < 2; tt++) {
 #pragma unroll
             for (int i = 0; i < 16; i++) { X[tt][i] = 0.f; Y[tt][i] = 0.f; }
-            const unsigned char* kr = im + Lay::oKt + (32 * tt + n32) * Lay::KP + 16 * half;
-            const unsigned char* qr = im + Lay::oQh + (32 * tt + n32) * Lay::KP + 16 * half;
 #pragma unroll
             for (int j = 0; j < JT; j++)
 #pragma unroll
                 for (int st = 0; st < 2; st++) {
-                    const u32x4 ka = *reinterpret_cast<const u32x4*>(kr + 32 * (2 * j + st));
-                    const u32x4 qa = *reinterpret_cast<const u32x4*>(qr + 32 * (2 * j + st));
-                    X[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, ka), __builtin_bit_cast(f16x8, sop[j][st]), X[tt], 0, 0, 0);
-                    Y[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, sop[j][st]), __builtin_bit_cast(f16x8, qa), Y[tt], 0, 0, 0);
-                    if (more && (tt * JT + j) * 2 + st < NIMG) issue_one(c + 1, (c + 1) & 1, (tt * JT + j) * 2 + st);
+                    const int f = 2 * JT * tt + 2 * j + st;
+                    X[tt] = mfma(kt[f], sop[j][st], X[tt]);
+                    Y[tt] = mfma(sop[j][st], qh[f], Y[tt]);
+                    kt[f] = frag(cn, Lay::fKt + f);
+                    qh[f] = frag(cn, Lay::fQh + f);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
         }
-#pragma unroll
-        for (int k = 2 * JT * 2; k < NIMG; k++) // (more loads than MFMA pairs: the rest goes out here)
-            if (more) issue_one(c + 1, (c + 1) & 1, k);
         // W^T = Vt - X, as B operands (token axis in slot order by construction)
         u32x4 wop[2][2];
 #pragma unroll
         for (int tt = 0; tt < 2; tt++)
 #pragma unroll
             for (int st = 0; st < 2; st++) {
+                const f16x8 v = __builtin_bit_cast(f16x8, vt[2 * tt + st]);
                 float w[8];
-                vt_of(im, tt, st, w);
 #pragma unroll
-                for (int e = 0; e < 8; e++) w[e] -= X[tt][8 * st + e];
+                for (int e = 0; e < 8; e++) w[e] = (float)v[e] - X[tt][8 * st + e];
                 wop[tt][st].x = pack_f16(w[0], w[1]); wop[tt][st].y = pack_f16(w[2], w[3]);
                 wop[tt][st].z = pack_f16(w[4], w[5]); wop[tt][st].w = pack_f16(w[6], w[7]);
+                vt[2 * tt + st] = frag(cn, Lay::fVt + 4 * dt + 2 * tt + st);
             }
         // O = Y + M W^T (M is lower triangular: tokens of tile 0 see only tile 0)
 #pragma unroll
-        for (int tt = 0; tt < 2; tt++) {
-            const unsigned char* mr = im + Lay::oM + (32 * tt + n32) * Lay::TP + 16 * half;
+        for (int tt = 0; tt < 2; tt++)
 #pragma unroll
             for (int t2 = 0; t2 <= tt; t2++)
 #pragma unroll
                 for (int st = 0; st < 2; st++) {
-                    const u32x4 ma = *reinterpret_cast<const u32x4*>(mr + 32 * (2 * t2 + st));
-                    Y[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, wop[t2][st]), __builtin_bit_cast(f16x8, ma), Y[tt], 0, 0, 0);
+                    Y[tt] = mfma(wop[t2][st], mm[2 * (tt + t2) + st], Y[tt]);
+                    mm[2 * (tt + t2) + st] = frag(cn, Lay::fM + 2 * (tt + t2) + st);
                 }
-            // lane = token n32 of this tile; element i = column 32 wave + 8 (i / 4) + 4 half + i % 4.  The two lanes of a
+        __builtin_amdgcn_sched_barrier(0);
+        // S^T <- e^{g_C} S^T + Kh^T W^T
+#pragma unroll
+        for (int j = 0; j < JT; j++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) St[j][i] *= gC;
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int j = 0; j < JT; j++) {
+                St[j] = mfma(kh[4 * j + s], wop[s >> 1][s & 1], St[j]);
+                kh[4 * j + s] = frag(cn, Lay::fKhT + 4 * j + s);
+            }
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++) {
+            // lane = token n32 of this tile; element i = column 32 dt + 8 (i / 4) + 4 half + i % 4.  The two lanes of a
             // token (half 0 and 1) swap two of their four 8-byte pieces so that each holds two whole 16-byte pieces:
             // half as many store instructions, and the address unit works through a store per lane and instruction.
-            {
-                u32x2 w[4];
+            u32x2 w[4];
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    float o[4];
+            for (int g = 0; g < 4; g++) {
+                float o[4];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) o[e] = fminf(fmaxf(Y[tt][4 * g + e], -65504.0f), 65504.0f); // saturating: an overflow must not become inf
-                    w[g].x = pack_f16(o[0], o[1]); w[g].y = pack_f16(o[2], o[3]);
-                }
-                // half 0 keeps pieces g = 0, 2 (and gets the partner's upper halves of them), half 1 keeps g = 1, 3
-                u32x2 give[2], got[2];
-                give[0] = half ? w[0] : w[1]; give[1] = half ? w[2] : w[3];
+                for (int e = 0; e < 4; e++) o[e] = fminf(fmaxf(Y[tt][4 * g + e], -65504.0f), 65504.0f); // saturating: an overflow must not become inf
+                w[g].x = pack_f16(o[0], o[1]); w[g].y = pack_f16(o[2], o[3]);
+            }
+            // half 0 keeps pieces g = 0, 2 (and gets the partner's upper halves of them), half 1 keeps g = 1, 3
+            u32x2 give[2], got[2];
+            give[0] = half ? w[0] : w[1]; give[1] = half ? w[2] : w[3];
 #pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    got[k].x = (uint32_t)__shfl_xor((int)give[k].x, 32, 64);
-                    got[k].y = (uint32_t)__shfl_xor((int)give[k].y, 32, 64);
-                }
-                if (n32 < len - (c * GD_C + 32 * tt)) {
-                    f16_t* orow = (f16_t*)P.Amix + (size_t)(row0 + c * GD_C + 32 * tt + n32) * P.aLd + h * DV + 32 * wave + 8 * half;
+            for (int k = 0; k < 2; k++) {
+                got[k].x = (uint32_t)__shfl_xor((int)give[k].x, 32, 64);
+                got[k].y = (uint32_t)__shfl_xor((int)give[k].y, 32, 64);
+            }
+            if (n32 < len - (c * GD_C + 32 * tt)) {
+                f16_t* orow = (f16_t*)P.Amix + (size_t)(row0 + c * GD_C + 32 * tt + n32) * P.aLd + h * DV + 32 * dt + 8 * half;
 #pragma unroll
-                    for (int k = 0; k < 2; k++) { // columns 16 k + 8 half .. + 7: lower four from the half-0 lane, upper four from the half-1 lane
-                        const u32x2 mine = w[2 * k + half];
-                        u32x4 v;
-                        v.x = half ? got[k].x : mine.x; v.y = half ? got[k].y : mine.y;
-                        v.z = half ? mine.x : got[k].x; v.w = half ? mine.y : got[k].y;
-                        *reinterpret_cast<u32x4*>(orow + 16 * k) = v;
-                    }
+                for (int k = 0; k < 2; k++) { // columns 16 k + 8 half .. + 7: lower four from the half-0 lane, upper four from the half-1 lane
+                    const u32x2 mine = half ? w[2 * k + 1] : w[2 * k];
+                    u32x4 v;
+                    v.x = half ? got[k].x : mine.x; v.y = half ? got[k].y : mine.y;
+                    v.z = half ? mine.x : got[k].x; v.w = half ? mine.y : got[k].y;
+                    *reinterpret_cast<u32x4*>(orow + 16 * k) = v;
                 }
             }
         }
-        // S^T <- e^{g_C} S^T + Kh^T W^T
-#pragma unroll
-        for (int j = 0; j < JT; j++) {
-#pragma unroll
-            for (int i = 0; i < 16; i++) St[j][i] *= gC;
-            const unsigned char* hr = im + Lay::oKhT + (32 * j + n32) * Lay::TP + 16 * half;
-#pragma unroll
-            for (int t2 = 0; t2 < 2; t2++)
-#pragma unroll
-                for (int st = 0; st < 2; st++) {
-                    const u32x4 ha = *reinterpret_cast<const u32x4*>(hr + 32 * (2 * t2 + st));
-                    St[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, ha), __builtin_bit_cast(f16x8, wop[t2][st]), St[j], 0, 0, 0);
-                }
-        }
-        __builtin_amdgcn_s_waitcnt(0x0F70);              // vmcnt(0): the next chunk's image has landed -- as a builtin, so that
-        asm volatile("" ::: "memory");                   // the compiler knows and does not wait again among the next loads
-        __syncthreads();                                  // ... for every wave; everyone is done with this image
+        gC = gN;
     }
 #pragma unroll
     for (int j = 0; j < JT; j++)
@@ -1498,8 +1482,6 @@ static size_t gdn_prep_lds(int dk) { return ((size_t)GD_C * GD_C + 12 * GD_C) * 
 int mlh_init_prefill_kernels(mlh_ctx* c) {
     MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gdn_prep<64>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_prep_lds(64)));
     MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gdn_prep<128>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_prep_lds(128)));
-    MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gdn_scan<64>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * GdLayout<64>::image));
-    MLH_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gdn_scan<128>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * GdLayout<128>::image));
     return 0;
 }
 
@@ -1662,10 +1644,10 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
                 const int *dcs = d_chunk, *dct = d_chunk + nchunk, *dcb = d_seg + 4 * nseg;
                 if (hp.gdnDk == 64) {
                     hipLaunchKernelGGL((k_gdn_prep<64>), dim3(nchunk, hp.gdnHeads), dim3(128), gdn_prep_lds(64), st, P, L, dcs, dct, (unsigned char*)c->pfGdnWs, c->pfGdnG);
-                    hipLaunchKernelGGL((k_gdn_scan<64>), dim3(hp.gdnHeads, nseg), dim3(128), (size_t)2 * GdLayout<64>::image, st, P, L, dcb, (const unsigned char*)c->pfGdnWs, c->pfGdnG);
+                    hipLaunchKernelGGL((k_gdn_scan<64>), dim3(hp.gdnHeads, nseg, 2), dim3(64), 0, st, P, L, dcb, (const unsigned char*)c->pfGdnWs, c->pfGdnG);
                 } else {
                     hipLaunchKernelGGL((k_gdn_prep<128>), dim3(nchunk, hp.gdnHeads), dim3(256), gdn_prep_lds(128), st, P, L, dcs, dct, (unsigned char*)c->pfGdnWs, c->pfGdnG);
-                    hipLaunchKernelGGL((k_gdn_scan<128>), dim3(hp.gdnHeads, nseg), dim3(256), (size_t)2 * GdLayout<128>::image, st, P, L, dcb, (const unsigned char*)c->pfGdnWs, c->pfGdnG);
+                    hipLaunchKernelGGL((k_gdn_scan<128>), dim3(hp.gdnHeads, nseg, 4), dim3(64), 0, st, P, L, dcb, (const unsigned char*)c->pfGdnWs, c->pfGdnG);
                 }
             }
         }

@@ -386,3 +386,30 @@ def test_prefill_fp32_attention_edges(pkg, orc, kind):
                 err = np.max(np.abs(dev.logits(s) - wants[s])) / np.max(np.abs(wants[s]))
                 assert err <= tol, (lens[s], cut, err, tol)
     dev.close()
+
+
+@pytest.mark.parametrize("kind", ["hybrid", "hd128"])
+def test_prefill_bf16_gdn_chunk_edges(pkg, orc, kind):
+    """The chunked gated delta net (chunks of 64 tokens, tiles of 32 tokens and 32 state columns): one chunk, one and a little, tile edges and a last
+    chunk of one token, several segments in one call and each appended to a state; the state is checked by the greedy steps that follow.  Tolerance: that
+    of the bf16 prefill above (half operands)."""
+    hp = small_cfg(pkg, kind, weightDtype=pkg.DTYPE_BF16, maxSeqs=6)
+    model, dev, w = make(pkg, orc, hp, seed=45, bf16=True)
+    lens = [64, 65, 96, 97, 128, 193]
+    prompts = [pkg.random_tokens(500 + n, 0, hp.vocabSize, n) for n in lens]
+    wants = [orc.forward_full(w, p, "f64", last_only=True)["logits"][-1] for p in prompts]
+    for cut in (0, 64):
+        dev.reset()
+        if cut:
+            dev.prefill_batch(list(range(6)), [p[:cut] for p in prompts])
+        seqs = [s for s, n in enumerate(lens) if n > cut]
+        dev.prefill_batch(seqs, [prompts[s][cut:] for s in seqs])
+        for s in seqs:
+            err = np.max(np.abs(dev.logits(s) - wants[s])) / np.max(np.abs(wants[s]))
+            assert err <= 4e-3, (lens[s], cut, err)
+    first = [dev.greedy_token(s) for s in range(6)]
+    out = dev.decode_loop(first, 1)
+    for s, p in enumerate(prompts):
+        want = orc.forward_full(w, np.append(p, first[s]).astype(np.int32), "f64", last_only=True)["logits"][-1]
+        assert want.max() - want[int(out[0, s])] <= BF16_RTOL * np.max(np.abs(want)), (lens[s], "after the state")
+    dev.close()
