@@ -61,6 +61,21 @@ def test_gemm_f16(pkg, m, n, k):
     assert np.max(np.abs(c - want)) <= 4e-6 * np.sqrt(k) * np.max(np.abs(want)) + 1e-5
 
 
+@pytest.mark.parametrize("m,n,k", [(900, 3700, 64), (1100, 3500, 128), (2000, 1990, 192), (2000, 2000, 256), (1300, 2500, 448), (1900, 2050, 576), (777, 2048, 5888)])
+def test_gemm_f16_four_stages(pkg, m, n, k):
+    """128 x 128 tiles with four stages (one workgroup a compute unit): fewer slices of K than stages, as many and more, ragged M and N, and K split
+    between workgroups.  Tolerance as above: products of halves are exact in fp32, their sum errs like sqrt(k) eps."""
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k), dtype=np.float32).astype(np.float16).astype(np.float32)
+    b = rng.standard_normal((n, k), dtype=np.float32).astype(np.float16).astype(np.float32)
+    r = rng.standard_normal((m, n), dtype=np.float32)
+    c, _ = pkg.selftest_gemm(a, b, r, f16=True)
+    c2, _ = pkg.selftest_gemm(a, b, r, iters=3, f16=True)
+    assert np.array_equal(c, c2)
+    want = a.astype(np.float64) @ b.astype(np.float64).T + r
+    assert np.max(np.abs(c - want)) <= 4e-6 * np.sqrt(k) * np.max(np.abs(want)) + 1e-5
+
+
 @pytest.mark.parametrize("kind", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("m,n,k", [(300, 512, 256), (257, 1000, 704), (130, 36, 128), (100, 256, 512), (64, 320, 256), (9, 128, 2048),
                                    (1100, 17000, 192)])
