@@ -81,13 +81,6 @@ template <typename AT> __device__ __forceinline__ void put_mix(const PfArgs& P, 
     if (P.rows) rows_put(P.rows, col, (int)row, P.lay, P.half != 0, v);
     else put_at<AT>(P.Amix, row, P.aLd, col, v);
 }
-// ... four of them
-template <typename AT> __device__ __forceinline__ void put_mix4(const PfArgs& P, size_t row, int col, const f32x4& v) {
-    if (P.rows) rows_put4(P.rows, col, (int)row, P.lay, P.half != 0, v.x, v.y, v.z, v.w);
-    else if constexpr (sizeof(AT) == 6) p3_put4((unsigned char*)P.Amix + row * P.aLd * 6, col, v.x, v.y, v.z, v.w);
-    else
-        for (int e = 0; e < 4; e++) put_at<AT>(P.Amix, row, P.aLd, col + e, v[e]);
-}
 template <typename WT> __device__ __forceinline__ float getw(const WT* p);
 template <> __device__ __forceinline__ float getw<float>(const float* p) { return *p; }
 template <> __device__ __forceinline__ float getw<bf16_t>(const bf16_t* p) { return __uint_as_float(((uint32_t)*p) << 16); }
@@ -113,6 +106,12 @@ template <> __device__ __forceinline__ void put4<f16_t>(f16_t* o, float a, float
 
 template <typename AT> __device__ __forceinline__ void put4_at(void* base, size_t row, int ld, int col, float a, float b, float c, float d) { put4<AT>((AT*)base + row * ld + col, a, b, c, d); }
 template <> __device__ __forceinline__ void put4_at<p3_t>(void* base, size_t row, int ld, int col, float a, float b, float c, float d) { p3_put4((unsigned char*)base + row * ld * 6, col, a, b, c, d); }
+// Four columns of the mixing output.
+template <typename AT> __device__ __forceinline__ void put_mix4(const PfArgs& P, size_t row, int col, const f32x4& v) {
+    if (P.rows) rows_put4(P.rows, col, (int)row, P.lay, P.half != 0, v.x, v.y, v.z, v.w);
+    else if constexpr (sizeof(AT) == 6) p3_put4((unsigned char*)P.Amix + row * P.aLd * 6, col, v.x, v.y, v.z, v.w);
+    else put4_at<AT>(P.Amix, row, P.aLd, col, v.x, v.y, v.z, v.w);
+}
 
 template <typename AT>
 __global__ void __launch_bounds__(PWG) k_pf_rmsnorm(const float* __restrict__ X, const float* __restrict__ gamma, void* out, int n, int d) {
@@ -609,43 +608,56 @@ __global__ void __launch_bounds__(PWG, H16 ? 2 : 1) k_pf_attn_mfma(PfArgs P, Lay
 // Gated-delta-net prefill.  The rows of a head's state evolve independently of each other
 //   S[r,:] <- alpha S[r,:] + beta (v_r - alpha u_r) k^T,  u_r = S[r,:].k,   o_r = S_new[r,:].q
 // (the decode kernel's update, regrouped; k, q L2-normalised), so one workgroup carries PF_GR rows of
-// one head of one segment in registers across the whole segment: 4 lanes per row, each with DK/4
-// columns.  The decay is kept out of the element loop: the registers hold S / a for a running scalar a
-// (the product of the alphas since the last renormalisation), so a token costs three FMAs per element
-// -- S.k, S.q and the rank-1 update -- instead of four.  Sixteen tokens of q, k, v and gate inputs are staged in LDS at a time, the next sixteen
-// being loaded into registers meanwhile.  With p = S_old[r,:].q the read-out needs no second pass:
+// one head of one segment in registers across the whole segment: eight lanes per two rows, each with DK/8
+// columns of both.  Sixteen tokens of q, k, v and gate inputs are staged in LDS at a time, the next sixteen
+// being loaded into registers meanwhile.  The decay is kept out of the element loop: within the sixteen the registers hold S / a,
+// a the product of their alphas so far, so a token costs three FMAs per element -- S.k, S.q and the rank-1 update --
+// instead of four.  With p = S_old[r,:].q the read-out needs no second pass:
 // o_r = (alpha p + w (k.q)) / |q|,  w = beta (v_r - alpha u_r) / |k|.
+// A token's constants are ready before the sixteen begin, nothing in them branches, and the outputs leave together behind them: what is left
+// from token to token is u's sum, two FMAs and the update.  Bound by that chain with one workgroup on a unit, by issue and by the LDS reads of
+// k and q (why a lane has two rows) with three.  Measured (12 heads of 64): 19 segments of up to 333 tokens 113 us (148 with a branch and the output's
+// conversion inside the token), 64 of up to 512 224 us (263).
 #define PF_GC 16
 #define PF_GR 64
 // Workgroup barrier that orders LDS traffic only: __syncthreads() also waits for every outstanding global
 // load (loads and stores share one counter), which would put the next chunk's prefetch on the critical path.
 __device__ __forceinline__ void pf_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-template <int CTRL> __device__ __forceinline__ float quad_swap(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+template <int CTRL> __device__ __forceinline__ float dpp_of(float v, float other = 0.f) { // lanes whose source lies outside the row of sixteen: `other`
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(other), __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float sum8(float v) { // over eight lanes, in all of them: in the vector ALU (a shuffle through LDS costs some 100 cycles)
+    v += dpp_of<0xB1>(v);         // lanes 0<->1, 2<->3
+    v += dpp_of<0x4E>(v);         // lanes 0<->2, 1<->3
+    return v + dpp_of<0x141>(v);  // lane i <-> 7 - i
 }
 template <int DK, typename AT>
 __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFrom) {
-    constexpr int DV = DK, TPR = PWG / PF_GR, CPT = DK / TPR;
-    static_assert(TPR == 4, "the row sum below is a quad reduction");
+    constexpr int DV = DK, TPR = 8, RPT = PF_GR * TPR / PWG, CPT = DK / TPR;
+    static_assert(RPT == 2, "a pair of rows per eight lanes");
     constexpr int NQK = PF_GC * DK / 4 / PWG; // f32x4 loads per thread for each of q and k
     __shared__ __attribute__((aligned(16))) float qs[PF_GC][DK];
     __shared__ __attribute__((aligned(16))) float ks[PF_GC][DK];
-    __shared__ float vs[PF_GC][PF_GR];
+    __shared__ __attribute__((aligned(16))) float vs[PF_GC][PF_GR];
+    __shared__ __attribute__((aligned(16))) float os[PF_GC][PF_GR];
     __shared__ float zs[PF_GC][2];
-    __shared__ float gate[PF_GC][6]; // alpha, beta, 1/|q|, 1/|k|, k.q, 1/alpha
+    __shared__ float gate[PF_GC][5]; // alpha, beta, 1/|q|, 1/|k|, k.q
+    __shared__ __attribute__((aligned(16))) f32x4 cst[PWG / 64][PF_GC]; // by wave: the factors of u, w, p in the read-out and w in the read-out
     const StepArgs& a = P.a;
-    const int h = blockIdx.x, seg = blockIdx.y, r0 = blockIdx.z * PF_GR, tid = threadIdx.x;
+    const int h = blockIdx.x, seg = blockIdx.y, r0 = blockIdx.z * PF_GR, tid = threadIdx.x, wave = tid >> 6;
     const int seq = P.segSeq[seg], len = P.segLen[seg], row0 = P.segStart[seg];
     if (len >= skipFrom) return; // taken by the chunk-parallel kernels
-    const int r = tid / TPR, cg = tid % TPR, c0 = cg * CPT;
+    const int r = tid / TPR * RPT, cg = tid % TPR, c0 = cg * CPT;
     float* Srow = L.S + (((size_t)seq * a.gdnHeads + h) * DV + r0 + r) * DK + c0;
-    float S[CPT];
+    float S[RPT][CPT];
 #pragma unroll
-    for (int c = 0; c < CPT; c += 4) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(Srow + c);
-        S[c] = v.x; S[c + 1] = v.y; S[c + 2] = v.z; S[c + 3] = v.w;
-    }
-    float ascale = 1.0f, ainv = 1.0f; // S (true state) = ascale * S[] (registers); ainv = 1 / ascale
+    for (int j = 0; j < RPT; j++)
+#pragma unroll
+        for (int c = 0; c < CPT; c += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(Srow + j * DK + c);
+            S[j][c] = v.x; S[j][c + 1] = v.y; S[j][c + 2] = v.z; S[j][c + 3] = v.w;
+        }
+    const float ba = L.gdnBa[h], bb = L.gdnBb[h]; // (loaded inside the loop they would wait for the next sixteen tokens, issued before them)
     f32x4 qreg[NQK], kreg[NQK];
     float vreg[PF_GC * PF_GR / PWG], zreg = 0.f;
     auto fetch = [&](int t0) {
@@ -667,6 +679,11 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
             zreg = P.QKV[(size_t)(row0 + t0 + min(c, last)) * P.qkvLd + ((tid & 1) ? L.offGb : L.offGa) + h];
         }
     };
+    static_assert(PF_GC * PF_GR == 4 * PWG, "the outputs of a chunk: four columns a thread");
+    auto put_outputs = [&](int t0, int nt) { // of the chunk from t0 on
+        const int c = tid / (PF_GR / 4), e4 = tid % (PF_GR / 4) * 4;
+        if (c < nt) put_mix4<AT>(P, (size_t)(row0 + t0 + c), h * DV + r0 + e4, *reinterpret_cast<const f32x4*>(&os[c][e4]));
+    };
     fetch(0);
     for (int t0 = 0; t0 < len; t0 += PF_GC) {
         const int nt = min(PF_GC, len - t0);
@@ -685,65 +702,107 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
         if (tid < 2 * PF_GC) zs[tid >> 1][tid & 1] = zreg;
         pf_lds_barrier();
         if (t0 + PF_GC < len) fetch(t0 + PF_GC); // in flight during this chunk's arithmetic
+        if (t0 > 0) put_outputs(t0 - PF_GC, PF_GC);
         { // per token: |q|, |k|, k.q and the gates -- 16 threads per token
             const int c = tid >> 4, sub = tid & 15;
             float sq = 0.f, sk = 0.f, kq = 0.f;
-            for (int e = sub; e < DK; e += 16) {
-                const float qv = qs[c][e], kv = ks[c][e];
-                sq = fmaf(qv, qv, sq); sk = fmaf(kv, kv, sk); kq = fmaf(kv, qv, kq);
-            }
 #pragma unroll
-            for (int o = 8; o > 0; o >>= 1) { sq += __shfl_xor(sq, o, 64); sk += __shfl_xor(sk, o, 64); kq += __shfl_xor(kq, o, 64); }
+            for (int e = sub * 4; e < DK; e += 64) {
+                const f32x4 qv = *reinterpret_cast<const f32x4*>(&qs[c][e]), kv = *reinterpret_cast<const f32x4*>(&ks[c][e]);
+#pragma unroll
+                for (int i = 0; i < 4; i++) { sq = fmaf(qv[i], qv[i], sq); sk = fmaf(kv[i], kv[i], sk); kq = fmaf(kv[i], qv[i], kq); }
+            }
+            sq = sum8(sq); sk = sum8(sk); kq = sum8(kq);
+            sq += dpp_of<0x140>(sq); sk += dpp_of<0x140>(sk); kq += dpp_of<0x140>(kq); // lane i <-> 15 - i
+            const float za = zs[c][0] + ba, zb = zs[c][1] + bb;
+            const float rq = 1.0f / sqrtf(sq + 1e-6f), rk = 1.0f / sqrtf(sk + 1e-6f);
+            const float sp = fmaxf(za, 0.f) + log1pf(expf(-fabsf(za)));
+            const bool past = c >= nt; // a token past the segment's end leaves the state as it is
             if (sub == 0) {
-                const float za = zs[c][0] + L.gdnBa[h], zb = zs[c][1] + L.gdnBb[h];
-                const float rq = 1.0f / sqrtf(sq + 1e-6f), rk = 1.0f / sqrtf(sk + 1e-6f);
-                const float sp = fmaxf(za, 0.f) + log1pf(expf(-fabsf(za)));
-                gate[c][0] = expf(-sp);
-                gate[c][5] = expf(sp);
-                gate[c][1] = pf_sigmoid(zb);
+                gate[c][0] = past ? 1.f : expf(-sp);
+                gate[c][1] = past ? 0.f : pf_sigmoid(zb);
                 gate[c][2] = rq; gate[c][3] = rk; gate[c][4] = kq * rq * rk; // k.q of the normalised vectors
             }
         }
         pf_lds_barrier();
-#pragma unroll 4
-        for (int c = 0; c < nt; c++) {
+        float aprod; // the product of the chunk's alphas
+        bool fold;   // ... is too small to carry: every token folds its alpha into the registers instead
+        { // a token's constants, by lane (each wave for itself; lanes that agree mod 16 alike)
+            const int c = tid & 15;
             const float alpha = gate[c][0], beta = gate[c][1], rq = gate[c][2], rk = gate[c][3], kqn = gate[c][4];
-            float kk[CPT];
-            float ua[4] = {0.f, 0.f, 0.f, 0.f}, pa[4] = {0.f, 0.f, 0.f, 0.f}; // four independent chains each
-#pragma unroll
-            for (int e = 0; e < CPT; e += 4) {
-                const f32x4 k4 = *reinterpret_cast<const f32x4*>(&ks[c][c0 + e]);
-                const f32x4 q4 = *reinterpret_cast<const f32x4*>(&qs[c][c0 + e]);
-                kk[e] = k4.x; kk[e + 1] = k4.y; kk[e + 2] = k4.z; kk[e + 3] = k4.w;
-                ua[0] = fmaf(S[e], k4.x, ua[0]); ua[1] = fmaf(S[e + 1], k4.y, ua[1]); ua[2] = fmaf(S[e + 2], k4.z, ua[2]); ua[3] = fmaf(S[e + 3], k4.w, ua[3]);
-                pa[0] = fmaf(S[e], q4.x, pa[0]); pa[1] = fmaf(S[e + 1], q4.y, pa[1]); pa[2] = fmaf(S[e + 2], q4.z, pa[2]); pa[3] = fmaf(S[e + 3], q4.w, pa[3]);
-            }
-            float u = (ua[0] + ua[1]) + (ua[2] + ua[3]), p = (pa[0] + pa[1]) + (pa[2] + pa[3]);
-            // sum over the 4 lanes of a row: quad permutes in the VALU (a cross-lane shuffle through LDS costs
-            // ~100 cycles each, and this is the serial path from one token to the next)
-            u += quad_swap<0xB1>(u); p += quad_swap<0xB1>(p);   // lanes 0<->1, 2<->3
-            u += quad_swap<0x4E>(u); p += quad_swap<0x4E>(p);   // lanes 0<->2, 1<->3
-            u *= rk * ascale; p *= rq * ascale;                // against the normalised k and q, with the decay put back
-            const float wn = beta * (vs[c][r] - alpha * u);    // coefficient of the normalised k
-            ascale *= alpha; ainv *= gate[c][5];               // gate[c][5] = 1 / alpha
-            if (ascale < 1.0e-12f) {                           // workgroup-uniform (one head): fold the decay into the registers
-#pragma unroll
-                for (int e = 0; e < CPT; e++) S[e] *= ascale;
-                ascale = 1.0f; ainv = 1.0f;
-            }
-            const float w = wn * rk * ainv;
-#pragma unroll
-            for (int e = 0; e < CPT; e++) S[e] = fmaf(w, kk[e], S[e]);
-            if (cg == 0) put_mix<AT>(P, (size_t)(row0 + t0 + c), h * DV + r0 + r, alpha * p + wn * kqn);
+            float pr = alpha; // of the alphas up to this token
+            pr *= dpp_of<0x111>(pr, 1.f); pr *= dpp_of<0x112>(pr, 1.f); pr *= dpp_of<0x114>(pr, 1.f); pr *= dpp_of<0x118>(pr, 1.f);
+            aprod = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pr), 15));
+            fold = !(aprod >= 1.0e-12f);
+            const float before = fold ? 1.f : dpp_of<0x111>(pr, 1.f), after = fold ? 1.f : pr;
+            f32x4 k4;
+            k4.x = alpha * rk * before; k4.y = beta * rk / after; k4.z = alpha * rq * before; k4.w = beta * kqn;
+            if ((tid & 63) < 16) cst[wave][c] = k4;
         }
-    }
+        f32x4 kept = (f32x4)(0.f); // outputs of tokens cg and cg + 8: rows r, r + 1 each
+        struct Token { f32x4 k[CPT / 4], q[CPT / 4], f; float2 v; };
+        auto load = [&](int c) __attribute__((always_inline)) {
+            Token t;
 #pragma unroll
-    for (int e = 0; e < CPT; e++) S[e] *= ascale;
+            for (int e = 0; e < CPT / 4; e++) {
+                t.k[e] = *reinterpret_cast<const f32x4*>(&ks[c][c0 + 4 * e]);
+                t.q[e] = *reinterpret_cast<const f32x4*>(&qs[c][c0 + 4 * e]);
+            }
+            t.f = cst[wave][c];
+            t.v = *reinterpret_cast<const float2*>(&vs[c][r]);
+            return t;
+        };
+        auto token = [&](int c, const Token& t, bool folding) __attribute__((always_inline)) {
+            float ua[RPT][2] = {}, pa[RPT][2] = {}; // two chains each
 #pragma unroll
-    for (int c = 0; c < CPT; c += 4) {
-        f32x4 v; v.x = S[c]; v.y = S[c + 1]; v.z = S[c + 2]; v.w = S[c + 3];
-        *reinterpret_cast<f32x4*>(Srow + c) = v;
+            for (int e = 0; e < CPT; e++)
+#pragma unroll
+                for (int j = 0; j < RPT; j++) {
+                    ua[j][e & 1] = fmaf(S[j][e], t.k[e / 4][e % 4], ua[j][e & 1]);
+                    pa[j][e & 1] = fmaf(S[j][e], t.q[e / 4][e % 4], pa[j][e & 1]);
+                }
+            const float w0 = fmaf(-t.f.x, sum8(ua[0][0] + ua[0][1]), t.v.x), w1 = fmaf(-t.f.x, sum8(ua[1][0] + ua[1][1]), t.v.y);
+            const float s0 = t.f.y * w0, s1 = t.f.y * w1; // coefficients of k
+            const float alpha = folding ? gate[c][0] : 1.f;
+#pragma unroll
+            for (int e = 0; e < CPT; e++) {
+                S[0][e] = fmaf(s0, t.k[e / 4][e % 4], folding ? alpha * S[0][e] : S[0][e]);
+                S[1][e] = fmaf(s1, t.k[e / 4][e % 4], folding ? alpha * S[1][e] : S[1][e]);
+            }
+            const float o0 = fmaf(t.f.z, sum8(pa[0][0] + pa[0][1]), t.f.w * w0), o1 = fmaf(t.f.z, sum8(pa[1][0] + pa[1][1]), t.f.w * w1);
+            if (c < 8) { kept.x = cg == c ? o0 : kept.x; kept.y = cg == c ? o1 : kept.y; }
+            else { kept.z = cg == c - 8 ? o0 : kept.z; kept.w = cg == c - 8 ? o1 : kept.w; }
+        };
+        if (!fold) {
+            Token t[2];
+            t[0] = load(0);
+#pragma unroll
+            for (int c = 0; c < PF_GC; c++) { // the next token's values are on their way out of LDS during this one
+                if (c + 1 < PF_GC) t[(c + 1) & 1] = load(c + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                token(c, t[c & 1], false);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int j = 0; j < RPT; j++)
+#pragma unroll
+                for (int e = 0; e < CPT; e++) S[j][e] *= aprod;
+        } else {
+            for (int c = 0; c < PF_GC; c++) token(c, load(c), true);
+        }
+        *reinterpret_cast<float2*>(&os[cg][r]) = make_float2(kept.x, kept.y);
+        *reinterpret_cast<float2*>(&os[cg + 8][r]) = make_float2(kept.z, kept.w);
     }
+    pf_lds_barrier();
+    const int tail = (len - 1) / PF_GC * PF_GC;
+    put_outputs(tail, len - tail);
+#pragma unroll
+    for (int j = 0; j < RPT; j++)
+#pragma unroll
+        for (int c = 0; c < CPT; c += 4) {
+            f32x4 v; v.x = S[j][c]; v.y = S[j][c + 1]; v.z = S[j][c + 2]; v.w = S[j][c + 3];
+            *reinterpret_cast<f32x4*>(Srow + j * DK + c) = v;
+        }
 }
 
 // ----------------------------------------------------------------------------
