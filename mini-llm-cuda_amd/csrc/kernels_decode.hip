@@ -1010,14 +1010,14 @@ int mlh_launch_mix(mlh_ctx* c, const StepArgs& a, const LayerDev& L) {
             return -1;
         }
     } else {
-        // few (head, sequence) pairs: a head's rows are split over four workgroups so that every compute unit has work
-        const bool split = a.gdnHeads * a.nseq <= 256;
+        // A head's rows over four workgroups: a state of 16 or 64 KB is latency more than bytes.  Many heads of 64: over two, the norms of q and k being
+        // each workgroup's own.  Measured (us): 12 heads x 19 sequences 5.8, 5.2, 5.0 over one, two, four; x 64 10.9, 8.7, 10.2; four layers of 16 heads
+        // of 128 with everything else, 17 sequences 389, 380, 371; 64 787, 782, 780.
         if (a.gdnDk == 64 && a.gdnDv == 64) {
-            if (split) hipLaunchKernelGGL((k_gdn<64, 64, 4>), dim3(a.gdnHeads, a.nseq, 4), dim3(WG), 0, st, a, L);
-            else hipLaunchKernelGGL((k_gdn<64, 64, 1>), dim3(a.gdnHeads, a.nseq), dim3(WG), 0, st, a, L);
+            if (a.gdnHeads * a.nseq <= 512) hipLaunchKernelGGL((k_gdn<64, 64, 4>), dim3(a.gdnHeads, a.nseq, 4), dim3(WG), 0, st, a, L);
+            else hipLaunchKernelGGL((k_gdn<64, 64, 2>), dim3(a.gdnHeads, a.nseq, 2), dim3(WG), 0, st, a, L);
         } else if (a.gdnDk == 128 && a.gdnDv == 128) {
-            if (split) hipLaunchKernelGGL((k_gdn<128, 128, 4>), dim3(a.gdnHeads, a.nseq, 4), dim3(WG), 0, st, a, L);
-            else hipLaunchKernelGGL((k_gdn<128, 128, 1>), dim3(a.gdnHeads, a.nseq), dim3(WG), 0, st, a, L);
+            hipLaunchKernelGGL((k_gdn<128, 128, 4>), dim3(a.gdnHeads, a.nseq, 4), dim3(WG), 0, st, a, L);
         }
         else {
             c->err = "GDN kernel supports dk = dv = 64 or 128";

@@ -457,3 +457,22 @@ def test_prefill_gdn_strong_decay(pkg, orc, kind):
             err = np.max(np.abs(dev.logits(s) - wants[s])) / np.max(np.abs(wants[s]))
             assert err <= tol, (lens[s], cut, err, tol)
     dev.close()
+
+
+@pytest.mark.parametrize("nseq", [42, 43])
+def test_batched_gdn_split(pkg, orc, nseq):
+    """512 (head, sequence) pairs are where a head's state goes over two workgroups instead of four: 504 and 516 pairs, logits after two steps against the
+    oracle.  Tolerance as for the fp32 prefill: some ten fp32 contractions a layer, each off by at most 2^-24 sqrt(K) of its largest term."""
+    hp = pkg.config(3, dim=256, attnHeads=4, headDim=64, ffnDim=704, transformers=2, vocabSize=1000, gdnHeads=12, maxL=40, maxSeqs=nseq)
+    pkg.set_layer_pattern(hp, 1)
+    model, dev, w = make(pkg, orc, hp, seed=49)
+    prompts = [pkg.random_tokens(700 + s, 0, hp.vocabSize, 1 + s % 5) for s in range(nseq)]
+    dev.prefill_batch(list(range(nseq)), prompts)
+    feed = [pkg.random_tokens(800 + i, 0, hp.vocabSize, nseq) for i in range(2)]
+    for f in feed:
+        dev.decode_step(f)
+    tol = 10 * hp.transformers * np.sqrt(hp.ffnDim) * 2.0 ** -24
+    for s in range(0, nseq, 6):
+        want = orc.forward_full(w, np.concatenate([prompts[s], [f[s] for f in feed]]).astype(np.int32), "f64", last_only=True)["logits"][-1]
+        assert np.max(np.abs(dev.logits(s) - want)) <= tol * np.max(np.abs(want)), s
+    dev.close()
