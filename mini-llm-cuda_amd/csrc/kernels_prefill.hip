@@ -930,6 +930,14 @@ __global__ void __launch_bounds__(2 * DK, 2) k_gdn_prep(PfArgs P, LayerDev L, co
             const int which = tix >> 2, tt = (tix >> 1) & 1, ti = tix & 1;
             const uint16_t* Aop = (which ? q16 : k16) + (32 * tt + n32) * (DK + 8) + 8 * half;
             const uint16_t* Bop = k16 + (32 * ti + n32) * (DK + 8) + 8 * half;
+            const int i_ = 32 * ti + n32;
+            f32x4 gt[4], bt[4]; // of the lane's sixteen tokens, read ahead: behind the stores below every one would wait for its way out of LDS
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                gt[q] = *reinterpret_cast<const f32x4*>(g + 32 * tt + 8 * q + 4 * half);
+                bt[q] = *reinterpret_cast<const f32x4*>(beta + 32 * tt + 8 * q + 4 * half);
+            }
+            const float gi = g[i_];
             f32x16 acc;
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[i] = 0.f;
@@ -937,12 +945,11 @@ __global__ void __launch_bounds__(2 * DK, 2) k_gdn_prep(PfArgs P, LayerDev L, co
             for (int s_ = 0; s_ < DK / 16; s_++)
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, *reinterpret_cast<const u32x4*>(Aop + 16 * s_)),
                                                              __builtin_bit_cast(f16x8, *reinterpret_cast<const u32x4*>(Bop + 16 * s_)), acc, 0, 0, 0);
-            const int i_ = 32 * ti + n32;
 #pragma unroll
             for (int e = 0; e < 16; e++) {
                 const int t = 32 * tt + 8 * (e >> 2) + 4 * half + (e & 3);
-                const float dec = expf(g[t] - g[i_]); // <= 1 where it is used (i <= t)
-                if (which == 0) Am[t * GD_C + i_] = i_ < t ? beta[t] * dec * acc[e] : 0.f;
+                const float dec = expf(gt[e >> 2][e & 3] - gi); // <= 1 where it is used (i <= t)
+                if (which == 0) Am[t * GD_C + i_] = i_ < t ? bt[e >> 2][e & 3] * dec * acc[e] : 0.f;
                 else if (ti <= tt) // (the tile above the diagonal is zero and not stored)
                     *reinterpret_cast<uint16_t*>(img + (Lay::fM + (tt + ti) * 2 + ((slot_of(i_) >> 4) & 1)) * 1024 + (((slot_of(i_) >> 3) & 1) * 32 + (t & 31)) * 16 + 2 * (slot_of(i_) & 7)) =
                         f16_bits(i_ <= t ? dec * acc[e] : 0.f);
@@ -1609,10 +1616,10 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     bool anyGdn = false, fresh = true; // fresh: every segment starts its sequence, all keys of the call are rows of the call
     for (const LayerDev& L : c->layers) anyGdn = anyGdn || L.kind == MLH_KIND_GDN;
     const bool gdnChunked = anyGdn && c->pfDtype == MLH_GEMM_F16 && !rowsPath; // segments of 64 tokens or more: chunk-parallel MFMA path
-    int nblk = 0, nchunk = 0;
+    int nblk = 0, nchunk = 0, chunked = 0; // chunked: segments on that path
     for (int s = 0; s < nseg; s++) {
         nblk += cdiv(lens[s], qb);
-        if (gdnChunked && lens[s] >= GD_C) nchunk += cdiv(lens[s], GD_C);
+        if (gdnChunked && lens[s] >= GD_C) { nchunk += cdiv(lens[s], GD_C); chunked++; }
     }
     int* const h = c->pinMeta.p;
     int *h_ids = h, *h_rowSeq = h + n, *h_rowPos = h + 2 * n, *h_seg = h + 3 * n, *h_blk = h_seg + 5 * nseg, *h_chunk = h_blk + 2 * nblk;
@@ -1690,9 +1697,10 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
                 else hipLaunchKernelGGL((k_pf_attn<128, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
             }
         } else {
-            const int skipFrom = nchunk > 0 ? GD_C : 0x7fffffff;
+            const int skipFrom = gdnChunked ? GD_C : 0x7fffffff;
             const dim3 gr(hp.gdnHeads, nseg, hp.gdnDv / PF_GR);
-            if (hp.gdnDk == 64) {
+            if (chunked == nseg) { // (a launch whose workgroups all return takes 4.7 us a layer)
+            } else if (hp.gdnDk == 64) {
                 PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<64, p3_t>), gr, dim3(PWG), 0, st, P, L, skipFrom),
                                hipLaunchKernelGGL((k_pf_gdn<64, f16_t>), gr, dim3(PWG), 0, st, P, L, skipFrom));
             } else {
