@@ -113,19 +113,24 @@ template <typename AT> __device__ __forceinline__ void put_mix4(const PfArgs& P,
     else put4_at<AT>(P.Amix, row, P.aLd, col, v.x, v.y, v.z, v.w);
 }
 
-template <typename AT>
+// KEEP: 16-byte pieces a lane keeps, rows of up to 256 KEEP elements.  All loads of a row and of the gains go out at once: a load under a comparison, or the
+// gains asked for behind the sum, each add a memory latency.  Measured: 777 rows of 2048 5.4 us (6.3), 517 rows of 768 5.0 us (4.9); 16384 rows of
+// 2048 32 us (37), 6.2 TB/s: part of it comes out of the caches.
+template <typename AT, int KEEP>
 __global__ void __launch_bounds__(PWG) k_pf_rmsnorm(const float* __restrict__ X, const float* __restrict__ gamma, void* out, int n, int d) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= n) return;
     const float* x = X + (size_t)row * d;
-    constexpr int KEEP = 16; // 16-byte pieces a lane keeps: rows of up to 64 * 4 * 16 = 4096 elements
-    f32x4 keep[KEEP];
+    f32x4 keep[KEEP], gain[KEEP];
+#pragma unroll
+    for (int k = 0; k < KEEP; k++) keep[k] = *reinterpret_cast<const f32x4*>(x + min(lane * 4 + k * 256, d - 4));
+#pragma unroll
+    for (int k = 0; k < KEEP; k++) gain[k] = *reinterpret_cast<const f32x4*>(gamma + min(lane * 4 + k * 256, d - 4));
     float s = 0.f;
 #pragma unroll
     for (int k = 0; k < KEEP; k++) {
-        const int i = lane * 4 + k * 256;
-        keep[k] = i < d ? *reinterpret_cast<const f32x4*>(x + i) : (f32x4)(0.f);
-        s = fmaf(keep[k].x, keep[k].x, s); s = fmaf(keep[k].y, keep[k].y, s); s = fmaf(keep[k].z, keep[k].z, s); s = fmaf(keep[k].w, keep[k].w, s);
+        const f32x4 v = lane * 4 + k * 256 < d ? keep[k] : (f32x4)(0.f);
+        s = fmaf(v.x, v.x, s); s = fmaf(v.y, v.y, s); s = fmaf(v.z, v.z, s); s = fmaf(v.w, v.w, s);
     }
     for (int i = lane * 4 + KEEP * 256; i < d; i += 256) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(x + i);
@@ -136,15 +141,19 @@ __global__ void __launch_bounds__(PWG) k_pf_rmsnorm(const float* __restrict__ X,
 #pragma unroll
     for (int k = 0; k < KEEP; k++) {
         const int i = lane * 4 + k * 256;
-        if (i < d) {
-            const f32x4 v = keep[k], g = *reinterpret_cast<const f32x4*>(gamma + i);
-            put4_at<AT>(out, (size_t)row, d, i, g.x * (v.x / r), g.y * (v.y / r), g.z * (v.z / r), g.w * (v.w / r));
-        }
+        const f32x4 v = keep[k], g = gain[k];
+        if (i < d) put4_at<AT>(out, (size_t)row, d, i, g.x * (v.x / r), g.y * (v.y / r), g.z * (v.z / r), g.w * (v.w / r));
     }
     for (int i = lane * 4 + KEEP * 256; i < d; i += 256) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(x + i), g = *reinterpret_cast<const f32x4*>(gamma + i);
         put4_at<AT>(out, (size_t)row, d, i, g.x * (v.x / r), g.y * (v.y / r), g.z * (v.z / r), g.w * (v.w / r));
     }
+}
+template <typename AT> static void launch_rmsnorm(hipStream_t st, const float* X, const float* gamma, void* out, int n, int d) {
+    const dim3 grid((n + 3) / 4);
+    if (d <= 1024) hipLaunchKernelGGL((k_pf_rmsnorm<AT, 4>), grid, dim3(PWG), 0, st, X, gamma, out, n, d);
+    else if (d <= 2048) hipLaunchKernelGGL((k_pf_rmsnorm<AT, 8>), grid, dim3(PWG), 0, st, X, gamma, out, n, d);
+    else hipLaunchKernelGGL((k_pf_rmsnorm<AT, 16>), grid, dim3(PWG), 0, st, X, gamma, out, n, d);
 }
 
 // Per (head, row): per-head RMSNorm of q and k (inference.cu:52-81, 97-111), RoPE on adjacent pairs at the
@@ -1678,8 +1687,8 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
             R.K = d_; R.A = c->rowsX; R.ssqIn = c->rowsSsqX; R.nparts = t == hp.transformers - 1 ? 1 : d_ / RW_TILE; R.C = P.QKV; R.ldc = P.qkvLd;
             mlh_rows_gemm(c, RW_PLAIN, L.WaR, L.rowsA, R);
         } else {
-            PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<p3_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, L.g1, P.Xn, n, d_),
-                           hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, L.g1, P.Xn, n, d_));
+            PF_DISPATCH_WT(c, launch_rmsnorm<p3_t>(st, P.X, L.g1, P.Xn, n, d_),
+                           launch_rmsnorm<f16_t>(st, P.X, L.g1, P.Xn, n, d_));
             GEMM(P.Xn, d_, L.WaP, L.sWa, d_, P.QKV, P.qkvLd, nullptr, 0, n, L.rowsA, d_);
         }
         if (L.kind == MLH_KIND_ATTENTION) {
@@ -1726,8 +1735,8 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
             continue;
         }
         GEMM(P.Amix, P.aLd, L.WoP, L.sWo, L.ad + hp.pleDim, P.H1, d_, P.X, d_, n, d_, L.ad + hp.pleDim); // Wo . a + pleUp . e + x
-        PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<p3_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.H1, L.g2, P.Xn, n, d_),
-                       hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.H1, L.g2, P.Xn, n, d_));
+        PF_DISPATCH_WT(c, launch_rmsnorm<p3_t>(st, P.H1, L.g2, P.Xn, n, d_),
+                       launch_rmsnorm<f16_t>(st, P.H1, L.g2, P.Xn, n, d_));
         { // gate/up projection with SiLU(gate) * up in the epilogue (inference.cu:262-281): U comes out in the GEMM input type
             hipError_t e_ = mlh_gemm_tn_epi(st, dt, 1, P.Xn, d_, L.W13P, d_, P.U, F, nullptr, 0, n, 2 * F, d_, c->gemmWs, L.sW13);
             if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
@@ -1740,8 +1749,8 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         R.K = d_; R.A = c->rowsX; R.ssqIn = c->rowsSsqX; R.nparts = d_ / RW_TILE; R.C = allLogits; R.ldc = hp.vocabSize;
         mlh_rows_gemm(c, RW_PLAIN, c->ER, hp.vocabSize, R);
     } else if (allLogits) {
-        PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_rmsnorm<p3_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, c->gF, P.Xn, n, d_),
-                       hipLaunchKernelGGL((k_pf_rmsnorm<f16_t>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P.X, c->gF, P.Xn, n, d_));
+        PF_DISPATCH_WT(c, launch_rmsnorm<p3_t>(st, P.X, c->gF, P.Xn, n, d_),
+                       launch_rmsnorm<f16_t>(st, P.X, c->gF, P.Xn, n, d_));
         hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, P.Xn, d_, c->EP, d_, allLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_, c->gemmWs, c->sE);
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
     }

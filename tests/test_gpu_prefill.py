@@ -476,3 +476,16 @@ def test_batched_gdn_split(pkg, orc, nseq):
         want = orc.forward_full(w, np.concatenate([prompts[s], [f[s] for f in feed]]).astype(np.int32), "f64", last_only=True)["logits"][-1]
         assert np.max(np.abs(dev.logits(s) - want)) <= tol * np.max(np.abs(want)), s
     dev.close()
+
+
+@pytest.mark.parametrize("heads", [1, 5, 16, 17, 32, 33, 65])
+def test_prefill_norm_widths(pkg, orc, heads):
+    """The row norms of tiled prefills keep 1024, 2048 or 4096 elements a wave and walk the rest: widths on both sides of each, whole and broken multiples of
+    256.  Tolerance as above: some ten fp32 contractions, each off by at most 2^-24 sqrt(K) of its largest term, K up to the width."""
+    hp = pkg.config(2, dim=64 * heads, attnHeads=heads, headDim=64, ffnDim=64, transformers=1, vocabSize=64, maxL=80, maxSeqs=1)
+    model, dev, w = make(pkg, orc, hp, seed=51)
+    prompt = pkg.random_tokens(51, 0, hp.vocabSize, 66)
+    want = orc.forward_full(w, prompt, "f64", last_only=True)["logits"][-1]
+    dev.prefill(0, prompt)
+    assert np.max(np.abs(dev.logits(0) - want)) <= 10 * np.sqrt(max(hp.dim, hp.ffnDim)) * 2.0 ** -24 * np.max(np.abs(want))
+    dev.close()
