@@ -1257,6 +1257,132 @@ __global__ void __launch_bounds__(64, 1) k_gdn_scan(PfArgs P, LayerDev L, const 
         for (int i = 0; i < 16; i++) Sg[(size_t)dv * DK + 32 * j + 8 * (i >> 2) + 4 * half + (i & 3)] = St[j][i];
 }
 
+// The same with one wave per 16 columns, on 16 x 16 x 32 products, where few heads times segments run: half the products, packing and outputs of a chunk
+// on a wave's chain, for twice the operands' way through the caches.  The operand image is the one above.  Its pieces hold the contraction's elements
+// {4 hh .. 4 hh + 3, 8 + 4 hh .. + 3} of step st; lane (n, q) takes those of st = q / 2, hh = q % 2, which makes row 4 q + i of a 16-row tile number
+// 16 (q / 2) + 4 (q % 2) + i of its 32 (tile 0 of a pair) or 8 more (tile 1): the state's dk and X's tokens are kept in that order, so that they are
+// operands as they stand here too.  Measured (head size 128, 13 chunks): 16 heads 16.8 us (26.2 with 32 columns a wave), 4 x 16 heads 24.4 (27.5).
+template <int DK>
+__global__ void __launch_bounds__(64, 1) k_gdn_scan16(PfArgs P, LayerDev L, const int* __restrict__ chunkBase, const unsigned char* __restrict__ ws,
+                                                        const float* __restrict__ gCexp) {
+    constexpr int DV = DK, JT = DK / 32;
+    typedef GdLayout<DK> Lay;
+    const StepArgs& a = P.a;
+    const int h = blockIdx.x, seg = blockIdx.y, dt = blockIdx.z, lane = threadIdx.x, n = lane & 15, q = lane >> 4;
+    const int len = P.segLen[seg];
+    if (len < GD_C) return; // short segments take the recurrent kernel
+    const int seq = P.segSeq[seg], row0 = P.segStart[seg], nch = (len + GD_C - 1) / GD_C, cb = chunkBase[seg];
+    auto place = [](int x) { return 16 * (x >> 3) + 4 * ((x >> 2) & 1) + (x & 3); }; // row x of a pair's first tile among its 32
+    unsigned offR[2], offN[2]; // this lane's piece: rows in that order (tile of the pair), columns in their own (half of the 32)
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        offR[t] = (q >> 1) * 1024 + ((q & 1) * 32 + place(n) + 8 * t) * 16;
+        offN[t] = (q >> 1) * 1024 + ((q & 1) * 32 + n + 16 * t) * 16;
+    }
+    float* Srow = L.S + (((size_t)seq * a.gdnHeads + h) * DV + 16 * dt + n) * DK + place(4 * q);
+    f32x4 St[JT][2]; // S^T: rows dk = 32 j + place(4 q) + 8 t + i, column dv = 16 dt + n
+#pragma unroll
+    for (int j = 0; j < JT; j++)
+#pragma unroll
+        for (int t = 0; t < 2; t++) St[j][t] = *reinterpret_cast<const f32x4*>(Srow + 32 * j + 8 * t);
+    u32x4 kt[2][2][JT], qh[4][JT], mm[3][2], kh[JT][2][2], vt[2]; // this chunk's pieces, each the next chunk's once it has been used
+    auto frag = [&](int c, int f, unsigned off) __attribute__((always_inline)) {
+        return *reinterpret_cast<const u32x4*>(ws + ((size_t)(cb + c) * a.gdnHeads + h) * Lay::total + f * 1024 + off);
+    };
+    auto get_kt = [&](int c, int u, int t, int j) __attribute__((always_inline)) { return frag(c, Lay::fKt + u * 2 * JT + 2 * j, offR[t]); };
+    auto get_qh = [&](int c, int v, int j) __attribute__((always_inline)) { return frag(c, Lay::fQh + (v >> 1) * 2 * JT + 2 * j, offN[v & 1]); };
+    auto get_mm = [&](int c, int p, int o) __attribute__((always_inline)) { return frag(c, Lay::fM + 2 * p, offN[o]); };
+    auto get_kh = [&](int c, int j, int t, int u) __attribute__((always_inline)) { return frag(c, Lay::fKhT + 4 * j + 2 * u, offR[t]); };
+    const unsigned offV = (dt >> 1) * 4096 + ((dt & 1) ? offN[1] : offN[0]);
+    auto get_vt = [&](int c, int u) __attribute__((always_inline)) { return frag(c, Lay::fVt + 2 * u, offV); };
+    auto mfma = [](const u32x4& x, const u32x4& y, const f32x4& z) __attribute__((always_inline)) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x), __builtin_bit_cast(f16x8, y), z, 0, 0, 0);
+    };
+#pragma unroll
+    for (int j = 0; j < JT; j++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) { kt[v >> 1][v & 1][j] = get_kt(0, v >> 1, v & 1, j); qh[v][j] = get_qh(0, v, j); kh[j][v & 1][v >> 1] = get_kh(0, j, v & 1, v >> 1); }
+#pragma unroll
+    for (int u = 0; u < 2; u++) vt[u] = get_vt(0, u);
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+#pragma unroll
+        for (int o = 0; o < 2; o++) mm[p][o] = get_mm(0, p, o);
+    float gC = gCexp[(size_t)cb * a.gdnHeads + h];
+    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0), as a builtin: as above
+    asm volatile("" ::: "memory");
+    for (int c = 0; c < nch; c++) {
+        const int cn = min(c + 1, nch - 1); // (behind the last chunk: that one again, dropped)
+        const float gN = gCexp[(size_t)(cb + cn) * a.gdnHeads + h];
+        u32x4 sop[JT];
+#pragma unroll
+        for (int j = 0; j < JT; j++) {
+            sop[j].x = pack_f16(St[j][0].x, St[j][0].y); sop[j].y = pack_f16(St[j][0].z, St[j][0].w);
+            sop[j].z = pack_f16(St[j][1].x, St[j][1].y); sop[j].w = pack_f16(St[j][1].z, St[j][1].w);
+        }
+        f32x4 X[2][2], Y[4]; // X = Kt S0^T: [tokens 32 u + .., dv];  Y^T = S0 (diag(e^g) Q)^T: [dv, tokens 16 v + ..]
+#pragma unroll
+        for (int v = 0; v < 4; v++) { X[v >> 1][v & 1] = (f32x4)(0.f); Y[v] = (f32x4)(0.f); }
+#pragma unroll
+        for (int j = 0; j < JT; j++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                X[v >> 1][v & 1] = mfma(kt[v >> 1][v & 1][j], sop[j], X[v >> 1][v & 1]);
+                kt[v >> 1][v & 1][j] = get_kt(cn, v >> 1, v & 1, j);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        u32x4 wop[2]; // W^T = Vt - X
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const f16x8 v = __builtin_bit_cast(f16x8, vt[u]);
+            wop[u].x = pack_f16((float)v[0] - X[u][0].x, (float)v[1] - X[u][0].y); wop[u].y = pack_f16((float)v[2] - X[u][0].z, (float)v[3] - X[u][0].w);
+            wop[u].z = pack_f16((float)v[4] - X[u][1].x, (float)v[5] - X[u][1].y); wop[u].w = pack_f16((float)v[6] - X[u][1].z, (float)v[7] - X[u][1].w);
+            vt[u] = get_vt(cn, u);
+        }
+        // S^T <- e^{g_C} S^T + Kh^T W^T: what the next chunk waits for
+#pragma unroll
+        for (int j = 0; j < JT; j++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) St[j][t] *= gC;
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int j = 0; j < JT; j++)
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    St[j][t] = mfma(kh[j][t][u], wop[u], St[j][t]);
+                    kh[j][t][u] = get_kh(cn, j, t, u);
+                }
+        __builtin_amdgcn_sched_barrier(0);
+        // O = Y + M W^T (M is lower triangular: tokens of the first 32 see only those)
+#pragma unroll
+        for (int j = 0; j < JT; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                Y[v] = mfma(sop[j], qh[v][j], Y[v]);
+                qh[v][j] = get_qh(cn, v, j);
+            }
+#pragma unroll
+        for (int p = 0; p < 3; p++) // (0, 0), (1, 0), (1, 1)
+#pragma unroll
+            for (int o = 0; o < 2; o++) {
+                const int v = (p ? 2 : 0) + o;
+                Y[v] = mfma(wop[p >> 1], mm[p][o], Y[v]);
+                mm[p][o] = get_mm(cn, p, o);
+            }
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (n < len - (c * GD_C + 16 * v))
+                put4<f16_t>((f16_t*)P.Amix + (size_t)(row0 + c * GD_C + 16 * v + n) * P.aLd + h * DV + 16 * dt + 4 * q, Y[v].x, Y[v].y, Y[v].z, Y[v].w); // saturating
+        gC = gN;
+    }
+#pragma unroll
+    for (int j = 0; j < JT; j++)
+#pragma unroll
+        for (int t = 0; t < 2; t++) *reinterpret_cast<f32x4*>(Srow + 32 * j + 8 * t) = St[j][t];
+}
+
 // e[row][j] = silu(ple gate output) * P[tok][j], appended to the row of the mixing output
 template <typename WT, typename AT>
 __global__ void k_pf_ple(PfArgs P, LayerDev L) {
@@ -1718,12 +1844,19 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
             }
             if (nchunk > 0) {
                 const int *dcs = d_chunk, *dct = d_chunk + nchunk, *dcb = d_seg + 4 * nseg;
+                // 16 columns a wave up to two waves a compute unit (4 segments of 16 heads of 128: 24.4 us, 27.5 with 32 columns); beyond, the operands'
+                // second way through the caches costs more than the shorter chain gives (8 segments: 51, 41).
+                const bool narrow = hp.gdnHeads * chunked * (hp.gdnDv / 16) <= 2 * c->numCUs;
+#define SCAN(K_, DK_, W_) hipLaunchKernelGGL((K_<DK_>), dim3(hp.gdnHeads, nseg, DK_ / W_), dim3(64), 0, st, P, L, dcb, (const unsigned char*)c->pfGdnWs, c->pfGdnG)
                 if (hp.gdnDk == 64) {
                     hipLaunchKernelGGL((k_gdn_prep<64>), dim3(nchunk, hp.gdnHeads), dim3(128), gdn_prep_lds(64), st, P, L, dcs, dct, (unsigned char*)c->pfGdnWs, c->pfGdnG);
-                    hipLaunchKernelGGL((k_gdn_scan<64>), dim3(hp.gdnHeads, nseg, 2), dim3(64), 0, st, P, L, dcb, (const unsigned char*)c->pfGdnWs, c->pfGdnG);
+                    if (narrow) SCAN(k_gdn_scan16, 64, 16);
+                    else SCAN(k_gdn_scan, 64, 32);
                 } else {
                     hipLaunchKernelGGL((k_gdn_prep<128>), dim3(nchunk, hp.gdnHeads), dim3(256), gdn_prep_lds(128), st, P, L, dcs, dct, (unsigned char*)c->pfGdnWs, c->pfGdnG);
-                    hipLaunchKernelGGL((k_gdn_scan<128>), dim3(hp.gdnHeads, nseg, 4), dim3(64), 0, st, P, L, dcb, (const unsigned char*)c->pfGdnWs, c->pfGdnG);
+                    if (narrow) SCAN(k_gdn_scan16, 128, 16);
+                    else SCAN(k_gdn_scan, 128, 32);
+#undef SCAN
                 }
             }
         }

@@ -403,12 +403,13 @@ def test_prefill_fp32_attention_edges(pkg, orc, kind):
     dev.close()
 
 
-@pytest.mark.parametrize("kind", ["hybrid", "hd128"])
-def test_prefill_bf16_gdn_chunk_edges(pkg, orc, kind):
-    """The chunked gated delta net (chunks of 64 tokens, tiles of 32 tokens and 32 state columns): one chunk, one and a little, tile edges and a last
-    chunk of one token, several segments in one call and each appended to a state; the state is checked by the greedy steps that follow.  Tolerance: that
-    of the bf16 prefill above (half operands)."""
+@pytest.mark.parametrize("kind,heads", [("hybrid", 4), ("hd128", 2), ("hybrid", 24), ("hd128", 12)])
+def test_prefill_bf16_gdn_chunk_edges(pkg, orc, kind, heads):
+    """The chunked gated delta net (chunks of 64 tokens, tiles of 16 or 32 tokens and state columns: the narrow form up to 512 waves, which the cases of
+    few heads stay below and those of many exceed): one chunk, one and a little, tile edges and a last chunk of one token, several segments in one call and
+    each appended to a state; the state is checked by the greedy steps that follow.  Tolerance: that of the bf16 prefill above (half operands)."""
     hp = small_cfg(pkg, kind, weightDtype=pkg.DTYPE_BF16, maxSeqs=6)
+    hp.gdnHeads = heads
     model, dev, w = make(pkg, orc, hp, seed=45, bf16=True)
     lens = [64, 65, 96, 97, 128, 193]
     prompts = [pkg.random_tokens(500 + n, 0, hp.vocabSize, n) for n in lens]
