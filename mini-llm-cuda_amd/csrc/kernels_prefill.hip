@@ -1834,13 +1834,13 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         } else {
             const int skipFrom = gdnChunked ? GD_C : 0x7fffffff;
             const dim3 gr(hp.gdnHeads, nseg, hp.gdnDv / PF_GR);
-            if (chunked == nseg) { // (a launch whose workgroups all return takes 4.7 us a layer)
-            } else if (hp.gdnDk == 64) {
-                PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<64, p3_t>), gr, dim3(PWG), 0, st, P, L, skipFrom),
-                               hipLaunchKernelGGL((k_pf_gdn<64, f16_t>), gr, dim3(PWG), 0, st, P, L, skipFrom));
-            } else {
-                PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<128, p3_t>), gr, dim3(PWG), 0, st, P, L, skipFrom),
-                               hipLaunchKernelGGL((k_pf_gdn<128, f16_t>), gr, dim3(PWG), 0, st, P, L, skipFrom));
+            if (chunked < nseg) { // (a launch whose workgroups all return takes 4.7 us a layer)
+                if (hp.gdnDk == 64)
+                    PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<64, p3_t>), gr, dim3(PWG), 0, st, P, L, skipFrom),
+                                   hipLaunchKernelGGL((k_pf_gdn<64, f16_t>), gr, dim3(PWG), 0, st, P, L, skipFrom));
+                else
+                    PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<128, p3_t>), gr, dim3(PWG), 0, st, P, L, skipFrom),
+                                   hipLaunchKernelGGL((k_pf_gdn<128, f16_t>), gr, dim3(PWG), 0, st, P, L, skipFrom));
             }
             if (nchunk > 0) {
                 const int *dcs = d_chunk, *dct = d_chunk + nchunk, *dcb = d_seg + 4 * nseg;
