@@ -616,19 +616,18 @@ __global__ void __launch_bounds__(PWG, H16 ? 2 : 1) k_pf_attn_mfma(PfArgs P, Lay
 
 // Gated-delta-net prefill.  The rows of a head's state evolve independently of each other
 //   S[r,:] <- alpha S[r,:] + beta (v_r - alpha u_r) k^T,  u_r = S[r,:].k,   o_r = S_new[r,:].q
-// (the decode kernel's update, regrouped; k, q L2-normalised), so one workgroup carries PF_GR rows of
-// one head of one segment in registers across the whole segment: eight lanes per two rows, each with DK/8
-// columns of both.  Sixteen tokens of q, k, v and gate inputs are staged in LDS at a time, the next sixteen
+// (the decode kernel's update, regrouped; k, q L2-normalised), so one workgroup carries GR rows of
+// one head of one segment in registers across the whole segment: eight lanes per two rows (GR = 64) or one (32), each with DK/8
+// columns of them.  Sixteen tokens of q, k, v and gate inputs are staged in LDS at a time, the next sixteen
 // being loaded into registers meanwhile.  The decay is kept out of the element loop: within the sixteen the registers hold S / a,
 // a the product of their alphas so far, so a token costs three FMAs per element -- S.k, S.q and the rank-1 update --
 // instead of four.  With p = S_old[r,:].q the read-out needs no second pass:
 // o_r = (alpha p + w (k.q)) / |q|,  w = beta (v_r - alpha u_r) / |k|.
 // A token's constants are ready before the sixteen begin, nothing in them branches, and the outputs leave together behind them: what is left
 // from token to token is u's sum, two FMAs and the update.  Bound by that chain with one workgroup on a unit, by issue and by the LDS reads of
-// k and q (why a lane has two rows) with three.  Measured (12 heads of 64): 19 segments of up to 333 tokens 113 us (148 with a branch and the output's
-// conversion inside the token), 64 of up to 512 224 us (263).
+// k and q (why a lane has two rows) with three.  Measured (12 heads of 64): 19 segments of up to 333 tokens 101 us with 64 rows, 82 with 32 (148 with a
+// branch and the output's conversion inside the token), 64 of up to 512 215 and 222 (263).
 #define PF_GC 16
-#define PF_GR 64
 // Workgroup barrier that orders LDS traffic only: __syncthreads() also waits for every outstanding global
 // load (loads and stores share one counter), which would put the next chunk's prefetch on the critical path.
 __device__ __forceinline__ void pf_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -640,20 +639,20 @@ __device__ __forceinline__ float sum8(float v) { // over eight lanes, in all of 
     v += dpp_of<0x4E>(v);         // lanes 0<->2, 1<->3
     return v + dpp_of<0x141>(v);  // lane i <-> 7 - i
 }
-template <int DK, typename AT>
+template <int DK, int GR, typename AT>
 __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFrom) {
-    constexpr int DV = DK, TPR = 8, RPT = PF_GR * TPR / PWG, CPT = DK / TPR;
-    static_assert(RPT == 2, "a pair of rows per eight lanes");
+    constexpr int DV = DK, TPR = 8, RPT = GR * TPR / PWG, CPT = DK / TPR;
+    static_assert(RPT == 1 || RPT == 2, "rows per eight lanes");
     constexpr int NQK = PF_GC * DK / 4 / PWG; // f32x4 loads per thread for each of q and k
     __shared__ __attribute__((aligned(16))) float qs[PF_GC][DK];
     __shared__ __attribute__((aligned(16))) float ks[PF_GC][DK];
-    __shared__ __attribute__((aligned(16))) float vs[PF_GC][PF_GR];
-    __shared__ __attribute__((aligned(16))) float os[PF_GC][PF_GR];
+    __shared__ __attribute__((aligned(16))) float vs[PF_GC][GR];
+    __shared__ __attribute__((aligned(16))) float os[PF_GC][GR];
     __shared__ float zs[PF_GC][2];
     __shared__ float gate[PF_GC][5]; // alpha, beta, 1/|q|, 1/|k|, k.q
     __shared__ __attribute__((aligned(16))) f32x4 cst[PWG / 64][PF_GC]; // by wave: the factors of u, w, p in the read-out and w in the read-out
     const StepArgs& a = P.a;
-    const int h = blockIdx.x, seg = blockIdx.y, r0 = blockIdx.z * PF_GR, tid = threadIdx.x, wave = tid >> 6;
+    const int h = blockIdx.x, seg = blockIdx.y, r0 = blockIdx.z * GR, tid = threadIdx.x, wave = tid >> 6;
     const int seq = P.segSeq[seg], len = P.segLen[seg], row0 = P.segStart[seg];
     if (len >= skipFrom) return; // taken by the chunk-parallel kernels
     const int r = tid / TPR * RPT, cg = tid % TPR, c0 = cg * CPT;
@@ -668,7 +667,7 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
         }
     const float ba = L.gdnBa[h], bb = L.gdnBb[h]; // (loaded inside the loop they would wait for the next sixteen tokens, issued before them)
     f32x4 qreg[NQK], kreg[NQK];
-    float vreg[PF_GC * PF_GR / PWG], zreg = 0.f;
+    float vreg[PF_GC * GR / PWG], zreg = 0.f;
     auto fetch = [&](int t0) {
         const int last = len - 1 - t0; // >= 0
 #pragma unroll
@@ -679,8 +678,8 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
             kreg[it] = *reinterpret_cast<const f32x4*>(qkv + L.offK + h * DK + e4);
         }
 #pragma unroll
-        for (int it = 0; it < PF_GC * PF_GR / PWG; it++) {
-            const int i = it * PWG + tid, c = i / PF_GR, e = i % PF_GR;
+        for (int it = 0; it < PF_GC * GR / PWG; it++) {
+            const int i = it * PWG + tid, c = i / GR, e = i % GR;
             vreg[it] = P.QKV[(size_t)(row0 + t0 + min(c, last)) * P.qkvLd + L.offV + h * DV + r0 + e];
         }
         if (tid < 2 * PF_GC) {
@@ -688,9 +687,8 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
             zreg = P.QKV[(size_t)(row0 + t0 + min(c, last)) * P.qkvLd + ((tid & 1) ? L.offGb : L.offGa) + h];
         }
     };
-    static_assert(PF_GC * PF_GR == 4 * PWG, "the outputs of a chunk: four columns a thread");
     auto put_outputs = [&](int t0, int nt) { // of the chunk from t0 on
-        const int c = tid / (PF_GR / 4), e4 = tid % (PF_GR / 4) * 4;
+        const int c = tid / (GR / 4), e4 = tid % (GR / 4) * 4;
         if (c < nt) put_mix4<AT>(P, (size_t)(row0 + t0 + c), h * DV + r0 + e4, *reinterpret_cast<const f32x4*>(&os[c][e4]));
     };
     fetch(0);
@@ -704,9 +702,9 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
             *reinterpret_cast<f32x4*>(&ks[c][e4]) = kreg[it];
         }
 #pragma unroll
-        for (int it = 0; it < PF_GC * PF_GR / PWG; it++) {
+        for (int it = 0; it < PF_GC * GR / PWG; it++) {
             const int i = it * PWG + tid;
-            vs[i / PF_GR][i % PF_GR] = vreg[it];
+            vs[i / GR][i % GR] = vreg[it];
         }
         if (tid < 2 * PF_GC) zs[tid >> 1][tid & 1] = zreg;
         pf_lds_barrier();
@@ -748,8 +746,8 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
             k4.x = alpha * rk * before; k4.y = beta * rk / after; k4.z = alpha * rq * before; k4.w = beta * kqn;
             if ((tid & 63) < 16) cst[wave][c] = k4;
         }
-        f32x4 kept = (f32x4)(0.f); // outputs of tokens cg and cg + 8: rows r, r + 1 each
-        struct Token { f32x4 k[CPT / 4], q[CPT / 4], f; float2 v; };
+        float kept[2][RPT] = {}; // outputs of tokens cg and cg + 8: row r (and r + 1)
+        struct Token { f32x4 k[CPT / 4], q[CPT / 4], f; float v[RPT]; };
         auto load = [&](int c) __attribute__((always_inline)) {
             Token t;
 #pragma unroll
@@ -758,7 +756,8 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
                 t.q[e] = *reinterpret_cast<const f32x4*>(&qs[c][c0 + 4 * e]);
             }
             t.f = cst[wave][c];
-            t.v = *reinterpret_cast<const float2*>(&vs[c][r]);
+#pragma unroll
+            for (int j = 0; j < RPT; j++) t.v[j] = vs[c][r + j];
             return t;
         };
         auto token = [&](int c, const Token& t, bool folding) __attribute__((always_inline)) {
@@ -770,17 +769,15 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
                     ua[j][e & 1] = fmaf(S[j][e], t.k[e / 4][e % 4], ua[j][e & 1]);
                     pa[j][e & 1] = fmaf(S[j][e], t.q[e / 4][e % 4], pa[j][e & 1]);
                 }
-            const float w0 = fmaf(-t.f.x, sum8(ua[0][0] + ua[0][1]), t.v.x), w1 = fmaf(-t.f.x, sum8(ua[1][0] + ua[1][1]), t.v.y);
-            const float s0 = t.f.y * w0, s1 = t.f.y * w1; // coefficients of k
             const float alpha = folding ? gate[c][0] : 1.f;
 #pragma unroll
-            for (int e = 0; e < CPT; e++) {
-                S[0][e] = fmaf(s0, t.k[e / 4][e % 4], folding ? alpha * S[0][e] : S[0][e]);
-                S[1][e] = fmaf(s1, t.k[e / 4][e % 4], folding ? alpha * S[1][e] : S[1][e]);
+            for (int j = 0; j < RPT; j++) {
+                const float w = fmaf(-t.f.x, sum8(ua[j][0] + ua[j][1]), t.v[j]), s = t.f.y * w; // s: the coefficient of k
+#pragma unroll
+                for (int e = 0; e < CPT; e++) S[j][e] = fmaf(s, t.k[e / 4][e % 4], folding ? alpha * S[j][e] : S[j][e]);
+                const float o = fmaf(t.f.z, sum8(pa[j][0] + pa[j][1]), t.f.w * w);
+                kept[c >> 3][j] = cg == (c & 7) ? o : kept[c >> 3][j];
             }
-            const float o0 = fmaf(t.f.z, sum8(pa[0][0] + pa[0][1]), t.f.w * w0), o1 = fmaf(t.f.z, sum8(pa[1][0] + pa[1][1]), t.f.w * w1);
-            if (c < 8) { kept.x = cg == c ? o0 : kept.x; kept.y = cg == c ? o1 : kept.y; }
-            else { kept.z = cg == c - 8 ? o0 : kept.z; kept.w = cg == c - 8 ? o1 : kept.w; }
         };
         if (!fold) {
             Token t[2];
@@ -799,8 +796,8 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
         } else {
             for (int c = 0; c < PF_GC; c++) token(c, load(c), true);
         }
-        *reinterpret_cast<float2*>(&os[cg][r]) = make_float2(kept.x, kept.y);
-        *reinterpret_cast<float2*>(&os[cg + 8][r]) = make_float2(kept.z, kept.w);
+#pragma unroll
+        for (int j = 0; j < RPT; j++) { os[cg][r + j] = kept[0][j]; os[cg + 8][r + j] = kept[1][j]; }
     }
     pf_lds_barrier();
     const int tail = (len - 1) / PF_GC * PF_GC;
@@ -1833,14 +1830,16 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
             }
         } else {
             const int skipFrom = gdnChunked ? GD_C : 0x7fffffff;
-            const dim3 gr(hp.gdnHeads, nseg, hp.gdnDv / PF_GR);
+            // 32 state rows a workgroup up to two heads a compute unit: half the products of a token on a wave's chain.  Measured (heads of 64; us, 64 and 32
+            // rows): 12 heads x 1 segment 44, 34; x 5 66, 47; x 19 101, 82; x 32 177, 141; x 64 215, 222.
             if (chunked < nseg) { // (a launch whose workgroups all return takes 4.7 us a layer)
-                if (hp.gdnDk == 64)
-                    PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<64, p3_t>), gr, dim3(PWG), 0, st, P, L, skipFrom),
-                                   hipLaunchKernelGGL((k_pf_gdn<64, f16_t>), gr, dim3(PWG), 0, st, P, L, skipFrom));
-                else
-                    PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_gdn<128, p3_t>), gr, dim3(PWG), 0, st, P, L, skipFrom),
-                                   hipLaunchKernelGGL((k_pf_gdn<128, f16_t>), gr, dim3(PWG), 0, st, P, L, skipFrom));
+                const bool half = hp.weightDtype == MLH_DTYPE_BF16, few = hp.gdnHeads * nseg <= 2 * c->numCUs;
+#define RECUR(DK_, GR_, AT_) hipLaunchKernelGGL((k_pf_gdn<DK_, GR_, AT_>), dim3(hp.gdnHeads, nseg, DK_ / GR_), dim3(PWG), 0, st, P, L, skipFrom)
+#define RECUR_ROWS(DK_, AT_) do { if (few) RECUR(DK_, 32, AT_); else RECUR(DK_, 64, AT_); } while (0)
+                if (hp.gdnDk == 64) { if (half) RECUR_ROWS(64, f16_t); else RECUR_ROWS(64, p3_t); }
+                else { if (half) RECUR_ROWS(128, f16_t); else RECUR_ROWS(128, p3_t); }
+#undef RECUR_ROWS
+#undef RECUR
             }
             if (nchunk > 0) {
                 const int *dcs = d_chunk, *dct = d_chunk + nchunk, *dcb = d_seg + 4 * nseg;

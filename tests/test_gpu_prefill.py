@@ -431,30 +431,33 @@ def test_prefill_bf16_gdn_chunk_edges(pkg, orc, kind, heads):
     dev.close()
 
 
-@pytest.mark.parametrize("kind", ["hybrid", "hd128"])
-def test_prefill_gdn_strong_decay(pkg, orc, kind):
+@pytest.mark.parametrize("kind,heads,nseg", [("hybrid", 4, 6), ("hd128", 2, 6), ("hybrid", 24, 22), ("hd128", 24, 22)])
+def test_prefill_gdn_strong_decay(pkg, orc, kind, heads, nseg):
     """The recurrent gated delta net carries the product of sixteen decays and folds them into the state one by one where that product is too small:
     heads that keep everything, that forget half, all but a hundredth and all but 1e-17 at every token, over lengths around the sixteen, in one call and
-    appended to a state.  Tolerance: every logit is the end of some ten fp32 contractions a layer, each off by at most 2^-24 sqrt(K) of its largest term."""
-    hp = small_cfg(pkg, kind, maxSeqs=6)
+    appended to a state, with 32 state rows a workgroup and (more than 512 heads of segments) 64.  Tolerance: every logit is the end of some ten fp32
+    contractions a layer, each off by at most 2^-24 sqrt(K) of its largest term."""
+    hp = small_cfg(pkg, kind, maxSeqs=nseg)
+    hp.gdnHeads = heads
     model = pkg.Model.generate(hp, 47).randomize_gains(47)
     for layer in range(hp.transformers):
         b = model.tensor(layer, pkg.T_GDN_ALPHA_B)
         if b is not None:
-            b[:] = np.resize(np.float32([-20.0, 40.0, 5.0, 0.37]), hp.gdnHeads) if layer % 2 else np.resize(np.float32([0.37, 5.0, -20.0, 40.0]), hp.gdnHeads)
+            b[:] = np.resize(np.float32([-20.0, 40.0, 5.0, 0.37]), heads) if layer % 2 else np.resize(np.float32([0.37, 5.0, -20.0, 40.0]), heads)
     dev = pkg.Device(hp, 0)
     dev.upload(model)
     w = orc.Weights.from_model(model)
-    tol = 10 * hp.transformers * np.sqrt(hp.ffnDim) * 2.0 ** -24
-    lens = [66, 79, 80, 81, 95, 130]
-    prompts = [pkg.random_tokens(600 + n, 0, hp.vocabSize, n) for n in lens]
-    wants = [orc.forward_full(w, p, "f64", last_only=True)["logits"][-1] for p in prompts]
+    tol = 10 * hp.transformers * np.sqrt(max(hp.ffnDim, heads * hp.gdnDv)) * 2.0 ** -24
+    lens = np.resize([66, 79, 80, 81, 95, 130], nseg)
+    prompts = [pkg.random_tokens(600 + s, 0, hp.vocabSize, int(n)) for s, n in enumerate(lens)]
+    checked = [0, 1, 2, 3, 4, 5] if nseg == 6 else [1, 11, nseg - 1]
+    wants = {s: orc.forward_full(w, prompts[s], "f64", last_only=True)["logits"][-1] for s in checked}
     for cut in (0, 65):
         dev.reset()
         if cut:
-            dev.prefill_batch(list(range(6)), [p[:cut] for p in prompts])
-        dev.prefill_batch(list(range(6)), [p[cut:] for p in prompts])
-        for s in range(6):
+            dev.prefill_batch(list(range(nseg)), [p[:cut] for p in prompts])
+        dev.prefill_batch(list(range(nseg)), [p[cut:] for p in prompts])
+        for s in checked:
             err = np.max(np.abs(dev.logits(s) - wants[s])) / np.max(np.abs(wants[s]))
             assert err <= tol, (lens[s], cut, err, tol)
     dev.close()
