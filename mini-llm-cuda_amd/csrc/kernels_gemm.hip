@@ -506,7 +506,7 @@ static double w4_us(int M, int N, int K, int cus) {
 // every workgroup writes its partial tile to a workspace and bumps the tile's counter; whichever
 // arrives last adds the partials in slice order -- the result does not depend on arrival order --
 // applies the epilogue and resets the counter.  Partials and counters move with agent-scope atomics
-// (memory-side), which is all the ordering this needs: no cache write-back or invalidate.
+// (memory-side), and every wave waits for its stores before the counter goes up: no cache write-back or invalidate.
 // ----------------------------------------------------------------------------
 __device__ __forceinline__ float g_ald(const float* p) {
     return __uint_as_float(__hip_atomic_load(reinterpret_cast<const unsigned*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
@@ -594,8 +594,8 @@ __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny(const T* __restr
                 g_ast(myPart + ((size_t)mb * 16 + i) * 64 + lane, red_sum(red, mb, i, lane));
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup"); // the stores above have been acknowledged ...
-        __syncthreads();                                        // ... for every wave of the workgroup
+        stores_landed();  // the partial tile is where the last to arrive will read it ...
+        __syncthreads();  // ... for every wave of the workgroup
         if (tid == 0) {
             const unsigned prev = __hip_atomic_fetch_add(counters + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             lastFlag = prev == (unsigned)(ks - 1);
@@ -746,7 +746,7 @@ __global__ void __launch_bounds__(GSK_WAVES * 64) k_gemm_skinny16(const float* _
 #pragma unroll
             for (int r = 0; r < 4; r++) g_ast(myPart + ((size_t)wave * 4 + r) * 64 + lane, wsum(wave, r));
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        stores_landed(); // (as in k_gemm_skinny)
         __syncthreads();
         if (tid == 0) {
             const unsigned prev = __hip_atomic_fetch_add(counters + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -17,9 +17,9 @@
 // eight XCDs).  Agent-scope fences are avoided on purpose: on this part they write back and
 // invalidate the L2 and cost tens of microseconds.  Instead every value that another workgroup
 // reads is written with an agent-scope atomic store (write-through) and read with an agent-scope
-// atomic load (served from the memory side), with workgroup-scope fences for ordering.  Weights are
+// atomic load (served from the memory side); each wave waits for its stores before its workgroup arrives.  Weights are
 // read-only and use ordinary cached loads; each wave issues the loads of its next phase's weight
-// rows before it enters the barrier, so HBM latency overlaps the synchronisation.
+// rows between its arrival at the barrier and the wait, so HBM latency overlaps the synchronisation.
 #include <stdlib.h>
 
 #include "mlh_internal.h"
@@ -174,7 +174,7 @@ struct PersistArgs {
 // XCD (blockIdx % 8) arrive on their group word, the last of a group arrives on the top word, the
 // last there publishes the epoch to the eight release words.
 __device__ __forceinline__ void grid_arrive(const PersistArgs& P, unsigned& epoch) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup"); // this thread's write-through stores have completed
+    stores_landed(); // this wave's write-through stores have completed (no weight loads are in flight: they go out behind the arrival)
     lds_barrier();
     epoch++;
     if (threadIdx.x == 0) {

@@ -176,8 +176,8 @@ __global__ void __launch_bounds__(128 * NW, NW / 2 * tile_wgs<T>(32 * WM + 16 * 
                 tl_ast(mine + (size_t)(2 * (i * WN + j)) * THREADS, (unsigned long long)__float_as_uint(acc[i][j].x) | ((unsigned long long)__float_as_uint(acc[i][j].y) << 32));
                 tl_ast(mine + (size_t)(2 * (i * WN + j) + 1) * THREADS, (unsigned long long)__float_as_uint(acc[i][j].z) | ((unsigned long long)__float_as_uint(acc[i][j].w) << 32));
             }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup"); // the stores above have been acknowledged ...
-        __syncthreads();                                        // ... for every wave of the workgroup
+        stores_landed();  // the partial tile is where the last to arrive will read it ...
+        __syncthreads();  // ... for every wave of the workgroup
         if (tid == 0) {
             const unsigned prev = __hip_atomic_fetch_add(counters + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             lastFlag = prev == (unsigned)(ks - 1);

@@ -23,6 +23,11 @@ struct f16_t { uint16_t bits; };
 #define MLH_GEMM_WS_PARTIALS (256 * 8 * 2 * 16 * 64) // ... and the partial sums (floats) behind them
 #define MLH_SELFTEST_SWIGLU 0x100 // mlh_selftest_gemm: flag beside the operand type, selects the SwiGLU epilogue
 
+// This wave's stores and atomics so far have reached the memory that other workgroups read, the memory side for agent-scope ones.  For
+// what is published by a counter: each storing wave waits here, then the workgroup meets at a barrier, then one thread counts.  A release
+// fence of workgroup scope is not that wait on this target: it orders the waves of one compute unit, and compiles to no wait for stores.
+__device__ __forceinline__ void stores_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // Device-side description of one transformer block.
 struct LayerDev {
     const void* Wa;       // fused first-phase matrix [rowsA, dim]: q|k|v|[g]|[pleGate]|[gdnA|gdnB]

@@ -1,0 +1,62 @@
+"""What the built gfx950 code has to show that no run of it can: listings of libmlh.so's own kernels.  CPU only."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+# Kernels whose workgroups publish partial results or phase outputs by bumping a counter.
+COUNTING = ("k_gemm_tile", "k_gemm_skinny", "k_gemm_skinny16", "k_decode_persistent")
+
+
+@pytest.fixture(scope="module")
+def listing(pkg, tmp_path_factory):
+    """{kernel: its instructions, in address order} of every device code object in the built library."""
+    where = tmp_path_factory.mktemp("code")
+    lib = shutil.copy(os.path.join(pkg.LIB_DIR, "libmlh.so"), where / "libmlh.so")
+    subprocess.run([OBJDUMP, "--offloading", str(lib)], cwd=where, check=True, capture_output=True)
+    out = {}
+    for f in sorted(os.listdir(where)):
+        if not f.endswith("gfx950"):
+            continue
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", f], cwd=where, check=True, capture_output=True, text=True).stdout
+        code = None
+        for line in text.splitlines():
+            head = re.match(r"<(\S+)>:$|^[0-9a-f]+ <(\S+)>:$", line)
+            if head:
+                code = out.setdefault(head.group(1) or head.group(2), [])
+            elif code is not None and line.strip():
+                code.append(line.split("//")[0].strip())
+    return out
+
+
+def kernel_name(symbol):
+    m = re.match(r"_Z(\d+)", symbol)
+    return symbol[m.end():m.end() + int(m.group(1))] if m else symbol
+
+
+def test_stores_have_landed_before_a_counter_says_so(listing):
+    """A counter that tells other workgroups (of another XCD as a rule) that partial sums are in memory may go up only when every
+    wave's stores have been acknowledged: in front of the barrier before the atomic, each wave waits for vmcnt(0) behind its last
+    store.  A workgroup-scope release fence compiles to no such wait on this target."""
+    seen, bad = {}, []
+    for symbol, code in listing.items():
+        name = kernel_name(symbol)
+        if name not in COUNTING:
+            continue
+        for i, ins in enumerate(code):
+            if not ins.startswith("global_atomic_add"):
+                continue
+            seen[name] = seen.get(name, 0) + 1
+            b = next(k for k in range(i, -1, -1) if code[k].startswith("s_barrier"))
+            for k in range(b - 1, -1, -1):
+                op = code[k].split()[0]
+                if op == "s_waitcnt" and re.search(r"vmcnt\(0\)", code[k]):
+                    break
+                if re.match(r"(global|flat|buffer|scratch)_(store|atomic)", op) or op.startswith(("s_cbranch", "s_branch", "s_setpc")):
+                    bad.append((symbol, i, code[k]))
+                    break
+    assert set(seen) == set(COUNTING), seen
+    assert not bad, f"{len(bad)} counters go up while stores may be on their way, the first: {bad[0]}"
