@@ -208,9 +208,9 @@ int mlh_set_graph(mlh_ctx* ctx, int stepsPerGraph);
  * leaves the context at mode 0 (mlh_get_persistent, mlh_persistent_fallbacks).
  * In mode 3 a call of up to 16 sequences (mlh_single_launch_sequences; without graph replays) runs its steps in one launch as
  * well: models with 8 to 16 heads of 64 or 128, gated-delta-net heads of the same size and number, per-layer embeddings of width
- * 32 (fp32), 64 or 128, dim up to 768 (fp32) / 2048 (bf16), ffnDim up to 2048 / 6144 in multiples of 256 / 512.  Its workgroups
- * meet before anything is written; when they do not, the call falls back in the same way.  A wait that expires behind the
- * meeting is an error (-2): the sequences of the call have to be reset.
+ * 32 (fp32), 64 or 128, dim up to 768 (fp32) / 2048 (bf16), ffnDim up to 2048 / 6144 in multiples of 256 / 512.  It gives up
+ * and falls back in the same way: its workgroups meet before anything is written, and it writes gated-delta-net states to a second
+ * place (mlh_create allocates it for the first 16 sequences), so that those from before the launch are there after a wait that expires later.
  * Mode 0, unsupported shapes and more sequences: a sequence of kernels issued as mlh_set_graph says. */
 int mlh_set_persistent(mlh_ctx* ctx, int mode);
 
@@ -226,7 +226,7 @@ int mlh_persistent_fallbacks(mlh_ctx* ctx);
  * any wait having to expire.  mlh_debug_set_xcd_tag: sets the XCD-rank kernel's running tag count (device word and
  * host mirror), to exercise the reset that precedes a wrap of the 32-bit tags. */
 int mlh_debug_inject_abort(mlh_ctx* ctx, int launches);
-/* mlh_debug_inject_abort_at_step: the next single-launch decode launch of one sequence gives up by itself when workgroup 0 reaches
+/* mlh_debug_inject_abort_at_step: the next single-launch decode launch gives up by itself when workgroup 0 reaches
  * decode step `step` (> 0; counted from 0 inside the launch) -- after the earlier steps have run and written what
  * they write -- so the test can see that the redo starts from the state before the launch.  0 switches it off. */
 int mlh_debug_inject_abort_at_step(mlh_ctx* ctx, int step);

@@ -26,7 +26,13 @@
 // 16 would be several blocks of rows one after the other in the same waves: at 19, two blocks took 464, the row kernels 414.
 //
 // The launch starts with a meeting of all 256 workgroups: if one is missing after a bounded wait nothing has been written and the
-// call runs as the sequence of row kernels instead.  Behind it every workgroup is resident, and every wait is bounded as well.
+// call runs as the sequence of row kernels instead.  Behind it every workgroup is resident, and every wait is bounded as well: when
+// one expires the launch ends early and the row kernels redo the steps.  What a redo cannot write anew, the gated-delta-net states, is
+// therefore read from one place in the first step and written to another, which counts when the launch has ended well (the host keeps
+// which one that is, mlh_ranks_done; other kernels know the first only, mlh_ranks_settle).  The same bytes as in place; a copy of the
+// rows made on the way cost 10 to 33 us a launch (d 2048 bf16, 1 and 8 sequences).
+#include <string.h>
+
 #include <algorithm>
 
 #include "mlh_internal.h"
@@ -60,6 +66,9 @@ struct RanksArgs {
     int rowsQ;         // words per token of the first phase's region
     int planeBytes;    // of the operand planes in LDS
     unsigned *abortFlag, *xcdCount;
+    int abortAtStep;   // test hook: workgroup 0 gives up when it reaches this step (> 0)
+    int otherAt;       // floats from a sequence's gated-delta-net states to their second place
+    unsigned sides;    // bit s: the states of sequence s are in the second place before the launch
     unsigned area, oPart, oMl, oMix, oX, oH, oU, oXP, oHP, oAmax, oTok; // bytes of exchange words per XCD and what lies where in them; oAmax, oTok: behind all of them
 };
 
@@ -135,8 +144,9 @@ struct RkShared {
         asm volatile("" : "+s"(X), "+s"(r), "+v"(lane)); \
     } while (0)
 #define RK_BAR() lds_barrier()
-// Once per layer, and not at every barrier (0.1 us each): whether a wait was given up.  Until then the waves go on with what they have,
-// no further wait waits, and nothing outside the launch's own buffers is written.
+// Once per layer, and not at every barrier (0.1 us each): whether a wait was given up.  Until then the waves go on with what they have and
+// no further wait waits; what they publish carries valid tags, so K/V rows from the first step's position on, the states' other
+// place, logits, picks and positions may all be written from it.  The redo writes them again (positions: mlh_ranks_failed).
 #define RK_CHECK()                  \
     do {                            \
         if (runi(S.ctl[0])) return; \
@@ -220,7 +230,7 @@ __device__ __forceinline__ void rk_communicator(const RanksArgs& P, const RkShar
     int rows = 4 * RPI; // of a pair per workgroup: the XCD's 32 workgroups share its pairs
     while (rows < 64 && pairs * HD > rows * RK_PER) rows *= 2;
     const int gPair = runi(r0 / (HD / rows)), gIts = gPair < pairs ? rows / (4 * RPI) : 0; // RPI rows a wave, gIts times; 0: none
-    const int gHead = runi(gPair / mb), gTok = gPair - gHead * mb, gRow = (r0 - gPair * (HD / rows)) * rows + cw * (rows / 4);
+    const int gHead = runi(gPair / mb), gTok = gPair - gHead * mb, gMove = runi((int)(P.sides >> S.seq[gTok])) & 1 ? -P.otherAt : P.otherAt, gRow = (r0 - gPair * (HD / rows)) * rows + cw * (rows / 4);
     const int aSplit = runi((cw * RK_PER + r0) / pairs), aPair = cw * RK_PER + r0 - aSplit * pairs, aHead = runi(aPair / mb), aTok = aPair - aHead * mb;
     int lanesLog = 6; // of the lanes that sum up a row's squares
     while ((mb << lanesLog) > 64) lanesLog--;
@@ -357,6 +367,7 @@ __device__ __forceinline__ void rk_communicator(const RanksArgs& P, const RkShar
         for (int k = 0; k < 2; k++) keep4(k, gain4(layers[NL - 1].g1, k)); // the first norm's gain
         RK_BAR(); // tokens, positions and the first gain in LDS
         RK_CHECK();
+        if (P.abortAtStep > 0 && step == P.abortAtStep && X0 == 0 && r0 == 0) ok = false;
         // A half layer is one product over the residual rows and what follows it: even ones the first phase, the token mixing and the
         // output projection, odd ones gate / up and the down projection; behind them the LM head.
 #pragma unroll 1
@@ -378,8 +389,8 @@ __device__ __forceinline__ void rk_communicator(const RanksArgs& P, const RkShar
                 const int longest = (int)pwave_max((float)S.pos[min(lane, mb - 1)]);
                 return max(1, min(min(RK_COMM * RK_PER / pairs, RK_SPLITS), (longest + BR - 1) / BR));
             };
-            // this wave's first state row (elements: below 2^31, 64 sequences of 16 heads)
-            unsigned stateAt = (unsigned)runi(((S.seq[gTok] * a.gdnHeads + X + RK_XCDS * gHead) * HD + gRow) * HD);
+            // this wave's first state row (elements, below 2^31: ranks_model), as it is read in this step
+            unsigned stateAt = (unsigned)(runi(((S.seq[gTok] * a.gdnHeads + X + RK_XCDS * gHead) * HD + gRow) * HD) + ((gMove > 0) == (step > 0) ? P.otherAt : 0));
             auto key_base = [&](int h, int j) { // row 0 of key block j
                 const int q = j * BR / MLH_KV_PAGE;
                 const int page = q < 64 ? __builtin_amdgcn_readlane(pages, q) : runi(a.pageTable[pageSeq * a.pagesPerSeq + q]);
@@ -520,6 +531,7 @@ __device__ __forceinline__ void rk_communicator(const RanksArgs& P, const RkShar
                             __builtin_amdgcn_raw_buffer_store_b64(z, W, ((((c >> 1) & 1) * ngm + (c >> 2)) * mb + gTok) * 16u + (c & 1) * 8u, own + P.oMix, ST_XCD);
                         }
                     }
+                if (step == 0) St += gMove;
                 if (ok)
 #pragma unroll
                     for (int i = 0; i < ITS; i++)
@@ -1173,6 +1185,16 @@ __global__ void k_ranks_prep(unsigned* abortFlag, unsigned* xcdCount, unsigned s
     if (threadIdx.x == 0) *abortFlag = 0u;
     if (threadIdx.x <= RK_XCDS) xcdCount[threadIdx.x] = threadIdx.x < RK_XCDS ? startCount : 0u;
 }
+// states of sequences that are in their second place, to the first (x: pieces, y: layer, z: sequence)
+__global__ void __launch_bounds__(256) k_ranks_settle(const LayerDev* layers, size_t otherAt4, unsigned which, size_t per4) {
+    f32x4* S = reinterpret_cast<f32x4*>(layers[blockIdx.y].S);
+    if (!S || !(which >> blockIdx.z & 1)) return;
+    S += blockIdx.z * per4;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < per4; i += (size_t)gridDim.x * 256) S[i] = S[otherAt4 + i];
+}
+__global__ void k_ranks_positions(const int* lens, int* pos, int nseq) {
+    if (threadIdx.x < nseq) pos[threadIdx.x] = lens[threadIdx.x];
+}
 __global__ void k_ranks_zero(u32x4* p, size_t n) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) p[i] = (u32x4)(0u);
 }
@@ -1225,12 +1247,19 @@ static bool ranks_plan(const mlh_ctx* c, int n, RanksPlan& p) {
     return at < ((size_t)1 << 31);
 }
 
-// Whether the kernel covers this context's model (memory for its exchange words apart).
-static bool ranks_shape(const mlh_ctx* c) {
+// Floats of one sequence's states of a layer (0: no layer has states).
+static size_t state_floats(const mlh_ctx* c) {
+    for (const LayerDev& L : c->layers)
+        if (L.kind == MLH_KIND_GDN) return (size_t)c->hp.gdnHeads * c->hp.gdnDk * c->hp.gdnDv;
+    return 0;
+}
+
+// Whether the kernel covers a model of these hyper-parameters on this device.
+static bool ranks_model(const mlh_ctx* c) {
     const mlh_hparams& hp = c->hp;
     const bool half = hp.weightDtype == MLH_DTYPE_BF16;
     const int ke = half ? 64 : 32, ca = half ? 4 : 3, tw = half ? 4 : 2, ns = RK_WORK / tw, cw = half ? 6 : 2, t13 = half ? 3 : 2;
-    if (c->numCUs != RK_XCDS * RK_PER || !mlh_rows_applicable(c, 1)) return false;
+    if (c->numCUs != RK_XCDS * RK_PER) return false;
     if (hp.headDim != 64 && hp.headDim != 128) return false;
     if (hp.attnHeads < RK_XCDS || hp.attnHeads > 2 * RK_XCDS || hp.dim != hp.attnHeads * hp.headDim) return false;
     for (const LayerDev& L : c->layers)
@@ -1243,8 +1272,14 @@ static bool ranks_shape(const mlh_ctx* c) {
         for (const LayerDev& L : c->layers)
             if (L.offPle % 16) return false;
     }
-    return true;
+    return (hp.maxSeqs + RK_MAX_SEQS) * state_floats(c) < (size_t)1 << 31; // (state rows: 32-bit offsets)
 }
+
+// Sequences whose states have a second place behind those of all maxSeqs (mlh_create allocates both).
+int mlh_ranks_other_seqs(const mlh_ctx* c) { return ranks_model(c) ? std::min(c->hp.maxSeqs, RK_MAX_SEQS) : 0; }
+
+// Whether the kernel covers this context's model as it has been finalized (memory for its exchange words apart).
+static bool ranks_shape(const mlh_ctx* c) { return ranks_model(c) && mlh_rows_applicable(c, 1); }
 
 bool mlh_ranks_applicable(const mlh_ctx* c, int nseq) { return c->ranksMax >= nseq && mlh_rows_applicable(c, nseq); }
 
@@ -1323,8 +1358,39 @@ int mlh_launch_ranks(mlh_ctx* c, int nseq, int steps) {
         if (const int rc = mlh_ranks_reset(c)) return rc;
     P.tagBase = (unsigned)c->ranksTag;
     c->ranksTag += need;
+    P.otherAt = (int)(hp.maxSeqs * state_floats(c));
+    P.sides = c->ranksSides;
+    P.abortAtStep = c->injectAbortStep;
+    c->injectAbortStep = 0;
     const unsigned startCount = c->injectAbort > 0 ? (unsigned)RK_PER : 0u; // test hook: no workgroup finds a place
     if (c->injectAbort > 0) c->injectAbort--;
     hipLaunchKernelGGL(k_ranks_prep, dim3(1), dim3(64), 0, c->stream, P.abortFlag, P.xcdCount, startCount);
     return ranks_launch(c, &P, p.lds);
+}
+
+// A launch of nseq sequences has ended well: their states are in the place they were not in.
+void mlh_ranks_done(mlh_ctx* c, int nseq) {
+    if (state_floats(c)) c->ranksSides ^= (1u << nseq) - 1u; // (16 at most)
+}
+
+// It has given up (and its stream has drained): positions are what they were, and no word of it is met again.
+int mlh_ranks_failed(mlh_ctx* c, int nseq) {
+    memcpy(c->pinIo.p, c->h_len.data(), (size_t)nseq * 4);
+    hipLaunchKernelGGL(k_ranks_positions, dim3(1), dim3(64), 0, c->stream, (const int*)c->pinIo.p, c->d_pos, nseq);
+    MLH_CHECK(c, hipGetLastError());
+    return mlh_ranks_reset(c);
+}
+
+// Before any other kernel works on sequences [s0, s1): their states are in the first place.
+int mlh_ranks_settle(mlh_ctx* c, int s0, int s1) {
+    s0 = std::min(s0, RK_MAX_SEQS);
+    s1 = std::min(s1, RK_MAX_SEQS);
+    const unsigned which = c->ranksSides & ((1u << s1) - (1u << s0));
+    if (!which) return 0;
+    const size_t per4 = state_floats(c) / 4;
+    hipLaunchKernelGGL(k_ranks_settle, dim3((unsigned)std::min<size_t>(16, (per4 + 255) / 256), c->hp.transformers, s1), dim3(256), 0, c->stream,
+                       (const LayerDev*)c->d_layers, c->hp.maxSeqs * per4, which, per4);
+    MLH_CHECK(c, hipGetLastError());
+    c->ranksSides &= ~which;
+    return 0;
 }

@@ -194,7 +194,6 @@ extern "C" int mlh_create(const mlh_hparams* hpIn, int device, mlh_ctx** out) {
             if ((rc = dev_alloc(c, &L.K, poolFloats)) || (rc = dev_alloc(c, &L.V, poolFloats))) return bail(rc);
         } else {
             if ((rc = dev_alloc(c, &ba, hp.gdnHeads)) || (rc = dev_alloc(c, &bb, hp.gdnHeads))) return bail(rc);
-            if ((rc = dev_alloc(c, &L.S, (size_t)S * hp.gdnHeads * hp.gdnDk * hp.gdnDv))) return bail(rc);
         }
         L.g1 = g1; L.g2 = g2; L.gq = gq; L.gk = gk; L.gdnBa = ba; L.gdnBb = bb;
     }
@@ -223,6 +222,9 @@ extern "C" int mlh_create(const mlh_hparams* hpIn, int device, mlh_ctx** out) {
         c->numCUs = prop.multiProcessorCount;
         c->coopLaunch = prop.cooperativeLaunch != 0;
     }
+    const size_t stateSeqs = (size_t)S + mlh_ranks_other_seqs(c); // states of S sequences, and second places of the first of them
+    for (LayerDev& L : c->layers)
+        if (L.kind == MLH_KIND_GDN && (rc = dev_alloc(c, &L.S, stateSeqs * hp.gdnHeads * hp.gdnDk * hp.gdnDv))) return bail(rc);
     if ((rc = dev_alloc(c, &c->d_layers, (size_t)hp.transformers)) || (rc = dev_alloc(c, &c->d_sync, 64 * 24)) ||
         (rc = dev_alloc(c, &c->pamaxVal, (size_t)c->numCUs)) || (rc = dev_alloc(c, &c->pamaxIdx, (size_t)c->numCUs)) ||
         (rc = dev_alloc(c, &c->kvPart, (size_t)hp.attnHeads * c->pagesPerSeq * (hp.headDim + 2))))
@@ -473,7 +475,10 @@ extern "C" int mlh_reset(mlh_ctx* c, int seq) {
         hipLaunchKernelGGL(k_reset, dim3(gdn ? (unsigned)std::min<size_t>(16, (per4 + 255) / 256) : 1, gdn ? hp.transformers : 1, e - s), dim3(256), 0, c->stream,
                            c->d_layers, c->d_pos, s, per4);
         MLH_CHECK(c, hipGetLastError());
-        for (; s < e; s++) { c->h_len[s] = 0; c->h_dirty[s] = 0; }
+        for (; s < e; s++) {
+            c->h_len[s] = 0; c->h_dirty[s] = 0;
+            if (s < 32) c->ranksSides &= ~(1u << s);
+        }
     }
     return 0;
 }
@@ -557,7 +562,10 @@ extern "C" int mlh_prefill_batch(mlh_ctx* c, int nseg, const int32_t* seqs, cons
     }
     for (long i = 0; i < total; i++)
         if (ids[i] < 0 || ids[i] >= hp.vocabSize) { c->err = "token id out of range"; return -1; }
-    for (int s = 0; s < nseg; s++) touch(c, seqs[s], seqs[s] + 1);
+    for (int s = 0; s < nseg; s++) {
+        touch(c, seqs[s], seqs[s] + 1);
+        if ((rc = mlh_ranks_settle(c, seqs[s], seqs[s] + 1))) return rc;
+    }
     if (c->prefillMode == 0 && total > 1 && mlh_prefill_gemm_supported(c)) // (a single token: the decode step, which splits the keys)
         return mlh_run_prefill_gemm(c, nseg, seqs, ids, lens, nullptr);
     long off = 0;
@@ -585,6 +593,7 @@ extern "C" int mlh_forward_full(mlh_ctx* c, int seq, const int32_t* ids, int n, 
     for (int i = 0; i < n; i++)
         if (ids[i] < 0 || ids[i] >= hp.vocabSize) { c->err = "token id out of range"; return -1; }
     touch(c, seq, seq + 1);
+    if ((rc = mlh_ranks_settle(c, seq, seq + 1))) return rc;
     // device results: logits, probabilities, targets, losses
     const size_t mat = (size_t)n * V * 4, need = mat * (probsOut ? 2 : 1) + (size_t)n * 8;
     if (need > c->fullBytes) {
@@ -687,16 +696,17 @@ static bool use_persistent(const mlh_ctx* c, int nseq) {
 // is then put back to where it was before the launch, so the caller can run the same steps again another way:
 // position, token and the tag counter are written at a kernel's normal end only; K/V rows of the steps that did run
 // are written again with the same values; the XCD-rank kernel keeps gated-delta-net states in LDS until its normal
-// end; the barrier kernel stores them at every step, and gets them back from the copy taken before its launch.
+// end; the barrier kernel stores them at every step, and gets them back from the copy taken before its launch; the kernel of several
+// sequences writes them to a second place, which then does not count, and gets its positions back (picks may have been made).
 static int check_persistent_abort(mlh_ctx* c, int nseq) {
     if (c->d_timing && !use_ranks(c, nseq)) mlh_dump_persistent_timing(c);
     const int flag = c->pinIo.p[c->hp.maxSeqs]; // (end_steps)
-    if (flag && use_ranks(c, nseq)) { // 1, 2: not all workgroups found a place, nothing was written; 3: a wait expired behind that
-        const int rc = mlh_ranks_reset(c);
-        if (rc) return rc;
+    if (use_ranks(c, nseq)) {
+        if (!flag) { mlh_ranks_done(c, nseq); return 0; }
+        if (const int rc = mlh_ranks_failed(c, nseq)) return rc;
         MLH_CHECK(c, hipStreamSynchronize(c->stream));
-        c->err = flag == 3 ? "decode kernel of several sequences abandoned a wait in mid-run: its sequences have to be reset" : "decode kernel of several sequences: not all workgroups were resident";
-        return flag == 3 ? -2 : -3;
+        c->err = flag == 3 ? "decode kernel of several sequences abandoned a wait" : "decode kernel of several sequences: not all workgroups were resident";
+        return -3;
     }
     if (flag) {
         c->err = flag == 2 ? "XCD-rank decode kernel: the workgroups did not spread evenly over the XCDs"
@@ -745,6 +755,7 @@ static int end_steps(mlh_ctx* c, int nout) {
 static int run_steps(mlh_ctx* c, int nseq, int steps) {
     int rc;
     if (use_ranks(c, nseq)) return mlh_launch_ranks(c, nseq, steps);
+    if ((rc = mlh_ranks_settle(c, 0, nseq))) return rc;
     if (use_persistent(c, nseq)) return (c->usePersistent == 3 && mlh_xcd_supported(c)) ? mlh_launch_xcd(c, steps) : mlh_launch_persistent(c, steps);
     if (c->graphSteps >= 1) {
         const int k = c->graphSteps;
@@ -849,6 +860,7 @@ extern "C" int mlh_profile_decode(mlh_ctx* c, const int32_t* first, int nseq, in
     int rc = check_decode(c, first, nseq, steps);
     if (rc) return rc;
     if (!usPerLaunch || !launchesPerStep || steps > 64) { c->err = "bad argument (at most 64 steps)"; return -1; }
+    if ((rc = mlh_ranks_settle(c, 0, nseq))) return rc;
     std::vector<hipEvent_t> events;
     std::vector<int> ids;
     hipEvent_t e0;
@@ -982,6 +994,7 @@ extern "C" int mlh_time_kernel(mlh_ctx* c, int kernel, int layer, int nseq, int 
     for (int s = 0; s < nseq; s++)
         if (c->h_len[s] >= c->hp.maxL) { c->err = "sequence is full"; return -1; }
     touch(c, 0, nseq);
+    if ((rc = mlh_ranks_settle(c, 0, nseq))) return rc;
     hipEvent_t e0, e1;
     MLH_CHECK(c, hipEventCreate(&e0));
     MLH_CHECK(c, hipEventCreate(&e1));

@@ -168,6 +168,7 @@ struct mlh_ctx {
     void* ranksBuf = nullptr;      // its exchange words
     size_t ranksBytes = 0;
     unsigned long long ranksTag = 0; // tags its launches have used
+    unsigned ranksSides = 0;       // bit s: the gated-delta-net states of sequence s are at their second place (slot maxSeqs + s)
     LayerDev* d_layers = nullptr;  // device copy of `layers`
     unsigned* d_sync = nullptr;    // barrier words + abort flag
     float* pamaxVal = nullptr;     // [numCUs]
@@ -275,8 +276,12 @@ void mlh_rows_lm_head(mlh_ctx* c, int n, const float* X, const int* segStart, co
 
 // kernels_ranks.hip: decode steps of several sequences in one launch
 bool mlh_ranks_applicable(const mlh_ctx* c, int nseq);
+int mlh_ranks_other_seqs(const mlh_ctx* c);
 int mlh_ranks_prepare(mlh_ctx* c);
 int mlh_ranks_reset(mlh_ctx* c);
+void mlh_ranks_done(mlh_ctx* c, int nseq);
+int mlh_ranks_failed(mlh_ctx* c, int nseq);
+int mlh_ranks_settle(mlh_ctx* c, int s0, int s1);
 int mlh_launch_ranks(mlh_ctx* c, int nseq, int steps);
 
 // kernels_persistent.hip

@@ -127,6 +127,33 @@ def test_gives_up_at_its_meeting_and_falls_back(pkg, orc):
         dev.close()
 
 
+@pytest.mark.parametrize("case,n,steps,at", [("hybrid16", 16, 4, 1), ("hybrid2", 2, 2, 1), ("half_hd128_one", 1, 3, 2), ("half_hd128", 8, 3, 1),
+                                             ("attn_flags8", 8, 5, 3)])
+def test_gives_up_in_mid_run_and_falls_back(pkg, orc, case, n, steps, at):
+    """A launch that is left in mid-run (forced from the host: workgroup 0 gives up when it reaches that step) has written states, K/V rows,
+    picks and perhaps positions.  The call puts the sequences back and redoes its steps: bit for bit what a context does that runs them
+    as row kernels from the start."""
+    hp = config(pkg, **CASES[case][0])
+    out = {}
+    for inject in (0, 1):
+        dev, _, prompts = start(pkg, orc, hp, n, 5, 80, 97)
+        got = [dev.decode_loop([dev.greedy_token(s) for s in range(n)], 2)]
+        assert dev.persistent_fallbacks() == 0
+        if inject:
+            dev.debug_inject_abort_at_step(at)
+        else:
+            dev.set_persistent(0)
+        got.append(dev.decode_loop([int(t) for t in got[-1][-1]], steps))
+        assert dev.persistent_fallbacks() == inject
+        assert [dev.seq_len(s) for s in range(n)] == [len(p) + 2 + steps for p in prompts]
+        dev.set_persistent(3)
+        got.append(dev.decode_loop([int(t) for t in got[-1][-1]], 2))  # positions, states and rows carried over
+        assert dev.persistent_fallbacks() == inject
+        out[inject] = np.concatenate(got), np.stack([dev.logits(s) for s in range(n)])
+        dev.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
 def test_batches_of_changing_size_share_the_exchange_words(pkg, orc):
     """Calls of 5, 2, 7 and 1 sequences in turn on one context: every size lays the exchange words out differently over what the others left."""
     hp = config(pkg, heads=12, hd=64, ffn=512, layers=4, vocab=1000, ple=64)
