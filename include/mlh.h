@@ -205,7 +205,7 @@ int mlh_set_graph(mlh_ctx* ctx, int stepsPerGraph);
  * by other work), the sequence is as it was before the launch (position, token and tags are written at a kernel's
  * normal end only; the XCD-rank kernel keeps gated-delta-net states in LDS until then, the barrier kernel's are put
  * back from a copy taken before its launch), and the call redoes its steps as the kernel sequence and
- * leaves the context at mode 0 (mlh_get_persistent, mlh_persistent_fallbacks).
+ * leaves the context at mode 0 (mlh_get_persistent, mlh_persistent_fallbacks; of the kernel of several sequences below, that kernel alone).
  * In mode 3 a call of up to 16 sequences (mlh_single_launch_sequences; without graph replays) runs its steps in one launch as
  * well: models with 8 to 16 heads of 64 or 128, gated-delta-net heads of the same size and number, per-layer embeddings of width
  * 32 (fp32), 64 or 128, dim up to 768 (fp32) / 2048 (bf16), ffnDim up to 2048 / 6144 in multiples of 256 / 512.  It gives up
@@ -214,9 +214,11 @@ int mlh_set_graph(mlh_ctx* ctx, int stepsPerGraph);
  * Mode 0, unsupported shapes and more sequences: a sequence of kernels issued as mlh_set_graph says. */
 int mlh_set_persistent(mlh_ctx* ctx, int mode);
 
-/* The mode in effect (it differs from what mlh_set_persistent was given after a fallback), and how many decode
- * calls so far were started as a single launch, gave up a wait and were redone as the kernel sequence.  After such
- * a call the context stays at mode 0; mlh_last_error keeps the reason. */
+/* The mode in effect for as many sequences as the last decode call had (it differs from what mlh_set_persistent was given
+ * after a fallback), and how many decode calls so far were started as a single launch, gave up a wait and were redone as the
+ * kernel sequence.  After such a call of the one-sequence kernels the context stays at mode 0; after one of the kernel of several
+ * sequences it is at mode 0 for the calls which that kernel would take, the others keep their mode.  mlh_set_persistent brings
+ * the kernels back; mlh_last_error keeps the reason. */
 int mlh_get_persistent(mlh_ctx* ctx);
 int mlh_persistent_fallbacks(mlh_ctx* ctx);
 

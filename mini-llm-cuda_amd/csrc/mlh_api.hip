@@ -677,10 +677,11 @@ static int ensure_graph(mlh_ctx* c, int slot, int nseq, int k) {
 
 // Up to 16 sequences, and one of a model that the XCD-rank kernel does not cover, in one launch of kernels_ranks.hip.  (A caller who
 // asked for graph replays gets those.)
-static bool use_ranks(const mlh_ctx* c, int nseq) {
+static bool for_ranks(const mlh_ctx* c, int nseq) {
     if (c->usePersistent != 3 || c->temperature > 0.f || c->graphSteps > 0 || !mlh_ranks_applicable(c, nseq)) return false;
     return nseq > 1 || !mlh_xcd_supported(c);
 }
+static bool use_ranks(const mlh_ctx* c, int nseq) { return !c->ranksOff && for_ranks(c, nseq); }
 
 static bool use_persistent(const mlh_ctx* c, int nseq) {
     if (use_ranks(c, nseq)) return true;
@@ -787,16 +788,18 @@ static int check_decode(mlh_ctx* c, const int32_t* ids, int nseq, int steps) {
         if (c->h_len[s] + steps > hp.maxL) { c->err = "sequence would exceed maxL"; return -1; }
     }
     touch(c, 0, nseq);
+    c->lastDecodeSeqs = nseq;
     return set_identity_slots(c, nseq);
 }
 
 // The single-launch kernels need every compute unit for themselves.  When one gives up (another process or stream
-// holds units), the call is redone as the kernel sequence and the context stays in that mode: the steps cost more,
-// the results are the same.  mlh_get_persistent shows the mode in effect, mlh_persistent_fallbacks how often it happened.
-static int fall_back_to_kernel_sequence(mlh_ctx* c) {
+// holds units), the call is redone as the kernel sequence, and so are the calls after it that the same kernel would take: the steps
+// cost more, the results are the same.  mlh_get_persistent shows the mode in effect, mlh_persistent_fallbacks how often it happened.
+// (The kernel of several sequences goes out of use alone: a call of many sequences does not cost the caller the one-sequence kernel.)
+static void fall_back_to_kernel_sequence(mlh_ctx* c, int nseq) {
     c->persistentFallbacks++;
-    c->usePersistent = 0;
-    return 0;
+    if (use_ranks(c, nseq)) c->ranksOff = true;
+    else c->usePersistent = 0;
 }
 
 extern "C" int mlh_decode_loop(mlh_ctx* c, const int32_t* first, int nseq, int steps, int32_t* out) {
@@ -810,7 +813,7 @@ extern "C" int mlh_decode_loop(mlh_ctx* c, const int32_t* first, int nseq, int s
         if ((rc = end_steps(c, steps * nseq))) return rc;
         if (!single || (rc = check_persistent_abort(c, nseq)) == 0) break;
         if (rc != -3) return rc;
-        fall_back_to_kernel_sequence(c); // and once more, as a sequence of kernels
+        fall_back_to_kernel_sequence(c, nseq); // and once more, as a sequence of kernels
     }
     memcpy(out, c->pinIo.p + c->hp.maxSeqs + 1, (size_t)steps * nseq * 4);
     for (int s = 0; s < nseq; s++) {
@@ -845,7 +848,7 @@ extern "C" int mlh_time_decode(mlh_ctx* c, const int32_t* first, int nseq, int s
         if (rc || (rc = end_steps(c, 0))) break;
         if (!single || (rc = check_persistent_abort(c, nseq)) == 0) break;
         if (rc != -3) break;
-        fall_back_to_kernel_sequence(c);
+        fall_back_to_kernel_sequence(c, nseq);
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -943,10 +946,11 @@ extern "C" int mlh_set_persistent(mlh_ctx* c, int enabled) {
     if (!c) return -1;
     if (enabled != 0 && enabled != 1 && enabled != 3) { c->err = "persistent mode must be 0, 1 or 3"; return -1; }
     c->usePersistent = enabled;
+    c->ranksOff = false;
     return 0;
 }
 
-extern "C" int mlh_get_persistent(mlh_ctx* c) { return c ? c->usePersistent : -1; }
+extern "C" int mlh_get_persistent(mlh_ctx* c) { return !c ? -1 : c->ranksOff && for_ranks(c, c->lastDecodeSeqs) ? 0 : c->usePersistent; }
 extern "C" int mlh_persistent_fallbacks(mlh_ctx* c) { return c ? c->persistentFallbacks : -1; }
 
 extern "C" int mlh_debug_inject_abort(mlh_ctx* c, int launches) {

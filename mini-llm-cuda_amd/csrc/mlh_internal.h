@@ -168,6 +168,8 @@ struct mlh_ctx {
     void* ranksBuf = nullptr;      // its exchange words
     size_t ranksBytes = 0;
     unsigned long long ranksTag = 0; // tags its launches have used
+    bool ranksOff = false;         // it has given up, and is not tried again before mlh_set_persistent
+    int lastDecodeSeqs = 0;        // sequences of the last decode call
     unsigned ranksSides = 0;       // bit s: the gated-delta-net states of sequence s are at their second place (slot maxSeqs + s)
     LayerDev* d_layers = nullptr;  // device copy of `layers`
     unsigned* d_sync = nullptr;    // barrier words + abort flag

@@ -154,6 +154,31 @@ def test_gives_up_in_mid_run_and_falls_back(pkg, orc, case, n, steps, at):
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
 
 
+def test_giving_up_costs_the_one_sequence_kernel_nothing(pkg, orc):
+    """Once the launch of several sequences has given up, calls that it would take run as row kernels; one sequence stays in its single
+    launch (a second forced start shows it: only a single launch takes it)."""
+    hp = config(pkg, heads=12, hd=64, ffn=512, layers=4, vocab=1000, ple=64)
+    dev, w, prompts = start(pkg, orc, hp, 4, 6, 30, 83)
+    assert dev.xcd_decode_supported()
+    hist = [list(p) for p in prompts]
+    nxt = [dev.greedy_token(s) for s in range(4)]
+    for n, arm, mode, fallbacks in ((4, 1, 0, 1), (1, 0, 3, 1), (4, 1, 0, 1), (1, 0, 0, 2), (4, 0, 0, 2)):
+        if arm:
+            dev.debug_inject_abort(1)
+        out = dev.decode_loop(nxt[:n], 2)
+        assert (dev.get_persistent(), dev.persistent_fallbacks()) == (mode, fallbacks)
+        for s in range(n):
+            hist[s] += [nxt[s], int(out[0, s])]
+            nxt[s] = int(out[1, s])
+    for s in range(4):
+        dec = orc.Decoder(w, "f64")
+        for t in hist[s]:
+            _, lg = dec.step(int(t))
+        assert_logits_close(dev.logits(s), lg, RTOL, f"sequence {s}")
+        dec.close()
+    dev.close()
+
+
 def test_batches_of_changing_size_share_the_exchange_words(pkg, orc):
     """Calls of 5, 2, 7 and 1 sequences in turn on one context: every size lays the exchange words out differently over what the others left."""
     hp = config(pkg, heads=12, hd=64, ffn=512, layers=4, vocab=1000, ple=64)
