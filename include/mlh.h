@@ -225,8 +225,8 @@ int mlh_persistent_fallbacks(mlh_ctx* ctx);
 /* Test hooks (no counterpart in the reference).  mlh_debug_inject_abort: the next `launches` single-launch decode
  * launches find their bounded wait already given up (XCD-rank kernels: arrival counters that start full; barrier
  * kernel: an abort flag that starts raised), so every workgroup leaves at once and the fallback path runs without
- * any wait having to expire.  mlh_debug_set_xcd_tag: sets the XCD-rank kernel's running tag count (device word and
- * host mirror), to exercise the reset that precedes a wrap of the 32-bit tags. */
+ * any wait having to expire.  mlh_debug_set_xcd_tag: sets the XCD-rank kernels' running tag counts (of one sequence: device
+ * word and host mirror; of several: host only), to exercise the reset that precedes a wrap of the 32-bit tags. */
 int mlh_debug_inject_abort(mlh_ctx* ctx, int launches);
 /* mlh_debug_inject_abort_at_step: the next single-launch decode launch gives up by itself when workgroup 0 reaches
  * decode step `step` (> 0; counted from 0 inside the launch) -- after the earlier steps have run and written what

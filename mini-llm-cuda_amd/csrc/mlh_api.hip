@@ -971,6 +971,7 @@ extern "C" int mlh_debug_set_xcd_tag(mlh_ctx* c, unsigned tagsUsed) {
     MLH_CHECK(c, hipStreamSynchronize(c->stream));
     MLH_CHECK(c, hipMemcpy(c->d_sync + 64 * 21, &tagsUsed, 4, hipMemcpyHostToDevice));
     c->xcdTagNext = tagsUsed;
+    c->ranksTag = tagsUsed;
     return 0;
 }
 

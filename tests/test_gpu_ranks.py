@@ -16,6 +16,7 @@ GAP_TOL = 2e-5
 CASES = {
     # name: (hyper-parameters, sequences, prompt lengths from .. to, steps)
     "hybrid2": (dict(heads=12, hd=64, ffn=512, layers=4, vocab=1000, ple=64), 2, 3, 40, 5),
+    "ple32": (dict(heads=12, hd=64, ffn=512, layers=4, vocab=700, ple=32), 3, 2, 40, 4),  # the narrowest per-layer embeddings
     "hybrid9": (dict(heads=12, hd=64, ffn=2048, layers=4, vocab=1003, ple=64), 9, 1, 130, 4),
     "hybrid16": (dict(heads=8, hd=64, ffn=256, layers=4, vocab=4111, ple=128), 16, 2, 70, 4),
     "attn_flags5": (dict(heads=9, hd=64, ffn=768, layers=2, vocab=520, ple=0, gdn=False, flags=True, dim_ok=False), 5, 5, 90, 4),
@@ -177,6 +178,58 @@ def test_giving_up_costs_the_one_sequence_kernel_nothing(pkg, orc):
         assert_logits_close(dev.logits(s), lg, RTOL, f"sequence {s}")
         dec.close()
     dev.close()
+
+
+def test_tags_are_cleared_before_they_wrap(pkg, orc):
+    """The 32-bit tags of the exchange words are a running count of layer passes.  With the count set just below 2^32 a launch whose tags
+    do not fit starts from cleared words and count 0; one whose tags just fit runs up to the last; both agree with the oracle."""
+    hp = config(pkg, heads=12, hd=64, ffn=512, layers=4, vocab=1000, ple=64)
+    dev, w, prompts = start(pkg, orc, hp, 3, 6, 40, 101)
+    hist = [list(p) for p in prompts]
+    nxt = [dev.greedy_token(s) for s in range(3)]
+    top, passes = 0xFFFFFFFF, hp.transformers + 1  # a launch of n steps takes n * passes + 1 tags; below `top` they fit
+    for n, tag in ((3, None), (4, top - 4 * passes - 1), (2, None), (5, top - 5 * passes - 2), (1, None), (3, top - 1), (2, None)):
+        if tag is not None:
+            dev.debug_set_xcd_tag(tag)
+        out = dev.decode_loop(nxt, n)
+        for s in range(3):
+            hist[s] += [nxt[s]] + [int(t) for t in out[:-1, s]]
+            nxt[s] = int(out[-1, s])
+    assert dev.get_persistent() == 3 and dev.persistent_fallbacks() == 0
+    for s in range(3):
+        dec = orc.Decoder(w, "f64")
+        check_greedy_against_oracle(dec, prompts[s], hist[s][len(prompts[s]):] + [nxt[s]], GAP_TOL, what=f"sequence {s}")
+        dec.reset()
+        for t in hist[s]:
+            _, lg = dec.step(int(t))
+        assert_logits_close(dev.logits(s), lg, RTOL, f"sequence {s}")
+        dec.close()
+    dev.close()
+
+
+def test_more_than_64_pages(pkg):
+    """A wave holds the first 64 page numbers of its sequence in registers and looks the others up: keys beyond 4096 positions, against the
+    row kernels over the same tokens (1e-4: two orders of fp32 sums; one of 66 pages in another's place moves a logit by some 1e-2)."""
+    hp = config(pkg, heads=8, hd=64, ffn=256, layers=2, vocab=300, ple=0, gdn=False, maxL=4400, maxSeqs=3)
+    out = {}
+    for mode in (3, 0):
+        model = pkg.Model.generate(hp, 7).randomize_gains(7)
+        dev = pkg.Device(hp, 0)
+        dev.upload(model)
+        dev.set_page_table(np.random.default_rng(7).permutation(3 * 69).astype(np.int32))
+        dev.prefill_batch([0, 1, 2], [pkg.random_tokens(7, s, hp.vocabSize, n) for s, n in enumerate((4200, 33, 4094))])
+        dev.set_persistent(mode)
+        assert dev.single_launch_sequences() >= 3
+        lg = []
+        for row in np.random.default_rng(8).integers(0, hp.vocabSize, size=(4, 3)):  # sequence 2 reaches its 65th page on the way
+            dev.decode_step([int(t) for t in row])
+            lg.append([dev.logits(s) for s in range(3)])
+        assert dev.persistent_fallbacks() == 0
+        out[mode] = np.array(lg)
+        dev.close()
+    for i in range(4):
+        for s in range(3):
+            assert_logits_close(out[3][i, s], out[0][i, s], 1e-4, f"step {i} sequence {s}")
 
 
 def test_batches_of_changing_size_share_the_exchange_words(pkg, orc):
