@@ -207,8 +207,9 @@ int mlh_set_graph(mlh_ctx* ctx, int stepsPerGraph);
  * back from a copy taken before its launch), and the call redoes its steps as the kernel sequence and
  * leaves the context at mode 0 (mlh_get_persistent, mlh_persistent_fallbacks; of the kernel of several sequences below, that kernel alone).
  * In mode 3 a call of up to 16 sequences (mlh_single_launch_sequences; without graph replays) runs its steps in one launch as
- * well: models with 8 to 16 heads of 64 or 128, gated-delta-net heads of the same size and number, per-layer embeddings of width
- * 32 (fp32), 64 or 128, dim up to 768 (fp32) / 2048 (bf16), ffnDim up to 2048 / 6144 in multiples of 256 / 512.  It gives up
+ * well: models with 8 to 16 heads of 64 or, with bf16 weights, 128 (more than 8 of them: up to 8 sequences),
+ * gated-delta-net heads of the same size and number, per-layer embeddings of width 32 (fp32), 64 or 128, dim a multiple of 128
+ * up to 768 (fp32) / 2048 (bf16), ffnDim up to 2048 / 6144 in multiples of 256 / 512.  It gives up
  * and falls back in the same way: its workgroups meet before anything is written, and it writes gated-delta-net states to a second
  * place (mlh_create allocates it for the first 16 sequences), so that those from before the launch are there after a wait that expires later.
  * Mode 0, unsupported shapes and more sequences: a sequence of kernels issued as mlh_set_graph says. */

@@ -123,7 +123,7 @@ __device__ __forceinline__ void rk_mul(const RkW<bf16_t>& w, const RkOp<bf16_t>&
 // w1b: a third tile of gate / up, then the rest of the down projection; w2: output projection, then the down projection, TW tiles of which
 // NS workers share one.
 template <typename WT, int HD> struct RkCfg;
-template <int HD> struct RkCfg<float, HD> { static constexpr int CA = 3, NTB = 0, TW = 2, CO = HD == 64 ? 2 : 3, CW = 2; };
+template <> struct RkCfg<float, 64> { static constexpr int CA = 3, NTB = 0, TW = 2, CO = 2, CW = 2; }; // (8 heads of 128 are wider than fp32 weights fit)
 template <int HD> struct RkCfg<bf16_t, HD> { static constexpr int CA = 4, NTB = 1, TW = 4, CO = HD == 64 ? 2 : 3, CW = 6; };
 
 struct RkShared {
@@ -1260,7 +1260,7 @@ static bool ranks_model(const mlh_ctx* c) {
     const bool half = hp.weightDtype == MLH_DTYPE_BF16;
     const int ke = half ? 64 : 32, ca = half ? 4 : 3, tw = half ? 4 : 2, ns = RK_WORK / tw, cw = half ? 6 : 2, t13 = half ? 3 : 2;
     if (c->numCUs != RK_XCDS * RK_PER) return false;
-    if (hp.headDim != 64 && hp.headDim != 128) return false;
+    if (hp.headDim != 64 && (!half || hp.headDim != 128)) return false;
     if (hp.attnHeads < RK_XCDS || hp.attnHeads > 2 * RK_XCDS || hp.dim != hp.attnHeads * hp.headDim) return false;
     for (const LayerDev& L : c->layers)
         if (L.kind != MLH_KIND_ATTENTION && (hp.gdnHeads != hp.attnHeads || hp.gdnDk != hp.headDim || hp.gdnDv != hp.headDim)) return false;
@@ -1299,7 +1299,7 @@ static int ranks_launch(mlh_ctx* c, const RanksArgs* P, size_t lds) {
 static int ranks_launch(mlh_ctx* c, const RanksArgs* P, size_t lds) {
     const bool half = c->hp.weightDtype == MLH_DTYPE_BF16, wide = c->hp.headDim == 128;
     if (half) return wide ? ranks_launch<bf16_t, 128>(c, P, lds) : ranks_launch<bf16_t, 64>(c, P, lds);
-    return wide ? ranks_launch<float, 128>(c, P, lds) : ranks_launch<float, 64>(c, P, lds);
+    return ranks_launch<float, 64>(c, P, lds);
 }
 
 int mlh_ranks_reset(mlh_ctx* c) {

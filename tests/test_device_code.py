@@ -60,3 +60,9 @@ def test_stores_have_landed_before_a_counter_says_so(listing):
                     break
     assert set(seen) == set(COUNTING), seen
     assert not bad, f"{len(bad)} counters go up while stores may be on their way, the first: {bad[0]}"
+
+
+def test_every_built_form_of_the_decode_of_several_sequences_is_reached(listing):
+    """fp32 weights with heads of 64, bf16 with 64 and 128: what the rule for a model lets through, and no kernel beside it."""
+    forms = {s[s.index("I") + 1:s.index("EE")] for s in listing if kernel_name(s) == "k_decode_ranks"}
+    assert forms == {"fLi64", "tLi64", "tLi128"}
