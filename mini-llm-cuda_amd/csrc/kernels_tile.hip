@@ -310,8 +310,8 @@ static hipError_t launch_tile(hipStream_t stream, int epi, const void* A, int ld
 // them on a unit takes slices * us[k - 1] + 3.  us: measured per K slice with one, two and three workgroups on every
 // unit (the loads, barriers and LDS reads of a workgroup hide behind the others' MFMAs).
 struct TileCost { int tm, tn, slots; double us[3]; };
-// Variants of the two-byte types: 64 x 64; 128 x 128 with two stages, two workgroups a unit; 128 x 128 with four stages, for launches that
-// put one on a unit: nothing but its own stages then covers the way of a slice from memory.  777 x 2048 x 5888, K split in two, weights cold
+// Variants of the two-byte types: 64 x 64; 128 x 128 with two stages, two workgroups a unit; halves only (what the models multiply): 128 x 128
+// with four stages, for launches that put one on a unit: nothing but its own stages then covers the way of a slice from memory.  777 x 2048 x 5888, K split in two, weights cold
 // (a prefill reads each once): 36.8 us against 48.3 with two stages; on 512 workgroups (3270 rows) 114 against 110.
 static const TileCost kCostHalf[3] = {{64, 64, 3, {0.26, 0.38, 0.58}}, {128, 128, 2, {0.64, 1.04, 0.0}}, {128, 128, 1, {0.58, 0.0, 0.0}}};
 static const TileCost kCostP3[2] = {{64, 64, 2, {0.39, 0.75, 0.0}}, {128, 128, 1, {1.28, 0.0, 0.0}}};
@@ -344,7 +344,7 @@ static double tile_choice(int dtype, int M, int N, int K, int cus, bool ws, Tile
     const bool p3 = dtype == MLH_GEMM_P3;
     const int slices = K / (p3 ? P3_BLOCK : 64);
     double best = 0.0;
-    for (int v = 0; v < (p3 ? 2 : 3); v++) {
+    for (int v = 0; v < (dtype == MLH_GEMM_F16 ? 3 : 2); v++) {
         int ks;
         const double us = best_split(p3 ? kCostP3[v] : kCostHalf[v], M, N, slices, cus, ws, ks);
         if (v == 0 || us < best) { best = us; c.variant = v; c.ks = ks; }
@@ -366,10 +366,10 @@ hipError_t mlh_gemm_tile(hipStream_t stream, int dtype, int epi, const void* A, 
     // Measured (517 x 768 x 3072, 517 x 6144 x 768, 17000 x 768 x 2048; us): planes 27, 35, 335 -- fp32 MFMA tiles of 256 x 256 took
     // 701, 187, 512 --, halves 13, 13, 69.  fp32: 64 x 64 by eight waves of 32 x 16, three stages (two workgroups a unit), or
     // 128 x 128 by eight waves of 64 x 32, two stages.  Two-byte operands: 64 x 64 by four waves of 32 x 32, three stages, or
-    // 128 x 128 by eight waves, two stages (two workgroups a unit) or four (one).
+    // 128 x 128 by eight waves, two stages (two workgroups a unit) or, halves, four (one).
     if (dtype == MLH_GEMM_P3) return c.variant == 0 ? TILE(p3_t, 2, 1, 4, 3) : TILE(p3_t, 4, 2, 4, 2);
     if (dtype == MLH_GEMM_F16) return c.variant == 0 ? TILE(f16_t, 2, 2, 2, 3) : c.variant == 1 ? TILE(f16_t, 4, 2, 4, 2) : TILE(f16_t, 4, 2, 4, 4);
-    return c.variant == 0 ? TILE(bf16_t, 2, 2, 2, 3) : c.variant == 1 ? TILE(bf16_t, 4, 2, 4, 2) : TILE(bf16_t, 4, 2, 4, 4);
+    return c.variant == 0 ? TILE(bf16_t, 2, 2, 2, 3) : TILE(bf16_t, 4, 2, 4, 2);
 #undef TILE
 }
 

@@ -66,3 +66,9 @@ def test_every_built_form_of_the_decode_of_several_sequences_is_reached(listing)
     """fp32 weights with heads of 64, bf16 with 64 and 128: what the rule for a model lets through, and no kernel beside it."""
     forms = {s[s.index("I") + 1:s.index("EE")] for s in listing if kernel_name(s) == "k_decode_ranks"}
     assert forms == {"fLi64", "tLi64", "tLi128"}
+
+
+def test_tiles_of_four_stages_exist_for_halves_only(listing):
+    """No model multiplies bf16 operands (they become scaled halves at finalize), and planes take two or three stages."""
+    forms = {s[s.index("I") + 1:s.index("EE")] for s in listing if kernel_name(s) == "k_gemm_tile"}
+    assert {f.split("Li")[0] for f in forms if f.split("Li")[4] == "4E"} == {"5f16_t"}, forms
