@@ -50,6 +50,7 @@ template <> struct GemmTraits<bf16_t> {
         const uint32_t u = __float_as_uint(v);
         return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
     }
+    static __device__ __forceinline__ uint32_t bits2(float lo, float hi) { return bits(lo) | (bits(hi) << 16); }
     static __device__ __forceinline__ void put(bf16_t* p, float v) { *p = (bf16_t)bits(v); }
 };
 
@@ -57,10 +58,11 @@ template <> struct GemmTraits<f16_t> {
     static __device__ __forceinline__ void mma(const u32x4& a, const u32x4& b, f32x16& c) {
         c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
     }
-    static __device__ __forceinline__ uint32_t bits(float v) { // saturating: an overflow must not become inf
-        const _Float16 h = (_Float16)fminf(fmaxf(v, -65504.0f), 65504.0f);
+    static __device__ __forceinline__ uint32_t bits(float v) {
+        const _Float16 h = (_Float16)half_range(v);
         return __builtin_bit_cast(uint16_t, h);
     }
+    static __device__ __forceinline__ uint32_t bits2(float lo, float hi) { return pack_f16(lo, hi); } // (under halves_saturate)
     static __device__ __forceinline__ void put(f16_t* p, float v) { p->bits = (uint16_t)bits(v); }
 };
 
@@ -389,12 +391,13 @@ __global__ void __launch_bounds__(GW_THREADS) k_gemm_tn_w4(const T* __restrict__
                         const float g0 = acc[bm][bn].x * alpha, u0 = acc[bm][bn].y * alpha;
                         const float g1 = acc[bm][bn].z * alpha, u1 = acc[bm][bn].w * alpha;
                         // silu(g) u = g u / (1 + e^-g) on the hardware's exp2 and reciprocal (1 ulp each: far inside the rounding
-                        // of the two-byte result); e^-g = inf gives 0, as the limit does
-                        const float o0 = g0 * u0 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * g0));
-                        const float o1 = g1 * u1 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * g1));
-                        *(lds_u32*)(pp + r16 * GW_EP + (bn * 8 + 2 * kq) * 2) = GemmTraits<T>::bits(o0) | (GemmTraits<T>::bits(o1) << 16);
+                        // of the two-byte result); e^-g = inf gives 0, as the limit does (g u first could be inf, and inf * 0 is NaN)
+                        const float o0 = g0 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * g0)) * u0;
+                        const float o1 = g1 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * g1)) * u1;
+                        *(lds_u32*)(pp + r16 * GW_EP + (bn * 8 + 2 * kq) * 2) = GemmTraits<T>::bits2(o0, o1);
                     }
                 };
+                halves_saturate(1); // (777 x 11264 x 2048: 43.5 us, 44.2 with half_range; 42.4 with a clamp that lost NaN)
                 if (inside) { // interior tile: block bm + 1 is formed and written into the other patch while block bm comes back
                     put(0, patch);
 #pragma unroll
@@ -431,6 +434,7 @@ __global__ void __launch_bounds__(GW_THREADS) k_gemm_tn_w4(const T* __restrict__
                         }
                     }
                 }
+                halves_saturate(0);
             }
         }
         id += (int)gridDim.x;

@@ -69,8 +69,8 @@ __device__ __forceinline__ float pf_silu(float v) { return v / (1.0f + expf(-v))
 
 // store a float as the GEMM input type (IEEE half for bf16 models, whose MFMA path runs in fp16)
 template <typename AT> __device__ __forceinline__ void put(AT* p, float v);
-template <> __device__ __forceinline__ void put<f16_t>(f16_t* p, float v) { // saturating: an overflow must not become inf
-    const _Float16 h = (_Float16)fminf(fmaxf(v, -65504.0f), 65504.0f);
+template <> __device__ __forceinline__ void put<f16_t>(f16_t* p, float v) {
+    const _Float16 h = (_Float16)half_range(v);
     p->bits = __builtin_bit_cast(uint16_t, h);
 }
 // element `col` of row `row` of a GEMM input matrix (leading dimension ld in elements; fp32 models: three bf16 planes, p3.h)
@@ -97,11 +97,8 @@ __global__ void k_pf_embed(PfArgs P) {
 // 4096 elements stay in registers between the sum of squares and the scaling (one pass over memory), and a lane's
 // four results leave as one store.
 template <typename AT> __device__ __forceinline__ void put4(AT* o, float a, float b, float c, float d);
-template <> __device__ __forceinline__ void put4<f16_t>(f16_t* o, float a, float b, float c, float d) { // saturating like put<f16_t>
-    auto h = [](float v) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)fminf(fmaxf(v, -65504.0f), 65504.0f)); };
-    uint2 w;
-    w.x = h(a) | (h(b) << 16); w.y = h(c) | (h(d) << 16);
-    *reinterpret_cast<uint2*>(o) = w;
+template <> __device__ __forceinline__ void put4<f16_t>(f16_t* o, float a, float b, float c, float d) {
+    *reinterpret_cast<uint2*>(o) = make_uint2(pack_half_range(a, b), pack_half_range(c, d));
 }
 
 template <typename AT> __device__ __forceinline__ void put4_at(void* base, size_t row, int ld, int col, float a, float b, float c, float d) { put4<AT>((AT*)base + row * ld + col, a, b, c, d); }
@@ -158,10 +155,6 @@ template <typename AT> static void launch_rmsnorm(hipStream_t st, const float* X
 
 // Per (head, row): per-head RMSNorm of q and k (inference.cu:52-81, 97-111), RoPE on adjacent pairs at the
 // row's position (inference.cu:113-134), q written back in place, k and v written to the KV pages.
-__device__ __forceinline__ uint32_t pack_f16(float lo, float hi) { // two floats -> two IEEE halves (round to nearest even)
-    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, f16x2{(_Float16)lo, (_Float16)hi}); // (one instruction; put together from two halves it is three)
-}
 
 template <int HD>
 __global__ void __launch_bounds__(64) k_pf_qk_rope_kv(PfArgs P, LayerDev L) {
@@ -1221,10 +1214,7 @@ __global__ void __launch_bounds__(64, 1) k_gdn_scan(PfArgs P, LayerDev L, const 
             u32x2 w[4];
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                float o[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) o[e] = fminf(fmaxf(Y[tt][4 * g + e], -65504.0f), 65504.0f); // saturating: an overflow must not become inf
-                w[g].x = pack_f16(o[0], o[1]); w[g].y = pack_f16(o[2], o[3]);
+                w[g].x = pack_half_range(Y[tt][4 * g], Y[tt][4 * g + 1]); w[g].y = pack_half_range(Y[tt][4 * g + 2], Y[tt][4 * g + 3]);
             }
             // half 0 keeps pieces g = 0, 2 (and gets the partner's upper halves of them), half 1 keeps g = 1, 3
             u32x2 give[2], got[2];
@@ -1371,7 +1361,7 @@ __global__ void __launch_bounds__(64, 1) k_gdn_scan16(PfArgs P, LayerDev L, cons
 #pragma unroll
         for (int v = 0; v < 4; v++)
             if (n < len - (c * GD_C + 16 * v))
-                put4<f16_t>((f16_t*)P.Amix + (size_t)(row0 + c * GD_C + 16 * v + n) * P.aLd + h * DV + 16 * dt + 4 * q, Y[v].x, Y[v].y, Y[v].z, Y[v].w); // saturating
+                put4<f16_t>((f16_t*)P.Amix + (size_t)(row0 + c * GD_C + 16 * v + n) * P.aLd + h * DV + 16 * dt + 4 * q, Y[v].x, Y[v].y, Y[v].z, Y[v].w);
         gC = gN;
     }
 #pragma unroll

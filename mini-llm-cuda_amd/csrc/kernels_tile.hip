@@ -250,16 +250,11 @@ __global__ void __launch_bounds__(128 * NW, NW / 2 * tile_wgs<T>(32 * WM + 16 * 
 #pragma unroll
                     for (int p = 0; p < 3; p++) *reinterpret_cast<uint32_t*>(row + p3_offset(j) + p * P3_PLANE) = w[p];
                 } else { // exp2 and reciprocal of the hardware (1 ulp each): far inside the rounding of a two-byte result
-                    float o[2] = {v.x * v.y * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * v.x)),
-                                  v.z * v.w * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * v.z))};
-                    uint32_t w = 0;
-#pragma unroll
-                    for (int e = 0; e < 2; e++) {
-                        uint32_t b;
-                        if (__is_same(T, f16_t)) b = __builtin_bit_cast(uint16_t, (_Float16)fminf(fmaxf(o[e], -65504.0f), 65504.0f)); // saturating
-                        else b = __builtin_bit_cast(uint16_t, (__bf16)o[e]);
-                        w |= b << (16 * e);
-                    }
+                    float o[2] = {v.x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * v.x)) * v.y, // (the factor that can be 0 before the one that could overflow)
+                                  v.z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * v.z)) * v.w};
+                    uint32_t w;
+                    if (__is_same(T, f16_t)) w = pack_half_range(o[0], o[1]);
+                    else w = __builtin_bit_cast(uint16_t, (__bf16)o[0]) | (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)o[1]) << 16;
                     *reinterpret_cast<uint32_t*>(row + j * 2) = w;
                 }
             }

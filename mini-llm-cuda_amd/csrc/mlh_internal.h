@@ -28,6 +28,21 @@ struct f16_t { uint16_t bits; };
 // fence of workgroup scope is not that wait on this target: it orders the waves of one compute unit, and compiles to no wait for stores.
 __device__ __forceinline__ void stores_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// A value on its way into an IEEE half: finite ones saturate (an overflow must not become an infinity), infinities and NaN stay what they
+// are.
+__device__ __forceinline__ float half_range(float v) {
+    const float s = __builtin_amdgcn_fmed3f(v, -65504.0f, 65504.0f);
+    return __builtin_amdgcn_classf(v, 0x207) ? v : s; // either NaN, either infinity
+}
+__device__ __forceinline__ uint32_t pack_f16(float lo, float hi) { // two floats -> two IEEE halves (round to nearest even)
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, f16x2{(_Float16)lo, (_Float16)hi}); // (one instruction; put together from two halves it is three)
+}
+__device__ __forceinline__ uint32_t pack_half_range(float lo, float hi) { return pack_f16(half_range(lo), half_range(hi)); }
+// The same from the conversion itself (FP16_OVFL of the wave's mode register), between halves_saturate(1) and (0): for an epilogue of nothing
+// but conversions.  Matrix products must not run under it: they would take an infinite operand for 65504 and NaN for 0.
+__device__ __forceinline__ void halves_saturate(int on) { __builtin_amdgcn_s_setreg(1 | 23 << 6, on); }
+
 // Device-side description of one transformer block.
 struct LayerDev {
     const void* Wa;       // fused first-phase matrix [rowsA, dim]: q|k|v|[g]|[pleGate]|[gdnA|gdnB]

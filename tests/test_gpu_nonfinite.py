@@ -3,7 +3,7 @@ float64 oracle, or float64 NumPy for the bare products), not the NaN of a produc
 import numpy as np
 import pytest
 
-from test_gpu_gemm_tiles import P3, selftest
+from test_gpu_gemm_tiles import F16, P3, selftest
 
 pytestmark = pytest.mark.gpu
 INF = np.inf
@@ -160,3 +160,59 @@ def test_planes(pkg, m, n, k):
     assert np.all(np.isfinite(got))
     ok = b[:, 5] != np.float32(3e-39)  # (a denormal factor: planes below the bf16 denormals are lost)
     assert np.max(np.abs(got - want)[:, ok] / np.abs(want)[:, ok]) <= 2.0 ** -22
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 320, 256), (300, 512, 256), (1100, 17000, 192)])  # the three kernels of halves
+def test_swiglu_to_halves(pkg, m, n, k):
+    """silu(gate) * up on its way into halves: NaN and infinities stay, finite values beyond the halves saturate, and a gate of minus a
+    lot gives 0 whatever the other factor is."""
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((m, k)).astype(np.float16).astype(np.float32)
+    b = (rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float16).astype(np.float32)
+    a[1, 2], a[2, 3], a[3, 4] = np.nan, INF, -INF
+    a[4], a[5], a[6] = 0, 0, 0
+    a[4, 5], a[5, 6], a[6, 7] = 60000, 300, -60000
+    b[0:8, 2:8] = np.array([1, 2, -1, 3, 0.5, -2, -4, -3], np.float32)[:, None]  # gate, up of units 0 .. 3
+    b[8:, 2:8] = np.where(b[8:, 2:8] == 0, 1, b[8:, 2:8])  # (no 0 against an infinity)
+    got = selftest(pkg, F16, a, b, swiglu=True).astype(np.float64)
+    with np.errstate(all="ignore"):
+        p = a.astype(np.float64) @ b.astype(np.float64).T
+        want = p[:, 0::2] / (1 + np.exp(-p[:, 0::2])) * p[:, 1::2]
+    assert np.isnan(want[1]).all() and np.isinf(want[2, 0]) and np.isnan(want[3, 0]) and want[4, 0] > 65504 and want[6, 1] == -1.08e10
+    want = np.where(np.isfinite(want), np.clip(want, -65504, 65504), want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf])
+    ok = np.isfinite(want)
+    # one rounding to halves, and the factors' fp32 sums (values up to 65504 come from factors of up to 3e5)
+    assert np.all(np.abs(got - want)[ok] <= 2.0 ** -11 * np.abs(want)[ok] + 2e-6 * np.sqrt(k))
+
+
+@pytest.mark.parametrize("kind", ["attn", "hybrid"])
+@pytest.mark.parametrize("n", [40, 90])  # tiled products; also segments in chunks
+def test_an_overflow_in_a_long_prompt_of_halves(pkg, kind, n):
+    """Finite weights and one token whose residual row overflows in the layer applied first: the next layer makes NaN of its key, value and
+    state update, and so are the logits of the tokens behind it, as they are token by token."""
+    hp = config(pkg, kind, 1)
+    m = model(pkg, hp, "")
+    top = hp.transformers - 1
+    E, g2 = m.tensor(0, pkg.T_TOKEN_EMBEDDINGS), m.tensor(top, pkg.T_RMS_GAMMA2)
+    E[:, 9], E[69, 9], g2[9] = -0.5, 0.5, 1.0
+    gate, up = m.tensor(top, pkg.T_FFN_1A), m.tensor(top, pkg.T_FFN_1B)
+    gate[0], up[0] = 0, 0
+    gate[0, 9] = up[0, 9] = 1000  # unit 0: silu(1000 x) 1000 x of the ninth normed column, x about 13 for token 69 and -13 for the others
+    m.tensor(top, pkg.T_FFN_2)[11, 0] = 3e38
+    dev = pkg.Device(hp, 0)
+    dev.upload(m)
+    assert dev.operand_bytes() > 0
+    ids = np.random.default_rng(3).integers(0, 60, n).astype(np.int32)
+    for odd in (False, True):
+        ids[3] = 69 if odd else 7
+        seen = {}
+        for mode in (0, 1):
+            dev.set_prefill_mode(mode)
+            dev.reset()
+            dev.prefill(0, ids)
+            seen[mode] = np.isnan(dev.logits(0))
+        assert np.all(seen[1] == odd) and np.all(seen[0] == odd)
+    dev.close()
