@@ -102,8 +102,8 @@ int mlh_upload_rope_table(mlh_ctx* ctx, const float* tab, int n);
 /* Must be called once after the uploads and before any forward call: checks
  * that every tensor the hyper-parameters require has arrived.
  * Infinities and NaN go through the products as fp32 arithmetic has them.  The MFMA kernels multiply sums of planes, where an
- * infinity would become NaN: a model with a matrix element that is infinite, NaN or (fp32) 3.3962e38 or more, or a gain of 2^60
- * or more, runs without them, its prompts token by token.  Limits that remain: an activation of 3.3962e38 or more counts as
+ * infinity would become NaN: a model with an element of a matrix or table that is infinite, NaN or (fp32) 3.3962e38 or more, or a gain or gate
+ * bias of 2^60 or more, runs without them, its prompts token by token.  Limits that remain: an activation of 3.3962e38 or more counts as
  * NaN (the next norm's sum of squares has overflowed by then); a sum with terms of 0.99 of the largest float may
  * be infinite; and prefill calls of more than 32 tokens of bf16 models hold activations as halves, where a finite one
  * beyond 65504 counts as 65504 (queries, keys and values: as infinite). */

@@ -1522,10 +1522,12 @@ static int build_mirror(mlh_ctx* c, const void* src, size_t n, const void** dst,
     return 0;
 }
 
-// Sets *found when the magnitude of an element (as bits: infinities and NaN are the largest) reaches `limit`.
+// Sets *found when the magnitude of one of n elements (as bits: infinities and NaN are the largest) reaches `limit`.
 template <typename WT>
-__global__ void __launch_bounds__(256) k_find_beyond(const uint4* __restrict__ w, size_t n16, uint32_t limit, unsigned* found) {
+__global__ void __launch_bounds__(256) k_find_beyond(const uint4* __restrict__ w, size_t n, uint32_t limit, unsigned* found) {
+    const size_t n16 = n / (16 / sizeof(WT));
     bool any = false;
+    if (sizeof(WT) == 4 && blockIdx.x == 0 && threadIdx.x < n - n16 * 4) any = (reinterpret_cast<const uint32_t*>(w)[n16 * 4 + threadIdx.x] & 0x7fffffffu) >= limit; // (a gate bias per head)
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) {
         const uint4 v = w[i];
         const uint32_t x[4] = {v.x, v.y, v.z, v.w};
@@ -1541,7 +1543,9 @@ __global__ void __launch_bounds__(256) k_find_beyond(const uint4* __restrict__ w
 // Whether the MFMA kernels may multiply this model's matrices.  Their products are sums over planes (of the activations, and of fp32
 // weights) or of scaled halves, which an infinite operand turns into NaN where inf * x is infinite; the GEMV and
 // single-launch kernels multiply in fp32 and keep it.  So no weight may lie beyond the planes, and no gain above 2^60: rows
-// are multiplied by it before they are normalised, and their squares overflow from 2^64 on.  One pass over the weights per finalize.
+// are multiplied by it before they are normalised, and their squares overflow from 2^64 on.  Nor may a per-layer embedding lie beyond the planes
+// (what it scales is multiplied by PLE up), or a gate bias above 2^60: the chunked delta rule adds up logarithms of decays and takes
+// differences of the sums.  One pass over the weights per finalize.
 static int operand_values(mlh_ctx* c, bool* within) {
     const mlh_hparams& hp = c->hp;
     const size_t d = hp.dim, F = hp.ffnDim, pl = hp.pleDim;
@@ -1550,16 +1554,18 @@ static int operand_values(mlh_ctx* c, bool* within) {
     MLH_CHECK(c, hipMalloc((void**)&found, 4));
     hipError_t e = hipMemsetAsync(found, 0, 4, c->stream);
     auto matrix = [&](const void* w, size_t n) { // (rows are multiples of 128 bytes)
-        if (c->wbytes == 4) hipLaunchKernelGGL((k_find_beyond<float>), dim3(2048), dim3(256), 0, c->stream, (const uint4*)w, n / 4, P3_BEYOND, found);
-        else hipLaunchKernelGGL((k_find_beyond<bf16_t>), dim3(2048), dim3(256), 0, c->stream, (const uint4*)w, n / 8, 0x7f80u, found);
+        if (c->wbytes == 4) hipLaunchKernelGGL((k_find_beyond<float>), dim3(2048), dim3(256), 0, c->stream, (const uint4*)w, n, P3_BEYOND, found);
+        else hipLaunchKernelGGL((k_find_beyond<bf16_t>), dim3(2048), dim3(256), 0, c->stream, (const uint4*)w, n, 0x7f80u, found);
     };
-    auto gain = [&](const float* g) { hipLaunchKernelGGL((k_find_beyond<float>), dim3(4), dim3(256), 0, c->stream, (const uint4*)g, d / 4, 0x5d800000u, found); };
+    auto vector = [&](const float* g, size_t n) { hipLaunchKernelGGL((k_find_beyond<float>), dim3(4), dim3(256), 0, c->stream, (const uint4*)g, n, 0x5d800000u, found); };
     matrix(c->E, (size_t)hp.vocabSize * d);
-    gain(c->gF);
+    vector(c->gF, d);
     for (const LayerDev& L : c->layers) {
         matrix(L.Wa, L.rowsA * d); matrix(L.Wo, d * L.ad); matrix(L.W13, 2 * F * d); matrix(L.W2, d * F);
-        if (pl) matrix(L.pleUp, d * pl);
-        gain(L.g1); gain(L.g2);
+        if (pl) { matrix(L.pleUp, d * pl); matrix(L.pleTable, (size_t)hp.vocabSize * pl); }
+        vector(L.g1, d); vector(L.g2, d);
+        if (L.gq) { vector(L.gq, d); vector(L.gk, d); }
+        if (L.gdnBa) { vector(L.gdnBa, hp.gdnHeads); vector(L.gdnBb, hp.gdnHeads); }
     }
     if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(&h, found, 4, hipMemcpyDeviceToHost, c->stream);

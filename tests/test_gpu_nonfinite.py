@@ -15,8 +15,11 @@ ODD = [77, 78, 79]        # vocabulary rows that the cases below change; never f
 def config(pkg, kind, bf16):
     if kind == "attn":  # what the XCD-rank kernel takes
         return pkg.config(2, dim=256, attnHeads=4, headDim=64, ffnDim=704, transformers=2, vocabSize=1000, maxL=160, maxSeqs=5, weightDtype=bf16)
-    hp = pkg.config(3, dim=256, attnHeads=4, headDim=64, ffnDim=704, transformers=4, vocabSize=1000, gdnHeads=4, pleDim=64, maxL=160,
-                    maxSeqs=5, weightDtype=bf16)
+    if kind == "flags":
+        return pkg.config(2, dim=256, attnHeads=4, headDim=64, ffnDim=704, transformers=2, vocabSize=1000, maxL=160, maxSeqs=5, weightDtype=bf16,
+                          qkRmsNorm=1, queryGating=1)
+    hp = pkg.config(3, dim=256, attnHeads=4, headDim=64, ffnDim=704, transformers=4, vocabSize=1000, gdnHeads=6 if kind == "heads6" else 4, pleDim=64,
+                    maxL=160, maxSeqs=5, weightDtype=bf16)
     pkg.set_layer_pattern(hp, 1)
     return hp
 
@@ -41,6 +44,22 @@ def model(pkg, hp, case):
             wa, wb = m.tensor(layer, pkg.T_GDN_ALPHA_W), m.tensor(layer, pkg.T_GDN_BETA_W)
             if wa is not None:
                 wa[0, 3], wa[1, 3], wb[2, 3], wb[3, 3] = INF, -INF, INF, 3e38
+    elif case == "embedding":  # of a token that the prompts hold
+        for layer in range(hp.transformers):
+            m.tensor(layer, pkg.T_PLE_TABLE)[7, 5] = INF
+    elif case == "bias":  # decays of 0 and 1, write strengths of 1 and 0
+        for layer in range(hp.transformers):
+            ba, bb = m.tensor(layer, pkg.T_GDN_ALPHA_B), m.tensor(layer, pkg.T_GDN_BETA_B)
+            if ba is not None:
+                ba[0], ba[1], bb[2], bb[3] = INF, -INF, INF, -INF
+    elif case == "large bias":  # sums of 64 logarithms of such a decay would overflow
+        for layer in range(hp.transformers):
+            ba = m.tensor(layer, pkg.T_GDN_ALPHA_B)
+            if ba is not None:
+                ba[-1] = 3e38
+    elif case == "query gain":
+        for layer in range(hp.transformers):
+            m.tensor(layer, pkg.T_QUERY_RMS_GAMMA)[9] = 2.0 ** 62
     return m
 
 
@@ -100,6 +119,13 @@ def test_paths_against_oracle(pkg, orc, kind, case, bf16):
             if not np.isnan(want[i]).any() and np.sum(want[i] == want[i].max()) == 1:
                 assert pick == want[i].argmax()
     dev.close()
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("kind,case", [("hybrid", "embedding"), ("hybrid", "bias"), ("heads6", "large bias"), ("flags", "query gain")])
+def test_tables_gains_and_biases_against_oracle(pkg, orc, kind, case, bf16):
+    """As above, of the parameters that are no operands of a product themselves (heads6: the last bias lies behind the whole 16-byte pieces)."""
+    test_paths_against_oracle(pkg, orc, kind, case, bf16)
 
 
 def test_finalize_with_and_without_operands(pkg):
