@@ -119,6 +119,8 @@ int mlh_finalize(mlh_ctx* ctx);
  * mlh_operand_bytes is what they take now. */
 int mlh_limit_operands(mlh_ctx* ctx, uint64_t bytes);
 uint64_t mlh_operand_bytes(const mlh_ctx* ctx);
+/* The bytes of work buffers that a prefill call over all maxSeqs * maxL positions takes (kept by the context for later calls). */
+uint64_t mlh_prefill_bytes(const mlh_ctx* ctx);
 
 /* Empties a sequence (length 0, GDN states zero).  seq = -1: all sequences.
  * The reference has one implicit sequence in seqTokenIndices (network_globals.h:147-148). */

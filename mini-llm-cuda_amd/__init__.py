@@ -74,6 +74,7 @@ _sigs_dev = {
     "mlh_finalize": (c_int, [c_void_p]),
     "mlh_limit_operands": (c_int, [c_void_p, c_uint64]),
     "mlh_operand_bytes": (c_uint64, [c_void_p]),
+    "mlh_prefill_bytes": (c_uint64, [c_void_p]),
     "mlh_reset": (c_int, [c_void_p, c_int]),
     "mlh_seq_len": (c_int, [c_void_p, c_int]),
     "mlh_max_len": (c_int, [c_void_p]),
@@ -294,6 +295,9 @@ class Device:
     def limit_operands(self, nbytes):
         """Most device bytes that the next finalize may spend on the copies of the matrices that the MFMA kernels read (0: none)."""
         self._check(dev.mlh_limit_operands(self._h, int(nbytes)))
+
+    def prefill_bytes(self):
+        return dev.mlh_prefill_bytes(self._h)
 
     def operand_bytes(self):
         return dev.mlh_operand_bytes(self._h)

@@ -1586,11 +1586,24 @@ static int build_planes(mlh_ctx* c, const void* src, int rows, int cols, const v
     return 0;
 }
 
-// Work buffers of a prefill call of that many rows (ensure_prefill_buffers), within a few percent.
+// A chunk's operands of all heads (bf16 models with gated-delta-net layers; else 0).
+static size_t gdn_chunk_bytes(const mlh_ctx* c) {
+    const mlh_hparams& hp = c->hp;
+    if (hp.weightDtype != MLH_DTYPE_BF16) return 0;
+    for (const LayerDev& L : c->layers)
+        if (L.kind == MLH_KIND_GDN) return (size_t)hp.gdnHeads * ((hp.gdnDk == 64 ? GdLayout<64>::total : GdLayout<128>::total) + 4);
+    return 0;
+}
+// Work buffers of a prefill call: per row, and of the chunks that segments of 64 rows or more are cut into (ensure_prefill_buffers).
 static size_t prefill_row_bytes(const mlh_ctx* c) {
     const mlh_hparams& hp = c->hp;
     const size_t wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 6, d = hp.dim;
     return d * (8 + wb + (wb == 2 ? 4 : 0)) + (size_t)c->maxRowsA * 4 + ((size_t)c->maxAd + hp.pleDim + hp.ffnDim) * wb + 64;
+}
+// ... of one over every position of the context, with the products' split-K workspace.
+size_t mlh_prefill_work_bytes(const mlh_ctx* c) {
+    const size_t rows = (size_t)c->hp.maxSeqs * c->hp.maxL, chunks = (size_t)c->hp.maxSeqs * cdiv(c->hp.maxL, GD_C);
+    return rows * prefill_row_bytes(c) + chunks * gdn_chunk_bytes(c) + mlh_gemm_workspace_bytes();
 }
 
 // Whether the copies fit: into the caller's limit, and onto the device with room left for a prefill call over every position of the
@@ -1605,7 +1618,8 @@ static int operand_room(mlh_ctx* c, bool* fits) {
         need += (rows16(L.rowsA) * d + rows16(d) * (L.ad + pl) + rows16(2 * F) * d + rows16(d) * F) * per + (pl ? d * (L.ad + pl) * wb : 0);
     size_t free = 0, total = 0;
     MLH_CHECK(c, hipMemGetInfo(&free, &total));
-    const size_t row = prefill_row_bytes(c), work = std::min((size_t)hp.maxSeqs * hp.maxL * row, total / 16), have = c->pfRows * row; // (of earlier calls)
+    const size_t have = c->pfRows * prefill_row_bytes(c) + c->pfGdnChunks * gdn_chunk_bytes(c) + (c->gemmWs ? mlh_gemm_workspace_bytes() : 0); // (of earlier calls)
+    const size_t work = std::min(mlh_prefill_work_bytes(c), total / 16);
     *fits = need <= c->operandLimit && need + (work > have ? work - have : 0) <= free;
     return 0;
 }

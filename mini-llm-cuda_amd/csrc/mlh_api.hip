@@ -434,6 +434,8 @@ extern "C" int mlh_limit_operands(mlh_ctx* c, uint64_t bytes) {
     return 0;
 }
 
+extern "C" uint64_t mlh_prefill_bytes(const mlh_ctx* c) { return c ? mlh_prefill_work_bytes(c) : 0; }
+
 extern "C" uint64_t mlh_operand_bytes(const mlh_ctx* c) { return c ? c->operandBytes : 0; }
 
 static int check_ready(mlh_ctx* c) {

@@ -272,6 +272,7 @@ void mlh_set_thread_error(const std::string& msg);
 
 // kernels_prefill.hip
 #define MLH_PREFILL_GEMM_MIN_ROWS 16 // bf16 models: calls of fewer tokens keep fp32 activations throughout
+size_t mlh_prefill_work_bytes(const mlh_ctx* c);
 bool mlh_prefill_gemm_supported(const mlh_ctx* c);
 int mlh_init_prefill_kernels(mlh_ctx* c);
 #define MLH_NO_ROOM (-4) // inside a finalize only: a copy does not fit on the device

@@ -93,3 +93,20 @@ def test_without_copies_of_the_matrices(pkg, bf16):
     for a, b in zip(answers(dev), fast):
         assert np.array_equal(a, b)
     dev.close()
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+def test_room_for_a_prefill_over_every_position(pkg, bf16):
+    """What finalize keeps free for prefill calls is what the largest one allocates: to 2 % and the granularity of a dozen allocations (2 MB each)."""
+    import torch
+
+    hp = pkg.config(3, dim=512, attnHeads=4, headDim=128, ffnDim=512, transformers=2, vocabSize=256, gdnHeads=16, gdnDk=128, gdnDv=128, pleDim=64,
+                    maxL=2100, maxSeqs=8, weightDtype=bf16)
+    pkg.set_layer_pattern(hp, 1)
+    dev = pkg.Device(hp, 0)
+    dev.upload(pkg.Model.generate(hp, 5))
+    before = torch.cuda.mem_get_info()[0]
+    dev.prefill_batch(list(range(8)), [pkg.random_tokens(5, s, hp.vocabSize, hp.maxL) for s in range(8)])
+    took = before - torch.cuda.mem_get_info()[0]
+    assert abs(took - dev.prefill_bytes()) <= 0.02 * took + (24 << 20), (took, dev.prefill_bytes())
+    dev.close()
