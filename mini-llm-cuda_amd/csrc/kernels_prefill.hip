@@ -398,9 +398,11 @@ __global__ void __launch_bounds__(PWG, H16 ? 2 : 1) k_pf_attn_mfma(PfArgs P, Lay
         const float qs = 1.44269504088896341f / sqrtf((float)HD);
 #pragma unroll
         for (int s = 0; s < KS; s++) {
-            const f32x4 lo = *reinterpret_cast<const f32x4*>(q + 16 * s) * qs, hi = *reinterpret_cast<const f32x4*>(q + 16 * s + 4) * qs;
-            qop[s].x = pack_f16(lo.x, lo.y); qop[s].y = pack_f16(lo.z, lo.w);
-            qop[s].z = pack_f16(hi.x, hi.y); qop[s].w = pack_f16(hi.z, hi.w);
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(q + 16 * s), hi = *reinterpret_cast<const f32x4*>(q + 16 * s + 4);
+            // one at a time: product and conversion are then one instruction (v_fma_mixlo_f16) and the product is rounded once
+            auto pair = [&](float a, float b) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(a * qs)) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(b * qs)) << 16); };
+            qop[s].x = pair(lo.x, lo.y); qop[s].y = pair(lo.z, lo.w);
+            qop[s].z = pair(hi.x, hi.y); qop[s].w = pair(hi.z, hi.w);
         }
     }
     f32x16 oacc[MB];

@@ -72,3 +72,12 @@ def test_tiles_of_four_stages_exist_for_halves_only(listing):
     """No model multiplies bf16 operands (they become scaled halves at finalize), and planes take two or three stages."""
     forms = {s[s.index("I") + 1:s.index("EE")] for s in listing if kernel_name(s) == "k_gemm_tile"}
     assert {f.split("Li")[0] for f in forms if f.split("Li")[4] == "4E"} == {"5f16_t"}, forms
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_scaled_queries_are_rounded_once(listing, hd):
+    """The prefill attention of halves scales its queries in fp32 and rounds to halves: HD / 2 of them a lane, each in one instruction."""
+    code = [code for s, code in listing.items() if kernel_name(s) == "k_pf_attn_mfma" and f"Li{hd}E" in s]
+    assert len(code) == 2
+    for c in code:
+        assert sum(bool(re.match(r"v_(fma|mad)_mix(lo|hi)_f16", ins)) for ins in c) >= hd // 2
