@@ -17,9 +17,10 @@
 //   the answer late.
 // The sides meet at workgroup barriers.
 //
-// What bounds it: the chain of exchanges and, at one instruction every four or five cycles, what a communicator executes between
-// them (d 768: 18 us a layer, 6 of them weights); for the widest models HBM as well (d 2048 bf16: 110 MB a layer, 30 us for one
-// sequence, 41 for eight, whose rows take the communicators longer).  Hence the care below for what is formed when: a value made
+// What bounds it: the chain of exchanges and what a communicator executes between them; for the widest models HBM as well.  Time stamps: d 768,
+// 5 sequences, a gated-delta-net layer 17.7 us, its bytes 6 at the copy kernel's rate: partial sums from all XCDs 2.3, residual rows gathered and
+// split 3.0, the products with their words' way out and in 7.2, delta rule 1.0, mixing output 1.0, barriers and 1 / rms 2.6.  d 2048 bf16: 28 us for
+// one sequence, 42 for eight (bytes 22 and 25), of which the residual rows are 2.7 and 10.6.  Hence the care below for what is formed when: a value made
 // of the thread's place that the compiler keeps, spills or moves behind a barrier costs more than forming it again.
 // Measured, us per step, here and as the row kernels' sequence: hybrid, fp32, d 768, 12 layers: 2 sequences 219 and 367, 5 sequences 232
 // and 373, 16 sequences 315 and 394; hybrid, bf16, d 2048, 24 layers: 1 sequence 705 and 1161, 8 sequences 1050 and 1265.  More than
