@@ -1382,14 +1382,15 @@ int mlh_ranks_failed(mlh_ctx* c, int nseq) {
     return mlh_ranks_reset(c);
 }
 
-// Before any other kernel works on sequences [s0, s1): their states are in the first place.
-int mlh_ranks_settle(mlh_ctx* c, int s0, int s1) {
-    s0 = std::min(s0, RK_MAX_SEQS);
-    s1 = std::min(s1, RK_MAX_SEQS);
-    const unsigned which = c->ranksSides & ((1u << s1) - (1u << s0));
+// Before any other kernel works on n sequences (seqs: which; null: the first n): their states are in the first place.
+int mlh_ranks_settle(mlh_ctx* c, const int* seqs, int n) {
+    if (!c->ranksSides) return 0;
+    unsigned which = 0;
+    for (int i = 0; i < n; i++)
+        if (const int s = seqs ? seqs[i] : i; s < RK_MAX_SEQS) which |= c->ranksSides & 1u << s;
     if (!which) return 0;
     const size_t per4 = state_floats(c) / 4;
-    hipLaunchKernelGGL(k_ranks_settle, dim3((unsigned)std::min<size_t>(16, (per4 + 255) / 256), c->hp.transformers, s1), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL(k_ranks_settle, dim3((unsigned)std::min<size_t>(16, (per4 + 255) / 256), c->hp.transformers, RK_MAX_SEQS), dim3(256), 0, c->stream,
                        (const LayerDev*)c->d_layers, c->hp.maxSeqs * per4, which, per4);
     MLH_CHECK(c, hipGetLastError());
     c->ranksSides &= ~which;

@@ -368,7 +368,7 @@ hipError_t mlh_gemm_tile(hipStream_t stream, int dtype, int epi, const void* A, 
 #undef TILE
 }
 
-// fp32 rows -> plane rows (weights at finalize; the self-test's operands).  ldd >= cols, columns past `cols` become zero.
+// fp32 rows -> plane rows (weights at finalize; the self-test's operands, which alone may lie beyond P3_BEYOND).  ldd >= cols, columns past `cols` become zero.
 __global__ void __launch_bounds__(256) k_split_p3(const float* __restrict__ src, int lds_, void* dst, int ldd, int rows, int cols) {
     const size_t n4 = (size_t)rows * (ldd / 4);
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {

@@ -564,10 +564,8 @@ extern "C" int mlh_prefill_batch(mlh_ctx* c, int nseg, const int32_t* seqs, cons
     }
     for (long i = 0; i < total; i++)
         if (ids[i] < 0 || ids[i] >= hp.vocabSize) { c->err = "token id out of range"; return -1; }
-    for (int s = 0; s < nseg; s++) {
-        touch(c, seqs[s], seqs[s] + 1);
-        if ((rc = mlh_ranks_settle(c, seqs[s], seqs[s] + 1))) return rc;
-    }
+    for (int s = 0; s < nseg; s++) touch(c, seqs[s], seqs[s] + 1);
+    if ((rc = mlh_ranks_settle(c, seqs, nseg))) return rc;
     if (c->prefillMode == 0 && total > 1 && mlh_prefill_gemm_supported(c)) // (a single token: the decode step, which splits the keys)
         return mlh_run_prefill_gemm(c, nseg, seqs, ids, lens, nullptr);
     long off = 0;
@@ -595,7 +593,7 @@ extern "C" int mlh_forward_full(mlh_ctx* c, int seq, const int32_t* ids, int n, 
     for (int i = 0; i < n; i++)
         if (ids[i] < 0 || ids[i] >= hp.vocabSize) { c->err = "token id out of range"; return -1; }
     touch(c, seq, seq + 1);
-    if ((rc = mlh_ranks_settle(c, seq, seq + 1))) return rc;
+    if ((rc = mlh_ranks_settle(c, &seq, 1))) return rc;
     // device results: logits, probabilities, targets, losses
     const size_t mat = (size_t)n * V * 4, need = mat * (probsOut ? 2 : 1) + (size_t)n * 8;
     if (need > c->fullBytes) {
@@ -758,7 +756,7 @@ static int end_steps(mlh_ctx* c, int nout) {
 static int run_steps(mlh_ctx* c, int nseq, int steps) {
     int rc;
     if (use_ranks(c, nseq)) return mlh_launch_ranks(c, nseq, steps);
-    if ((rc = mlh_ranks_settle(c, 0, nseq))) return rc;
+    if ((rc = mlh_ranks_settle(c, nullptr, nseq))) return rc;
     if (use_persistent(c, nseq)) return (c->usePersistent == 3 && mlh_xcd_supported(c)) ? mlh_launch_xcd(c, steps) : mlh_launch_persistent(c, steps);
     if (c->graphSteps >= 1) {
         const int k = c->graphSteps;
@@ -865,7 +863,7 @@ extern "C" int mlh_profile_decode(mlh_ctx* c, const int32_t* first, int nseq, in
     int rc = check_decode(c, first, nseq, steps);
     if (rc) return rc;
     if (!usPerLaunch || !launchesPerStep || steps > 64) { c->err = "bad argument (at most 64 steps)"; return -1; }
-    if ((rc = mlh_ranks_settle(c, 0, nseq))) return rc;
+    if ((rc = mlh_ranks_settle(c, nullptr, nseq))) return rc;
     std::vector<hipEvent_t> events;
     std::vector<int> ids;
     hipEvent_t e0;
@@ -1001,7 +999,7 @@ extern "C" int mlh_time_kernel(mlh_ctx* c, int kernel, int layer, int nseq, int 
     for (int s = 0; s < nseq; s++)
         if (c->h_len[s] >= c->hp.maxL) { c->err = "sequence is full"; return -1; }
     touch(c, 0, nseq);
-    if ((rc = mlh_ranks_settle(c, 0, nseq))) return rc;
+    if ((rc = mlh_ranks_settle(c, nullptr, nseq))) return rc;
     hipEvent_t e0, e1;
     MLH_CHECK(c, hipEventCreate(&e0));
     MLH_CHECK(c, hipEventCreate(&e1));

@@ -299,7 +299,7 @@ int mlh_ranks_prepare(mlh_ctx* c);
 int mlh_ranks_reset(mlh_ctx* c);
 void mlh_ranks_done(mlh_ctx* c, int nseq);
 int mlh_ranks_failed(mlh_ctx* c, int nseq);
-int mlh_ranks_settle(mlh_ctx* c, int s0, int s1);
+int mlh_ranks_settle(mlh_ctx* c, const int* seqs, int n);
 int mlh_launch_ranks(mlh_ctx* c, int nseq, int steps);
 
 // kernels_persistent.hip

@@ -232,6 +232,58 @@ def test_more_than_64_pages(pkg):
             assert_logits_close(out[3][i, s], out[0][i, s], 1e-4, f"step {i} sequence {s}")
 
 
+def test_other_kernels_go_on_where_it_left_the_states(pkg, orc):
+    """After a launch the delta-rule states may be in their second place: prompts that continue a sequence, a teacher-forced forward, a new
+    prompt after a reset, row kernels, the one-sequence launch and kernels without copies of the matrices all find them."""
+    hp = config(pkg, heads=12, hd=64, ffn=512, layers=4, vocab=1000, ple=64, maxSeqs=18, maxL=200)
+    dev, w, prompts = start(pkg, orc, hp, 17, 4, 40, 107)
+    hist = [list(p) for p in prompts]
+    nxt = [dev.greedy_token(s) for s in range(17)]
+
+    def decode(n, steps):
+        out = dev.decode_loop(nxt[:n], steps)
+        for s in range(n):
+            hist[s] += [nxt[s]] + [int(t) for t in out[:-1, s]]
+            nxt[s] = int(out[-1, s])
+
+    def prompt(seqs, n):
+        more = [pkg.random_tokens(n, s, hp.vocabSize, n + s) for s in seqs]
+        dev.prefill_batch(seqs, more)
+        for s, ids in zip(seqs, more):
+            hist[s] += list(ids)
+            nxt[s] = dev.greedy_token(s)
+
+    assert dev.single_launch_sequences() == 16
+    decode(5, 2)               # 0 .. 4 in the second place
+    prompt([0, 2], 7)          # row kernels
+    prompt([16, 1], 40)        # tiled products
+    lg, _, _ = dev.forward_full(3, np.arange(9, dtype=np.int32), want_probs=False)
+    hist[3] += list(range(9))
+    nxt[3] = dev.greedy_token(3)
+    assert nxt[3] == int(np.argmax(lg[-1]))
+    dev.reset(4)
+    hist[4] = []
+    prompt([4], 11)
+    decode(4, 3)
+    decode(17, 2)              # row kernels
+    decode(3, 1)
+    decode(1, 2)               # one sequence
+    decode(2, 1)
+    dev.limit_operands(0)
+    dev.finalize()
+    assert dev.single_launch_sequences() <= 1
+    decode(3, 2)
+    for s in range(17):
+        dec = orc.Decoder(w, "f64")
+        for t in hist[s]:
+            _, want = dec.step(int(t))
+        assert dev.seq_len(s) == len(hist[s])
+        assert_logits_close(dev.logits(s), want, RTOL, f"sequence {s}")
+        dec.close()
+    assert dev.persistent_fallbacks() == 0
+    dev.close()
+
+
 def test_batches_of_changing_size_share_the_exchange_words(pkg, orc):
     """Calls of 5, 2, 7 and 1 sequences in turn on one context: every size lays the exchange words out differently over what the others left."""
     hp = config(pkg, heads=12, hd=64, ffn=512, layers=4, vocab=1000, ple=64)
