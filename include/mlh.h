@@ -214,7 +214,9 @@ int mlh_set_graph(mlh_ctx* ctx, int stepsPerGraph);
  * gated-delta-net heads of the same size and number, per-layer embeddings of width 32 (fp32), 64 or 128, dim a multiple of 128
  * up to 768 (fp32) / 2048 (bf16), ffnDim up to 2048 / 6144 in multiples of 256 / 512.  It gives up
  * and falls back in the same way: its workgroups meet before anything is written, and it writes gated-delta-net states to a second
- * place (mlh_create allocates it for the first 16 sequences), so that those from before the launch are there after a wait that expires later.
+ * place (mlh_create allocates it for the first 16 sequences, 64 where the next sentence applies), so that those from before the launch are there
+ * after a wait that expires later.  Calls of up to 64 sequences run as one launch too for fp32 models of those whose dim is 512 or more and whose heads have
+ * at most 32 tiles of 16 first-phase rows to a pair (no query gating beside per-layer embeddings or more than 8 heads).
  * Mode 0, unsupported shapes and more sequences: a sequence of kernels issued as mlh_set_graph says. */
 int mlh_set_persistent(mlh_ctx* ctx, int mode);
 
@@ -251,7 +253,8 @@ int mlh_set_sampling(mlh_ctx* ctx, float temperature, unsigned long long seed);
 /* 1 when mode 3 of mlh_set_persistent applies to this context's model and device, else 0
  * (no counterpart in the reference: its decode loop is one kernel sequence, inference_orchestrator.cu:120-165). */
 int mlh_xcd_decode_supported(mlh_ctx* ctx);
-/* The largest nseq whose decode calls run as a single launch in mode 3 (0: none; no counterpart in the reference). */
+/* The largest nseq whose decode calls run as a single launch in mode 3 for every covered model (0: none; 16 at most: fp32 models may go on to 64,
+ * see mlh_set_persistent; no counterpart in the reference). */
 int mlh_single_launch_sequences(mlh_ctx* ctx);
 
 int mlh_synchronize(mlh_ctx* ctx);

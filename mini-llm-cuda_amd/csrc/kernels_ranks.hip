@@ -24,7 +24,7 @@
 // of the thread's place that the compiler keeps, spills or moves behind a barrier costs more than forming it again.
 // Measured, us per step, here and as the row kernels' sequence: hybrid, fp32, d 768, 12 layers: 2 sequences 219 and 367, 5 sequences 232
 // and 373, 16 sequences 315 and 394; hybrid, bf16, d 2048, 24 layers: 1 sequence 705 and 1161, 8 sequences 1050 and 1265.  More than
-// 16 would be several blocks of rows one after the other in the same waves: at 19, two blocks took 464, the row kernels 414.
+// 16, and from 6 on where it covers the model: kernels_wide.hip.
 //
 // The launch starts with a meeting of all 256 workgroups: if one is missing after a bounded wait nothing has been written and the
 // call runs as the sequence of row kernels instead.  Behind it every workgroup is resident, and every wait is bounded as well: when
@@ -37,25 +37,15 @@
 #include <algorithm>
 
 #include "mlh_internal.h"
-#include "persist_common.h"
+#include "xcd_exchange.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
 #define RK_WORK 8                             // worker waves
 #define RK_COMM 4                             // communicator waves
 #define RK_CT (RK_COMM * 64)                  // their threads
 #define RK_THREADS ((RK_WORK + RK_COMM) * 64)
-#define RK_XCDS 8
-#define RK_PER 32                             // workgroups per XCD
-#define RK_SPIN (1u << 20)
-#define RK_MEET_SPIN (1u << 14)               // of the meeting at the start (about 20 ms)
-#define RK_LEFT 0x10000u                      // in the word that counts them: somebody has gone
-#define RK_LDS (160 * 1024)
 #define RK_SPLITS 16                          // key splits of a (head, sequence) at most
-#define RK_MAX_SEQS 16                        // one block of MFMA columns
-
-enum { LD_XCD = 2, LD_CROSS = 16, ST_XCD = 0, ST_CROSS = 16 }; // cache policy of exchange loads and stores: nt stays out of the L1, sc1 goes past the L2
 
 struct RanksArgs {
     StepArgs a;
@@ -73,17 +63,6 @@ struct RanksArgs {
     unsigned area, oPart, oMl, oMix, oX, oH, oU, oXP, oHP, oAmax, oTok; // bytes of exchange words per XCD and what lies where in them; oAmax, oTok: behind all of them
 };
 
-__device__ __forceinline__ int runi(int v) { return __builtin_amdgcn_readfirstlane(v); }
-// The layer table is read by scalar loads where it is used.
-typedef const __attribute__((address_space(4))) LayerDev* LayerPtr;
-
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-template <int POL> __device__ __forceinline__ u32x4 xget(rsrc_t r, unsigned lane, unsigned base) { return __builtin_amdgcn_raw_buffer_load_b128(r, lane, base, POL); }
-template <int POL> __device__ __forceinline__ void xput(rsrc_t r, unsigned lane, unsigned base, float a, float b, unsigned tag) { // two words
-    const u32x4 v = {__float_as_uint(a), tag, __float_as_uint(b), tag};
-    __builtin_amdgcn_raw_buffer_store_b128(v, r, lane, base, POL);
-}
-__device__ __forceinline__ bool xfresh(const u32x4& v, unsigned tag) { return v.y == tag && v.w == tag; }
 // ---- weights ----
 template <typename WT> struct RkW { u32x4 raw[2]; }; // this lane's share of a chunk: 16 rows x 128 bytes
 template <typename WT> struct RkOp;                  // ... ready to multiply
@@ -162,15 +141,6 @@ __device__ __forceinline__ void rk_put4(unsigned char* planes, int k, int t, int
     unsigned char* p = planes + (k >> 5) * 3 * stride + (q * mb + t) * 16 + e * 2;
 #pragma unroll
     for (int pl = 0; pl < 3; pl++) *reinterpret_cast<uint2*>(p + pl * stride) = make_uint2(x[pl], y[pl]);
-}
-
-template <int W> __device__ __forceinline__ float rk_row_sum(float v) { // over aligned groups of 16 or 32 lanes
-    v = pgroup_sum<16>(v);
-    if (W == 32) { // the rows of 16 in pairs
-        const u32x2 t = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = __uint_as_float(t.x) + __uint_as_float(t.y);
-    }
-    return v;
 }
 
 // Four neighbouring values of a matrix row, fetched now and converted when they are used.
@@ -1139,30 +1109,8 @@ __global__ void __launch_bounds__(RK_THREADS) k_decode_ranks(RanksArgs P) {
         S.pos[threadIdx.x] = P.a.pos[s];
     }
     if (threadIdx.x < 64) {
-        // the XCD from the hardware register, the rank inside it from the order of arrival; then a meeting of all
-        unsigned xcc, rank = RK_PER;
-        asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
-        xcc &= 15u;
-        if (xcc < RK_XCDS && threadIdx.x == 0) rank = __hip_atomic_fetch_add(P.xcdCount + xcc, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        rank = (unsigned)runi((int)rank);
-        // One word decides: the 256th arrival makes it 256 for good, a workgroup that waits no longer (or has no place) adds
-        // RK_LEFT before that, and then nobody goes on.
-        unsigned* meet = P.xcdCount + RK_XCDS;
-        unsigned code = rank >= RK_PER ? 2u : 0u;
-        if (threadIdx.x == 0) {
-            if (code) __hip_atomic_fetch_or(meet, RK_LEFT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            else __hip_atomic_fetch_add(meet, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            for (unsigned spins = 0; !code; spins++) {
-                unsigned n = aldu(meet);
-                if (n == RK_XCDS * RK_PER) break;
-                if (n & RK_LEFT) code = 1u;
-                else if (spins > RK_MEET_SPIN) {
-                    if (__hip_atomic_compare_exchange_strong(meet, &n, n | RK_LEFT, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) code = 1u;
-                    else spins = RK_MEET_SPIN; // somebody arrived just now: look again
-                }
-                __builtin_amdgcn_s_sleep(2);
-            }
-        }
+        unsigned xcc, rank;
+        const unsigned code = rk_meeting(P.xcdCount, xcc, rank);
         if (threadIdx.x == 0) {
             if (code) astu(P.abortFlag, code);
             S.ctl[0] = code ? 1 : 0;
@@ -1187,7 +1135,7 @@ __global__ void k_ranks_prep(unsigned* abortFlag, unsigned* xcdCount, unsigned s
     if (threadIdx.x <= RK_XCDS) xcdCount[threadIdx.x] = threadIdx.x < RK_XCDS ? startCount : 0u;
 }
 // states of sequences that are in their second place, to the first (x: pieces, y: layer, z: sequence)
-__global__ void __launch_bounds__(256) k_ranks_settle(const LayerDev* layers, size_t otherAt4, unsigned which, size_t per4) {
+__global__ void __launch_bounds__(256) k_ranks_settle(const LayerDev* layers, size_t otherAt4, unsigned long long which, size_t per4) {
     f32x4* S = reinterpret_cast<f32x4*>(layers[blockIdx.y].S);
     if (!S || !(which >> blockIdx.z & 1)) return;
     S += blockIdx.z * per4;
@@ -1218,7 +1166,7 @@ static bool ranks_plan(const mlh_ctx* c, int n, RanksPlan& p) {
     p.lds = (size_t)p.planeBytes + 2 * slots * RK_WORK * 1024 + RK_CT * 8 + (RK_CT + 16 + 64 * 4 + d + 3 * 16 + 16) * 4;
     // n tokens are the columns of one MFMA; a residual element per communicator thread, state rows of a pair of a head and a sequence per workgroup,
     // a group of the PLE chunk's columns per thread
-    if (n > RK_MAX_SEQS || n > RK_CT / (d / 64) || n * nh * hp.headDim > RK_PER * 64 || n > RK_CT / (ke / 4) || p.lds > RK_LDS) return false;
+    if (n > MLH_RANKS_MAX_SEQS || n > RK_CT / (d / 64) || n * nh * hp.headDim > RK_PER * 64 || n > RK_CT / (ke / 4) || p.lds > RK_LDS) return false;
     p.lds = std::max(p.lds, (size_t)RK_LDS / 2 + 1024); // one workgroup per compute unit
     int tiles = 0;
     for (const LayerDev& L : c->layers) {
@@ -1255,6 +1203,9 @@ static size_t state_floats(const mlh_ctx* c) {
     return 0;
 }
 
+// Sequences whose states have a second place, in a model that the kernel covers: those of a launch of this kernel or of kernels_wide.hip.
+static int other_seqs(const mlh_ctx* c) { return std::min(c->hp.maxSeqs, mlh_wide_model(c) ? MLH_WIDE_MAX_SEQS : MLH_RANKS_MAX_SEQS); }
+
 // Whether the kernel covers a model of these hyper-parameters on this device.
 static bool ranks_model(const mlh_ctx* c) {
     const mlh_hparams& hp = c->hp;
@@ -1273,16 +1224,21 @@ static bool ranks_model(const mlh_ctx* c) {
         for (const LayerDev& L : c->layers)
             if (L.offPle % 16) return false;
     }
-    return (hp.maxSeqs + RK_MAX_SEQS) * state_floats(c) < (size_t)1 << 31; // (state rows: 32-bit offsets)
+    return (hp.maxSeqs + other_seqs(c)) * state_floats(c) < (size_t)1 << 31; // (state rows: 32-bit offsets)
 }
 
 // Sequences whose states have a second place behind those of all maxSeqs (mlh_create allocates both).
-int mlh_ranks_other_seqs(const mlh_ctx* c) { return ranks_model(c) ? std::min(c->hp.maxSeqs, RK_MAX_SEQS) : 0; }
+int mlh_ranks_other_seqs(const mlh_ctx* c) { return ranks_model(c) ? other_seqs(c) : 0; }
 
 // Whether the kernel covers this context's model as it has been finalized (memory for its exchange words apart).
 static bool ranks_shape(const mlh_ctx* c) { return ranks_model(c) && mlh_rows_applicable(c, 1); }
 
-bool mlh_ranks_applicable(const mlh_ctx* c, int nseq) { return c->ranksMax >= nseq && mlh_rows_applicable(c, nseq); }
+// From how many sequences on kernels_wide.hip takes them.  Measured, us per step, here and there (hybrid, fp32, d 768, 12 layers): 2 sequences
+// 224 and 250, 5 241 and 253, 6 269 and 256, 7 275 and 257, 8 273 and 258, 12 327 and 263, 16 339 and 267.
+#define WIDE_FROM 6
+static bool use_wide(const mlh_ctx* c, int nseq) { return nseq >= WIDE_FROM && c->wideMax >= nseq; }
+
+bool mlh_ranks_applicable(const mlh_ctx* c, int nseq) { return (use_wide(c, nseq) || c->ranksMax >= nseq) && mlh_rows_applicable(c, nseq); }
 
 template <typename WT, int HD>
 static int ranks_launch(mlh_ctx* c, const RanksArgs* P, size_t lds) {
@@ -1305,22 +1261,26 @@ static int ranks_launch(mlh_ctx* c, const RanksArgs* P, size_t lds) {
 
 int mlh_ranks_reset(mlh_ctx* c) {
     c->ranksTag = 0;
-    if (!c->ranksBuf) return 0;
-    hipLaunchKernelGGL(k_ranks_zero, dim3(1024), dim3(256), 0, c->stream, (u32x4*)c->ranksBuf, c->ranksBytes / 16);
-    MLH_CHECK(c, hipGetLastError());
+    void* const bufs[] = {c->ranksBuf, c->wideBuf};
+    const size_t bytes[] = {c->ranksBytes, c->wideBytes};
+    for (int i = 0; i < 2; i++) {
+        if (!bufs[i]) continue;
+        hipLaunchKernelGGL(k_ranks_zero, dim3(1024), dim3(256), 0, c->stream, (u32x4*)bufs[i], bytes[i] / 16);
+        MLH_CHECK(c, hipGetLastError());
+    }
     return 0;
 }
 
 // At finalize: how many sequences the kernel takes (none where the model or the device does not suit it), and its exchange words.
 int mlh_ranks_prepare(mlh_ctx* c) {
-    c->ranksMax = 0;
+    c->ranksMax = c->wideMax = 0;
     if (!ranks_shape(c)) return 0;
-    const int rc = ranks_launch(c, nullptr, 0);
+    int rc = ranks_launch(c, nullptr, 0);
     if (rc) return rc < 0 ? rc : 0;
     int most = 0;
     size_t bytes = 0;
     RanksPlan p;
-    for (int n = 1; n <= std::min(c->hp.maxSeqs, RK_MAX_SEQS) && ranks_plan(c, n, p); n++) { most = n; bytes = std::max(bytes, p.words); }
+    for (int n = 1; n <= std::min(c->hp.maxSeqs, MLH_RANKS_MAX_SEQS) && ranks_plan(c, n, p); n++) { most = n; bytes = std::max(bytes, p.words); }
     if (bytes > c->ranksBytes) {
         void* q = nullptr;
         if (hipMalloc(&q, bytes) != hipSuccess) { // no room: the row kernels
@@ -1332,14 +1292,28 @@ int mlh_ranks_prepare(mlh_ctx* c) {
         c->ranksBytes = bytes;
     }
     c->ranksMax = most;
+    if ((rc = mlh_wide_prepare(c))) return rc;
     return mlh_ranks_reset(c);
 }
 
 // `steps` decode steps of sequences 0 .. nseq - 1 in one launch.
 int mlh_launch_ranks(mlh_ctx* c, int nseq, int steps) {
     const mlh_hparams& hp = c->hp;
+    const bool wide = use_wide(c, nseq);
     RanksPlan p;
-    if (!ranks_plan(c, nseq, p) || p.words > c->ranksBytes) { c->err = "decode of several sequences: no plan"; return -1; }
+    if (!wide && (!ranks_plan(c, nseq, p) || p.words > c->ranksBytes)) { c->err = "decode of several sequences: no plan"; return -1; }
+    // tags are a running count of layer passes; before it could wrap and meet a stale word, everything goes back to zero
+    const unsigned long long need = (unsigned long long)steps * (hp.transformers + 1) + 1;
+    if (c->ranksTag + need >= 0xFFFFFFFFull)
+        if (const int rc = mlh_ranks_reset(c)) return rc;
+    const unsigned tagBase = (unsigned)c->ranksTag;
+    c->ranksTag += need;
+    const int otherAt = (int)(hp.maxSeqs * state_floats(c));
+    const unsigned startCount = c->injectAbort > 0 ? (unsigned)RK_PER : 0u; // test hook: no workgroup finds a place
+    if (c->injectAbort > 0) c->injectAbort--;
+    hipLaunchKernelGGL(k_ranks_prep, dim3(1), dim3(64), 0, c->stream, c->d_sync + 64 * 20, c->d_sync + 64 * 23, startCount);
+    MLH_CHECK(c, hipGetLastError());
+    if (wide) return mlh_launch_wide(c, nseq, steps, tagBase, otherAt);
     RanksArgs P;
     mlh_fill_args(c, P.a, nseq, c->d_tok);
     P.layers = c->d_layers;
@@ -1353,25 +1327,17 @@ int mlh_launch_ranks(mlh_ctx* c, int nseq, int steps) {
     P.xcdCount = c->d_sync + 64 * 23;
     P.area = p.area; P.oPart = p.oPart; P.oMl = p.oMl; P.oMix = p.oMix; P.oX = p.oX; P.oH = p.oH; P.oU = p.oU; P.oXP = p.oXP; P.oHP = p.oHP;
     P.oAmax = p.oAmax; P.oTok = p.oTok;
-    // tags are a running count of layer passes; before it could wrap and meet a stale word, everything goes back to zero
-    const unsigned long long need = (unsigned long long)steps * (hp.transformers + 1) + 1;
-    if (c->ranksTag + need >= 0xFFFFFFFFull)
-        if (const int rc = mlh_ranks_reset(c)) return rc;
-    P.tagBase = (unsigned)c->ranksTag;
-    c->ranksTag += need;
-    P.otherAt = (int)(hp.maxSeqs * state_floats(c));
-    P.sides = c->ranksSides;
+    P.tagBase = tagBase;
+    P.otherAt = otherAt;
+    P.sides = (unsigned)c->ranksSides;
     P.abortAtStep = c->injectAbortStep;
     c->injectAbortStep = 0;
-    const unsigned startCount = c->injectAbort > 0 ? (unsigned)RK_PER : 0u; // test hook: no workgroup finds a place
-    if (c->injectAbort > 0) c->injectAbort--;
-    hipLaunchKernelGGL(k_ranks_prep, dim3(1), dim3(64), 0, c->stream, P.abortFlag, P.xcdCount, startCount);
     return ranks_launch(c, &P, p.lds);
 }
 
 // A launch of nseq sequences has ended well: their states are in the place they were not in.
 void mlh_ranks_done(mlh_ctx* c, int nseq) {
-    if (state_floats(c)) c->ranksSides ^= (1u << nseq) - 1u; // (16 at most)
+    if (state_floats(c)) c->ranksSides ^= ~0ull >> (64 - nseq); // (64 at most)
 }
 
 // It has given up (and its stream has drained): positions are what they were, and no word of it is met again.
@@ -1385,12 +1351,12 @@ int mlh_ranks_failed(mlh_ctx* c, int nseq) {
 // Before any other kernel works on n sequences (seqs: which; null: the first n): their states are in the first place.
 int mlh_ranks_settle(mlh_ctx* c, const int* seqs, int n) {
     if (!c->ranksSides) return 0;
-    unsigned which = 0;
+    unsigned long long which = 0;
     for (int i = 0; i < n; i++)
-        if (const int s = seqs ? seqs[i] : i; s < RK_MAX_SEQS) which |= c->ranksSides & 1u << s;
+        if (const int s = seqs ? seqs[i] : i; s < MLH_WIDE_MAX_SEQS) which |= c->ranksSides & 1ull << s;
     if (!which) return 0;
     const size_t per4 = state_floats(c) / 4;
-    hipLaunchKernelGGL(k_ranks_settle, dim3((unsigned)std::min<size_t>(16, (per4 + 255) / 256), c->hp.transformers, RK_MAX_SEQS), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL(k_ranks_settle, dim3((unsigned)std::min<size_t>(16, (per4 + 255) / 256), c->hp.transformers, MLH_WIDE_MAX_SEQS), dim3(256), 0, c->stream,
                        (const LayerDev*)c->d_layers, c->hp.maxSeqs * per4, which, per4);
     MLH_CHECK(c, hipGetLastError());
     c->ranksSides &= ~which;

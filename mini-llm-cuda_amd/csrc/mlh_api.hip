@@ -479,7 +479,7 @@ extern "C" int mlh_reset(mlh_ctx* c, int seq) {
         MLH_CHECK(c, hipGetLastError());
         for (; s < e; s++) {
             c->h_len[s] = 0; c->h_dirty[s] = 0;
-            if (s < 32) c->ranksSides &= ~(1u << s);
+            if (s < MLH_WIDE_MAX_SEQS) c->ranksSides &= ~(1ull << s);
         }
     }
     return 0;
@@ -675,7 +675,7 @@ static int ensure_graph(mlh_ctx* c, int slot, int nseq, int k) {
     return 0;
 }
 
-// Up to 16 sequences, and one of a model that the XCD-rank kernel does not cover, in one launch of kernels_ranks.hip.  (A caller who
+// Several sequences, and one of a model that the XCD-rank kernel does not cover, in one launch of kernels_ranks.hip or kernels_wide.hip.  (A caller who
 // asked for graph replays gets those.)
 static bool for_ranks(const mlh_ctx* c, int nseq) {
     if (c->usePersistent != 3 || c->temperature > 0.f || c->graphSteps > 0 || !mlh_ranks_applicable(c, nseq)) return false;

@@ -185,7 +185,10 @@ struct mlh_ctx {
     unsigned long long ranksTag = 0; // tags its launches have used
     bool ranksOff = false;         // it has given up, and is not tried again before mlh_set_persistent
     int lastDecodeSeqs = 0;        // sequences of the last decode call
-    unsigned ranksSides = 0;       // bit s: the gated-delta-net states of sequence s are at their second place (slot maxSeqs + s)
+    int wideMax = 0;               // ... and the one of more sequences (kernels_wide.hip)
+    void* wideBuf = nullptr;       // its exchange memory
+    size_t wideBytes = 0;
+    unsigned long long ranksSides = 0; // bit s: the gated-delta-net states of sequence s are at their second place (slot maxSeqs + s)
     LayerDev* d_layers = nullptr;  // device copy of `layers`
     unsigned* d_sync = nullptr;    // barrier words + abort flag
     float* pamaxVal = nullptr;     // [numCUs]
@@ -293,6 +296,8 @@ void mlh_rows_rest_of_layer(mlh_ctx* c, int t, const RowsArgs& base, float* x, f
 void mlh_rows_lm_head(mlh_ctx* c, int n, const float* X, const int* segStart, const int* segLen, const int* segSeq, float* amaxVal, int* amaxIdx);
 
 // kernels_ranks.hip: decode steps of several sequences in one launch
+#define MLH_RANKS_MAX_SEQS 16 // one block of MFMA columns
+#define MLH_WIDE_MAX_SEQS 64  // four (kernels_wide.hip)
 bool mlh_ranks_applicable(const mlh_ctx* c, int nseq);
 int mlh_ranks_other_seqs(const mlh_ctx* c);
 int mlh_ranks_prepare(mlh_ctx* c);
@@ -301,6 +306,10 @@ void mlh_ranks_done(mlh_ctx* c, int nseq);
 int mlh_ranks_failed(mlh_ctx* c, int nseq);
 int mlh_ranks_settle(mlh_ctx* c, const int* seqs, int n);
 int mlh_launch_ranks(mlh_ctx* c, int nseq, int steps);
+// kernels_wide.hip: ... of 6 to 64 sequences (mlh_launch_ranks decides)
+bool mlh_wide_model(const mlh_ctx* c);
+int mlh_wide_prepare(mlh_ctx* c);
+int mlh_launch_wide(mlh_ctx* c, int nseq, int steps, unsigned tagBase, int otherAt);
 
 // kernels_persistent.hip
 bool mlh_persistent_supported(const mlh_ctx* c);

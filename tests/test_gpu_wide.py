@@ -1,0 +1,132 @@
+"""Decode of 6 to 64 sequences in one launch (kernels_wide.hip) against the CPU oracle: the smallest and largest batches of every number of
+token blocks, heads of which a second one has 1, 2, 4 or no sharers, flags, layer mixes, per-layer embeddings, ragged lengths on shuffled pages,
+vocabularies that end inside a tile, and the way out.
+
+Bounds: as in the other decode tests (1e-3 relative, ids by a gap of 2e-5)."""
+import numpy as np
+import pytest
+
+from conftest import assert_logits_close, check_greedy_against_oracle
+from test_gpu_ranks import config, start
+
+pytestmark = pytest.mark.gpu
+
+RTOL = 1e-3
+GAP_TOL = 2e-5
+
+CASES = {
+    # name: (hyper-parameters, sequences, prompt lengths from .. to, steps)
+    "hybrid6": (dict(heads=12, hd=64, ffn=1024, layers=4, vocab=300, ple=64), 6, 2, 50, 4),
+    "attn_flags7": (dict(heads=8, hd=64, ffn=768, layers=2, vocab=520, ple=0, gdn=False, flags=True), 7, 5, 120, 3),
+    "hybrid16": (dict(heads=10, hd=64, ffn=256, layers=2, vocab=4999, ple=32), 16, 2, 40, 3),
+    "hybrid17": (dict(heads=12, hd=64, ffn=2048, layers=4, vocab=1003, ple=64), 17, 1, 90, 4),
+    "hybrid32": (dict(heads=8, hd=64, ffn=256, layers=4, vocab=4111, ple=128), 32, 2, 60, 3),
+    "hybrid33": (dict(heads=10, hd=64, ffn=512, layers=2, vocab=700, ple=32), 33, 2, 40, 3),
+    "hybrid48": (dict(heads=12, hd=64, ffn=768, layers=2, vocab=520, ple=0), 48, 2, 30, 2),
+    "hybrid64": (dict(heads=12, hd=64, ffn=512, layers=2, vocab=1000, ple=64), 64, 1, 70, 3),
+    "attn_flags49": (dict(heads=8, hd=64, ffn=768, layers=2, vocab=520, ple=32, gdn=False, flags=True), 49, 3, 200, 2),
+}
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_batches_against_the_oracle(pkg, orc, case):
+    shape, n, lo, hi, steps = CASES[case]
+    hp = config(pkg, maxSeqs=n, maxL=256, **shape)
+    dev, w, prompts = start(pkg, orc, hp, n, lo, hi, 60 + n)
+    first = [dev.greedy_token(s) for s in range(n)]
+    a = dev.decode_loop(first, steps)                # a run of steps in one launch
+    b = dev.decode_loop([int(t) for t in a[-1]], 1)  # and a step of its own: cache, states, positions carried over
+    assert dev.persistent_fallbacks() == 0
+    got = np.concatenate([np.array([first]), a, b])
+    for s in sorted(s for s in {0, 1, 15, 16, n // 4, n // 2 - 1, n // 2, n - 2, n - 1} if s < n):
+        dec = orc.Decoder(w, "f64")
+        check_greedy_against_oracle(dec, prompts[s], got[:, s].tolist(), GAP_TOL, what=f"{case} sequence {s}")
+        dec.reset()
+        for t in list(prompts[s]) + got[:-1, s].tolist():
+            _, lg = dec.step(int(t))
+        assert_logits_close(dev.logits(s), lg, RTOL, f"{case} sequence {s}")
+        assert dev.seq_len(s) == len(prompts[s]) + steps + 1
+        dec.close()
+    dev.close()
+
+
+@pytest.mark.parametrize("n", [6, 17, 40, 64])
+def test_every_sequence_against_the_row_kernels(pkg, orc, n):
+    """All logits over the same tokens in both, two orders of fp32 sums apart, and no further from the float64 oracle than theirs (a factor
+    of two of rounding noise)."""
+    hp = config(pkg, heads=12, hd=64, ffn=1024, layers=8, vocab=1024, ple=64, maxSeqs=64, maxL=256)
+    out, feed = {}, np.random.default_rng(4).integers(0, hp.vocabSize, size=(5, n))
+    for mode in (3, 0):
+        dev, w, prompts = start(pkg, orc, hp, n, 3, 60, 71)
+        dev.set_persistent(mode)
+        for row in feed:
+            dev.decode_step([int(t) for t in row])
+        assert dev.persistent_fallbacks() == 0
+        out[mode] = np.stack([dev.logits(s) for s in range(n)])
+        dev.close()
+    for s in range(n):
+        assert_logits_close(out[3][s], out[0][s], 1e-4, f"sequence {s}")
+    err = {3: [], 0: []}
+    for s in range(0, n, 5):
+        dec = orc.Decoder(w, "f64")
+        for t in list(prompts[s]) + feed[:, s].tolist():
+            _, lg = dec.step(int(t))
+        dec.close()
+        for mode in err:
+            err[mode].append(np.linalg.norm(out[mode][s] - lg) / np.linalg.norm(lg))
+    rms = {mode: float(np.sqrt(np.mean(np.square(e)))) for mode, e in err.items()}
+    print(f"distance from float64: one launch {rms[3]:.2e}, row kernels {rms[0]:.2e}")
+    assert rms[3] <= 2 * rms[0]
+
+
+@pytest.mark.parametrize("where", ["meeting", "mid-run"])
+def test_gives_up_and_falls_back(pkg, orc, where):
+    """A launch that gives up (places taken from the host; a workgroup that leaves at step 2) is redone as row kernels from the states
+    before it, also where an earlier launch has left those in their second place; the kernel comes back once it is asked for."""
+    hp = config(pkg, heads=12, hd=64, ffn=512, layers=4, vocab=1000, ple=64, maxSeqs=20, maxL=128)
+    ids, logits = {}, {}
+    for inject in (False, True):
+        dev, w, prompts = start(pkg, orc, hp, 20, 3, 30, 83)
+        nxt = [dev.greedy_token(s) for s in range(20)]
+        out = []
+        for k in range(3):
+            if inject and k == 1:
+                dev.debug_inject_abort(1) if where == "meeting" else dev.debug_inject_abort_at_step(2)
+            if inject and k == 2:
+                assert dev.get_persistent() == 0 and dev.persistent_fallbacks() == 1
+                dev.set_persistent(3)
+            out.append(dev.decode_loop(nxt, 4))
+            nxt = [int(t) for t in out[-1][-1]]
+        assert dev.persistent_fallbacks() == int(inject)
+        ids[inject] = np.concatenate(out)
+        logits[inject] = np.stack([dev.logits(s) for s in range(20)])
+        dev.close()
+    assert (ids[True] == ids[False]).mean() > 0.99  # (two orders of fp32 sums: a tie may part)
+    for s in range(20):
+        if (ids[True][:, s] == ids[False][:, s]).all():
+            assert_logits_close(logits[True][s], logits[False][s], 1e-4, f"sequence {s}")
+
+
+def test_batches_of_changing_size_share_the_exchange_memory(pkg, orc):
+    """Calls of 40, 17, 64, 5, 9, 33 and 64 sequences in turn on one context, with a tag count that wraps on the way: every size lays the data
+    out over what the others left, and the kernel of few sequences works on the same states."""
+    hp = config(pkg, heads=12, hd=64, ffn=512, layers=4, vocab=1000, ple=64, maxSeqs=64, maxL=128)
+    dev, w, prompts = start(pkg, orc, hp, 64, 2, 40, 91)
+    hist = [list(p) for p in prompts]
+    nxt = [dev.greedy_token(s) for s in range(64)]
+    for n in (40, 17, 64, 5, 9, 33, 64):
+        if n == 5:
+            dev.debug_set_xcd_tag(0xFFFFFFF0)
+        out = dev.decode_loop(nxt[:n], 2)
+        for s in range(n):
+            hist[s] += [nxt[s], int(out[0, s])]
+            nxt[s] = int(out[1, s])
+    assert dev.persistent_fallbacks() == 0
+    for s in (0, 4, 5, 8, 9, 16, 17, 32, 39, 40, 63):
+        dec = orc.Decoder(w, "f64")
+        for t in hist[s]:
+            _, lg = dec.step(int(t))
+        assert_logits_close(dev.logits(s), lg, RTOL, f"sequence {s}")
+        assert dev.seq_len(s) == len(hist[s])
+        dec.close()
+    dev.close()
