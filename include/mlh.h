@@ -313,8 +313,8 @@ int mlh_time_decode(mlh_ctx* ctx, const int32_t* first_ids, int nseq, int steps,
 
 /* Stand-alone run of the prefill's MFMA GEMM (no context needed):
  * C[M,N] = A[M,K] . B[N,K]^T (+ R[M,N]), host fp32 arrays in and out; with MLH_DTYPE_BF16 (or 2 = IEEE half) both
- * operands are rounded to that type first; 3 takes fp32 through the three-bf16-plane products of the prefill (at fp32
- * precision; so does MLH_DTYPE_F32 from 65 rows on).  K*4 (fp32) or K*2 (bf16, half) must be a multiple of 128.
+ * operands are rounded to that type first; 3 takes fp32 through products of three bf16 planes (at fp32
+ * precision; so does MLH_DTYPE_F32 from 65 rows on), 4 through the scaled halves of the prefill (K a multiple of 32; the SwiGLU epilogue then gives fp32).  K*4 (fp32) or K*2 (bf16, half) must be a multiple of 128.
  * dtype | 0x100 selects the SwiGLU epilogue of the gate/up projection instead (R must be null, N even): columns 2j and
  * 2j+1 of the product are gate and up of unit j and C is [M, N/2] with C[m, j] = silu(gate) * up, rounded to the
  * operand type as the prefill pass stores it (inference.cu:262-281).

@@ -12,6 +12,7 @@
 // Here: the 256 x 256-tile kernel of the long two-byte products (k_gemm_tn_w4), the weight-streaming kernels for up to
 // 64 rows (k_gemm_skinny*: bf16 models' prompts of 33 to 64 tokens as halves; every type through mlh_gemm_device and the self-test,
 // which alone uses k_gemm_tn_w4 with bf16) and the dispatch; kernels_tile.hip has what lies between, and every longer fp32 product.
+#include <math.h>
 #include <string.h>
 
 #include <algorithm>
@@ -849,10 +850,12 @@ static hipError_t launch_gemm_skinny(hipStream_t stream, int epi, const void* A,
 // ws: optional zero-initialised workspace of mlh_gemm_workspace_bytes() (enables split-K for M <= 64); launches that
 // share a workspace must be ordered on one stream.
 hipError_t mlh_gemm_tn_epi(hipStream_t stream, int dtype, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                           const float* R, int ldr, int M, int N, int K, void* ws, float alpha) {
+                           const float* R, int ldr, int M, int N, int K, void* ws, float alpha, const int* eA, const int* eB, const int* eC) {
     const size_t esz = dtype == MLH_GEMM_P3 ? 6 : dtype == MLH_DTYPE_F32 ? 4 : 2;
-    if (dtype == MLH_GEMM_P3 && (M <= 0 || N <= 0 || K <= 0 || K % 32 || lda % 32 || ldb % 32)) return hipErrorInvalidValue;
-    if (dtype == MLH_GEMM_P3) return mlh_gemm_tile(stream, dtype, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha);
+    if (dtype == MLH_GEMM_P3 || dtype == MLH_GEMM_H2) {
+        if (M <= 0 || N <= 0 || K <= 0 || K % 32 || lda % 32 || ldb % 32 || (dtype == MLH_GEMM_H2 && (!eB || (epi == GEMM_EPI_SWIGLU && !eC)))) return hipErrorInvalidValue;
+        return mlh_gemm_tile(stream, dtype, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha, eA, eB, eC);
+    }
     if (M <= 0 || N <= 0 || K <= 0 || ((size_t)K * esz) % GKB != 0 || ((size_t)lda * esz) % 16 != 0 || ((size_t)ldb * esz) % 16 != 0)
         return hipErrorInvalidValue;
     if (epi == GEMM_EPI_SWIGLU && (N & 1)) return hipErrorInvalidValue;
@@ -869,7 +872,7 @@ hipError_t mlh_gemm_tn_epi(hipStream_t stream, int dtype, int epi, const void* A
         GEMM_BY_TYPE((launch_gemm_skinny<float, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)),
                      (launch_gemm_skinny<bf16_t, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)),
                      (launch_gemm_skinny<f16_t, 2>(stream, epi, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, ws, alpha)));
-    if (dtype == MLH_DTYPE_F32) return hipErrorInvalidValue; // longer fp32 products take their operands as planes (MLH_GEMM_P3)
+    if (dtype == MLH_DTYPE_F32) return hipErrorInvalidValue; // longer fp32 products take their operands as pairs (MLH_GEMM_H2) or planes (MLH_GEMM_P3)
     // Two-byte operands: 256 x 256 tiles walked by one workgroup per unit where there are enough of them, smaller tiles
     // (kernels_tile.hip) otherwise: the estimates decide.
     const int cus = mlh_gemm_num_cus();
@@ -910,22 +913,30 @@ static void host_to_f16(const float* src, f16_t* dst, size_t n) {
     }
 }
 
+static int unit_exponent(double bound) { // (k_unit_exps on the host)
+    int e = 0;
+    frexp(bound, &e);
+    return bound > 0.0 ? e - 15 : 0;
+}
+
 // Stand-alone check and timing of the GEMM kernel: host fp32 inputs (rounded to bf16 first when
 // dtype says so), result back on the host, mean launch time over `iters` launches from HIP events.
 extern "C" int mlh_selftest_gemm(int dtypeAndEpilogue, int M, int N, int K, const float* A, const float* B, const float* R, float* C,
                                  int iters, double* avgUs) {
     int dtype = dtypeAndEpilogue & 0xff;
-    if (dtype == MLH_DTYPE_F32 && M > 64) dtype = MLH_GEMM_P3; // as the prefill pass does
-    const bool p3 = dtype == MLH_GEMM_P3;
+    if (dtype == MLH_DTYPE_F32 && M > 64) dtype = MLH_GEMM_P3;
+    const bool p3 = dtype == MLH_GEMM_P3, h2 = dtype == MLH_GEMM_H2;
     const bool swiglu = (dtypeAndEpilogue & MLH_SELFTEST_SWIGLU) != 0; // C is then [M, N / 2]: silu(gate) * up of the column pairs
     if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0 || (swiglu && (R || (N & 1)))) return -1;
     if (mlh_device_count() <= 0) return -1;
-    if (p3 && K % 32) return -1;
-    const size_t esz = p3 ? 6 : dtype == MLH_DTYPE_F32 ? 4 : 2;
-    const int NC = !swiglu ? N : p3 ? (N / 2 + 31) / 32 * 32 : N / 2; // (rows of planes are whole blocks)
+    if ((p3 || h2) && K % 32) return -1;
+    const size_t esz = p3 ? 6 : h2 || dtype == MLH_DTYPE_F32 ? 4 : 2;
+    const int NC = !swiglu ? N : p3 || h2 ? (N / 2 + 31) / 32 * 32 : N / 2; // (rows of planes are whole blocks)
     const size_t csz = swiglu ? esz : 4; // the SwiGLU epilogue writes the operand type
     void *dA = nullptr, *dB = nullptr, *dW = nullptr, *dC = nullptr;
     float *dR = nullptr, *dF = nullptr;
+    int* dE = nullptr; // exponents of the rows of A, then of B, then of the units
+    std::vector<int> he;
     int rc = 0;
     std::vector<bf16_t> ha, hb;
     std::vector<uint16_t> hc;
@@ -942,10 +953,29 @@ extern "C" int mlh_selftest_gemm(int dtypeAndEpilogue, int M, int N, int K, cons
     const int epi = swiglu ? GEMM_EPI_SWIGLU : GEMM_EPI_PLAIN;
     hipEvent_t e0 = nullptr, e1 = nullptr;
 #define ST(x) do { if ((x) != hipSuccess) { rc = -2; goto done; } } while (0)
-    ST(hipMalloc(&dA, (size_t)M * K * esz)); ST(hipMalloc(&dB, (size_t)N * K * esz));
+    ST(hipMalloc(&dA, (size_t)M * K * esz)); ST(hipMalloc(&dB, (size_t)N * K * (h2 ? 6 : esz)));
     ST(hipMalloc(&dC, (size_t)M * NC * csz));
     if (R) { ST(hipMalloc((void**)&dR, (size_t)M * N * 4)); ST(hipMemcpy(dR, R, (size_t)M * N * 4, hipMemcpyHostToDevice)); }
-    if (p3) {
+    if (h2) {
+        ST(hipMalloc((void**)&dE, ((size_t)M + N + N / 2) * 4));
+        if (swiglu) { // |silu(gate) up| <= |a|^2 |gate row| |up row|
+            auto norm2 = [&](const float* x) { double s = 0.0; for (int k = 0; k < K; k++) s += (double)x[k] * x[k]; return s; };
+            double most = 0.0;
+            for (int m = 0; m < M; m++) most = std::max(most, norm2(A + (size_t)m * K));
+            he.resize(N / 2);
+            for (int j = 0; j < N / 2; j++) he[j] = unit_exponent(most * sqrt(norm2(B + (size_t)2 * j * K) * norm2(B + ((size_t)2 * j + 1) * K)));
+            ST(hipMemcpy(dE + M + N, he.data(), he.size() * 4, hipMemcpyHostToDevice));
+        }
+        ST(hipMalloc((void**)&dF, (size_t)N * K * 4));
+        ST(hipMemcpy(dF, B, (size_t)N * K * 4, hipMemcpyHostToDevice));
+        ST(mlh_split_h2(nullptr, true, dF, K, dB, K, nullptr, dE + M, N, K));
+        ST(hipDeviceSynchronize());
+        (void)hipFree(dF);
+        dF = nullptr;
+        ST(hipMalloc((void**)&dF, (size_t)M * K * 4));
+        ST(hipMemcpy(dF, A, (size_t)M * K * 4, hipMemcpyHostToDevice));
+        ST(mlh_split_h2(nullptr, false, dF, K, dA, K, nullptr, dE, M, K));
+    } else if (p3) {
         ST(hipMalloc((void**)&dF, (size_t)std::max(M, N) * K * 4));
         ST(hipMemcpy(dF, A, (size_t)M * K * 4, hipMemcpyHostToDevice));
         ST(mlh_split_p3(nullptr, dF, K, dA, K, M, K));
@@ -958,20 +988,30 @@ extern "C" int mlh_selftest_gemm(int dtypeAndEpilogue, int M, int N, int K, cons
     }
     ST(hipMalloc(&dW, mlh_gemm_workspace_bytes()));
     ST(hipMemset(dW, 0, mlh_gemm_workspace_bytes()));
-    ST(mlh_gemm_tn_epi(nullptr, dtype, epi, dA, K, dB, K, dC, NC, dR, N, M, N, K, dW));
+    ST(mlh_gemm_tn_epi(nullptr, dtype, epi, dA, K, dB, K, dC, NC, dR, N, M, N, K, dW, 1.0f, dE, dE ? dE + M : nullptr, dE ? dE + M + N : nullptr));
     ST(hipDeviceSynchronize());
     if (iters > 0 && avgUs) {
         ST(hipEventCreate(&e0)); ST(hipEventCreate(&e1));
         ST(hipEventRecord(e0, nullptr));
-        for (int i = 0; i < iters; i++) ST(mlh_gemm_tn_epi(nullptr, dtype, epi, dA, K, dB, K, dC, NC, dR, N, M, N, K, dW));
+        for (int i = 0; i < iters; i++) ST(mlh_gemm_tn_epi(nullptr, dtype, epi, dA, K, dB, K, dC, NC, dR, N, M, N, K, dW, 1.0f, dE, dE ? dE + M : nullptr, dE ? dE + M + N : nullptr));
         ST(hipEventRecord(e1, nullptr));
         ST(hipEventSynchronize(e1));
         float ms = 0.f;
         ST(hipEventElapsedTime(&ms, e0, e1));
         *avgUs = (double)ms * 1000.0 / iters;
     }
-    if (csz == 4) {
+    if (!swiglu || dtype == MLH_DTYPE_F32) {
         ST(hipMemcpy(C, dC, (size_t)M * NC * 4, hipMemcpyDeviceToHost));
+    } else if (h2) { // the sum of a pair, at its column's scale
+        hc.resize((size_t)M * NC * 2);
+        ST(hipMemcpy(hc.data(), dC, hc.size() * 2, hipMemcpyDeviceToHost));
+        for (int m = 0; m < M; m++)
+            for (int j = 0; j < N / 2; j++) {
+                const uint16_t* b = hc.data() + ((size_t)m * (NC / 32) + j / 32) * 64 + j % 32;
+                _Float16 hi, lo;
+                memcpy(&hi, b, 2); memcpy(&lo, b + 32, 2);
+                C[(size_t)m * (N / 2) + j] = ldexpf((float)hi + (float)lo, he[j]);
+            }
     } else if (p3) { // the sum of the planes is the fp32 result
         hc.resize((size_t)M * NC * 3);
         ST(hipMemcpy(hc.data(), dC, hc.size() * 2, hipMemcpyDeviceToHost));
@@ -994,7 +1034,7 @@ extern "C" int mlh_selftest_gemm(int dtypeAndEpilogue, int M, int N, int K, cons
 done:
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
-    (void)hipFree(dA); (void)hipFree(dB); (void)hipFree(dC); (void)hipFree(dR); (void)hipFree(dW); (void)hipFree(dF);
+    (void)hipFree(dA); (void)hipFree(dB); (void)hipFree(dC); (void)hipFree(dR); (void)hipFree(dW); (void)hipFree(dF); (void)hipFree(dE);
     return rc;
 }
 

@@ -1,7 +1,7 @@
 // Prefill: many tokens of one or more sequences through the stack at once.
 //
 // Rows of the activation matrices are tokens (all segments concatenated); the projections are MFMA
-// GEMMs (kernels_gemm.hip, kernels_tile.hip) against copies of the weights as planes or halves, or, in short calls, the row
+// GEMMs (kernels_gemm.hip, kernels_tile.hip) against copies of the weights as halves, or, in short calls, the row
 // kernels of the decode step (kernels_rows.hip); per layer
 //
 //   rmsnorm rows -> GEMM Wa -> attention: per-head QK-norm + RoPE + KV-page write, tiled causal attention
@@ -11,16 +11,18 @@
 //
 // and at the end the LM head runs for the last row of every segment only (the reference computes
 // logits for all L columns, inference.cu:723-743, and uses the last one).  With bf16 weights the GEMM
-// inputs (normed activations, mixing output, FFN activations) are rounded to half; with fp32 weights they and the
-// weights are stored as three bf16 planes that add up to the fp32 value (p3.h).  Accumulation, the
+// inputs (normed activations, mixing output, FFN activations) are rounded to half; with fp32 weights they are
+// stored as two halves, the weights as three that add up to the scaled fp32 value (h2.h).  Accumulation, the
 // residual stream, K/V and GDN states stay fp32.  This is what runInference(L) (inference.cu:376-751)
 // does for L columns, minus the columns that are already in the cache.
 #include <string.h>
 
 #include <algorithm>
 
+#include "h2.h"
 #include "mlh_internal.h"
 #include "p3.h"
+#include "persist_common.h"
 #include "sample.h"
 
 #define PWG 256
@@ -40,10 +42,11 @@ struct PfArgs {
     const int* blkSeg; // attention query blocks: segment and first query of the block
     const int* blkQ0;
     float* X;          // [n, dim] residual stream
-    void* Xn;          // [n, dim] GEMM input (planes or halves)
+    void* Xn;          // [n, dim] GEMM input (fp32 models: pairs of halves, h2.h; else halves)
+    int* exps;         // exponents of pairs' rows
     float* QKV;        // [n, qkvLd]
     int qkvLd;
-    void* Amix;        // [n, aLd] GEMM input of the output projection: mixing output, then (at column L.ad) the PLE row
+    void* Amix;        // [n, aLd] GEMM input of the output projection: mixing output, then (at column L.ad) the PLE row (fp32 models: floats first)
     int aLd;
     float* H1;         // [n, dim]
     void* U;           // [n, ffn]
@@ -64,6 +67,7 @@ __device__ __forceinline__ float pf_wave_max(float v) {
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
     return v;
 }
+__device__ __forceinline__ int pf_wave_max(int v) { return (int)pwave_max((float)v); } // (exponents: exact)
 __device__ __forceinline__ float pf_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); } // inference.cu:248
 __device__ __forceinline__ float pf_silu(float v) { return v / (1.0f + expf(-v)); }       // inference.cu:270
 
@@ -73,9 +77,9 @@ template <> __device__ __forceinline__ void put<f16_t>(f16_t* p, float v) {
     const _Float16 h = (_Float16)half_range(v);
     p->bits = __builtin_bit_cast(uint16_t, h);
 }
-// element `col` of row `row` of a GEMM input matrix (leading dimension ld in elements; fp32 models: three bf16 planes, p3.h)
+template <> __device__ __forceinline__ void put<float>(float* p, float v) { *p = v; }
+// element `col` of row `row` of a GEMM input matrix (leading dimension ld in elements)
 template <typename AT> __device__ __forceinline__ void put_at(void* base, size_t row, int ld, int col, float v) { put<AT>((AT*)base + row * ld + col, v); }
-template <> __device__ __forceinline__ void put_at<p3_t>(void* base, size_t row, int ld, int col, float v) { p3_put((unsigned char*)base + row * ld * 6, col, v); }
 // element `col` of a token's mixing output (behind it: its PLE columns)
 template <typename AT> __device__ __forceinline__ void put_mix(const PfArgs& P, size_t row, int col, float v) {
     if (P.rows) rows_put(P.rows, col, (int)row, P.lay, P.half != 0, v);
@@ -101,12 +105,12 @@ template <> __device__ __forceinline__ void put4<f16_t>(f16_t* o, float a, float
     *reinterpret_cast<uint2*>(o) = make_uint2(pack_half_range(a, b), pack_half_range(c, d));
 }
 
+template <> __device__ __forceinline__ void put4<float>(float* o, float a, float b, float c, float d) { *reinterpret_cast<f32x4*>(o) = f32x4{a, b, c, d}; }
+
 template <typename AT> __device__ __forceinline__ void put4_at(void* base, size_t row, int ld, int col, float a, float b, float c, float d) { put4<AT>((AT*)base + row * ld + col, a, b, c, d); }
-template <> __device__ __forceinline__ void put4_at<p3_t>(void* base, size_t row, int ld, int col, float a, float b, float c, float d) { p3_put4((unsigned char*)base + row * ld * 6, col, a, b, c, d); }
 // Four columns of the mixing output.
 template <typename AT> __device__ __forceinline__ void put_mix4(const PfArgs& P, size_t row, int col, const f32x4& v) {
     if (P.rows) rows_put4(P.rows, col, (int)row, P.lay, P.half != 0, v.x, v.y, v.z, v.w);
-    else if constexpr (sizeof(AT) == 6) p3_put4((unsigned char*)P.Amix + row * P.aLd * 6, col, v.x, v.y, v.z, v.w);
     else put4_at<AT>(P.Amix, row, P.aLd, col, v.x, v.y, v.z, v.w);
 }
 
@@ -114,7 +118,7 @@ template <typename AT> __device__ __forceinline__ void put_mix4(const PfArgs& P,
 // gains asked for behind the sum, each add a memory latency.  Measured: 777 rows of 2048 5.4 us (6.3), 517 rows of 768 5.0 us (4.9); 16384 rows of
 // 2048 32 us (37), 6.2 TB/s: part of it comes out of the caches.
 template <typename AT, int KEEP>
-__global__ void __launch_bounds__(PWG) k_pf_rmsnorm(const float* __restrict__ X, const float* __restrict__ gamma, void* out, int n, int d) {
+__global__ void __launch_bounds__(PWG) k_pf_rmsnorm(const float* __restrict__ X, const float* __restrict__ gamma, void* out, int* exps, int n, int d) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= n) return;
     const float* x = X + (size_t)row * d;
@@ -135,22 +139,36 @@ __global__ void __launch_bounds__(PWG) k_pf_rmsnorm(const float* __restrict__ X,
     }
     s = pf_wave_sum(s);
     const float r = sqrtf(s / (float)d + 1e-8f);
+    auto normed = [&](const f32x4& v, const f32x4& g) { return f32x4{g.x * (v.x / r), g.y * (v.y / r), g.z * (v.z / r), g.w * (v.w / r)}; };
+    auto later = [&](int i) { return normed(*reinterpret_cast<const f32x4*>(x + i), *reinterpret_cast<const f32x4*>(gamma + i)); }; // past the kept ones
 #pragma unroll
-    for (int k = 0; k < KEEP; k++) {
-        const int i = lane * 4 + k * 256;
-        const f32x4 v = keep[k], g = gain[k];
-        if (i < d) put4_at<AT>(out, (size_t)row, d, i, g.x * (v.x / r), g.y * (v.y / r), g.z * (v.z / r), g.w * (v.w / r));
+    for (int k = 0; k < KEEP; k++) keep[k] = normed(keep[k], gain[k]);
+    int e = 0;
+    if constexpr (__is_same(AT, h2_t)) { // the row's scale
+        int most = -100000;
+#pragma unroll
+        for (int k = 0; k < KEEP; k++) most = max(most, h2_size4(keep[k].x, keep[k].y, keep[k].z, keep[k].w)); // (past the end: the last columns once more)
+        for (int i = lane * 4 + KEEP * 256; i < d; i += 256) {
+            const f32x4 v = later(i);
+            most = max(most, h2_size4(v.x, v.y, v.z, v.w));
+        }
+        e = h2_exponent(pf_wave_max(most));
+        if (lane == 0) exps[row] = e;
     }
-    for (int i = lane * 4 + KEEP * 256; i < d; i += 256) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(x + i), g = *reinterpret_cast<const f32x4*>(gamma + i);
-        put4_at<AT>(out, (size_t)row, d, i, g.x * (v.x / r), g.y * (v.y / r), g.z * (v.z / r), g.w * (v.w / r));
-    }
+    auto store = [&](int i, const f32x4& v) {
+        if constexpr (__is_same(AT, h2_t)) h2_put4<false>((unsigned char*)out + (size_t)row * d * 4, i, ldexpf(v.x, -e), ldexpf(v.y, -e), ldexpf(v.z, -e), ldexpf(v.w, -e));
+        else put4_at<AT>(out, (size_t)row, d, i, v.x, v.y, v.z, v.w);
+    };
+#pragma unroll
+    for (int k = 0; k < KEEP; k++)
+        if (lane * 4 + k * 256 < d) store(lane * 4 + k * 256, keep[k]);
+    for (int i = lane * 4 + KEEP * 256; i < d; i += 256) store(i, later(i));
 }
-template <typename AT> static void launch_rmsnorm(hipStream_t st, const float* X, const float* gamma, void* out, int n, int d) {
+template <typename AT> static void launch_rmsnorm(hipStream_t st, const float* X, const float* gamma, void* out, int* exps, int n, int d) {
     const dim3 grid((n + 3) / 4);
-    if (d <= 1024) hipLaunchKernelGGL((k_pf_rmsnorm<AT, 4>), grid, dim3(PWG), 0, st, X, gamma, out, n, d);
-    else if (d <= 2048) hipLaunchKernelGGL((k_pf_rmsnorm<AT, 8>), grid, dim3(PWG), 0, st, X, gamma, out, n, d);
-    else hipLaunchKernelGGL((k_pf_rmsnorm<AT, 16>), grid, dim3(PWG), 0, st, X, gamma, out, n, d);
+    if (d <= 1024) hipLaunchKernelGGL((k_pf_rmsnorm<AT, 4>), grid, dim3(PWG), 0, st, X, gamma, out, exps, n, d);
+    else if (d <= 2048) hipLaunchKernelGGL((k_pf_rmsnorm<AT, 8>), grid, dim3(PWG), 0, st, X, gamma, out, exps, n, d);
+    else hipLaunchKernelGGL((k_pf_rmsnorm<AT, 16>), grid, dim3(PWG), 0, st, X, gamma, out, exps, n, d);
 }
 
 // Per (head, row): per-head RMSNorm of q and k (inference.cu:52-81, 97-111), RoPE on adjacent pairs at the
@@ -1381,6 +1399,57 @@ __global__ void k_pf_ple(PfArgs P, LayerDev L) {
     put_mix<AT>(P, (size_t)row, L.ad + j, pf_silu(g) * getw<WT>((const WT*)L.pleTable + (size_t)P.ids[row] * P.a.ple + j));
 }
 
+// fp32 models: the row of mixing output (floats, from several workgroups) and its PLE columns as pairs (h2.h) and the row's exponent, in place: 32
+// columns take 128 bytes either way, and a block's eight lanes read it in an instruction before the one that writes it.  A wave a row; up to 256 KEEP
+// columns stay in registers between the maximum and the split.
+template <int KEEP>
+__global__ void __launch_bounds__(PWG) k_pf_pairs(PfArgs P, LayerDev L) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, cols = L.ad + P.a.ple;
+    if (row >= P.n) return;
+    float* x = (float*)P.Amix + (size_t)row * P.aLd;
+    const float* gate = P.QKV + (size_t)row * P.qkvLd + L.offPle;
+    const float* table = (const float*)L.pleTable + (size_t)P.ids[row] * P.a.ple;
+    auto value = [&](int i) {
+        if (i < L.ad) return *reinterpret_cast<const f32x4*>(x + i);
+        const int j = i - L.ad;
+        return f32x4{pf_silu(gate[j]) * table[j], pf_silu(gate[j + 1]) * table[j + 1], pf_silu(gate[j + 2]) * table[j + 2], pf_silu(gate[j + 3]) * table[j + 3]};
+    };
+    f32x4 keep[KEEP];
+    int most = -100000;
+#pragma unroll
+    for (int k = 0; k < KEEP; k++) keep[k] = value(min(lane * 4 + k * 256, cols - 4));
+#pragma unroll
+    for (int k = 0; k < KEEP; k++) most = max(most, h2_size4(keep[k].x, keep[k].y, keep[k].z, keep[k].w));
+    for (int i = lane * 4 + KEEP * 256; i < cols; i += 256) {
+        const f32x4 v = value(i);
+        most = max(most, h2_size4(v.x, v.y, v.z, v.w));
+    }
+    const int e = h2_exponent(pf_wave_max(most));
+    if (lane == 0) P.exps[row] = e;
+    auto store = [&](int i, const f32x4& v) { h2_put4<false>(x, i, ldexpf(v.x, -e), ldexpf(v.y, -e), ldexpf(v.z, -e), ldexpf(v.w, -e)); };
+#pragma unroll
+    for (int k = 0; k < KEEP; k++)
+        if (lane * 4 + k * 256 < cols) store(lane * 4 + k * 256, keep[k]);
+    for (int i = lane * 4 + KEEP * 256; i < cols; i += 256) store(i, value(i));
+}
+
+// Exponents of the FFN units' columns, a wave each: |x / rms| <= sqrt(d), so by Cauchy and Schwarz a gate or up value is at most sqrt(d) |row (.) gain| and the
+// unit, |silu(g)| <= |g|, the product of the two.  It is brought under 2^15; the largest half is twice that.
+__global__ void __launch_bounds__(PWG) k_unit_exps(const float* __restrict__ W13, const float* __restrict__ gain, int* exps, int units, int d) {
+    const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (j >= units) return;
+    const float *g = W13 + (size_t)2 * j * d, *u = g + d;
+    double sg = 0.0, su = 0.0;
+    for (int i = lane; i < d; i += 64) {
+        const double a = (double)g[i] * gain[i], b = (double)u[i] * gain[i];
+        sg += a * a; su += b * b;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) { sg += __shfl_xor(sg, o, 64); su += __shfl_xor(su, o, 64); }
+    const double bound = (double)d * sqrt(sg) * sqrt(su);
+    if (lane == 0) exps[j] = bound > 0.0 ? __builtin_amdgcn_frexp_exp(bound) - 15 : 0;
+}
+
 // One workgroup per segment: argmax over the LM head's partial maxima of its last row (lowest index on ties); the
 // sequence's length advances by the segment's.  picks: pinned host memory, by sequence.
 __global__ void __launch_bounds__(PWG) k_pf_finish(PfArgs P, int nparts, int* picks) {
@@ -1579,12 +1648,14 @@ static int operand_values(mlh_ctx* c, bool* within) {
     return 0;
 }
 
-// An fp32 matrix as three bf16 planes, what the tiled products of the prefill multiply.
-static int build_planes(mlh_ctx* c, const void* src, int rows, int cols, const void** dst) {
-    void* buf = nullptr;
-    if (const int rc = mlh_operand_alloc(c, &buf, (size_t)rows * cols * 6)) return rc;
-    MLH_CHECK(c, mlh_split_p3(c->stream, (const float*)src, cols, buf, cols, rows, cols));
+// An fp32 matrix as triples of halves, what the tiled products of the prefill multiply.
+static int build_triples(mlh_ctx* c, const void* src, int rows, int cols, const int* colExps, const void** dst, const int** exps) {
+    void *buf = nullptr, *e = nullptr;
+    int rc;
+    if ((rc = mlh_operand_alloc(c, &buf, (size_t)rows * cols * 6)) || (rc = mlh_operand_alloc(c, &e, (size_t)rows * 4))) return rc;
+    MLH_CHECK(c, mlh_split_h2(c->stream, true, (const float*)src, cols, buf, cols, colExps, (int*)e, rows, cols));
     *dst = buf;
+    *exps = (const int*)e;
     return 0;
 }
 
@@ -1599,8 +1670,8 @@ static size_t gdn_chunk_bytes(const mlh_ctx* c) {
 // Work buffers of a prefill call: per row, and of the chunks that segments of 64 rows or more are cut into (ensure_prefill_buffers).
 static size_t prefill_row_bytes(const mlh_ctx* c) {
     const mlh_hparams& hp = c->hp;
-    const size_t wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 6, d = hp.dim;
-    return d * (8 + wb + (wb == 2 ? 4 : 0)) + (size_t)c->maxRowsA * 4 + ((size_t)c->maxAd + hp.pleDim + hp.ffnDim) * wb + 64;
+    const size_t wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 4, d = hp.dim;
+    return d * (8 + wb + (wb == 2 ? 4 : 0)) + (size_t)c->maxRowsA * 4 + ((size_t)c->maxAd + hp.pleDim + hp.ffnDim) * wb + 68;
 }
 // ... of one over every position of the context, with the products' split-K workspace.
 size_t mlh_prefill_work_bytes(const mlh_ctx* c) {
@@ -1631,11 +1702,12 @@ void mlh_drop_operands(mlh_ctx* c) {
     for (void* p : c->mirrorAllocs) (void)hipFree(p);
     c->mirrorAllocs.clear();
     c->operandBytes = 0;
-    for (LayerDev& L : c->layers) L.WaP = L.WoP = L.W13P = L.W2P = L.WaR = L.WoR = L.W13R = L.W2R = nullptr;
+    for (LayerDev& L : c->layers) L.eWa = L.eWo = L.eW13 = L.eW2 = L.eU = nullptr, L.WaP = L.WoP = L.W13P = L.W2P = L.WaR = L.WoR = L.W13R = L.W2R = nullptr;
     c->EP = c->ER = nullptr;
+    c->eE = nullptr;
 }
 
-// The planes or halves; on MLH_NO_ROOM what has been allocated so far is still there.
+// The halves; on MLH_NO_ROOM what has been allocated so far is still there.
 static int build_operands(mlh_ctx* c, unsigned* d_scratch) {
     const mlh_hparams& hp = c->hp;
     const bool mirror = hp.weightDtype == MLH_DTYPE_BF16;
@@ -1659,13 +1731,18 @@ static int build_operands(mlh_ctx* c, unsigned* d_scratch) {
                 (rc = build_mirror(c, L.W2, d * F, &L.W2P, &L.sW2, d_scratch)))
                 return rc;
         } else {
-            if ((rc = build_planes(c, L.Wa, L.rowsA, (int)d, &L.WaP)) || (rc = build_planes(c, wo, (int)d, L.ad + (int)pl, &L.WoP)) ||
-                (rc = build_planes(c, L.W13, 2 * (int)F, (int)d, &L.W13P)) || (rc = build_planes(c, L.W2, (int)d, (int)F, &L.W2P)))
+            void* units = nullptr;
+            if ((rc = mlh_operand_alloc(c, &units, F * 4))) return rc;
+            hipLaunchKernelGGL(k_unit_exps, dim3(cdiv((int)F, 4)), dim3(PWG), 0, c->stream, (const float*)L.W13, L.g2, (int*)units, (int)F, (int)d);
+            MLH_CHECK(c, hipGetLastError());
+            L.eU = (const int*)units;
+            if ((rc = build_triples(c, L.Wa, L.rowsA, (int)d, nullptr, &L.WaP, &L.eWa)) || (rc = build_triples(c, wo, (int)d, L.ad + (int)pl, nullptr, &L.WoP, &L.eWo)) ||
+                (rc = build_triples(c, L.W13, 2 * (int)F, (int)d, nullptr, &L.W13P, &L.eW13)) || (rc = build_triples(c, L.W2, (int)d, (int)F, L.eU, &L.W2P, &L.eW2)))
                 return rc;
         }
     }
     c->sE = 1.0f;
-    return mirror ? build_mirror(c, c->E, (size_t)hp.vocabSize * hp.dim, &c->EP, &c->sE, d_scratch) : build_planes(c, c->E, hp.vocabSize, hp.dim, &c->EP);
+    return mirror ? build_mirror(c, c->E, (size_t)hp.vocabSize * hp.dim, &c->EP, &c->sE, d_scratch) : build_triples(c, c->E, hp.vocabSize, hp.dim, nullptr, &c->EP, &c->eE);
 }
 
 int mlh_build_gemm_operands(mlh_ctx* c) {
@@ -1675,7 +1752,7 @@ int mlh_build_gemm_operands(mlh_ctx* c) {
     int rc = 0;
     bool ok = false;
     if ((rc = operand_values(c, &ok)) || !ok || (rc = operand_room(c, &ok)) || !ok) return rc;
-    c->pfDtype = c->hp.weightDtype == MLH_DTYPE_BF16 ? MLH_GEMM_F16 : MLH_GEMM_P3;
+    c->pfDtype = c->hp.weightDtype == MLH_DTYPE_BF16 ? MLH_GEMM_F16 : MLH_GEMM_H2;
     unsigned* d_scratch = nullptr;
     MLH_CHECK(c, hipMalloc((void**)&d_scratch, 8));
     rc = build_operands(c, d_scratch);
@@ -1702,7 +1779,7 @@ static int ensure_prefill_buffers(mlh_ctx* c, int rows) {
     for (void* p : c->pfAllocs) (void)hipFree(p);
     c->pfAllocs.clear();
     c->pfRows = 0;
-    const size_t n = (size_t)rows, wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 6; // GEMM input elements: halves, or three bf16 planes
+    const size_t n = (size_t)rows, wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 4; // GEMM input elements: halves, or pairs of them
     auto alloc = [&](void** p, size_t bytes) -> int {
         MLH_CHECK(c, hipMalloc(p, std::max<size_t>(bytes, 16)));
         c->pfAllocs.push_back(*p);
@@ -1713,7 +1790,7 @@ static int ensure_prefill_buffers(mlh_ctx* c, int rows) {
     const size_t meta = 3 * n + 5 * (size_t)hp.maxSeqs + 2 * nblk + 2 * nchunk; // ids, sequence and position of every row; segments; attention blocks; GDN chunks
     if ((rc = alloc((void**)&c->pfX, n * hp.dim * 4)) || (rc = alloc(&c->pfXn, n * hp.dim * wb)) ||
         (rc = alloc((void**)&c->pfQKV, n * c->maxRowsA * 4)) || (rc = alloc(&c->pfA, n * (c->maxAd + hp.pleDim) * wb)) ||
-        (rc = alloc((void**)&c->pfH1, n * hp.dim * 4)) ||
+        (rc = alloc((void**)&c->pfH1, n * hp.dim * 4)) || (rc = alloc((void**)&c->pfExp, n * 4)) ||
         (rc = alloc(&c->pfU, n * hp.ffnDim * wb)) ||
         (hp.weightDtype == MLH_DTYPE_BF16 && ((rc = alloc((void**)&c->pfKh, n * hp.dim * 2)) || (rc = alloc((void**)&c->pfVh, n * hp.dim * 2)))) ||
         (rc = alloc((void**)&c->pfMeta, meta * 4)))
@@ -1799,16 +1876,16 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     P.segStart = d_seg; P.segLen = d_seg + nseg; P.segSeq = d_seg + 2 * nseg; P.segPos0 = d_seg + 3 * nseg;
     P.blkSeg = d_blk; P.blkQ0 = d_blk + nblk;
     P.X = c->pfX; P.Xn = c->pfXn; P.QKV = c->pfQKV; P.qkvLd = c->maxRowsA; P.Amix = c->pfA; P.aLd = c->maxAd + hp.pleDim;
-    P.H1 = c->pfH1; P.U = c->pfU;
+    P.H1 = c->pfH1; P.U = c->pfU; P.exps = c->pfExp;
     P.Kh = mfmaAttn && fresh ? c->pfKh : nullptr;
     P.Vh = mfmaAttn && fresh ? c->pfVh : nullptr;
     P.lay = rows_layout(std::min(n, 64)); P.rows = rowsPath ? c->rowsMix : nullptr; P.half = hp.weightDtype == MLH_DTYPE_BF16;
     RowsArgs base = {};
     base.M = n; base.lay = P.lay; base.normDim = hp.dim;
     const int d_ = hp.dim, F = hp.ffnDim, dt = c->pfDtype;
-#define GEMM(A, lda, B, alpha, ldb, C, ldc, R, ldr, M, N, K)                                                \
-    do {                                                                                                    \
-        hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, c->gemmWs, alpha); \
+#define GEMM(A, lda, eA, B, alpha, eB, ldb, C, ldc, R, ldr, M, N, K)                                                           \
+    do {                                                                                                                     \
+        hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, c->gemmWs, alpha, eA, eB); \
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; } \
     } while (0)
 
@@ -1822,9 +1899,9 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
             R.K = d_; R.A = c->rowsX; R.ssqIn = c->rowsSsqX; R.nparts = t == hp.transformers - 1 ? 1 : d_ / RW_TILE; R.C = P.QKV; R.ldc = P.qkvLd;
             mlh_rows_gemm(c, RW_PLAIN, L.WaR, L.rowsA, R);
         } else {
-            PF_DISPATCH_WT(c, launch_rmsnorm<p3_t>(st, P.X, L.g1, P.Xn, n, d_),
-                           launch_rmsnorm<f16_t>(st, P.X, L.g1, P.Xn, n, d_));
-            GEMM(P.Xn, d_, L.WaP, L.sWa, d_, P.QKV, P.qkvLd, nullptr, 0, n, L.rowsA, d_);
+            PF_DISPATCH_WT(c, launch_rmsnorm<h2_t>(st, P.X, L.g1, P.Xn, P.exps, n, d_),
+                           launch_rmsnorm<f16_t>(st, P.X, L.g1, P.Xn, nullptr, n, d_));
+            GEMM(P.Xn, d_, P.exps, L.WaP, L.sWa, L.eWa, d_, P.QKV, P.qkvLd, nullptr, 0, n, L.rowsA, d_);
         }
         if (L.kind == MLH_KIND_ATTENTION) {
             if (hp.headDim == 64) {
@@ -1832,13 +1909,13 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<64, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<64, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (P.half) hipLaunchKernelGGL((k_pf_attn<64, f16_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
-                else hipLaunchKernelGGL((k_pf_attn<64, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
+                else hipLaunchKernelGGL((k_pf_attn<64, float>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
             } else {
                 hipLaunchKernelGGL((k_pf_qk_rope_kv<128>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<128, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<128, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (P.half) hipLaunchKernelGGL((k_pf_attn<128, f16_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
-                else hipLaunchKernelGGL((k_pf_attn<128, p3_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
+                else hipLaunchKernelGGL((k_pf_attn<128, float>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
             }
         } else {
             const int skipFrom = gdnChunked ? GD_C : 0x7fffffff;
@@ -1848,8 +1925,8 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
                 const bool half = hp.weightDtype == MLH_DTYPE_BF16, few = hp.gdnHeads * nseg <= 2 * c->numCUs;
 #define RECUR(DK_, GR_, AT_) hipLaunchKernelGGL((k_pf_gdn<DK_, GR_, AT_>), dim3(hp.gdnHeads, nseg, DK_ / GR_), dim3(PWG), 0, st, P, L, skipFrom)
 #define RECUR_ROWS(DK_, AT_) do { if (few) RECUR(DK_, 32, AT_); else RECUR(DK_, 64, AT_); } while (0)
-                if (hp.gdnDk == 64) { if (half) RECUR_ROWS(64, f16_t); else RECUR_ROWS(64, p3_t); }
-                else { if (half) RECUR_ROWS(128, f16_t); else RECUR_ROWS(128, p3_t); }
+                if (hp.gdnDk == 64) { if (half) RECUR_ROWS(64, f16_t); else RECUR_ROWS(64, float); }
+                else { if (half) RECUR_ROWS(128, f16_t); else RECUR_ROWS(128, float); }
 #undef RECUR_ROWS
 #undef RECUR
             }
@@ -1871,21 +1948,25 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
                 }
             }
         }
-        if (hp.pleDim > 0)
-            PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_ple<float, p3_t>), dim3(n), dim3(std::max(64, hp.pleDim)), 0, st, P, L),
+        if (dt == MLH_GEMM_H2 && !rowsPath) {
+            const int cols = L.ad + hp.pleDim;
+            if (cols <= 1024) hipLaunchKernelGGL((k_pf_pairs<4>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P, L);
+            else hipLaunchKernelGGL((k_pf_pairs<8>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P, L);
+        } else if (hp.pleDim > 0)
+            PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_ple<float, float>), dim3(n), dim3(std::max(64, hp.pleDim)), 0, st, P, L),
                            hipLaunchKernelGGL((k_pf_ple<bf16_t, f16_t>), dim3(n), dim3(std::max(64, hp.pleDim)), 0, st, P, L));
         if (rowsPath) {
             mlh_rows_rest_of_layer(c, t, base, P.X, P.H1);
             continue;
         }
-        GEMM(P.Amix, P.aLd, L.WoP, L.sWo, L.ad + hp.pleDim, P.H1, d_, P.X, d_, n, d_, L.ad + hp.pleDim); // Wo . a + pleUp . e + x
-        PF_DISPATCH_WT(c, launch_rmsnorm<p3_t>(st, P.H1, L.g2, P.Xn, n, d_),
-                       launch_rmsnorm<f16_t>(st, P.H1, L.g2, P.Xn, n, d_));
+        GEMM(P.Amix, P.aLd, P.exps, L.WoP, L.sWo, L.eWo, L.ad + hp.pleDim, P.H1, d_, P.X, d_, n, d_, L.ad + hp.pleDim); // Wo . a + pleUp . e + x
+        PF_DISPATCH_WT(c, launch_rmsnorm<h2_t>(st, P.H1, L.g2, P.Xn, P.exps, n, d_),
+                       launch_rmsnorm<f16_t>(st, P.H1, L.g2, P.Xn, nullptr, n, d_));
         { // gate/up projection with SiLU(gate) * up in the epilogue (inference.cu:262-281): U comes out in the GEMM input type
-            hipError_t e_ = mlh_gemm_tn_epi(st, dt, 1, P.Xn, d_, L.W13P, d_, P.U, F, nullptr, 0, n, 2 * F, d_, c->gemmWs, L.sW13);
+            hipError_t e_ = mlh_gemm_tn_epi(st, dt, 1, P.Xn, d_, L.W13P, d_, P.U, F, nullptr, 0, n, 2 * F, d_, c->gemmWs, L.sW13, P.exps, L.eW13, L.eU);
             if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
         }
-        GEMM(P.U, F, L.W2P, L.sW2, F, P.X, d_, P.H1, d_, n, d_, F);
+        GEMM(P.U, F, nullptr, L.W2P, L.sW2, L.eW2, F, P.X, d_, P.H1, d_, n, d_, F);
     }
 #undef GEMM
     if (allLogits && rowsPath) { // tied LM head of every normalised row (inference.cu:705-743 computes all L columns)
@@ -1893,9 +1974,9 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         R.K = d_; R.A = c->rowsX; R.ssqIn = c->rowsSsqX; R.nparts = d_ / RW_TILE; R.C = allLogits; R.ldc = hp.vocabSize;
         mlh_rows_gemm(c, RW_PLAIN, c->ER, hp.vocabSize, R);
     } else if (allLogits) {
-        PF_DISPATCH_WT(c, launch_rmsnorm<p3_t>(st, P.X, c->gF, P.Xn, n, d_),
-                       launch_rmsnorm<f16_t>(st, P.X, c->gF, P.Xn, n, d_));
-        hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, P.Xn, d_, c->EP, d_, allLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_, c->gemmWs, c->sE);
+        PF_DISPATCH_WT(c, launch_rmsnorm<h2_t>(st, P.X, c->gF, P.Xn, P.exps, n, d_),
+                       launch_rmsnorm<f16_t>(st, P.X, c->gF, P.Xn, nullptr, n, d_));
+        hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, P.Xn, d_, c->EP, d_, allLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_, c->gemmWs, c->sE, P.exps, c->eE);
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
     }
     for (int s0 = 0; s0 < nseg; s0 += 64)

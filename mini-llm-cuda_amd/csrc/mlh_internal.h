@@ -18,7 +18,8 @@ typedef uint16_t bf16_t;
 // IEEE half, as the MFMA path stores weights and activations of bf16 models (see MLH_GEMM_F16)
 struct f16_t { uint16_t bits; };
 #define MLH_GEMM_F16 2 // GEMM operand type code beside MLH_DTYPE_F32 / MLH_DTYPE_BF16
-#define MLH_GEMM_P3 3  // ... and for fp32 operands stored as three bf16 planes (p3.h)
+#define MLH_GEMM_P3 3  // ... and for fp32 operands stored as three bf16 planes (p3.h; the GEMM self-test)
+#define MLH_GEMM_H2 4  // ... and fp32 as halves, pairs times triples, with an exponent per row (h2.h)
 #define MLH_GEMM_WS_COUNTERS 1024 // tile counters at the head of a split-K workspace ...
 #define MLH_GEMM_WS_PARTIALS (256 * 8 * 2 * 16 * 64) // ... and the partial sums (floats) behind them
 #define MLH_SELFTEST_SWIGLU 0x100 // mlh_selftest_gemm: flag beside the operand type, selects the SwiGLU epilogue
@@ -63,11 +64,13 @@ struct LayerDev {
     int kind;
     int rowsA, offK, offV, offG, offPle, offGa, offGb;
     int ad;               // width of the mixing output fed to Wo
-    // What the prefill's products multiply: fp32 matrices as three bf16 planes (p3.h); for bf16 models IEEE-half
+    // What the prefill's products multiply: fp32 matrices as triples of halves (h2.h); for bf16 models IEEE-half
     // mirrors scaled by a power of two (exact), with the inverse scale applied to the product.
     // WoP is [dim, ad + pleDim]: Wo with pleUp appended along K, so that h1 = [a | e] . WoP^T is one product.
     const void *WaP, *WoP, *W13P, *W2P;
     float sWa, sWo, sW13, sW2;
+    const int *eWa, *eWo, *eW13, *eW2; // fp32: exponents of their rows ...
+    const int* eU;                     // ... and of the FFN units
     const void *WaR, *WoR, *W13R, *W2R; // for the row step: the matrices ([Wo | pleUp] as one) in its fetch order (rows.h)
 };
 
@@ -205,6 +208,7 @@ struct mlh_ctx {
     std::vector<void*> pfAllocs;
     float *pfX = nullptr, *pfQKV = nullptr, *pfH1 = nullptr;
     void *pfXn = nullptr, *pfA = nullptr, *pfU = nullptr;
+    int* pfExp = nullptr; // fp32: exponents of the rows of the product input at hand
     uint16_t *pfKh = nullptr, *pfVh = nullptr; // half copies of a call's K and V rows for the MFMA attention of a fresh prefill
     int* pfMeta = nullptr;
     void* pfGdnWs = nullptr;   // chunk operands of the chunk-parallel GDN prefill
@@ -212,8 +216,9 @@ struct mlh_ctx {
     size_t pfGdnChunks = 0;
     const void* EP = nullptr;  // LM-head matrix as the prefill's products read it (see LayerDev::WaP)
     float sE = 1.0f;
+    const int* eE = nullptr;
     const void* ER = nullptr;  // ... and in the row step's fetch order
-    int pfDtype = MLH_DTYPE_F32; // operand type of those: MLH_GEMM_P3 or MLH_GEMM_F16
+    int pfDtype = MLH_DTYPE_F32; // operand type of those: MLH_GEMM_H2 or MLH_GEMM_F16
     bool operands = false;     // the copies of the matrices that the MFMA kernels read (LayerDev::WaP .. W2R) exist
     std::vector<void*> mirrorAllocs;
     size_t operandBytes = 0, operandLimit = SIZE_MAX; // what they take and may take
@@ -253,20 +258,21 @@ int mlh_launch_probs(mlh_ctx* c, int seq);
 int mlh_init_kernels(mlh_ctx* c);
 
 // kernels_gemm.hip
-// C[M,N] = A[M,K] . B[N,K]^T (+ R[M,N]); dtype: operand type code (fp32 operands: M <= 64; MLH_GEMM_P3 has no limit).
+// C[M,N] = A[M,K] . B[N,K]^T (+ R[M,N]); dtype: operand type code (fp32 operands: M <= 64; MLH_GEMM_P3 and MLH_GEMM_H2 have no limit).
 // epi 0: C, R fp32.  epi 1 (SwiGLU): columns 2j / 2j+1 of the product are gate / up of unit j and
-// C is [M, N/2] in the operand type: C[m, j] = silu(gate) * up.
+// C is [M, N/2] in the operand type (H2: pairs): C[m, j] = silu(gate) * up.
 // ws: zero-initialised workspace of mlh_gemm_workspace_bytes() or null; with it, M <= 64 products of matrices
 // with few rows are split along K over workgroups (deterministically reduced).
 // alpha scales the product before the epilogue (the power of two an fp16 weight mirror was scaled by, inverted).
 hipError_t mlh_gemm_tn_epi(hipStream_t stream, int dtype, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                           const float* R, int ldr, int M, int N, int K, void* ws, float alpha = 1.0f);
-// kernels_tile.hip: the same product in 128 x 128 / 64 x 64 tiles (operands half, bf16 or P3), and fp32 -> P3 rows
+                           const float* R, int ldr, int M, int N, int K, void* ws, float alpha = 1.0f, const int* eA = nullptr, const int* eB = nullptr, const int* eC = nullptr);
+// kernels_tile.hip: the same product in 128 x 128 / 64 x 64 tiles (operands half, bf16, P3, or H2 with exponents eA, null: none, and eB; epi 1: of the units, eC), and fp32 -> P3 and H2 rows
 hipError_t mlh_gemm_tile(hipStream_t stream, int dtype, int epi, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
-                         const float* R, int ldr, int M, int N, int K, void* ws, float alpha);
+                         const float* R, int ldr, int M, int N, int K, void* ws, float alpha, const int* eA = nullptr, const int* eB = nullptr, const int* eC = nullptr);
 double mlh_gemm_tile_us(int dtype, int M, int N, int K, int cus, bool ws); // what that product is expected to take
 int mlh_gemm_num_cus(void); // kernels_gemm.hip: compute units of the current device, a multiple of eight; 0: unknown
 hipError_t mlh_split_p3(hipStream_t stream, const float* src, int lds, void* dst, int ldd, int rows, int cols);
+hipError_t mlh_split_h2(hipStream_t stream, bool triples, const float* src, int lds, void* dst, int ldd, const int* colExps, int* exps, int rows, int cols);
 size_t mlh_gemm_workspace_bytes(void);
 extern "C" int mlh_gemm_device_init(int device);
 
@@ -281,7 +287,7 @@ int mlh_init_prefill_kernels(mlh_ctx* c);
 #define MLH_NO_ROOM (-4) // inside a finalize only: a copy does not fit on the device
 int mlh_operand_alloc(mlh_ctx* c, void** p, size_t bytes); // memory of the copies: 0, MLH_NO_ROOM or an error
 void mlh_drop_operands(mlh_ctx* c);
-int mlh_build_gemm_operands(mlh_ctx* c); // at finalize: planes or halves and packed rows of every matrix, where the model's widths, its weights and memory allow
+int mlh_build_gemm_operands(mlh_ctx* c); // at finalize: halves and packed rows of every matrix, where the model's widths, its weights and memory allow
 int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_t* ids, const int32_t* lens, float* allLogits);
 int mlh_launch_softmax_rows(mlh_ctx* c, const float* logits, float* probs, const int* target, float* nll, int rows);
 

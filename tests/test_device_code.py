@@ -62,6 +62,30 @@ def test_stores_have_landed_before_a_counter_says_so(listing):
     assert not bad, f"{len(bad)} counters go up while stores may be on their way, the first: {bad[0]}"
 
 
+def _registers(operand):
+    m = re.match(r"v\[(\d+):(\d+)\]|v(\d+)\b", operand)
+    if not m:
+        return set()
+    return {int(m.group(3))} if m.group(3) else set(range(int(m.group(1)), int(m.group(2)) + 1))
+
+
+def test_no_wide_stores_data_is_overwritten_by_the_next_instruction(listing):
+    """A store of 12 or 16 bytes reads its data after it has been issued.  The compiler keeps an instruction between it and a write of
+    those registers except where a buffer store has a scalar offset, and there lanes have stored the overwritten value."""
+    stores, bad = 0, []
+    for symbol, code in listing.items():
+        for ins, after in zip(code, code[1:]):
+            m = re.match(r"(buffer|global|flat|scratch)_store_dwordx[34] (.*)", ins)
+            if not m:
+                continue
+            stores += 1
+            operands = [o.strip() for o in m.group(2).split(",")]
+            if after.startswith("v_") and _registers(after.split(None, 1)[1]) & _registers(operands[0 if m.group(1) == "buffer" else 1]):
+                bad.append((symbol, ins, after))
+    assert stores > 100
+    assert not bad, f"{len(bad)} stores, the first: {bad[0]}"
+
+
 def test_every_built_form_of_the_decode_of_several_sequences_is_reached(listing):
     """fp32 weights with heads of 64, bf16 with 64 and 128: what the rule for a model lets through, and no kernel beside it."""
     forms = {s[s.index("I") + 1:s.index("EE")] for s in listing if kernel_name(s) == "k_decode_ranks"}
