@@ -370,8 +370,10 @@ static hipError_t launch_tile(hipStream_t stream, int epi, const void* A, int ld
 struct TileCost { int tm, tn, slots; double us[3], split, part; };
 // Variants of the two-byte types: 64 x 64; 128 x 128 with two stages, two workgroups a unit; halves only (what the models multiply): 128 x 128
 // with four stages, for launches that put one on a unit: nothing but its own stages then covers the way of a slice from memory.  777 x 2048 x 5888, K split in two, weights cold
-// (a prefill reads each once): 36.8 us against 48.3 with two stages; on 512 workgroups (3270 rows) 114 against 110.
-static const TileCost kCostHalf[3] = {{64, 64, 3, {0.26, 0.38, 0.58}, 4.0, 0.5}, {128, 128, 2, {0.64, 1.04, 0.0}, 4.0, 0.5}, {128, 128, 1, {0.58, 0.0, 0.0}, 4.0, 0.5}};
+// (a prefill reads each once): 36.8 us against 48.3 with two stages; on 512 workgroups (3270 rows) 114 against 110; and 64 x 64 by two groups of four
+// waves with four stages of two slices, for launches that put one on a unit.  Prefills of 24 layers, weights cold (us): 100 x 6336 x 2048 12.6 (four waves, three stages:
+// 14.9), 300 x 2048 x 2048 12.2 (15.2); whole prefills of 70, 150, 300, 500 tokens 2124 (2318), 2546 (2718), 3122 (3218), 3483 (3647).
+static const TileCost kCostHalf[4] = {{64, 64, 3, {0.26, 0.38, 0.58}, 4.0, 0.5}, {128, 128, 2, {0.64, 1.04, 0.0}, 4.0, 0.5}, {128, 128, 1, {0.58, 0.0, 0.0}, 4.0, 0.5}, {64, 64, 1, {0.22, 0.0, 0.0}, 1.6, 0.1}};
 // Pairs by triples: 64 x 64 by four waves, three stages (60 KB: two workgroups a unit); 128 x 128 by eight, two
 // stages (80 KB, two a unit to the byte; three stages, one a unit: 0.98); 64 x 64 by two groups of four, three stages of two slices, for launches that put one on a
 // unit.  What bounds a slice of 128 x 128: its 40 KB on the way into LDS and the reads behind them
@@ -410,7 +412,7 @@ static double tile_choice(int dtype, int M, int N, int K, int cus, bool ws, Tile
     const TileCost* cost = dtype == MLH_GEMM_P3 ? kCostP3 : dtype == MLH_GEMM_H2 ? kCostH2 : kCostHalf;
     const int slices = K / (dtype == MLH_GEMM_P3 || dtype == MLH_GEMM_H2 ? 32 : 64);
     double best = 0.0;
-    for (int v = 0; v < (dtype == MLH_GEMM_F16 || dtype == MLH_GEMM_H2 ? 3 : 2); v++) {
+    for (int v = 0; v < (dtype == MLH_GEMM_F16 ? 4 : dtype == MLH_GEMM_H2 ? 3 : 2); v++) {
         int ks;
         const double us = best_split(cost[v], M, N, slices, cus, ws, ks);
         if (v == 0 || us < best) { best = us; c.variant = v; c.ks = ks; }
@@ -435,7 +437,7 @@ hipError_t mlh_gemm_tile(hipStream_t stream, int dtype, int epi, const void* A, 
     // 128 x 128 by eight waves, two stages (two workgroups a unit) or, halves, four (one).
     if (dtype == MLH_GEMM_P3) return c.variant == 0 ? TILE(p3_t, 2, 1, 4, 3) : TILE(p3_t, 4, 2, 4, 2);
     if (dtype == MLH_GEMM_H2) return c.variant == 0 ? TILE(h2_t, 2, 2, 2, 3) : c.variant == 1 ? TILE(h2_t, 4, 2, 4, 2) : TILE(h2_t, 2, 2, 2, 3, 2);
-    if (dtype == MLH_GEMM_F16) return c.variant == 0 ? TILE(f16_t, 2, 2, 2, 3) : c.variant == 1 ? TILE(f16_t, 4, 2, 4, 2) : TILE(f16_t, 4, 2, 4, 4);
+    if (dtype == MLH_GEMM_F16) return c.variant == 0 ? TILE(f16_t, 2, 2, 2, 3) : c.variant == 1 ? TILE(f16_t, 4, 2, 4, 2) : c.variant == 2 ? TILE(f16_t, 4, 2, 4, 4) : TILE(f16_t, 2, 2, 2, 4, 2);
     return c.variant == 0 ? TILE(bf16_t, 2, 2, 2, 3) : TILE(bf16_t, 4, 2, 4, 2);
 #undef TILE
 }

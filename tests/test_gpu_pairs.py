@@ -74,3 +74,14 @@ def test_a_row_that_is_not_finite_spoils_that_row_alone(pkg):
     bad = np.zeros(100, bool)
     bad[[17, 40, 99]] = True
     assert not np.isfinite(got[bad]).any() and np.array_equal(got[~bad], want[~bad])
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 64, 64), (70, 66, 192), (90, 2048, 2048), (150, 2048, 5888), (300, 200, 320)])
+def test_halves_in_slices_shared_by_two_groups(pkg, m, n, k):
+    """One slice (the second group has none), an odd number, K splits of unequal parts; products of halves are exact in fp32, so only the accumulation rounds."""
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k)).astype(np.float16).astype(np.float32)
+    b = (rng.standard_normal((n, k)) * 0.02).astype(np.float16).astype(np.float32)
+    want = a.astype(np.float64) @ b.astype(np.float64).T
+    got, _ = pkg.selftest_gemm(a, b, f16=True)
+    assert np.all(np.abs(got - want) <= (k / 16 + 8) * 2.0 ** -23 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T))
