@@ -238,16 +238,17 @@ __global__ void __launch_bounds__(64) k_pf_qk_rope_kv(PfArgs P, LayerDev L) {
 // Causal attention for 16 queries of one head at fp32 precision (inference.cu:136-239, 511-573 for these columns), optional sigmoid gate
 // (:241-250), on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: every product and sum fp32).
 //
-// The four waves of a workgroup take key tiles of 16 in turn, each with an online softmax of its own, and meet once at the end; nothing goes through
+// The four or eight waves of a workgroup take key tiles of 16 in turn, each with an online softmax of its own, and meet once at the end; nothing goes through
 // LDS on the way.  S^T[key, query] = K . Q^T: lane 16 g + n holds a key's (a query's) columns [g HD/4, (g + 1) HD/4), the order of the contraction being
 // free.  The accumulator leaves the lane the scores of keys 4 g .. 4 g + 3 of query n, which is the operand P of O^T += V^T . P^T as it stands; row m of the
 // V operand of block b is dimension m HD/16 + b, so V comes in 16-byte pieces as well.  Loads of the wave's next tile go out before this one's products.
-// Bound by the matrix cores' fp32 rate and, for few rows, by the longest chain of tiles.  Measured: 517 rows, 6 heads of 128: 30 us (107 on the
-// vector ALU through LDS tiles of 64 keys); 17 376 rows of 64 sequences, 12 heads of 64: 178 us (899).
+// Bound by the matrix cores' fp32 rate and, for few rows, by the longest chain of tiles: eight waves where that leaves a unit one workgroup (84 rows, 6 heads
+// of 128: 9.0 us, 11.4 by four; 517: 21.6, 31.4).  Measured: 517 rows 107 us on the vector ALU through LDS tiles of 64 keys; 17 376 rows of 64 sequences,
+// 12 heads of 64: 170 us (899; 178 while the compiler put a tile's loads behind the products they were to run under).
 #define PF_QB 16
-template <int HD, typename AT>
-__global__ void __launch_bounds__(PWG) k_pf_attn(PfArgs P, LayerDev L) {
-    constexpr int NW = PWG / 64, KC = HD / 4, VB = HD / 16, LDO = HD + 4;
+template <int HD, int NW, typename AT>
+__global__ void __launch_bounds__(NW * 64) k_pf_attn(PfArgs P, LayerDev L) {
+    constexpr int KC = HD / 4, VB = HD / 16, LDO = HD + 4;
     __shared__ float part[NW][PF_QB][LDO], stat[NW][2][PF_QB];
     const StepArgs& a = P.a;
     const int h = blockIdx.x, blk = blockIdx.y, tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = lane & 15, g = lane >> 4;
@@ -316,10 +317,12 @@ __global__ void __launch_bounds__(PWG) k_pf_attn(PfArgs P, LayerDev L) {
     if (t < ntiles) fetch(t, 0);
     while (t < ntiles) { // (no further tile: the same loads again, dropped)
         fetch(min(t + NW, ntiles - 1), 1);
+        __builtin_amdgcn_sched_barrier(0); // (the compiler would put the loads behind the products)
         tile(t, 0);
         t += NW;
         if (t >= ntiles) break;
         fetch(min(t + NW, ntiles - 1), 0);
+        __builtin_amdgcn_sched_barrier(0);
         tile(t, 1);
         t += NW;
     }
@@ -339,7 +342,7 @@ __global__ void __launch_bounds__(PWG) k_pf_attn(PfArgs P, LayerDev L) {
                 *reinterpret_cast<f32x4*>(&part[wave][n][(4 * g + i) * VB + b]) = f32x4{acc[b][i], acc[b + 1][i], acc[b + 2][i], acc[b + 3][i]} * f;
     }
     __syncthreads();
-    for (int i = tid; i < nq * (HD / 4); i += PWG) {
+    for (int i = tid; i < nq * (HD / 4); i += NW * 64) {
         const int qi = i / (HD / 4), c4 = (i % (HD / 4)) * 4;
         float M = stat[0][0][qi], den = 0.f;
 #pragma unroll
@@ -1904,18 +1907,23 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
             GEMM(P.Xn, d_, P.exps, L.WaP, L.sWa, L.eWa, d_, P.QKV, P.qkvLd, nullptr, 0, n, L.rowsA, d_);
         }
         if (L.kind == MLH_KIND_ATTENTION) {
+#define ATTN_ROWS(HD_, AT_)                                                                                                    \
+    do {                                                                                                                     \
+        if (hp.attnHeads * nblk <= c->numCUs) hipLaunchKernelGGL((k_pf_attn<HD_, 8, AT_>), dim3(hp.attnHeads, nblk), dim3(512), 0, st, P, L); \
+        else hipLaunchKernelGGL((k_pf_attn<HD_, 4, AT_>), dim3(hp.attnHeads, nblk), dim3(256), 0, st, P, L);                 \
+    } while (0)
             if (hp.headDim == 64) {
                 hipLaunchKernelGGL((k_pf_qk_rope_kv<64>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<64, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<64, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
-                else if (P.half) hipLaunchKernelGGL((k_pf_attn<64, f16_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
-                else hipLaunchKernelGGL((k_pf_attn<64, float>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
+                else if (P.half) ATTN_ROWS(64, f16_t);
+                else ATTN_ROWS(64, float);
             } else {
                 hipLaunchKernelGGL((k_pf_qk_rope_kv<128>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<128, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<128, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
-                else if (P.half) hipLaunchKernelGGL((k_pf_attn<128, f16_t>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
-                else hipLaunchKernelGGL((k_pf_attn<128, float>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
+                else if (P.half) ATTN_ROWS(128, f16_t);
+                else ATTN_ROWS(128, float);
             }
         } else {
             const int skipFrom = gdnChunked ? GD_C : 0x7fffffff;

@@ -109,3 +109,22 @@ def test_bf16_prefill_against_oracle(pkg, orc, kind, n):
     last = rel(dev.logits(0), want[-1])
     assert last < (1e-5 if n < 16 else 2 * np.sqrt(8 * hp.transformers) * 2.0 ** -11 / np.sqrt(3))  # (a single row: up to twice the rms)
     dev.close()
+
+
+@pytest.mark.parametrize("head", [64, 128])
+def test_attention_by_eight_and_by_four_waves(pkg, head):
+    """Up to one workgroup a compute unit eight waves share the keys of 16 queries, beyond it four: either side of the line and lengths of less than a tile
+    per wave, against prefill mode 1."""
+    heads = 512 // head
+    n = 16 * 256 // heads + 1  # at 256 units: the first length beyond it
+    hp = pkg.config(2, dim=512, attnHeads=heads, headDim=head, ffnDim=128, transformers=2, vocabSize=300, maxL=n + 8, maxSeqs=1)
+    dev = pkg.Device(hp, 0)
+    dev.upload(pkg.Model.generate(hp, 5).randomize_gains(5))
+    ids = pkg.random_tokens(9, 0, 300, n)
+    dev.set_prefill_mode(1)
+    want = dev.forward_full(0, ids)[0]
+    dev.set_prefill_mode(0)
+    for m in (2, 17, 66, 130, n - 1, n):
+        dev.reset()
+        assert rel(dev.forward_full(0, ids[:m])[0], want[:m]) < 2e-5
+    dev.close()
