@@ -111,6 +111,25 @@ def test_bf16_prefill_against_oracle(pkg, orc, kind, n):
     dev.close()
 
 
+@pytest.mark.parametrize("vocab", [999, 1024, 8192, 8193, 20480, 20481, 32768, 32770])
+def test_probabilities_of_rows_of_every_length(pkg, vocab):
+    """Probabilities and loss against float64 from the same call's logits.  Bound: a logit's difference and its exponential are right to 2^-23 (1 + |x|) and
+    2^-22, a sum of positive terms to 2^-24 times the longest chain of additions (33 in a thread, 22 across them)."""
+    hp = hybrid(pkg, dim=64, attnHeads=1, ffnDim=96, transformers=2, vocabSize=vocab, gdnHeads=1, maxL=80, maxSeqs=1)
+    dev = pkg.Device(hp, 0)
+    dev.upload(pkg.Model.generate(hp, 5).randomize_gains(5))
+    ids = pkg.random_tokens(7, 0, vocab, 70)
+    logits, probs, nll = dev.forward_full(0, ids)
+    x = logits.astype(np.float64)
+    x -= x.max(axis=1, keepdims=True)
+    want = np.exp(x) / np.exp(x).sum(axis=1, keepdims=True)
+    bound = 2.0 ** -23 * (1 + np.abs(x)) + 2.0 ** -21 + 60 * 2.0 ** -24
+    assert np.all(np.abs(probs - want) <= bound * want + 1e-37)
+    loss = -np.log(np.maximum(want[np.arange(69), ids[1:]], 1e-4)).mean()
+    assert abs(nll - loss) <= 1e-5 * loss
+    dev.close()
+
+
 @pytest.mark.parametrize("head", [64, 128])
 def test_attention_by_eight_and_by_four_waves(pkg, head):
     """Up to one workgroup a compute unit eight waves share the keys of 16 queries, beyond it four: either side of the line and lengths of less than a tile
