@@ -416,7 +416,7 @@ def vendor_gemm(a, b, iters, reps, flop):
 
 def products_leg(m, iters=20):
     """The products of the prefill passes alone, at the row counts of ordinary prompts: us per launch (HIP events, back to
-    back), planes for fp32 models and halves for bf16 ones."""
+    back), pairs by triples for fp32 models and halves for bf16 ones."""
     out = {}
     rng = np.random.default_rng(7)
     for rows in (128, 256, 517, 777, 1024, 2048):
@@ -424,7 +424,7 @@ def products_leg(m, iters=20):
                                   ("half d2048", True, ((6240, 2048), (2048, 2112), (11264, 2048), (2048, 5632)))):
             for n, k in shapes:
                 a, b = rng.standard_normal((rows, k), dtype=np.float32), rng.standard_normal((n, k), dtype=np.float32)
-                us = stats([m.selftest_gemm(a, b, None, f16=f16, iters=iters)[1] for _ in range(3)])["median"]
+                us = stats([m.selftest_gemm(a, b, None, f16=f16, pairs=not f16, iters=iters)[1] for _ in range(3)])["median"]
                 out[f"{what} {rows} x {n} x {k}"] = {"us": round(us, 2), "TFLOPs": round(2e-6 * rows * n * k / us, 1)}
     return out
 

@@ -110,7 +110,7 @@ int mlh_upload_rope_table(mlh_ctx* ctx, const float* tab, int n);
 int mlh_finalize(mlh_ctx* ctx);
 
 /* Device memory: mlh_create allocates the matrices as uploaded (4 or 2 bytes an element).  mlh_finalize adds what the MFMA kernels
- * read, where the widths allow them (mlh_set_prefill_mode): in fp32 10 bytes an element (three bf16 planes; the matrix in
+ * read, where the widths allow them (mlh_set_prefill_mode): in fp32 10 bytes an element (three halves, csrc/h2.h; the matrix in
  * the decode step's order), with bf16 weights 4 (halves; that order), and [output projection | PLE up] once more.  So a context
  * holds its matrices 3.5 times in fp32, 3 times in bf16.  The copies are made only if a prefill call over all
  * maxSeqs * maxL positions (or a sixteenth of the device's memory, if that is less) still has room beside them; without
