@@ -10,8 +10,8 @@
 // inference.cu:401-465, 487-507, 582-602, 624-695 and 723-743 for L > 1 columns.
 //
 // Here: the 256 x 256-tile kernel of the long two-byte products (k_gemm_tn_w4), the weight-streaming kernels for up to
-// 64 rows (k_gemm_skinny*: bf16 models' prompts of 33 to 64 tokens as halves; every type through mlh_gemm_device and the self-test,
-// which alone uses k_gemm_tn_w4 with bf16) and the dispatch; kernels_tile.hip has what lies between, and every longer fp32 product.
+// 64 rows of mlh_gemm_device and the self-test (k_gemm_skinny*; the self-test alone uses k_gemm_tn_w4 with bf16) and the dispatch;
+// kernels_tile.hip has what lies between, every longer fp32 product, and the prefill's of 33 to 64 rows of halves.
 #include <math.h>
 #include <string.h>
 
@@ -859,7 +859,7 @@ hipError_t mlh_gemm_tn_epi(hipStream_t stream, int dtype, int epi, const void* A
     if (M <= 0 || N <= 0 || K <= 0 || ((size_t)K * esz) % GKB != 0 || ((size_t)lda * esz) % 16 != 0 || ((size_t)ldb * esz) % 16 != 0)
         return hipErrorInvalidValue;
     if (epi == GEMM_EPI_SWIGLU && (N & 1)) return hipErrorInvalidValue;
-    // M <= 64 (short prefills of bf16 models, mlh_gemm_device): weight-streaming skinny kernel; more rows: tiles
+    // M <= 64 (mlh_gemm_device, the self-test): weight-streaming skinny kernel; more rows: tiles
 #define GEMM_BY_TYPE(call_f32, call_bf16, call_f16) \
     return dtype == MLH_DTYPE_BF16 ? (call_bf16) : dtype == MLH_GEMM_F16 ? (call_f16) : (call_f32)
     if (M <= 32)

@@ -1928,9 +1928,12 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     RowsArgs base = {};
     base.M = n; base.lay = P.lay; base.normDim = hp.dim;
     const int d_ = hp.dim, F = hp.ffnDim, dt = c->pfDtype;
+    // Up to 64 rows of halves are one row of 64 x 64 tiles: their two groups of waves keep four stages in flight, where a wave of the weight-streaming kernel (what
+    // mlh_gemm_tn_epi takes) has one chunk.  Whole prefills, 24 layers of width 2048, us: 33 rows 2237 -> 1756, 48 2406 -> 1819, 64 2707 -> 2002 (65: 2084).
+    auto* const product = dt == MLH_GEMM_F16 && n <= 64 ? mlh_gemm_tile : mlh_gemm_tn_epi;
 #define GEMM(A, lda, eA, B, alpha, eB, ldb, C, ldc, R, ldr, M, N, K)                                                           \
     do {                                                                                                                     \
-        hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, c->gemmWs, alpha, eA, eB); \
+        hipError_t e_ = product(st, dt, 0, A, lda, B, ldb, C, ldc, R, ldr, M, N, K, c->gemmWs, alpha, eA, eB, nullptr); \
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; } \
     } while (0)
 
@@ -2013,7 +2016,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         PF_DISPATCH_WT(c, launch_rmsnorm<h2_t>(st, P.H1, L.g2, P.Xn, P.exps, n, d_),
                        launch_rmsnorm<f16_t>(st, P.H1, L.g2, P.Xn, nullptr, n, d_));
         { // gate/up projection with SiLU(gate) * up in the epilogue (inference.cu:262-281): U comes out in the GEMM input type
-            hipError_t e_ = mlh_gemm_tn_epi(st, dt, 1, P.Xn, d_, L.W13P, d_, P.U, F, nullptr, 0, n, 2 * F, d_, c->gemmWs, L.sW13, P.exps, L.eW13, L.eU);
+            hipError_t e_ = product(st, dt, 1, P.Xn, d_, L.W13P, d_, P.U, F, nullptr, 0, n, 2 * F, d_, c->gemmWs, L.sW13, P.exps, L.eW13, L.eU);
             if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
         }
         GEMM(P.U, F, nullptr, L.W2P, L.sW2, L.eW2, F, P.X, d_, P.H1, d_, n, d_, F);
@@ -2026,7 +2029,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     } else if (allLogits) {
         PF_DISPATCH_WT(c, launch_rmsnorm<h2_t>(st, P.X, c->gF, P.Xn, P.exps, n, d_),
                        launch_rmsnorm<f16_t>(st, P.X, c->gF, P.Xn, nullptr, n, d_));
-        hipError_t e_ = mlh_gemm_tn_epi(st, dt, 0, P.Xn, d_, c->EP, d_, allLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_, c->gemmWs, c->sE, P.exps, c->eE);
+        hipError_t e_ = product(st, dt, 0, P.Xn, d_, c->EP, d_, allLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_, c->gemmWs, c->sE, P.exps, c->eE, nullptr);
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
     }
     for (int s0 = 0; s0 < nseg; s0 += 64)

@@ -58,3 +58,20 @@ def test_forward_full_against_steps(pkg, bf16, vocab, n):
     assert np.allclose(out[0][1].sum(1), 1, atol=1e-4)
     assert abs(out[0][2] - out[1][2]) < 1e-3
     dev.close()
+
+
+@pytest.mark.parametrize("lens", [[34], [47], [64], [20, 31], [17, 1, 40]])
+def test_tiles_of_33_to_64_halves_against_steps(pkg, lens):
+    """Models of halves multiply 33 to 64 rows as one row of 64 x 64 tiles, K split or not, whose last rows are past the end.  Bound: that of the calls above (three
+    roundings to half, 2^-11, on the way through each of two layers)."""
+    dev = device(pkg, dim=512, attnHeads=8, headDim=64, ffnDim=1472, vocabSize=1000, gdnHeads=8, gdnDk=64, gdnDv=64, pleDim=64, maxSeqs=len(lens), weightDtype=1)
+    rng = np.random.default_rng(sum(lens))
+    ids = [rng.integers(0, 1000, n).astype(np.int32) for n in lens]
+    seqs, out = list(range(len(lens))), []
+    for mode in (1, 0):
+        dev.reset()
+        dev.set_prefill_mode(mode)
+        dev.prefill_batch(seqs, ids)
+        out.append(np.stack([dev.logits(s) for s in seqs]))
+    assert rel(out[1], out[0]) < 3e-3
+    dev.close()
