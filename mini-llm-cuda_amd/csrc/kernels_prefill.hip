@@ -114,6 +114,22 @@ template <typename AT> __device__ __forceinline__ void put_mix4(const PfArgs& P,
     else put4_at<AT>(P.Amix, row, P.aLd, col, v.x, v.y, v.z, v.w);
 }
 
+// PLE columns of `rows` rows from row0 on, e[row][j] = silu(ple gate output) * P[tok][j], behind the mixing output (fp32 models' calls of more rows than the row
+// kernels take: k_pf_pairs).  Workgroups of their own in the launches that mix: a launch for them took 4.4 us a layer, whatever it did.  24 bf16 layers of width
+// 2048, us: 17 rows 1945 -> 1884, 70 2094 -> 2019, 300 3081 -> 3006, 777 4512 -> 4442; 16 384 rows the same.
+template <typename WT, typename AT> __device__ __forceinline__ void ple_columns(const PfArgs& P, const LayerDev& L, int row0, int rows, int tid, int threads) {
+    const int ple = P.a.ple;
+    for (int i = tid; i < rows * ple; i += threads) {
+        const int r = i / ple, j = i - r * ple;
+        const size_t row = (size_t)row0 + r;
+        put_mix<AT>(P, row, L.ad + j, pf_silu(P.QKV[row * P.qkvLd + L.offPle + j]) * getw<WT>((const WT*)L.pleTable + (size_t)P.ids[row] * ple + j));
+    }
+}
+__device__ __forceinline__ void ple_columns(const PfArgs& P, const LayerDev& L, int row0, int rows, int tid, int threads) {
+    if (P.half) ple_columns<bf16_t, f16_t>(P, L, row0, rows, tid, threads);
+    else ple_columns<float, float>(P, L, row0, rows, tid, threads);
+}
+
 // KEEP: 16-byte pieces a lane keeps, rows of up to 256 KEEP elements.  All loads of a row and of the gains go out at once: a load under a comparison, or the
 // gains asked for behind the sum, each add a memory latency.  Measured: 777 rows of 2048 5.4 us (6.3), 517 rows of 768 5.0 us (4.9); 16384 rows of
 // 2048 32 us (37), 6.2 TB/s: part of it comes out of the caches.
@@ -179,6 +195,7 @@ __global__ void __launch_bounds__(64) k_pf_qk_rope_kv(PfArgs P, LayerDev L) {
     constexpr int EPL = HD / 64;
     const StepArgs& a = P.a;
     const int h = blockIdx.x, row = blockIdx.y, lane = threadIdx.x;
+    if (h == a.heads) { ple_columns(P, L, row, 1, lane, 64); return; }
     const int seq = P.rowSeq[row], pos = P.rowPos[row];
     float* qkv = P.QKV + (size_t)row * P.qkvLd;
     float qv[EPL], kv[EPL], vv[EPL];
@@ -671,6 +688,11 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
     const int h = blockIdx.x, seg = blockIdx.y, r0 = blockIdx.z * GR, tid = threadIdx.x, wave = tid >> 6;
     const int seq = P.segSeq[seg], len = P.segLen[seg], row0 = P.segStart[seg];
     if (len >= skipFrom) return; // taken by the chunk-parallel kernels
+    if (h == a.gdnHeads) { // the segment's PLE columns, a share of its rows each
+        const int share = (len + gridDim.z - 1) / gridDim.z, from = min((int)blockIdx.z * share, len);
+        ple_columns(P, L, row0 + from, min(share, len - from), tid, PWG);
+        return;
+    }
     const int r = tid / TPR * RPT, cg = tid % TPR, c0 = cg * CPT;
     float* Srow = L.S + (((size_t)seq * a.gdnHeads + h) * DV + r0 + r) * DK + c0;
     float S[RPT][CPT];
@@ -877,6 +899,7 @@ __global__ void __launch_bounds__(2 * DK, 2) k_gdn_prep(PfArgs P, LayerDev L, co
     const int chunk = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int seg = chunkSeg[chunk], t0 = chunkT0[chunk];
     const int nv = min(GD_C, P.segLen[seg] - t0), row0 = P.segStart[seg] + t0;
+    if (h == a.gdnHeads) { ple_columns(P, L, row0, nv, tid, NT); return; }
     unsigned char* img = ws + ((size_t)chunk * a.gdnHeads + h) * Lay::total;
     float* g = gs; float* beta = gs + GD_C; float* sp = gs + 2 * GD_C; float* rk = gs + 3 * GD_C; float* rq = gs + 4 * GD_C;
     float* part = gs + 5 * GD_C;
@@ -1391,15 +1414,6 @@ __global__ void __launch_bounds__(64, 1) k_gdn_scan16(PfArgs P, LayerDev L, cons
     for (int j = 0; j < JT; j++)
 #pragma unroll
         for (int t = 0; t < 2; t++) *reinterpret_cast<f32x4*>(Srow + 32 * j + 8 * t) = St[j][t];
-}
-
-// e[row][j] = silu(ple gate output) * P[tok][j], appended to the row of the mixing output
-template <typename WT, typename AT>
-__global__ void k_pf_ple(PfArgs P, LayerDev L) {
-    const int row = blockIdx.x, j = threadIdx.x;
-    if (j >= P.a.ple) return;
-    const float g = P.QKV[(size_t)row * P.qkvLd + L.offPle + j];
-    put_mix<AT>(P, (size_t)row, L.ad + j, pf_silu(g) * getw<WT>((const WT*)L.pleTable + (size_t)P.ids[row] * P.a.ple + j));
 }
 
 // fp32 models: the row of mixing output (floats, from several workgroups) and its PLE columns as pairs (h2.h) and the row's exponent, in place: 32
@@ -1937,6 +1951,8 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; } \
     } while (0)
 
+    const int pleWgs = hp.pleDim > 0 && (dt != MLH_GEMM_H2 || rowsPath) ? 1 : 0; // a row's (segment's, chunk's) workgroup for the PLE columns
+
     if (rowsPath) mlh_rows_embed(c, P.ids, n, P.X, P.lay);
     else PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_embed<float>), dim3(cdiv(d_, PWG), n), dim3(PWG), 0, st, P),
                    hipLaunchKernelGGL((k_pf_embed<bf16_t>), dim3(cdiv(d_, PWG), n), dim3(PWG), 0, st, P));
@@ -1958,13 +1974,13 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         else hipLaunchKernelGGL((k_pf_attn<HD_, 4, AT_>), dim3(hp.attnHeads, nblk), dim3(256), 0, st, P, L);                 \
     } while (0)
             if (hp.headDim == 64) {
-                hipLaunchKernelGGL((k_pf_qk_rope_kv<64>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
+                hipLaunchKernelGGL((k_pf_qk_rope_kv<64>), dim3(hp.attnHeads + pleWgs, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<64, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<64, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (P.half) ATTN_ROWS(64, f16_t);
                 else ATTN_ROWS(64, float);
             } else {
-                hipLaunchKernelGGL((k_pf_qk_rope_kv<128>), dim3(hp.attnHeads, n), dim3(64), 0, st, P, L);
+                hipLaunchKernelGGL((k_pf_qk_rope_kv<128>), dim3(hp.attnHeads + pleWgs, n), dim3(64), 0, st, P, L);
                 if (mfmaAttn && P.Kh) hipLaunchKernelGGL((k_pf_attn_mfma<128, true>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (mfmaAttn) hipLaunchKernelGGL((k_pf_attn_mfma<128, false>), dim3(hp.attnHeads, nblk), dim3(PWG), 0, st, P, L);
                 else if (P.half) ATTN_ROWS(128, f16_t);
@@ -1976,7 +1992,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
             // rows): 12 heads x 1 segment 44, 34; x 5 66, 47; x 19 101, 82; x 32 177, 141; x 64 215, 222.
             if (chunked < nseg) { // (a launch whose workgroups all return takes 4.7 us a layer)
                 const bool half = hp.weightDtype == MLH_DTYPE_BF16, few = hp.gdnHeads * nseg <= 2 * c->numCUs;
-#define RECUR(DK_, GR_, AT_) hipLaunchKernelGGL((k_pf_gdn<DK_, GR_, AT_>), dim3(hp.gdnHeads, nseg, DK_ / GR_), dim3(PWG), 0, st, P, L, skipFrom)
+#define RECUR(DK_, GR_, AT_) hipLaunchKernelGGL((k_pf_gdn<DK_, GR_, AT_>), dim3(hp.gdnHeads + pleWgs, nseg, DK_ / GR_), dim3(PWG), 0, st, P, L, skipFrom)
 #define RECUR_ROWS(DK_, AT_) do { if (few) RECUR(DK_, 32, AT_); else RECUR(DK_, 64, AT_); } while (0)
                 if (hp.gdnDk == 64) { if (half) RECUR_ROWS(64, f16_t); else RECUR_ROWS(64, float); }
                 else { if (half) RECUR_ROWS(128, f16_t); else RECUR_ROWS(128, float); }
@@ -1990,11 +2006,11 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
                 const bool narrow = hp.gdnHeads * chunked * (hp.gdnDv / 16) <= 2 * c->numCUs;
 #define SCAN(K_, DK_, W_) hipLaunchKernelGGL((K_<DK_>), dim3(hp.gdnHeads, nseg, DK_ / W_), dim3(64), 0, st, P, L, dcb, (const unsigned char*)c->pfGdnWs, c->pfGdnG)
                 if (hp.gdnDk == 64) {
-                    hipLaunchKernelGGL((k_gdn_prep<64>), dim3(nchunk, hp.gdnHeads), dim3(128), gdn_prep_lds(64), st, P, L, dcs, dct, (unsigned char*)c->pfGdnWs, c->pfGdnG);
+                    hipLaunchKernelGGL((k_gdn_prep<64>), dim3(nchunk, hp.gdnHeads + pleWgs), dim3(128), gdn_prep_lds(64), st, P, L, dcs, dct, (unsigned char*)c->pfGdnWs, c->pfGdnG);
                     if (narrow) SCAN(k_gdn_scan16, 64, 16);
                     else SCAN(k_gdn_scan, 64, 32);
                 } else {
-                    hipLaunchKernelGGL((k_gdn_prep<128>), dim3(nchunk, hp.gdnHeads), dim3(256), gdn_prep_lds(128), st, P, L, dcs, dct, (unsigned char*)c->pfGdnWs, c->pfGdnG);
+                    hipLaunchKernelGGL((k_gdn_prep<128>), dim3(nchunk, hp.gdnHeads + pleWgs), dim3(256), gdn_prep_lds(128), st, P, L, dcs, dct, (unsigned char*)c->pfGdnWs, c->pfGdnG);
                     if (narrow) SCAN(k_gdn_scan16, 128, 16);
                     else SCAN(k_gdn_scan, 128, 32);
 #undef SCAN
@@ -2005,9 +2021,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
             const int cols = L.ad + hp.pleDim;
             if (cols <= 1024) hipLaunchKernelGGL((k_pf_pairs<4>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P, L);
             else hipLaunchKernelGGL((k_pf_pairs<8>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P, L);
-        } else if (hp.pleDim > 0)
-            PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_ple<float, float>), dim3(n), dim3(std::max(64, hp.pleDim)), 0, st, P, L),
-                           hipLaunchKernelGGL((k_pf_ple<bf16_t, f16_t>), dim3(n), dim3(std::max(64, hp.pleDim)), 0, st, P, L));
+        }
         if (rowsPath) {
             mlh_rows_rest_of_layer(c, t, base, P.X, P.H1);
             continue;

@@ -75,3 +75,19 @@ def test_tiles_of_33_to_64_halves_against_steps(pkg, lens):
         out.append(np.stack([dev.logits(s) for s in seqs]))
     assert rel(out[1], out[0]) < 3e-3
     dev.close()
+
+
+@pytest.mark.parametrize("bf16,hd,lens", [(1, 64, [70, 20]), (1, 128, [64, 63, 1]), (1, 64, [150]), (0, 64, [1, 30, 20]), (1, 128, [3, 20])])
+def test_embedding_columns_of_mixed_segments_against_steps(pkg, bf16, hd, lens):
+    """The per-layer embedding's columns come from workgroups beside the heads': chunked segments (64 tokens and more), recurrent ones and the row kernels.  Bounds: as above."""
+    dev = device(pkg, dim=256, attnHeads=256 // hd, headDim=hd, ffnDim=704, vocabSize=1000, gdnHeads=256 // hd, gdnDk=hd, gdnDv=hd, pleDim=128, maxSeqs=len(lens), weightDtype=bf16)
+    rng = np.random.default_rng(sum(lens))
+    ids = [rng.integers(0, 1000, n).astype(np.int32) for n in lens]
+    seqs, out = list(range(len(lens))), []
+    for mode in (1, 0):
+        dev.reset()
+        dev.set_prefill_mode(mode)
+        dev.prefill_batch(seqs, ids)
+        out.append(np.stack([dev.logits(s) for s in seqs]))
+    assert rel(out[1], out[0]) < (3e-3 if bf16 else 1e-5)
+    dev.close()
