@@ -42,12 +42,11 @@
 
 #include "mlh_internal.h"
 #include "rows_mul.h"
+#include "wide_places.h"
 #include "xcd_exchange.h"
 
-#define WD_WAVES 8
 #define WD_THREADS (WD_WAVES * 64)
 #define WD_GRID (RK_XCDS * RK_PER)
-#define WD_CA 3          // chunks of 32 columns a wave has of a product over the whole width: dim <= 768
 #define WD_HD 64
 #define WD_BR 16         // keys of a block: four loads of a wave each for K and V
 
@@ -135,7 +134,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) k_decode_wide(WideArgs P) {
     {
         group = r / TS; block0 = r % TS * MW;                       // tiles TS group .., blocks block0 ..
         fin = wave - (WD_WAVES - MB);
-        cnt = (nch - wave + WD_WAVES - 1) / WD_WAVES;                 // chunks wave, wave + 8, ... of a product over the whole width
+        cnt = wd_count(wave, nch);                                    // chunks wave, wave + 8, ... of a product over the whole width
         slot2 = wave >> 2; part2 = wave & 3;                        // output and down projection: tile r, or a share of the blocks of a later one; chunks part2, part2 + 4
         tile2 = slot2 ? min(RK_PER + r / share, dt - 1) : r;
         const int from1 = MB * (r % share) / share;
@@ -205,7 +204,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) k_decode_wide(WideArgs P) {
     // ---- weights ----
     typedef RowsW<float> Wt;
     Wt w1[TS][WD_CA], w2[2];
-    // (a wave with fewer chunks multiplies its matrix's last operands by zeros)
+    // (a wave with fewer chunks multiplies its own last operands once more, by zeros)
     const unsigned char* zeros = P.xw + P.oZero;
     auto chunk = [&](Wt& w, const void* m, size_t index, bool real) __attribute__((always_inline)) {
         w.load((real ? (const unsigned char*)m + index * 2048 : zeros) + (unsigned)lane * 16u);
@@ -251,23 +250,19 @@ __global__ void __launch_bounds__(WD_THREADS, 2) k_decode_wide(WideArgs P) {
         for (int i = 0; i < 2; i++) chunk(w2[i], L->W2R, (size_t)tile2 * (RK_XCDS * k) + X * k + part2 + 4 * i, part2 + 4 * i < k);
     };
 
-    // Where the flags lie that this lane reads: of the pieces of residual planes, of the mixing output (a chunk's two units for 64 sequences, or
-    // the PLE columns' blocks; past the last chunk, or without a sequence in it, the PLE's or the first head's) and of the FFN units.
+    // Where the flags lie that this lane reads (wide_places.h): of the pieces of residual planes, of the mixing output (a chunk's two units for 64
+    // sequences, or the PLE columns' blocks) and of the FFN units.
     unsigned flag1, flagM[4], flagU;
     {
-        const int i = min(lane, max(cnt, 1) * 2 * MW - 1), c = i / (2 * MW), j = i - c * 2 * MW;
-        flag1 = (unsigned)(((wave + WD_WAVES * c) * 2 + j / MW) * MB + block0 + j % MW) * 4u;
+        flag1 = (unsigned)wd_flag1(lane, wave, cnt, MB, MW, block0) * 4u;
 #pragma unroll
         for (int k = 0; k < 2; k++) {
-            int c2 = min(part2 + 4 * k, ko - 1);
-            if (c2 >= 2 && c2 < nh * 2 && lo >= hi) c2 -= 2;
-            const int hl = c2 >> 1, from = hl ? lo : 0, to = hl ? hi : n;
+            const int c2 = wd_mix_chunk(part2, k, ko, nh, lo >= hi), hl = c2 >> 1;
             const bool ple = c2 >= nh * 2;
-            flagM[2 * k] = ple ? P.fE + (unsigned)min(lane, MB - 1) * 4u : P.fM + (unsigned)((hl * 4 + (c2 & 1) * 2) * 64 + min(from + lane, to - 1)) * 4u;
+            flagM[2 * k] = ple ? P.fE + (unsigned)min(lane, MB - 1) * 4u : P.fM + (unsigned)wd_flagM(lane, c2, hl ? lo : 0, hl ? hi : n) * 4u;
             flagM[2 * k + 1] = flagM[2 * k] + (ple ? 0u : 256u);
         }
-        const int ku = fs / 32, iu = min(lane, 8 * MB - 1), cu = min(part2 + 4 * (iu / (4 * MB)), ku - 1);
-        flagU = (unsigned)(cu * 4 * MB + iu % (4 * MB)) * 4u;
+        flagU = (unsigned)wd_flagU(lane, part2, fs / 32, MB) * 4u;
         asm volatile("" : "+v"(flag1), "+v"(flagM[0]), "+v"(flagM[1]), "+v"(flagM[2]), "+v"(flagM[3]), "+v"(flagU));
     }
 
@@ -293,13 +288,13 @@ __global__ void __launch_bounds__(WD_THREADS, 2) k_decode_wide(WideArgs P) {
         float s[2 * WD_CA];
 #pragma unroll
         for (int k = 0; k < WD_CA; k++) {
-            const unsigned at = own + ssq + (unsigned)min(wave + WD_WAVES * k, nch - 1) * 512u + (unsigned)block0 * 64u;
+            const unsigned at = own + ssq + (unsigned)wd_chunk(wave, k, cnt) * 512u + (unsigned)block0 * 64u;
             s[2 * k] = loadF((unsigned)min(lane, MW * 16 - 1) * 4u, at);
             s[2 * k + 1] = loadF((unsigned)min(lane, MW * 16 - 1) * 4u, at + 256u);
         }
         u32x4 av[NA][1][3][MW] = {};
 #pragma unroll
-        for (int k = 0; k < NA; k++) operand(av[k], min(wave + WD_WAVES * k, nch - 1), block0, planes);
+        for (int k = 0; k < NA; k++) operand(av[k], wd_chunk(wave, k, cnt), block0, planes);
         f32x4 acc[TS][MW];
 #pragma unroll
         for (int t = 0; t < TS; t++)
@@ -310,7 +305,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) k_decode_wide(WideArgs P) {
 #pragma unroll
             for (int t = 0; t < TS; t++) times(w1[t][k], av[k % NA], acc[t]);
             __builtin_amdgcn_sched_barrier(0);
-            if (k + NA < WD_CA) operand(av[k % NA], min(wave + WD_WAVES * (k + NA), nch - 1), block0, planes);
+            if (k + NA < WD_CA) operand(av[k % NA], wd_chunk(wave, k + NA, cnt), block0, planes);
             if (k == 0) { // (the last operands are on their way)
                 asm volatile("" ::: "memory");
                 behind();
@@ -339,7 +334,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) k_decode_wide(WideArgs P) {
         constexpr int N = decltype(blocks)::value;
         u32x4 av[2][1][3][N] = {};
 #pragma unroll
-        for (int i = 0; i < 2; i++) operand(av[i], min(part2 + 4 * i, k - 1), b0, planes);
+        for (int i = 0; i < 2; i++) operand(av[i], wd_part(part2, i, k), b0, planes);
         asm volatile("" ::: "memory");
         behind();
         f32x4 acc[N];
@@ -347,7 +342,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) k_decode_wide(WideArgs P) {
         for (int mb = 0; mb < N; mb++) acc[mb] = (f32x4)(0.f);
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            const int c = min(part2 + 4 * i, k - 1);
+            const int c = wd_part(part2, i, k);
             if (mixed) { // sequences of the second head that another XCD has
                 const bool some = c >= 2 && c < nh * 2;
 #pragma unroll

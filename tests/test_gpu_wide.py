@@ -130,3 +130,27 @@ def test_batches_of_changing_size_share_the_exchange_memory(pkg, orc):
         assert dev.seq_len(s) == len(hist[s])
         dec.close()
     dev.close()
+
+
+@pytest.mark.parametrize("heads,ffn", [(8, 2048), (8, 1280), (10, 2048), (10, 1280)])
+def test_widths_whose_waves_have_fewer_chunks(pkg, orc, heads, ffn):
+    """Widths 512 and 640, where waves have two chunks of a product and not three, over borders of token blocks in both directions: what a launch of another
+    size has left in the exchange memory (fp32 sums where this one has planes) is multiplied nowhere."""
+    hp = config(pkg, heads=heads, hd=64, ffn=ffn, layers=2, vocab=600, ple=64, maxSeqs=64, maxL=96)
+    dev, w, prompts = start(pkg, orc, hp, 64, 2, 24, 97)
+    hist = [list(p) for p in prompts]
+    nxt = [dev.greedy_token(s) for s in range(64)]
+    for n in (20, 10, 40, 10, 64, 20, 48, 6, 33):
+        out = dev.decode_loop(nxt[:n], 2)
+        for s in range(n):
+            hist[s] += [nxt[s], int(out[0, s])]
+            nxt[s] = int(out[1, s])
+            assert np.isfinite(dev.logits(s)).all(), f"{n} sequences, sequence {s}"
+    assert dev.persistent_fallbacks() == 0
+    for s in range(0, 64, 3):
+        dec = orc.Decoder(w, "f64")
+        for t in hist[s]:
+            _, lg = dec.step(int(t))
+        assert_logits_close(dev.logits(s), lg, RTOL, f"sequence {s}")
+        dec.close()
+    dev.close()
