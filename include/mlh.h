@@ -110,7 +110,7 @@ int mlh_upload_rope_table(mlh_ctx* ctx, const float* tab, int n);
 int mlh_finalize(mlh_ctx* ctx);
 
 /* Device memory: mlh_create allocates the matrices as uploaded (4 or 2 bytes an element).  mlh_finalize adds what the MFMA kernels
- * read, where the widths allow them (mlh_set_prefill_mode): in fp32 10 bytes an element (three halves, csrc/h2.h; the matrix in
+ * read, where the widths allow them (mlh_set_prefill_mode): in fp32 10 bytes an element (three halves or bf16 planes, csrc/h2.h, p3.h; the matrix in
  * the decode step's order), with bf16 weights 4 (halves; that order), and [output projection | PLE up] once more.  So a context
  * holds its matrices 3.5 times in fp32, 3 times in bf16.  The copies are made only if a prefill call over all
  * maxSeqs * maxL positions (or a sixteenth of the device's memory, if that is less) still has room beside them; without
@@ -164,6 +164,13 @@ int mlh_forward_full(mlh_ctx* ctx, int seq, const int32_t* ids, int n, float* lo
  * pleDim and the mixing widths are multiples of 32 (fp32) / 64 (bf16), and in decode steps of up to 64 sequences;
  * 1: always token by token, and decode steps through the GEMV kernels. */
 int mlh_set_prefill_mode(mlh_ctx* ctx, int mode);
+/* What multiplies in a prefill call of `tokens` tokens as the context stands: the decode step's kernels token by token, the row kernels (fp32
+ * precision), tiles of halves (bf16 models), or, in fp32 models, pairs of scaled halves by triples (csrc/h2.h), or three bf16 planes (csrc/p3.h) where
+ * mlh_finalize finds the model's weights, gains or tables to spread further than halves reach (rows of weights with a typical
+ * element 2^12 below their largest, rows of activations, as far as that follows from the model, 2^8).  -1: not finalized, or no tokens.  (No counterpart in the
+ * reference, which has one path.) */
+enum { MLH_PREFILL_BY_TOKEN = 0, MLH_PREFILL_ROWS = 1, MLH_PREFILL_HALVES = 2, MLH_PREFILL_PAIRS = 3, MLH_PREFILL_PLANES = 4 };
+int mlh_prefill_route(const mlh_ctx* ctx, int tokens);
 
 /* One greedy decode step for sequences 0..nseq-1: feeds last_ids[s] at each
  * sequence's current position, appends it, returns argmax of the logits

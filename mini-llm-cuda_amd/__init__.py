@@ -22,6 +22,7 @@ MAX_LAYERS = 64
 
 KIND_ATTENTION, KIND_GDN = 0, 1
 DTYPE_F32, DTYPE_BF16 = 0, 1
+PREFILL_BY_TOKEN, PREFILL_ROWS, PREFILL_HALVES, PREFILL_PAIRS, PREFILL_PLANES = range(5)  # Device.prefill_route
 
 # tensor ids (include/mlh.h)
 (T_TOKEN_EMBEDDINGS, T_FINAL_RMS_GAMMA, T_RMS_GAMMA, T_QUERY, T_KEY, T_VALUE, T_OUTPUT_PROJ, T_RMS_GAMMA2,
@@ -99,6 +100,7 @@ _sigs_dev = {
     "mlh_debug_inject_abort_at_step": (c_int, [c_void_p, c_int]),
     "mlh_debug_set_xcd_tag": (c_int, [c_void_p, ctypes.c_uint]),
     "mlh_xcd_decode_supported": (c_int, [c_void_p]),
+    "mlh_prefill_route": (c_int, [c_void_p, c_int]),
     "mlh_single_launch_sequences": (c_int, [c_void_p]),
     "mlh_synchronize": (c_int, [c_void_p]),
     "mlh_time_kernel": (c_int, [c_void_p, c_int, c_int, c_int, c_int, _P(c_double), _P(c_double)]),
@@ -335,6 +337,10 @@ class Device:
 
     def set_prefill_mode(self, mode):
         self._check(dev.mlh_set_prefill_mode(self._h, int(mode)))
+
+    def prefill_route(self, tokens):
+        """What multiplies in a prefill call of that many tokens: one of PREFILL_BY_TOKEN .. PREFILL_PLANES."""
+        return dev.mlh_prefill_route(self._h, int(tokens))
 
     def decode_step(self, last_ids):
         a = np.ascontiguousarray(last_ids, dtype=np.int32)

@@ -1,7 +1,7 @@
 // Prefill: many tokens of one or more sequences through the stack at once.
 //
 // Rows of the activation matrices are tokens (all segments concatenated); the projections are MFMA
-// GEMMs (kernels_gemm.hip, kernels_tile.hip) against copies of the weights as halves, or, in short calls, the row
+// GEMMs (kernels_gemm.hip, kernels_tile.hip) against copies of the weights as halves or planes, or, in short calls, the row
 // kernels of the decode step (kernels_rows.hip); per layer
 //
 //   rmsnorm rows -> GEMM Wa -> attention: per-head QK-norm + RoPE + KV-page write, tiled causal attention
@@ -12,9 +12,11 @@
 // and at the end the LM head runs for the last row of every segment only (the reference computes
 // logits for all L columns, inference.cu:723-743, and uses the last one).  With bf16 weights the GEMM
 // inputs (normed activations, mixing output, FFN activations) are rounded to half; with fp32 weights they are
-// stored as two halves, the weights as three that add up to the scaled fp32 value (h2.h).  Accumulation, the
+// stored as two halves, the weights as three (h2.h), or, where a model's weights spread further than halves reach
+// (operand_spread), both as three bf16 planes that add up to the fp32 value (p3.h).  Accumulation, the
 // residual stream, K/V and GDN states stay fp32.  This is what runInference(L) (inference.cu:376-751)
 // does for L columns, minus the columns that are already in the cache.
+#include <math.h>
 #include <string.h>
 
 #include <algorithm>
@@ -42,11 +44,11 @@ struct PfArgs {
     const int* blkSeg; // attention query blocks: segment and first query of the block
     const int* blkQ0;
     float* X;          // [n, dim] residual stream
-    void* Xn;          // [n, dim] GEMM input (fp32 models: pairs of halves, h2.h; else halves)
+    void* Xn;          // [n, dim] GEMM input (fp32 models: pairs of halves, h2.h, or planes, p3.h; else halves); planes: that of the output projection too, [n, aLd]
     int* exps;         // exponents of pairs' rows
     float* QKV;        // [n, qkvLd]
     int qkvLd;
-    void* Amix;        // [n, aLd] GEMM input of the output projection: mixing output, then (at column L.ad) the PLE row (fp32 models: floats first)
+    void* Amix;        // [n, aLd] GEMM input of the output projection: mixing output, then (at column L.ad) the PLE row (fp32 models: floats, then pairs in place)
     int aLd;
     float* H1;         // [n, dim]
     void* U;           // [n, ffn]
@@ -108,6 +110,7 @@ template <> __device__ __forceinline__ void put4<f16_t>(f16_t* o, float a, float
 template <> __device__ __forceinline__ void put4<float>(float* o, float a, float b, float c, float d) { *reinterpret_cast<f32x4*>(o) = f32x4{a, b, c, d}; }
 
 template <typename AT> __device__ __forceinline__ void put4_at(void* base, size_t row, int ld, int col, float a, float b, float c, float d) { put4<AT>((AT*)base + row * ld + col, a, b, c, d); }
+template <> __device__ __forceinline__ void put4_at<p3_t>(void* base, size_t row, int ld, int col, float a, float b, float c, float d) { p3_put4((unsigned char*)base + row * ld * 6, col, a, b, c, d); }
 // Four columns of the mixing output.
 template <typename AT> __device__ __forceinline__ void put_mix4(const PfArgs& P, size_t row, int col, const f32x4& v) {
     if (P.rows) rows_put4(P.rows, col, (int)row, P.lay, P.half != 0, v.x, v.y, v.z, v.w);
@@ -115,7 +118,7 @@ template <typename AT> __device__ __forceinline__ void put_mix4(const PfArgs& P,
 }
 
 // PLE columns of `rows` rows from row0 on, e[row][j] = silu(ple gate output) * P[tok][j], behind the mixing output (fp32 models' calls of more rows than the row
-// kernels take: k_pf_pairs).  Workgroups of their own in the launches that mix: a launch for them took 4.4 us a layer, whatever it did.  24 bf16 layers of width
+// kernels take: k_pf_operand_rows).  Workgroups of their own in the launches that mix: a launch for them took 4.4 us a layer, whatever it did.  24 bf16 layers of width
 // 2048, us: 17 rows 1945 -> 1884, 70 2094 -> 2019, 300 3081 -> 3006, 777 4512 -> 4442; 16 384 rows the same.
 template <typename WT, typename AT> __device__ __forceinline__ void ple_columns(const PfArgs& P, const LayerDev& L, int row0, int rows, int tid, int threads) {
     const int ple = P.a.ple;
@@ -1417,10 +1420,10 @@ __global__ void __launch_bounds__(64, 1) k_gdn_scan16(PfArgs P, LayerDev L, cons
 }
 
 // fp32 models: the row of mixing output (floats, from several workgroups) and its PLE columns as pairs (h2.h) and the row's exponent, in place: 32
-// columns take 128 bytes either way, and a block's eight lanes read it in an instruction before the one that writes it.  A wave a row; up to 256 KEEP
-// columns stay in registers between the maximum and the split.
-template <int KEEP>
-__global__ void __launch_bounds__(PWG) k_pf_pairs(PfArgs P, LayerDev L) {
+// columns take 128 bytes either way, and a block's eight lanes read it in an instruction before the one that writes it; or as planes (p3.h), to Xn.  A wave a
+// row; up to 256 KEEP columns stay in registers between the maximum and the split.
+template <typename T, int KEEP>
+__global__ void __launch_bounds__(PWG) k_pf_operand_rows(PfArgs P, LayerDev L) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, cols = L.ad + P.a.ple;
     if (row >= P.n) return;
     float* x = (float*)P.Amix + (size_t)row * P.aLd;
@@ -1431,6 +1434,13 @@ __global__ void __launch_bounds__(PWG) k_pf_pairs(PfArgs P, LayerDev L) {
         const int j = i - L.ad;
         return f32x4{pf_silu(gate[j]) * table[j], pf_silu(gate[j + 1]) * table[j + 1], pf_silu(gate[j + 2]) * table[j + 2], pf_silu(gate[j + 3]) * table[j + 3]};
     };
+    if constexpr (__is_same(T, p3_t)) {
+        for (int i = lane * 4; i < cols; i += 256) {
+            const f32x4 v = value(i);
+            put4_at<p3_t>(P.Xn, (size_t)row, P.aLd, i, v.x, v.y, v.z, v.w);
+        }
+        return;
+    }
     f32x4 keep[KEEP];
     int most = -100000;
 #pragma unroll
@@ -1707,7 +1717,162 @@ static int operand_values(mlh_ctx* c, bool* within) {
     return 0;
 }
 
-// An fp32 matrix as triples of halves, what the tiled products of the prefill multiply.
+// Whether scaled halves reach over an fp32 model's operands.  A row of halves ends 2^-40 below its largest element (h2.h), where floats and planes end
+// at 2^-126: elements far below the largest are kept in fewer bits, and where the large ones meet zeros the sum is made of those.  So
+//   - a row of weights has its typical element (mean of the exponents, zeros apart) within 2^12 of its largest: with its columns' scales in W2, whose
+//     columns the units' exponents go into;
+//   - the rows that are multiplied have theirs within 2^8, as far as that follows from the model: residual columns (E's columns, rows of [Wo | pleUp] and W2, each
+//     about its own mean) with the gain in front of a product; value rows and PLE columns (gate row and table) beside each other;
+//   - an FFN unit, whose scale comes from its bound, is dim below that on rows without a direction; on rows as uneven as the residual columns at most 2^6 more.
+// What ends at 2^-40 is then 2^-24 or less of what is typical in all of them.
+// Models beyond multiply planes.  Random and trained weights have 3 to 6 in all of them.  Exponents and integer sums: the answer is the same at every finalize.
+#define SPREAD_WEIGHTS 12
+#define SPREAD_ROWS 8
+#define SPREAD_UNITS 6
+#define SPREAD_NONE (-100000)
+// the exponents of rows of [W | U] with those of the columns: the largest of each row to rowMost, and the largest distance of one from its row's mean to worst
+__global__ void __launch_bounds__(PWG) k_spread_rows(const float* __restrict__ W, int cols, const float* __restrict__ U, int cols2, const int* __restrict__ colExps, int* rowMost, int* worst, int rows) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    int most = SPREAD_NONE, sum = 0, count = 0;
+    for (int i = lane; i < cols + cols2; i += 64) {
+        const float x = i < cols ? W[(size_t)row * cols + i] : U[(size_t)row * cols2 + i - cols];
+        if (x == 0.f) continue;
+        const int e = h2_size(x) + (colExps ? colExps[i] : 0);
+        most = max(most, e); sum += e; count++;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) { most = max(most, __shfl_xor(most, o, 64)); sum += __shfl_xor(sum, o, 64); count += __shfl_xor(count, o, 64); }
+    if (lane) return;
+    if (rowMost) rowMost[row] = most;
+    if (count) atomicMax(worst, most - (int)floorf((float)sum / (float)count));
+}
+// ... the largest of each column to colMost (x: columns, y: strips of rows)
+__global__ void __launch_bounds__(PWG) k_spread_cols(const float* __restrict__ W, int rows, int cols, int* colMost) {
+    const int col = blockIdx.x * PWG + threadIdx.x, strip = (rows + gridDim.y - 1) / gridDim.y, end = min(rows, (int)(blockIdx.y + 1) * strip);
+    if (col >= cols) return;
+    int most = SPREAD_NONE;
+    for (int r = blockIdx.y * strip; r < end; r++) most = max(most, h2_size(W[(size_t)r * cols + col]));
+    atomicMax(colMost + col, most);
+}
+// ... and how far a unit's bound lies above dim times its size on rows of elements `like`, of mean square 1 (a power of two, the largest to worst)
+__global__ void __launch_bounds__(PWG) k_spread_units(const float* __restrict__ W13, const float* __restrict__ gain, const float* __restrict__ like, int* worst, int units, int d) {
+    const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (j >= units) return;
+    const float *g = W13 + (size_t)2 * j * d, *u = g + d;
+    double s[4] = {};
+    for (int i = lane; i < d; i += 64) {
+        const double a = (double)g[i] * gain[i], b = (double)u[i] * gain[i], x = like[i];
+        s[0] += a * a; s[1] += b * b; s[2] += a * a * x * x; s[3] += b * b * x * x;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int k = 0; k < 4; k++) s[k] += __shfl_xor(s[k], o, 64);
+    if (lane || s[0] == 0.0 || s[1] == 0.0) return; // (a unit that is always 0)
+    const double size = sqrt(s[2]) * sqrt(s[3]);
+    atomicMax(worst, size > 0.0 ? __builtin_amdgcn_frexp_exp(sqrt(s[0]) * sqrt(s[1]) / size) : -SPREAD_NONE);
+}
+static int spread_mean(const int* v, int n) { // rounded down; of the elements there are
+    long sum = 0, count = 0;
+    for (int i = 0; i < n; i++)
+        if (v[i] > SPREAD_NONE / 2) { sum += v[i]; count++; }
+    return count ? (int)floor((double)sum / (double)count) : SPREAD_NONE;
+}
+static bool spread_even(const std::vector<int>& v) {
+    const int mean = spread_mean(v.data(), (int)v.size());
+    return mean == SPREAD_NONE || *std::max_element(v.begin(), v.end()) - mean <= SPREAD_ROWS;
+}
+static int operand_spread(mlh_ctx* c, bool* within) {
+    const mlh_hparams& hp = c->hp;
+    const int d = hp.dim, F = hp.ffnDim, p = hp.pleDim, V = hp.vocabSize, n = (int)c->layers.size(), per = c->maxRowsA + p + 2 * d;
+    // ints: the worst row, E's columns, units; a layer's rows of Wa, table columns, rows of [Wo | pleUp] and W2
+    const size_t ints = 1 + 2 * (size_t)d + F + (size_t)n * per; // (at the end floats: a row like the residual's)
+    int* dev = nullptr;
+    std::vector<int> h(ints);
+    std::vector<float> gains((size_t)(2 * n + 1) * d);
+    MLH_CHECK(c, hipMalloc((void**)&dev, ints * 4));
+    hipError_t e = hipMemsetAsync(dev, 0x80, ints * 4, c->stream); // (far below SPREAD_NONE)
+    int *const worst = dev, *const colE = dev + 1, *const units = colE + d, *const first = units + F;
+    float* const like = (float*)(first + (size_t)n * per);
+    auto rows = [&](const void* W, int cols, const void* U, int cols2, const int* colExps, int* most, int count) {
+        hipLaunchKernelGGL(k_spread_rows, dim3(cdiv(count, 4)), dim3(PWG), 0, c->stream, (const float*)W, cols, (const float*)U, cols2, colExps, most, worst, count);
+    };
+    auto cols = [&](const void* W, int count, int width, int* most) { hipLaunchKernelGGL(k_spread_cols, dim3(cdiv(width, PWG), 64), dim3(PWG), 0, c->stream, (const float*)W, count, width, most); };
+    rows(c->E, d, nullptr, 0, nullptr, nullptr, V);
+    cols(c->E, V, d, colE);
+    for (int t = 0; t < n; t++) {
+        const LayerDev& L = c->layers[t];
+        int *a = first + (size_t)t * per, *table = a + c->maxRowsA, *o = table + p, *w2 = o + d;
+        rows(L.Wa, d, nullptr, 0, nullptr, a, L.rowsA);
+        rows(L.Wo, L.ad, L.pleUp, p, nullptr, o, d);
+        rows(L.W13, d, nullptr, 0, nullptr, nullptr, 2 * F);
+        hipLaunchKernelGGL(k_unit_exps, dim3(cdiv(F, 4)), dim3(PWG), 0, c->stream, (const float*)L.W13, L.g2, units, F, d);
+        rows(L.W2, F, nullptr, 0, units, w2, d);
+        if (p) { rows(L.pleTable, p, nullptr, 0, nullptr, nullptr, V); cols(L.pleTable, V, p, table); }
+        if (e == hipSuccess) e = hipMemcpyAsync(gains.data() + (size_t)2 * t * d, L.g1, (size_t)d * 4, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(gains.data() + (size_t)(2 * t + 1) * d, L.g2, (size_t)d * 4, hipMemcpyDeviceToHost, c->stream);
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(gains.data() + (size_t)2 * n * d, c->gF, (size_t)d * 4, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(h.data(), dev, ints * 4, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    bool ok = h[0] <= SPREAD_WEIGHTS;
+    std::vector<int> resid(d, SPREAD_NONE); // how far a residual column may lie above the others
+    auto contributes = [&](const int* v) {
+        const int mean = spread_mean(v, d);
+        for (int j = 0; j < d; j++)
+            if (v[j] > SPREAD_NONE / 2) resid[j] = std::max(resid[j], v[j] - mean);
+    };
+    contributes(h.data() + 1);
+    for (int t = 0; t < n; t++) {
+        const LayerDev& L = c->layers[t];
+        const int *a = h.data() + (first - dev) + (size_t)t * per, *table = a + c->maxRowsA, *o = table + p, *w2 = o + d;
+        contributes(o);
+        contributes(w2);
+        std::vector<int> mix(a + L.offV, a + L.offV + L.ad);
+        for (int j = 0; j < p; j++) mix.push_back(a[L.offPle + j] > SPREAD_NONE / 2 && table[j] > SPREAD_NONE / 2 ? a[L.offPle + j] + table[j] : SPREAD_NONE);
+        ok = ok && spread_even(mix);
+    }
+    for (int g = 0; g < 2 * n + 1; g++) {
+        std::vector<int> x(d, SPREAD_NONE);
+        for (int j = 0; j < d; j++) {
+            const float v = gains[(size_t)g * d + j];
+            int ex = 0;
+            (void)frexpf(v, &ex);
+            if (v != 0.f && resid[j] > SPREAD_NONE / 2) x[j] = ex + resid[j];
+        }
+        ok = ok && spread_even(x);
+    }
+    if (e == hipSuccess && ok) {
+        const int most = *std::max_element(resid.begin(), resid.end());
+        std::vector<float> row(d);
+        double ss = 0.0;
+        for (int j = 0; j < d; j++) { const double x = resid[j] > SPREAD_NONE / 2 ? ldexp(1.0, resid[j] - most) : 0.0; row[j] = (float)x; ss += x * x; }
+        for (float& x : row) x = ss > 0.0 ? (float)(x / sqrt(ss / d)) : 1.f;
+        e = hipMemcpyAsync(like, row.data(), (size_t)d * 4, hipMemcpyHostToDevice, c->stream);
+        if (e == hipSuccess) e = hipMemsetAsync(worst, 0, 4, c->stream);
+        for (const LayerDev& L : c->layers) hipLaunchKernelGGL(k_spread_units, dim3(cdiv(F, 4)), dim3(PWG), 0, c->stream, (const float*)L.W13, L.g2, (const float*)like, worst, F, d);
+        if (e == hipSuccess) e = hipGetLastError();
+        if (e == hipSuccess) e = hipMemcpyAsync(h.data(), worst, 4, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        ok = h[0] <= SPREAD_UNITS;
+    }
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipFree(dev);
+    MLH_CHECK(c, e);
+    *within = ok;
+    return 0;
+}
+
+// An fp32 matrix as three bf16 planes or as triples of halves, what the tiled products of the prefill multiply.
+static int build_planes(mlh_ctx* c, const void* src, int rows, int cols, const void** dst) {
+    void* buf = nullptr;
+    if (const int rc = mlh_operand_alloc(c, &buf, (size_t)rows * cols * 6)) return rc;
+    MLH_CHECK(c, mlh_split_p3(c->stream, (const float*)src, cols, buf, cols, rows, cols));
+    *dst = buf;
+    return 0;
+}
 static int build_triples(mlh_ctx* c, const void* src, int rows, int cols, const int* colExps, const void** dst, const int** exps) {
     void *buf = nullptr, *e = nullptr;
     int rc;
@@ -1726,11 +1891,15 @@ static size_t gdn_chunk_bytes(const mlh_ctx* c) {
         if (L.kind == MLH_KIND_GDN) return (size_t)hp.gdnHeads * ((hp.gdnDk == 64 ? GdLayout<64>::total : GdLayout<128>::total) + 4);
     return 0;
 }
+// Elements of the products' inputs: halves, pairs of them or planes; of the mixing output, which becomes planes in Xn; columns of Xn.
+static size_t input_bytes(const mlh_ctx* c) { return c->hp.weightDtype == MLH_DTYPE_BF16 ? 2 : c->pfDtype == MLH_GEMM_P3 ? 6 : 4; }
+static size_t mix_bytes(const mlh_ctx* c) { return std::min<size_t>(input_bytes(c), 4); }
+static size_t xn_cols(const mlh_ctx* c) { return c->pfDtype == MLH_GEMM_P3 ? std::max(c->hp.dim, c->maxAd + c->hp.pleDim) : c->hp.dim; }
 // Work buffers of a prefill call: per row, and of the chunks that segments of 64 rows or more are cut into (ensure_prefill_buffers).
 static size_t prefill_row_bytes(const mlh_ctx* c) {
     const mlh_hparams& hp = c->hp;
-    const size_t wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 4, d = hp.dim;
-    return d * (8 + wb + (wb == 2 ? 4 : 0)) + (size_t)c->maxRowsA * 4 + ((size_t)c->maxAd + hp.pleDim + hp.ffnDim) * wb + 68;
+    const size_t wb = input_bytes(c), d = hp.dim;
+    return d * (8 + (wb == 2 ? 4 : 0)) + xn_cols(c) * wb + (size_t)c->maxRowsA * 4 + ((size_t)c->maxAd + hp.pleDim) * mix_bytes(c) + hp.ffnDim * wb + 68;
 }
 // ... of one over every position of the context, with the products' split-K workspace.
 size_t mlh_prefill_work_bytes(const mlh_ctx* c) {
@@ -1766,7 +1935,7 @@ void mlh_drop_operands(mlh_ctx* c) {
     c->eE = nullptr;
 }
 
-// The halves; on MLH_NO_ROOM what has been allocated so far is still there.
+// The halves or planes; on MLH_NO_ROOM what has been allocated so far is still there.
 static int build_operands(mlh_ctx* c, unsigned* d_scratch) {
     const mlh_hparams& hp = c->hp;
     const bool mirror = hp.weightDtype == MLH_DTYPE_BF16;
@@ -1789,6 +1958,10 @@ static int build_operands(mlh_ctx* c, unsigned* d_scratch) {
                 (rc = build_mirror(c, L.W13, 2 * F * d, &L.W13P, &L.sW13, d_scratch)) ||
                 (rc = build_mirror(c, L.W2, d * F, &L.W2P, &L.sW2, d_scratch)))
                 return rc;
+        } else if (c->pfDtype == MLH_GEMM_P3) {
+            if ((rc = build_planes(c, L.Wa, L.rowsA, (int)d, &L.WaP)) || (rc = build_planes(c, wo, (int)d, L.ad + (int)pl, &L.WoP)) ||
+                (rc = build_planes(c, L.W13, 2 * (int)F, (int)d, &L.W13P)) || (rc = build_planes(c, L.W2, (int)d, (int)F, &L.W2P)))
+                return rc;
         } else {
             void* units = nullptr;
             if ((rc = mlh_operand_alloc(c, &units, F * 4))) return rc;
@@ -1801,7 +1974,14 @@ static int build_operands(mlh_ctx* c, unsigned* d_scratch) {
         }
     }
     c->sE = 1.0f;
-    return mirror ? build_mirror(c, c->E, (size_t)hp.vocabSize * hp.dim, &c->EP, &c->sE, d_scratch) : build_triples(c, c->E, hp.vocabSize, hp.dim, nullptr, &c->EP, &c->eE);
+    return mirror ? build_mirror(c, c->E, (size_t)hp.vocabSize * hp.dim, &c->EP, &c->sE, d_scratch) :
+           c->pfDtype == MLH_GEMM_P3 ? build_planes(c, c->E, hp.vocabSize, hp.dim, &c->EP) : build_triples(c, c->E, hp.vocabSize, hp.dim, nullptr, &c->EP, &c->eE);
+}
+
+static void drop_prefill_buffers(mlh_ctx* c) { // (hipFree waits for the device)
+    for (void* p : c->pfAllocs) (void)hipFree(p);
+    c->pfAllocs.clear();
+    c->pfRows = 0;
 }
 
 int mlh_build_gemm_operands(mlh_ctx* c) {
@@ -1809,9 +1989,13 @@ int mlh_build_gemm_operands(mlh_ctx* c) {
     c->f16Inexact = 0;
     if (!operand_widths(c)) return 0;
     int rc = 0;
-    bool ok = false;
-    if ((rc = operand_values(c, &ok)) || !ok || (rc = operand_room(c, &ok)) || !ok) return rc;
-    c->pfDtype = c->hp.weightDtype == MLH_DTYPE_BF16 ? MLH_GEMM_F16 : MLH_GEMM_H2;
+    bool ok = false, halves = true;
+    if ((rc = operand_values(c, &ok)) || !ok) return rc;
+    if (c->wbytes == 4 && (rc = operand_spread(c, &halves))) return rc;
+    const int form = c->wbytes == 2 ? MLH_GEMM_F16 : halves ? MLH_GEMM_H2 : MLH_GEMM_P3;
+    if (form != c->pfDtype) drop_prefill_buffers(c); // (their rows' size follows from it)
+    c->pfDtype = form;
+    if ((rc = operand_room(c, &ok)) || !ok) return rc;
     unsigned* d_scratch = nullptr;
     MLH_CHECK(c, hipMalloc((void**)&d_scratch, 8));
     rc = build_operands(c, d_scratch);
@@ -1835,10 +2019,8 @@ static int ensure_prefill_buffers(mlh_ctx* c, int rows) {
     if (rows <= c->pfRows) return 0;
     const mlh_hparams& hp = c->hp;
     (void)hipStreamSynchronize(c->stream);
-    for (void* p : c->pfAllocs) (void)hipFree(p);
-    c->pfAllocs.clear();
-    c->pfRows = 0;
-    const size_t n = (size_t)rows, wb = hp.weightDtype == MLH_DTYPE_BF16 ? 2 : 4; // GEMM input elements: halves, or pairs of them
+    drop_prefill_buffers(c);
+    const size_t n = (size_t)rows, wb = input_bytes(c);
     auto alloc = [&](void** p, size_t bytes) -> int {
         MLH_CHECK(c, hipMalloc(p, std::max<size_t>(bytes, 16)));
         c->pfAllocs.push_back(*p);
@@ -1847,8 +2029,8 @@ static int ensure_prefill_buffers(mlh_ctx* c, int rows) {
     int rc;
     const size_t nblk = cdiv(rows, PF_QB) + hp.maxSeqs, nchunk = cdiv(rows, GD_C) + hp.maxSeqs;
     const size_t meta = 3 * n + 5 * (size_t)hp.maxSeqs + 2 * nblk + 2 * nchunk; // ids, sequence and position of every row; segments; attention blocks; GDN chunks
-    if ((rc = alloc((void**)&c->pfX, n * hp.dim * 4)) || (rc = alloc(&c->pfXn, n * hp.dim * wb)) ||
-        (rc = alloc((void**)&c->pfQKV, n * c->maxRowsA * 4)) || (rc = alloc(&c->pfA, n * (c->maxAd + hp.pleDim) * wb)) ||
+    if ((rc = alloc((void**)&c->pfX, n * hp.dim * 4)) || (rc = alloc(&c->pfXn, n * xn_cols(c) * wb)) ||
+        (rc = alloc((void**)&c->pfQKV, n * c->maxRowsA * 4)) || (rc = alloc(&c->pfA, n * (c->maxAd + hp.pleDim) * mix_bytes(c))) ||
         (rc = alloc((void**)&c->pfH1, n * hp.dim * 4)) || (rc = alloc((void**)&c->pfExp, n * 4)) ||
         (rc = alloc(&c->pfU, n * hp.ffnDim * wb)) ||
         (hp.weightDtype == MLH_DTYPE_BF16 && ((rc = alloc((void**)&c->pfKh, n * hp.dim * 2)) || (rc = alloc((void**)&c->pfVh, n * hp.dim * 2)))) ||
@@ -1878,6 +2060,7 @@ static int ensure_gemm_workspace(mlh_ctx* c) {
 // 16 / 32 / 48 tokens 1511 / 2155 / 3767 -- 1953 / 2255 / 2723: three plane products against one of halves.
 #define MLH_ROWS_PREFILL_F32 64
 #define MLH_ROWS_PREFILL_BF16 32
+bool mlh_prefill_by_rows(const mlh_ctx* c, int tokens) { return tokens <= (c->hp.weightDtype == MLH_DTYPE_F32 ? MLH_ROWS_PREFILL_F32 : MLH_ROWS_PREFILL_BF16); }
 
 // Appends lens[s] tokens to sequence seqs[s] for every segment s (token ids concatenated in `ids`).
 // allLogits: null, or a device buffer [rows, vocab] that receives the logits of every position.
@@ -1888,7 +2071,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     int rc = ensure_prefill_buffers(c, n);
     if (rc == 0) rc = ensure_gemm_workspace(c);
     if (rc) return rc;
-    const bool rowsPath = n <= (hp.weightDtype == MLH_DTYPE_F32 ? MLH_ROWS_PREFILL_F32 : MLH_ROWS_PREFILL_BF16);
+    const bool rowsPath = mlh_prefill_by_rows(c, n);
     // ---- metadata: laid out in pinned memory as on the device, one copy ----
     // bf16 models: fp16 MFMA attention, 128 queries per workgroup; below 16 tokens as precise as the token-by-token path
     const bool mfmaAttn = hp.weightDtype == MLH_DTYPE_BF16 && n >= MLH_PREFILL_GEMM_MIN_ROWS;
@@ -1951,7 +2134,13 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; } \
     } while (0)
 
-    const int pleWgs = hp.pleDim > 0 && (dt != MLH_GEMM_H2 || rowsPath) ? 1 : 0; // a row's (segment's, chunk's) workgroup for the PLE columns
+#define NORM(X_, gain_)                                                                                                        \
+    do {                                                                                                                     \
+        if (dt == MLH_GEMM_F16) launch_rmsnorm<f16_t>(st, X_, gain_, P.Xn, nullptr, n, d_);                                   \
+        else if (dt == MLH_GEMM_P3) launch_rmsnorm<p3_t>(st, X_, gain_, P.Xn, nullptr, n, d_);                                \
+        else launch_rmsnorm<h2_t>(st, X_, gain_, P.Xn, P.exps, n, d_);                                                        \
+    } while (0)
+    const int pleWgs = hp.pleDim > 0 && (P.half || rowsPath) ? 1 : 0; // a row's (segment's, chunk's) workgroup for the PLE columns
 
     if (rowsPath) mlh_rows_embed(c, P.ids, n, P.X, P.lay);
     else PF_DISPATCH_WT(c, hipLaunchKernelGGL((k_pf_embed<float>), dim3(cdiv(d_, PWG), n), dim3(PWG), 0, st, P),
@@ -1963,8 +2152,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
             R.K = d_; R.A = c->rowsX; R.ssqIn = c->rowsSsqX; R.nparts = t == hp.transformers - 1 ? 1 : d_ / RW_TILE; R.C = P.QKV; R.ldc = P.qkvLd;
             mlh_rows_gemm(c, RW_PLAIN, L.WaR, L.rowsA, R);
         } else {
-            PF_DISPATCH_WT(c, launch_rmsnorm<h2_t>(st, P.X, L.g1, P.Xn, P.exps, n, d_),
-                           launch_rmsnorm<f16_t>(st, P.X, L.g1, P.Xn, nullptr, n, d_));
+            NORM(P.X, L.g1);
             GEMM(P.Xn, d_, P.exps, L.WaP, L.sWa, L.eWa, d_, P.QKV, P.qkvLd, nullptr, 0, n, L.rowsA, d_);
         }
         if (L.kind == MLH_KIND_ATTENTION) {
@@ -2017,18 +2205,18 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
                 }
             }
         }
-        if (dt == MLH_GEMM_H2 && !rowsPath) {
+        if (!P.half && !rowsPath) {
             const int cols = L.ad + hp.pleDim;
-            if (cols <= 1024) hipLaunchKernelGGL((k_pf_pairs<4>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P, L);
-            else hipLaunchKernelGGL((k_pf_pairs<8>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P, L);
+            if (dt == MLH_GEMM_P3) hipLaunchKernelGGL((k_pf_operand_rows<p3_t, 1>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P, L);
+            else if (cols <= 1024) hipLaunchKernelGGL((k_pf_operand_rows<h2_t, 4>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P, L);
+            else hipLaunchKernelGGL((k_pf_operand_rows<h2_t, 8>), dim3(cdiv(n, 4)), dim3(PWG), 0, st, P, L);
         }
         if (rowsPath) {
             mlh_rows_rest_of_layer(c, t, base, P.X, P.H1);
             continue;
         }
-        GEMM(P.Amix, P.aLd, P.exps, L.WoP, L.sWo, L.eWo, L.ad + hp.pleDim, P.H1, d_, P.X, d_, n, d_, L.ad + hp.pleDim); // Wo . a + pleUp . e + x
-        PF_DISPATCH_WT(c, launch_rmsnorm<h2_t>(st, P.H1, L.g2, P.Xn, P.exps, n, d_),
-                       launch_rmsnorm<f16_t>(st, P.H1, L.g2, P.Xn, nullptr, n, d_));
+        GEMM(dt == MLH_GEMM_P3 ? P.Xn : P.Amix, P.aLd, P.exps, L.WoP, L.sWo, L.eWo, L.ad + hp.pleDim, P.H1, d_, P.X, d_, n, d_, L.ad + hp.pleDim); // Wo . a + pleUp . e + x
+        NORM(P.H1, L.g2);
         { // gate/up projection with SiLU(gate) * up in the epilogue (inference.cu:262-281): U comes out in the GEMM input type
             hipError_t e_ = product(st, dt, 1, P.Xn, d_, L.W13P, d_, P.U, F, nullptr, 0, n, 2 * F, d_, c->gemmWs, L.sW13, P.exps, L.eW13, L.eU);
             if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
@@ -2041,8 +2229,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
         R.K = d_; R.A = c->rowsX; R.ssqIn = c->rowsSsqX; R.nparts = d_ / RW_TILE; R.C = allLogits; R.ldc = hp.vocabSize;
         mlh_rows_gemm(c, RW_PLAIN, c->ER, hp.vocabSize, R);
     } else if (allLogits) {
-        PF_DISPATCH_WT(c, launch_rmsnorm<h2_t>(st, P.X, c->gF, P.Xn, P.exps, n, d_),
-                       launch_rmsnorm<f16_t>(st, P.X, c->gF, P.Xn, nullptr, n, d_));
+        NORM(P.X, c->gF);
         hipError_t e_ = product(st, dt, 0, P.Xn, d_, c->EP, d_, allLogits, hp.vocabSize, nullptr, 0, n, hp.vocabSize, d_, c->gemmWs, c->sE, P.exps, c->eE, nullptr);
         if (e_ != hipSuccess) { c->err = std::string("prefill GEMM: ") + hipGetErrorString(e_); return -2; }
     }

@@ -656,6 +656,13 @@ extern "C" int mlh_set_prefill_mode(mlh_ctx* c, int mode) {
     return 0;
 }
 
+extern "C" int mlh_prefill_route(const mlh_ctx* c, int tokens) {
+    if (!c || !c->finalized || tokens < 1) return -1;
+    if (c->prefillMode != 0 || tokens == 1 || !mlh_prefill_gemm_supported(c)) return MLH_PREFILL_BY_TOKEN;
+    if (mlh_prefill_by_rows(c, tokens)) return MLH_PREFILL_ROWS;
+    return c->pfDtype == MLH_GEMM_F16 ? MLH_PREFILL_HALVES : c->pfDtype == MLH_GEMM_P3 ? MLH_PREFILL_PLANES : MLH_PREFILL_PAIRS;
+}
+
 // Captures `k` consecutive decode steps into one executable graph (slot 0: one step, slot 1: graphSteps steps).
 static int ensure_graph(mlh_ctx* c, int slot, int nseq, int k) {
     if (c->graphExec[slot] && c->graphNseqOf[slot] == nseq && c->graphStepsOf[slot] == k) return 0;

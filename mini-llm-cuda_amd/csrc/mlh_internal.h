@@ -18,7 +18,7 @@ typedef uint16_t bf16_t;
 // IEEE half, as the MFMA path stores weights and activations of bf16 models (see MLH_GEMM_F16)
 struct f16_t { uint16_t bits; };
 #define MLH_GEMM_F16 2 // GEMM operand type code beside MLH_DTYPE_F32 / MLH_DTYPE_BF16
-#define MLH_GEMM_P3 3  // ... and for fp32 operands stored as three bf16 planes (p3.h; the GEMM self-test)
+#define MLH_GEMM_P3 3  // ... and for fp32 operands stored as three bf16 planes (p3.h; models that spread further than halves reach)
 #define MLH_GEMM_H2 4  // ... and fp32 as halves, pairs times triples, with an exponent per row (h2.h)
 #define MLH_GEMM_WS_COUNTERS 1024 // tile counters at the head of a split-K workspace ...
 #define MLH_GEMM_WS_PARTIALS (256 * 8 * 2 * 16 * 64) // ... and the partial sums (floats) behind them
@@ -64,12 +64,12 @@ struct LayerDev {
     int kind;
     int rowsA, offK, offV, offG, offPle, offGa, offGb;
     int ad;               // width of the mixing output fed to Wo
-    // What the prefill's products multiply: fp32 matrices as triples of halves (h2.h); for bf16 models IEEE-half
+    // What the prefill's products multiply: fp32 matrices as triples of halves (h2.h) or as planes (p3.h); for bf16 models IEEE-half
     // mirrors scaled by a power of two (exact), with the inverse scale applied to the product.
     // WoP is [dim, ad + pleDim]: Wo with pleUp appended along K, so that h1 = [a | e] . WoP^T is one product.
     const void *WaP, *WoP, *W13P, *W2P;
     float sWa, sWo, sW13, sW2;
-    const int *eWa, *eWo, *eW13, *eW2; // fp32: exponents of their rows ...
+    const int *eWa, *eWo, *eW13, *eW2; // triples: exponents of their rows ...
     const int* eU;                     // ... and of the FFN units
     const void *WaR, *WoR, *W13R, *W2R; // for the row step: the matrices ([Wo | pleUp] as one) in its fetch order (rows.h)
 };
@@ -208,7 +208,7 @@ struct mlh_ctx {
     std::vector<void*> pfAllocs;
     float *pfX = nullptr, *pfQKV = nullptr, *pfH1 = nullptr;
     void *pfXn = nullptr, *pfA = nullptr, *pfU = nullptr;
-    int* pfExp = nullptr; // fp32: exponents of the rows of the product input at hand
+    int* pfExp = nullptr; // exponents of the rows of the product input at hand
     uint16_t *pfKh = nullptr, *pfVh = nullptr; // half copies of a call's K and V rows for the MFMA attention of a fresh prefill
     int* pfMeta = nullptr;
     void* pfGdnWs = nullptr;   // chunk operands of the chunk-parallel GDN prefill
@@ -218,7 +218,7 @@ struct mlh_ctx {
     float sE = 1.0f;
     const int* eE = nullptr;
     const void* ER = nullptr;  // ... and in the row step's fetch order
-    int pfDtype = MLH_DTYPE_F32; // operand type of those: MLH_GEMM_H2 or MLH_GEMM_F16
+    int pfDtype = MLH_DTYPE_F32; // operand type of those: MLH_GEMM_H2, MLH_GEMM_P3 or MLH_GEMM_F16
     bool operands = false;     // the copies of the matrices that the MFMA kernels read (LayerDev::WaP .. W2R) exist
     std::vector<void*> mirrorAllocs;
     size_t operandBytes = 0, operandLimit = SIZE_MAX; // what they take and may take
@@ -283,6 +283,7 @@ void mlh_set_thread_error(const std::string& msg);
 #define MLH_PREFILL_GEMM_MIN_ROWS 16 // bf16 models: calls of fewer tokens keep fp32 activations throughout
 size_t mlh_prefill_work_bytes(const mlh_ctx* c);
 bool mlh_prefill_gemm_supported(const mlh_ctx* c);
+bool mlh_prefill_by_rows(const mlh_ctx* c, int tokens); // through the row kernels
 int mlh_init_prefill_kernels(mlh_ctx* c);
 #define MLH_NO_ROOM (-4) // inside a finalize only: a copy does not fit on the device
 int mlh_operand_alloc(mlh_ctx* c, void** p, size_t bytes); // memory of the copies: 0, MLH_NO_ROOM or an error
