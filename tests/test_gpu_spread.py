@@ -50,11 +50,10 @@ def gains(octaves):
 
 
 def column(pkg, model, hp):
-    """A residual column 2^10 above the others that no product but the residual's own reads."""
+    """A residual column 2^9 above the others, from the embeddings on, that no product but the residual's own reads."""
+    model.tensor(0, pkg.T_TOKEN_EMBEDDINGS)[:, 3] = 20.0
     model.tensor(0, pkg.T_FINAL_RMS_GAMMA).reshape(-1)[3] = 0
     for layer in range(hp.transformers):
-        for tid in (pkg.T_OUTPUT_PROJ, pkg.T_FFN_2, pkg.T_PLE_UP):
-            model.tensor(layer, tid)[3] *= 2.0 ** 10
         for tid in (pkg.T_QUERY, pkg.T_KEY, pkg.T_VALUE, pkg.T_PLE_GATE, pkg.T_GDN_ALPHA_W, pkg.T_GDN_BETA_W, pkg.T_FFN_1A, pkg.T_FFN_1B):
             if model.tensor(layer, tid) is not None:
                 model.tensor(layer, tid)[:, 3] = 0
