@@ -1914,9 +1914,10 @@ static int operand_room(mlh_ctx* c, bool* fits) {
     const mlh_hparams& hp = c->hp;
     const size_t d = hp.dim, F = hp.ffnDim, pl = hp.pleDim, wb = c->wbytes, per = wb == 4 ? 10 : 4;
     auto rows16 = [](size_t n) { return (n + 15) / 16 * 16; };
-    size_t need = rows16(hp.vocabSize) * d * per;
+    const size_t exps = c->pfDtype == MLH_GEMM_H2 ? 4 : 0; // of every row, and of the FFN units
+    size_t need = rows16(hp.vocabSize) * d * per + hp.vocabSize * exps;
     for (const LayerDev& L : c->layers)
-        need += (rows16(L.rowsA) * d + rows16(d) * (L.ad + pl) + rows16(2 * F) * d + rows16(d) * F) * per + (pl ? d * (L.ad + pl) * wb : 0);
+        need += (rows16(L.rowsA) * d + rows16(d) * (L.ad + pl) + rows16(2 * F) * d + rows16(d) * F) * per + (pl ? d * (L.ad + pl) * wb : 0) + (L.rowsA + 2 * d + 3 * F) * exps;
     size_t free = 0, total = 0;
     MLH_CHECK(c, hipMemGetInfo(&free, &total));
     const size_t have = c->pfRows * prefill_row_bytes(c) + c->pfGdnChunks * gdn_chunk_bytes(c) + (c->gemmWs ? mlh_gemm_workspace_bytes() : 0); // (of earlier calls)

@@ -110,3 +110,18 @@ def test_room_for_a_prefill_over_every_position(pkg, bf16):
     took = before - torch.cuda.mem_get_info()[0]
     assert abs(took - dev.prefill_bytes()) <= 0.02 * took + (24 << 20), (took, dev.prefill_bytes())
     dev.close()
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+def test_a_limit_just_below_the_copies(pkg, bf16):
+    """What the copies take never exceeds the limit, their rows' exponents included (widths of whole tiles: no padding in between)."""
+    hp = pkg.config(3, dim=512, attnHeads=8, headDim=64, ffnDim=1024, transformers=2, vocabSize=1024, gdnHeads=8, pleDim=64, maxL=100, maxSeqs=2, weightDtype=bf16)
+    pkg.set_layer_pattern(hp, 1)
+    dev = pkg.Device(hp, 0)
+    dev.upload(pkg.Model.generate(hp, 5))
+    full = dev.operand_bytes()
+    for limit in (full - 1, full - 4096):
+        dev.limit_operands(limit)
+        dev.finalize()
+        assert dev.operand_bytes() <= limit
+    dev.close()
