@@ -12,7 +12,7 @@ typedef __amdgpu_buffer_rsrc_t rsrc_t;
 #define RK_LEFT 0x10000u                      // in the word that counts them: somebody has gone
 #define RK_LDS (160 * 1024)
 
-enum { LD_XCD = 2, LD_CROSS = 16, ST_XCD = 0, ST_CROSS = 16 }; // cache policy of exchange loads and stores: nt stays out of the L1, sc1 goes past the L2
+enum { LD_XCD = 2, LD_CROSS = 16, ST_XCD = 0, ST_CROSS = 16 }; // cache policy of exchange loads and stores: nt leaves no line in the L1 (measured, not promised: words with tags, that are loaded until they are new), sc1 goes past the L2
 
 __device__ __forceinline__ int runi(int v) { return __builtin_amdgcn_readfirstlane(v); }
 // The layer table is read by scalar loads where it is used.

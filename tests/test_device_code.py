@@ -105,3 +105,13 @@ def test_scaled_queries_are_rounded_once(listing, hd):
     assert len(code) == 2
     for c in code:
         assert sum(bool(re.match(r"v_(fma|mad)_mix(lo|hi)_f16", ins)) for ins in c) >= hd // 2
+
+
+def test_untagged_operands_are_read_past_the_l1(listing):
+    """k_decode_wide reads planes and partial sums that other workgroups of the XCD have stored, behind flags and without tags of their own.  Each of the five
+    products that does (first phase, output projection, gate / up, down projection, LM head) drops the compute unit's L1 lines once its flags are there."""
+    forms = {s: code for s, code in listing.items() if kernel_name(s) == "k_decode_wide"}
+    assert len(forms) == 4
+    for symbol, code in forms.items():
+        drops = [i for i, ins in enumerate(code) if ins.startswith("buffer_inv sc0") and "sc1" not in ins]
+        assert len(drops) >= 5, (symbol, len(drops))
