@@ -17,7 +17,9 @@
 //   gate / up     -> planes of silu(gate) up                                                     (planes in the XCD)
 //   down proj., residual                                                                       (as above)
 // Weights, and the mixing's states, are issued one product ahead, behind the operand loads of the product before: loads return in order on this
-// ISA, so a poll behind them would be answered late, and by the time of the next poll they have come.  (A ninth wave that brought them
+// ISA, so a poll behind them would be answered late, and by the time of the next poll they have come.  The down projection's go out in front of the poll for
+// gate / up, which waits for other workgroups anyway: behind its operands, in the waves that store nothing, a step took 1 to 3 % more (us, 6 / 16 / 48 / 64
+// sequences: 253, 262, 430, 474 in front; 257, 265, 433, 488 behind).  (A ninth wave that brought them
 // into the L2 instead met the others too late at the barriers: 480 us a step of 19 sequences, not 346; weights issued before the wait for
 // other XCDs slow that exchange down, 5.1 us for 3.3.)  64 sequences: a workgroup has two tiles and half the tokens of a product over the whole
 // width, which loads 240 KB and not 340.
@@ -183,7 +185,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) k_decode_wide(WideArgs P) {
     constexpr std::integral_constant<int, LD_XCD> InXcd = {};
     // Behind the flags of what other workgroups have stored: nothing of it is taken from the compute unit's L1, whatever was loaded before.  (Values with tags
     // show what is old, planes and sums do not, and that a non-temporal load leaves no line behind is nothing the instruction set promises.  A launch takes what it took
-    // without: 16 sequences 266 and 265 us a step, 32 326 and 328, 64 490 and 488.)
+    // without: 16 sequences 266 and 265 us a step, 32 326 and 328, 64 479 and 476.)
     auto past_l1 = [&]() __attribute__((always_inline)) { asm volatile("buffer_inv sc0" ::: "memory"); };
     auto flag = [&](auto pol, unsigned off, unsigned base, unsigned tag, bool mine) __attribute__((always_inline)) { // behind this wave's stores
         stores_landed();
@@ -724,12 +726,10 @@ __global__ void __launch_bounds__(WD_THREADS, 2) k_decode_wide(WideArgs P) {
             const f32x4 g2 = gain_of(L->g2);
             publish2(P.oHP, lt);
             residual(P.oHP, lt, g2, P.oH, P.oSH, P.fH, lt);
-            if (fin >= 0) issueW2(L); // (behind the product's operands its stores would wait for these)
-            issueW2(L);
+            issueW2(L); // in front of the poll: behind the product's operands its stores would wait for these
             // ---------------------------------------------------------------- gate / up of the XCD's FFN units (inference.cu:612-672)
             forget();
-            if (group * TS < fs / 8) product1(0, P.oH, P.oSH, true, P.fH, lt, [&]() __attribute__((always_inline)) { if (fin < 0) issueW2(L); });
-            else if (fin < 0) issueW2(L);
+            if (group * TS < fs / 8) product1(0, P.oH, P.oSH, true, P.fH, lt, [&]() {});
             lds_barrier();
             if (fin >= 0) {
                 const int tile = group * TS + fin / MW, block = block0 + fin % MW;
