@@ -263,6 +263,12 @@ int mlh_xcd_decode_supported(mlh_ctx* ctx);
 /* The largest nseq whose decode calls run as a single launch in mode 3 for every covered model (0: none; 16 at most: fp32 models may go on to 64,
  * see mlh_set_persistent; no counterpart in the reference). */
 int mlh_single_launch_sequences(mlh_ctx* ctx);
+/* What a decode call of sequences 0 .. nseq - 1 runs as the context stands (mode, sampling, graph replays, kernels that have given up): launches of the
+ * GEMV kernels or of the row kernels, or one launch for all steps of the barrier kernel, of the XCD-rank kernel (one sequence), or of one of the two kernels of several
+ * sequences (few rows, many rows).  -1: not finalized, or nseq out of range.  (No counterpart in the reference: its decode loop is one
+ * kernel sequence, inference_orchestrator.cu:120-165.) */
+enum { MLH_DECODE_GEMV = 0, MLH_DECODE_ROWS = 1, MLH_DECODE_BARRIER = 2, MLH_DECODE_XCD = 3, MLH_DECODE_RANKS = 4, MLH_DECODE_WIDE = 5 };
+int mlh_decode_route(const mlh_ctx* ctx, int nseq);
 
 int mlh_synchronize(mlh_ctx* ctx);
 

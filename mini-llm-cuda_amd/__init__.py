@@ -24,6 +24,8 @@ KIND_ATTENTION, KIND_GDN = 0, 1
 DTYPE_F32, DTYPE_BF16 = 0, 1
 PREFILL_BY_TOKEN, PREFILL_ROWS, PREFILL_HALVES, PREFILL_PAIRS, PREFILL_PLANES = range(5)  # Device.prefill_route
 
+DECODE_GEMV, DECODE_ROWS, DECODE_BARRIER, DECODE_XCD, DECODE_RANKS, DECODE_WIDE = range(6)  # Device.decode_route
+
 # tensor ids (include/mlh.h)
 (T_TOKEN_EMBEDDINGS, T_FINAL_RMS_GAMMA, T_RMS_GAMMA, T_QUERY, T_KEY, T_VALUE, T_OUTPUT_PROJ, T_RMS_GAMMA2,
  T_FFN_1A, T_FFN_1B, T_FFN_2, T_QUERY_RMS_GAMMA, T_KEY_RMS_GAMMA, T_GATED_QUERY, T_GDN_ALPHA_W, T_GDN_ALPHA_B,
@@ -100,6 +102,7 @@ _sigs_dev = {
     "mlh_debug_inject_abort_at_step": (c_int, [c_void_p, c_int]),
     "mlh_debug_set_xcd_tag": (c_int, [c_void_p, ctypes.c_uint]),
     "mlh_xcd_decode_supported": (c_int, [c_void_p]),
+    "mlh_decode_route": (c_int, [c_void_p, c_int]),
     "mlh_prefill_route": (c_int, [c_void_p, c_int]),
     "mlh_single_launch_sequences": (c_int, [c_void_p]),
     "mlh_synchronize": (c_int, [c_void_p]),
@@ -341,6 +344,10 @@ class Device:
     def prefill_route(self, tokens):
         """What multiplies in a prefill call of that many tokens: one of PREFILL_BY_TOKEN .. PREFILL_PLANES."""
         return dev.mlh_prefill_route(self._h, int(tokens))
+
+    def decode_route(self, nseq):
+        """What a decode call of that many sequences runs: one of DECODE_GEMV .. DECODE_WIDE."""
+        return dev.mlh_decode_route(self._h, int(nseq))
 
     def decode_step(self, last_ids):
         a = np.ascontiguousarray(last_ids, dtype=np.int32)

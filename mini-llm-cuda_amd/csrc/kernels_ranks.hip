@@ -1236,9 +1236,9 @@ static bool ranks_shape(const mlh_ctx* c) { return ranks_model(c) && mlh_rows_ap
 // From how many sequences on kernels_wide.hip takes them.  Measured, us per step, here and there (hybrid, fp32, d 768, 12 layers): 2 sequences
 // 224 and 250, 5 241 and 253, 6 269 and 256, 7 275 and 257, 8 273 and 258, 12 327 and 263, 16 339 and 267.
 #define WIDE_FROM 6
-static bool use_wide(const mlh_ctx* c, int nseq) { return nseq >= WIDE_FROM && c->wideMax >= nseq; }
+bool mlh_ranks_wide(const mlh_ctx* c, int nseq) { return nseq >= WIDE_FROM && c->wideMax >= nseq; }
 
-bool mlh_ranks_applicable(const mlh_ctx* c, int nseq) { return (use_wide(c, nseq) || c->ranksMax >= nseq) && mlh_rows_applicable(c, nseq); }
+bool mlh_ranks_applicable(const mlh_ctx* c, int nseq) { return (mlh_ranks_wide(c, nseq) || c->ranksMax >= nseq) && mlh_rows_applicable(c, nseq); }
 
 template <typename WT, int HD>
 static int ranks_launch(mlh_ctx* c, const RanksArgs* P, size_t lds) {
@@ -1299,7 +1299,7 @@ int mlh_ranks_prepare(mlh_ctx* c) {
 // `steps` decode steps of sequences 0 .. nseq - 1 in one launch.
 int mlh_launch_ranks(mlh_ctx* c, int nseq, int steps) {
     const mlh_hparams& hp = c->hp;
-    const bool wide = use_wide(c, nseq);
+    const bool wide = mlh_ranks_wide(c, nseq);
     RanksPlan p;
     if (!wide && (!ranks_plan(c, nseq, p) || p.words > c->ranksBytes)) { c->err = "decode of several sequences: no plan"; return -1; }
     // tags are a running count of layer passes; before it could wrap and meet a stale word, everything goes back to zero

@@ -987,6 +987,13 @@ extern "C" int mlh_single_launch_sequences(mlh_ctx* c) {
     return std::max(c->ranksMax, mlh_xcd_supported(c) ? 1 : 0);
 }
 
+extern "C" int mlh_decode_route(const mlh_ctx* c, int nseq) {
+    if (!c || !c->finalized || nseq < 1 || nseq > c->hp.maxSeqs) return -1;
+    if (use_ranks(c, nseq)) return mlh_ranks_wide(c, nseq) ? MLH_DECODE_WIDE : MLH_DECODE_RANKS;
+    if (use_persistent(c, nseq)) return c->usePersistent == 3 && mlh_xcd_supported(c) ? MLH_DECODE_XCD : MLH_DECODE_BARRIER;
+    return mlh_rows_applicable(c, nseq) ? MLH_DECODE_ROWS : MLH_DECODE_GEMV;
+}
+
 extern "C" int mlh_xcd_decode_supported(mlh_ctx* c) { return c && mlh_xcd_supported(c) ? 1 : 0; }
 
 extern "C" int mlh_synchronize(mlh_ctx* c) {

@@ -306,6 +306,7 @@ void mlh_rows_lm_head(mlh_ctx* c, int n, const float* X, const int* segStart, co
 #define MLH_RANKS_MAX_SEQS 16 // one block of MFMA columns
 #define MLH_WIDE_MAX_SEQS 64  // four (kernels_wide.hip)
 bool mlh_ranks_applicable(const mlh_ctx* c, int nseq);
+bool mlh_ranks_wide(const mlh_ctx* c, int nseq); // ... by kernels_wide.hip
 int mlh_ranks_other_seqs(const mlh_ctx* c);
 int mlh_ranks_prepare(mlh_ctx* c);
 int mlh_ranks_reset(mlh_ctx* c);

@@ -20,6 +20,7 @@ CASES = {
     "hybrid9": (dict(heads=12, hd=64, ffn=2048, layers=4, vocab=1003, ple=64), 9, 1, 130, 4),
     "hybrid16": (dict(heads=8, hd=64, ffn=256, layers=4, vocab=4111, ple=128), 16, 2, 70, 4),
     "attn_flags5": (dict(heads=9, hd=64, ffn=768, layers=2, vocab=520, ple=0, gdn=False, flags=True, dim_ok=False), 5, 5, 90, 4),
+    "gated_ple16": (dict(heads=12, hd=64, ffn=512, layers=2, vocab=600, ple=64, gdn=False, flags=True), 16, 5, 100, 4),  # fp32 rows that kernels_wide.hip refuses
     "attn_flags8": (dict(heads=8, hd=64, ffn=768, layers=2, vocab=520, ple=0, gdn=False, flags=True), 8, 5, 300, 4),
     "half_hd64": (dict(heads=16, hd=64, ffn=1024, layers=4, vocab=800, ple=64, half=True), 16, 2, 50, 4),
     "half_hd128_one": (dict(heads=8, hd=128, ffn=1536, layers=4, vocab=8200, ple=64, half=True), 1, 9, 9, 5),
@@ -61,6 +62,8 @@ def test_batches_against_the_oracle(pkg, orc, case):
     dev, w, prompts = start(pkg, orc, hp, n, lo, hi, 60 + len(case))
     covered = dev.single_launch_sequences() >= n
     assert covered == shape.get("dim_ok", True)  # (dim 576: not a multiple of 128, the row kernels)
+    wide = n >= 6 and not hp.weightDtype and covered and not (shape.get("flags") and shape["ple"])
+    assert dev.decode_route(n) == (pkg.DECODE_ROWS if not covered else pkg.DECODE_WIDE if wide else pkg.DECODE_RANKS)  # (kernels_wide.hip takes fp32 models from 6 on)
     first = [dev.greedy_token(s) for s in range(n)]
     a = dev.decode_loop(first, steps)           # a run of steps in one launch
     b = dev.decode_loop([int(t) for t in a[-1]], 1)  # and a step of its own: cache, states, positions carried over
@@ -83,15 +86,16 @@ def test_distance_from_float64_is_that_of_the_row_kernels(pkg, orc, half):
     """The same arithmetic precision as the sequence of row kernels: over the same tokens the rms distance of the logits from the float64
     oracle may exceed theirs by the spread of two orders of summation (a factor of two of rounding noise), no more."""
     hp = config(pkg, heads=8 if half else 12, hd=128 if half else 64, ffn=1024, layers=8, vocab=1024, ple=64, half=half)
-    err = {}
+    err, n = {}, 6 if half else 5
     for mode in (3, 0):
-        dev, w, prompts = start(pkg, orc, hp, 6, 10, 60, 71)
+        dev, w, prompts = start(pkg, orc, hp, n, 10, 60, 71)
         dev.set_persistent(mode)
-        feed = np.random.default_rng(4).integers(0, hp.vocabSize, size=(6, 6))
+        assert dev.decode_route(n) == (pkg.DECODE_RANKS if mode == 3 else pkg.DECODE_ROWS)
+        feed = np.random.default_rng(4).integers(0, hp.vocabSize, size=(6, n))
         for row in feed:
             dev.decode_step([int(t) for t in row])
         e = []
-        for s in range(6):
+        for s in range(n):
             dec = orc.Decoder(w, "f64")
             for t in list(prompts[s]) + feed[:, s].tolist():
                 _, lg = dec.step(int(t))
@@ -254,6 +258,7 @@ def test_other_kernels_go_on_where_it_left_the_states(pkg, orc):
             nxt[s] = dev.greedy_token(s)
 
     assert dev.single_launch_sequences() == 16
+    assert [dev.decode_route(m) for m in (1, 5, 17)] == [pkg.DECODE_XCD, pkg.DECODE_RANKS, pkg.DECODE_WIDE]
     decode(5, 2)               # 0 .. 4 in the second place
     prompt([0, 2], 7)          # row kernels
     prompt([16, 1], 40)        # tiled products
@@ -265,7 +270,11 @@ def test_other_kernels_go_on_where_it_left_the_states(pkg, orc):
     hist[4] = []
     prompt([4], 11)
     decode(4, 3)
+    decode(17, 2)              # one launch for more rows
+    decode(4, 1)
+    dev.set_persistent(0)
     decode(17, 2)              # row kernels
+    dev.set_persistent(3)
     decode(3, 1)
     decode(1, 2)               # one sequence
     decode(2, 1)

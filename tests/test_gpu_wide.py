@@ -33,6 +33,7 @@ def test_batches_against_the_oracle(pkg, orc, case):
     shape, n, lo, hi, steps = CASES[case]
     hp = config(pkg, maxSeqs=n, maxL=256, **shape)
     dev, w, prompts = start(pkg, orc, hp, n, lo, hi, 60 + n)
+    assert dev.decode_route(n) == pkg.DECODE_WIDE
     first = [dev.greedy_token(s) for s in range(n)]
     a = dev.decode_loop(first, steps)                # a run of steps in one launch
     b = dev.decode_loop([int(t) for t in a[-1]], 1)  # and a step of its own: cache, states, positions carried over
@@ -59,6 +60,7 @@ def test_every_sequence_against_the_row_kernels(pkg, orc, n):
     for mode in (3, 0):
         dev, w, prompts = start(pkg, orc, hp, n, 3, 60, 71)
         dev.set_persistent(mode)
+        assert dev.decode_route(n) == (pkg.DECODE_WIDE if mode == 3 else pkg.DECODE_ROWS)
         for row in feed:
             dev.decode_step([int(t) for t in row])
         assert dev.persistent_fallbacks() == 0
@@ -94,7 +96,9 @@ def test_gives_up_and_falls_back(pkg, orc, where):
                 dev.debug_inject_abort(1) if where == "meeting" else dev.debug_inject_abort_at_step(2)
             if inject and k == 2:
                 assert dev.get_persistent() == 0 and dev.persistent_fallbacks() == 1
+                assert dev.decode_route(20) == pkg.DECODE_ROWS
                 dev.set_persistent(3)
+            assert dev.decode_route(20) == pkg.DECODE_WIDE
             out.append(dev.decode_loop(nxt, 4))
             nxt = [int(t) for t in out[-1][-1]]
         assert dev.persistent_fallbacks() == int(inject)
@@ -117,6 +121,7 @@ def test_batches_of_changing_size_share_the_exchange_memory(pkg, orc):
     for n in (40, 17, 64, 5, 9, 33, 64):
         if n == 5:
             dev.debug_set_xcd_tag(0xFFFFFFF0)
+        assert dev.decode_route(n) == (pkg.DECODE_RANKS if n == 5 else pkg.DECODE_WIDE)
         out = dev.decode_loop(nxt[:n], 2)
         for s in range(n):
             hist[s] += [nxt[s], int(out[0, s])]
@@ -140,7 +145,8 @@ def test_widths_whose_waves_have_fewer_chunks(pkg, orc, heads, ffn):
     dev, w, prompts = start(pkg, orc, hp, 64, 2, 24, 97)
     hist = [list(p) for p in prompts]
     nxt = [dev.greedy_token(s) for s in range(64)]
-    for n in (20, 10, 40, 10, 64, 20, 48, 6, 33):
+    for n in (20, 10, 40, 10, 64, 20, 48, 9, 33):
+        assert dev.decode_route(n) == pkg.DECODE_WIDE
         out = dev.decode_loop(nxt[:n], 2)
         for s in range(n):
             hist[s] += [nxt[s], int(out[0, s])]
@@ -154,3 +160,57 @@ def test_widths_whose_waves_have_fewer_chunks(pkg, orc, heads, ffn):
         assert_logits_close(dev.logits(s), lg, RTOL, f"sequence {s}")
         dec.close()
     dev.close()
+
+
+def test_more_than_64_pages(pkg):
+    """A wave holds the first 64 page numbers of its sequence in registers and looks the others up: keys beyond 4096 positions, against the row kernels over the
+    same tokens (1e-4: two orders of fp32 sums)."""
+    n, hp = 9, config(pkg, heads=8, hd=64, ffn=256, layers=2, vocab=300, ple=0, gdn=False, maxL=4400, maxSeqs=9)
+    lens, out = (4200, 33, 4094, 70, 4160, 5, 900, 4095, 64), {}
+    for mode in (3, 0):
+        dev = pkg.Device(hp, 0)
+        dev.upload(pkg.Model.generate(hp, 7).randomize_gains(7))
+        dev.set_page_table(np.random.default_rng(7).permutation(n * 69).astype(np.int32))
+        dev.prefill_batch(list(range(n)), [pkg.random_tokens(7, s, hp.vocabSize, m) for s, m in enumerate(lens)])
+        dev.set_persistent(mode)
+        assert dev.decode_route(n) == (pkg.DECODE_WIDE if mode == 3 else pkg.DECODE_ROWS)
+        lg = []
+        for row in np.random.default_rng(8).integers(0, hp.vocabSize, size=(4, n)):  # sequences 2 and 7 reach their 65th page on the way
+            dev.decode_step([int(t) for t in row])
+            lg.append([dev.logits(s) for s in range(n)])
+        assert dev.persistent_fallbacks() == 0
+        out[mode] = np.array(lg)
+        dev.close()
+    for i in range(4):
+        for s in range(n):
+            assert_logits_close(out[3][i, s], out[0][i, s], 1e-4, f"step {i} sequence {s}")
+
+
+def test_calls_that_the_kernel_does_not_take(pkg, orc):
+    """What a caller sees of the route: one and few sequences, sampling, graph replays, prompts token by token, and a first phase of more tiles than workgroups
+    (query gating beside per-layer embeddings in models of more than 8 heads)."""
+    def context(**kw):
+        hp = config(pkg, **{**dict(heads=12, hd=64, ffn=512, layers=2, vocab=300, ple=64, maxSeqs=70, maxL=64), **kw})
+        dev = pkg.Device(hp, 0)
+        dev.upload(pkg.Model.generate(hp, 3))
+        return dev
+
+    dev = context()
+    assert [dev.decode_route(n) for n in (0, 1, 2, 5, 16, 17, 64, 65, 70, 71)] == [
+        -1, pkg.DECODE_XCD, pkg.DECODE_RANKS, pkg.DECODE_RANKS, pkg.DECODE_WIDE, pkg.DECODE_WIDE, pkg.DECODE_WIDE, pkg.DECODE_GEMV, pkg.DECODE_GEMV, -1]
+    dev.set_sampling(0.8, 1)
+    assert dev.decode_route(16) == pkg.DECODE_ROWS
+    dev.set_sampling(0.0)
+    dev.set_graph(4)
+    assert dev.decode_route(16) == pkg.DECODE_ROWS
+    dev.set_graph(0)
+    dev.set_prefill_mode(1)
+    assert dev.decode_route(16) == pkg.DECODE_GEMV
+    dev.set_prefill_mode(0)
+    assert dev.decode_route(16) == pkg.DECODE_WIDE
+    dev.close()
+    for kw, n16, n17 in ((dict(gdn=False, flags=True), pkg.DECODE_RANKS, pkg.DECODE_ROWS), (dict(half=True), pkg.DECODE_RANKS, pkg.DECODE_ROWS),
+                         (dict(gdn=False, flags=True, ple=0), pkg.DECODE_WIDE, pkg.DECODE_WIDE), (dict(gdn=False, flags=True, heads=8), pkg.DECODE_WIDE, pkg.DECODE_WIDE)):
+        dev = context(**kw)
+        assert (dev.decode_route(16), dev.decode_route(17)) == (n16, n17), kw
+        dev.close()
