@@ -24,7 +24,7 @@
 // of the thread's place that the compiler keeps, spills or moves behind a barrier costs more than forming it again.
 // Measured, us per step, here and as the row kernels' sequence: hybrid, fp32, d 768, 12 layers: 2 sequences 219 and 367, 5 sequences 232
 // and 373, 16 sequences 315 and 394; hybrid, bf16, d 2048, 24 layers: 1 sequence 705 and 1161, 8 sequences 1050 and 1265.  More than
-// 16, and from 6 on where it covers the model: kernels_wide.hip.
+// 16, and from 6 to 9 on where it covers the model and is faster: kernels_wide.hip.
 //
 // The launch starts with a meeting of all 256 workgroups: if one is missing after a bounded wait nothing has been written and the
 // call runs as the sequence of row kernels instead.  Behind it every workgroup is resident, and every wait is bounded as well: when
@@ -1233,10 +1233,22 @@ int mlh_ranks_other_seqs(const mlh_ctx* c) { return ranks_model(c) ? other_seqs(
 // Whether the kernel covers this context's model as it has been finalized (memory for its exchange words apart).
 static bool ranks_shape(const mlh_ctx* c) { return ranks_model(c) && mlh_rows_applicable(c, 1); }
 
-// From how many sequences on kernels_wide.hip takes them.  Measured, us per step, here and there (hybrid, fp32, d 768, 12 layers): 2 sequences
-// 224 and 250, 5 241 and 253, 6 269 and 256, 7 275 and 257, 8 273 and 258, 12 327 and 263, 16 339 and 267.
-#define WIDE_FROM 6
-bool mlh_ranks_wide(const mlh_ctx* c, int nseq) { return nseq >= WIDE_FROM && c->wideMax >= nseq; }
+// Whether kernels_wide.hip takes a call.  Here a pair of a head and a sequence has four workgroups of its XCD up to 64 pairs, fewer beyond; there it has one or a share
+// of one whatever their number, and attention layers cost a little more, the others less.  Measured, us per step, here and there (12 layers, fp32, 100 keys; in
+// brackets 350 keys):
+//   hybrid (3 in 4 gated delta net)  8 heads   6: 212, 209 (216, 216)   8: 216, 211 (221, 219)   9: 243, 211
+//                                   10 heads   6: 232, 242 (238, 249)   7: 257, 242 (264, 250)   9: 272, 244
+//                                   12 heads   5: 241, 253              6: 267, 255 (272, 263)   12: 321, 260   16: 328, 263
+//   attention only                   8 heads   6: 224, 239 (249, 267)   8: 237, 240 (264, 269)   9: 266, 240   8, gated and normed (272, 272)
+//                                   10 heads   6: 247, 261 (266, 285)   7: 275, 262 (299, 287)
+//              gated and normed     12 heads   6: 302, 303 (322, 331)   7: 310, 304 (338, 333)   8: 307, 306 (333, 337)   9: 339, 306 (374, 340)
+static bool wide_is_faster(const mlh_ctx* c, int nseq) {
+    int gdn = 0;
+    for (const LayerDev& L : c->layers) gdn += L.kind != MLH_KIND_ATTENTION;
+    const bool hybrid = 2 * gdn >= (int)c->layers.size();
+    return nseq >= (hybrid ? 6 : 7) && (nseq * c->hp.attnHeads > 64 || (hybrid && c->hp.attnHeads == RK_XCDS));
+}
+bool mlh_ranks_wide(const mlh_ctx* c, int nseq) { return c->wideMax >= nseq && (wide_is_faster(c, nseq) || nseq > std::max(c->ranksMax, 5)); }
 
 bool mlh_ranks_applicable(const mlh_ctx* c, int nseq) { return (mlh_ranks_wide(c, nseq) || c->ranksMax >= nseq) && mlh_rows_applicable(c, nseq); }
 

@@ -62,8 +62,7 @@ def test_batches_against_the_oracle(pkg, orc, case):
     dev, w, prompts = start(pkg, orc, hp, n, lo, hi, 60 + len(case))
     covered = dev.single_launch_sequences() >= n
     assert covered == shape.get("dim_ok", True)  # (dim 576: not a multiple of 128, the row kernels)
-    wide = n >= 6 and not hp.weightDtype and covered and not (shape.get("flags") and shape["ple"])
-    assert dev.decode_route(n) == (pkg.DECODE_ROWS if not covered else pkg.DECODE_WIDE if wide else pkg.DECODE_RANKS)  # (kernels_wide.hip takes fp32 models from 6 on)
+    assert dev.decode_route(n) == (pkg.DECODE_ROWS if not covered else pkg.DECODE_WIDE if case in ("hybrid9", "hybrid16") else pkg.DECODE_RANKS)
     first = [dev.greedy_token(s) for s in range(n)]
     a = dev.decode_loop(first, steps)           # a run of steps in one launch
     b = dev.decode_loop([int(t) for t in a[-1]], 1)  # and a step of its own: cache, states, positions carried over

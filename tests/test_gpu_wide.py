@@ -18,6 +18,7 @@ CASES = {
     # name: (hyper-parameters, sequences, prompt lengths from .. to, steps)
     "hybrid6": (dict(heads=12, hd=64, ffn=1024, layers=4, vocab=300, ple=64), 6, 2, 50, 4),
     "attn_flags7": (dict(heads=8, hd=64, ffn=768, layers=2, vocab=520, ple=0, gdn=False, flags=True), 7, 5, 120, 3),
+    "attn_flags9": (dict(heads=8, hd=64, ffn=768, layers=2, vocab=520, ple=0, gdn=False, flags=True), 9, 5, 120, 3),
     "hybrid16": (dict(heads=10, hd=64, ffn=256, layers=2, vocab=4999, ple=32), 16, 2, 40, 3),
     "hybrid17": (dict(heads=12, hd=64, ffn=2048, layers=4, vocab=1003, ple=64), 17, 1, 90, 4),
     "hybrid32": (dict(heads=8, hd=64, ffn=256, layers=4, vocab=4111, ple=128), 32, 2, 60, 3),
@@ -33,7 +34,7 @@ def test_batches_against_the_oracle(pkg, orc, case):
     shape, n, lo, hi, steps = CASES[case]
     hp = config(pkg, maxSeqs=n, maxL=256, **shape)
     dev, w, prompts = start(pkg, orc, hp, n, lo, hi, 60 + n)
-    assert dev.decode_route(n) == pkg.DECODE_WIDE
+    assert dev.decode_route(n) == (pkg.DECODE_RANKS if case == "attn_flags7" else pkg.DECODE_WIDE)  # (8 heads of attention only: from 9 on)
     first = [dev.greedy_token(s) for s in range(n)]
     a = dev.decode_loop(first, steps)                # a run of steps in one launch
     b = dev.decode_loop([int(t) for t in a[-1]], 1)  # and a step of its own: cache, states, positions carried over
@@ -195,6 +196,11 @@ def test_calls_that_the_kernel_does_not_take(pkg, orc):
         dev.upload(pkg.Model.generate(hp, 3))
         return dev
 
+    # from how many sequences on: pairs of a head and a sequence, and the share of attention layers
+    for kw, first in ((dict(heads=8), 6), (dict(heads=10), 7), (dict(heads=12), 6), (dict(heads=8, gdn=False), 9), (dict(heads=10, gdn=False), 7), (dict(heads=12, gdn=False), 7)):
+        dev = context(**kw)
+        assert [dev.decode_route(n) for n in range(2, 17)] == [pkg.DECODE_RANKS] * (first - 2) + [pkg.DECODE_WIDE] * (17 - first), kw
+        dev.close()
     dev = context()
     assert [dev.decode_route(n) for n in (0, 1, 2, 5, 16, 17, 64, 65, 70, 71)] == [
         -1, pkg.DECODE_XCD, pkg.DECODE_RANKS, pkg.DECODE_RANKS, pkg.DECODE_WIDE, pkg.DECODE_WIDE, pkg.DECODE_WIDE, pkg.DECODE_GEMV, pkg.DECODE_GEMV, -1]
