@@ -1204,7 +1204,12 @@ static size_t state_floats(const mlh_ctx* c) {
 }
 
 // Sequences whose states have a second place, in a model that the kernel covers: those of a launch of this kernel or of kernels_wide.hip.
-static int other_seqs(const mlh_ctx* c) { return std::min(c->hp.maxSeqs, mlh_wide_model(c) ? MLH_WIDE_MAX_SEQS : MLH_RANKS_MAX_SEQS); }
+// (Both places of all states lie within 32-bit offsets; where 64 more do not, 16 may.)
+static bool places_fit(const mlh_ctx* c, int others) { return (c->hp.maxSeqs + others) * state_floats(c) < (size_t)1 << 31; }
+static int other_seqs(const mlh_ctx* c) {
+    const int wide = std::min(c->hp.maxSeqs, MLH_WIDE_MAX_SEQS);
+    return mlh_wide_model(c) && places_fit(c, wide) ? wide : std::min(c->hp.maxSeqs, MLH_RANKS_MAX_SEQS);
+}
 
 // Whether the kernel covers a model of these hyper-parameters on this device.
 static bool ranks_model(const mlh_ctx* c) {
@@ -1224,7 +1229,7 @@ static bool ranks_model(const mlh_ctx* c) {
         for (const LayerDev& L : c->layers)
             if (L.offPle % 16) return false;
     }
-    return (hp.maxSeqs + other_seqs(c)) * state_floats(c) < (size_t)1 << 31; // (state rows: 32-bit offsets)
+    return places_fit(c, other_seqs(c));
 }
 
 // Sequences whose states have a second place behind those of all maxSeqs (mlh_create allocates both).

@@ -957,7 +957,7 @@ static int wide_launch(mlh_ctx* c, int mb, const WideArgs* P, size_t lds) {
 // At finalize: how many sequences the kernel takes (none where the model or the device does not suit it), and its exchange memory.
 int mlh_wide_prepare(mlh_ctx* c) {
     c->wideMax = 0;
-    const int most = std::min(c->hp.maxSeqs, MLH_WIDE_MAX_SEQS);
+    const int most = mlh_ranks_other_seqs(c); // (whose states have a second place)
     if (!mlh_wide_model(c) || !mlh_rows_applicable(c, 1)) return 0;
     size_t bytes = 0;
     WidePlan p;

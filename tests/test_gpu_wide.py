@@ -187,6 +187,29 @@ def test_more_than_64_pages(pkg):
             assert_logits_close(out[3][i, s], out[0][i, s], 1e-4, f"step {i} sequence {s}")
 
 
+def test_states_near_the_end_of_their_offsets(pkg):
+    """65 500 sequences of 8 heads: a second place of the states for 64 of them would lie beyond 32-bit offsets, one for 16 does not, so calls of up to 16 stay in
+    one launch (both kernels) and more rows run as row kernels; the first and last sequences of a call, and what follows on it, as without."""
+    hp = config(pkg, heads=8, hd=64, ffn=256, layers=1, vocab=300, ple=0, maxSeqs=65500, maxL=40)
+    hp.layerKinds[0] = pkg.KIND_GDN
+    out, feed = {}, np.random.default_rng(4).integers(0, 300, size=(3, 17))
+    for mode in (3, 0):
+        dev = pkg.Device(hp, 0)
+        dev.upload(pkg.Model.generate(hp, 7).randomize_gains(7))
+        dev.set_persistent(mode)
+        want = [pkg.DECODE_RANKS, pkg.DECODE_WIDE, pkg.DECODE_WIDE, pkg.DECODE_ROWS]
+        assert [dev.decode_route(n) for n in (5, 6, 16, 17)] == (want if mode == 3 else [pkg.DECODE_ROWS] * 4)
+        dev.prefill_batch(list(range(17)), [pkg.random_tokens(7, s, 300, 5 + s % 3) for s in range(17)])
+        for n in (16, 17, 5):
+            for row in feed:
+                dev.decode_step([int(t) for t in row[:n]])
+        assert dev.persistent_fallbacks() == 0
+        out[mode] = np.stack([dev.logits(s) for s in range(17)])
+        dev.close()
+    for s in range(17):
+        assert_logits_close(out[3][s], out[0][s], 1e-4, f"sequence {s}")
+
+
 def test_calls_that_the_kernel_does_not_take(pkg, orc):
     """What a caller sees of the route: one and few sequences, sampling, graph replays, prompts token by token, and a first phase of more tiles than workgroups
     (query gating beside per-layer embeddings in models of more than 8 heads)."""
