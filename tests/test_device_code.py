@@ -69,21 +69,49 @@ def _registers(operand):
     return {int(m.group(3))} if m.group(3) else set(range(int(m.group(1)), int(m.group(2)) + 1))
 
 
-def test_no_wide_stores_data_is_overwritten_by_the_next_instruction(listing):
-    """A store of 12 or 16 bytes reads its data after it has been issued.  The compiler keeps an instruction between it and a write of
+def _overwrites(code, i, data, states=2):
+    """The first vector instruction within `states` wait states behind code[i] that writes one of the registers `data` (s_nop N is N + 1 of them, any other
+    instruction one; a taken branch takes longer than two)."""
+    for ins in code[i + 1:]:
+        if states <= 0 or ins.startswith(("s_branch", "s_setpc", "s_endpgm")):
+            return None
+        m = re.match(r"s_nop (\w+)", ins)
+        states -= int(m.group(1), 0) + 1 if m else 1
+        if ins.startswith("v_"):
+            operands = ins.split(None, 1)[1].split(",")
+            written = operands[:2] if "swap" in ins.split()[0] else operands[:1]
+            if any(_registers(o.strip()) & data for o in written):
+                return ins
+    return None
+
+
+def test_no_wide_stores_data_is_overwritten_while_it_is_read(listing):
+    """A store of 12 or 16 bytes reads its data after it has been issued.  The compiler keeps two wait states between it and a write of
     those registers except where a buffer store has a scalar offset, and there lanes have stored the overwritten value."""
     stores, bad = 0, []
     for symbol, code in listing.items():
-        for ins, after in zip(code, code[1:]):
+        for i, ins in enumerate(code):
             m = re.match(r"(buffer|global|flat|scratch)_store_dwordx[34] (.*)", ins)
             if not m:
                 continue
             stores += 1
             operands = [o.strip() for o in m.group(2).split(",")]
-            if after.startswith("v_") and _registers(after.split(None, 1)[1]) & _registers(operands[0 if m.group(1) == "buffer" else 1]):
+            after = _overwrites(code, i, _registers(operands[0 if m.group(1) == "buffer" else 1]))
+            if after:
                 bad.append((symbol, ins, after))
     assert stores > 100
     assert not bad, f"{len(bad)} stores, the first: {bad[0]}"
+
+
+def test_the_wait_states_behind_a_store():
+    """What the check above counts: the instruction behind the next one, not what two or an s_nop of two wait states keep away, and both results of a swap."""
+    data = _registers("v[4:7]")
+    assert _overwrites(["store", "s_nop 0", "v_add_f32_e32 v5, v1, v2"], 0, data)
+    assert _overwrites(["store", "v_mov_b32_e32 v1, v4", "v_add_f32_e32 v7, v1, v2"], 0, data)
+    assert _overwrites(["store", "v_permlane16_swap_b32_e32 v1, v6"], 0, data)
+    assert not _overwrites(["store", "s_branch 65115", "v_add_f32_e32 v5, v1, v2"], 0, data)
+    assert not _overwrites(["store", "s_nop 1", "v_add_f32_e32 v5, v1, v2"], 0, data)
+    assert not _overwrites(["store", "v_mov_b32_e32 v1, v4", "v_mov_b32_e32 v8, v4", "v_add_f32_e32 v7, v1, v2"], 0, data)
 
 
 def test_every_built_form_of_the_decode_of_several_sequences_is_reached(listing):
