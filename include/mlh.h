@@ -222,8 +222,8 @@ int mlh_set_graph(mlh_ctx* ctx, int stepsPerGraph);
  * up to 768 (fp32) / 2048 (bf16), ffnDim up to 2048 / 6144 in multiples of 256 / 512.  It gives up
  * and falls back in the same way: its workgroups meet before anything is written, and it writes gated-delta-net states to a second
  * place (mlh_create allocates it for the first 16 sequences, 64 where the next sentence applies), so that those from before the launch are there
- * after a wait that expires later.  Calls of up to 64 sequences run as one launch too for fp32 models of those whose dim is 512 or more and whose heads have
- * at most 32 tiles of 16 first-phase rows to a pair (no query gating beside per-layer embeddings or more than 8 heads).
+ * after a wait that expires later.  Calls of up to 64 sequences run as one launch too for fp32 models of those with 8, 10 or 12 heads, except with query gating beside
+ * per-layer embeddings and more than 8 heads (mlh_decode_route says what a call runs).
  * Mode 0, unsupported shapes and more sequences: a sequence of kernels issued as mlh_set_graph says. */
 int mlh_set_persistent(mlh_ctx* ctx, int mode);
 
@@ -261,7 +261,7 @@ int mlh_set_sampling(mlh_ctx* ctx, float temperature, unsigned long long seed);
  * (no counterpart in the reference: its decode loop is one kernel sequence, inference_orchestrator.cu:120-165). */
 int mlh_xcd_decode_supported(mlh_ctx* ctx);
 /* The largest nseq whose decode calls run as a single launch in mode 3 for every covered model (0: none; 16 at most: fp32 models may go on to 64,
- * see mlh_set_persistent; no counterpart in the reference). */
+ * which mlh_decode_route shows; no counterpart in the reference). */
 int mlh_single_launch_sequences(mlh_ctx* ctx);
 /* What a decode call of sequences 0 .. nseq - 1 runs as the context stands (mode, sampling, graph replays, kernels that have given up): launches of the
  * GEMV kernels or of the row kernels, or one launch for all steps of the barrier kernel, of the XCD-rank kernel (one sequence), or of one of the two kernels of several

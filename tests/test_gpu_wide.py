@@ -25,6 +25,9 @@ CASES = {
     "hybrid33": (dict(heads=10, hd=64, ffn=512, layers=2, vocab=700, ple=32), 33, 2, 40, 3),
     "hybrid48": (dict(heads=12, hd=64, ffn=768, layers=2, vocab=520, ple=0), 48, 2, 30, 2),
     "hybrid64": (dict(heads=12, hd=64, ffn=512, layers=2, vocab=1000, ple=64), 64, 1, 70, 3),
+    "gated12_17": (dict(heads=12, hd=64, ffn=512, layers=2, vocab=600, ple=0, gdn=False, flags=True), 17, 3, 90, 3),  # 32 tiles of the first phase: all there are
+    "gated12_64": (dict(heads=12, hd=64, ffn=512, layers=2, vocab=600, ple=0, gdn=False, flags=True), 64, 1, 70, 2),
+    "gated10_50": (dict(heads=10, hd=64, ffn=1280, layers=2, vocab=600, ple=0, gdn=False, flags=True), 50, 1, 70, 2),
     "attn_flags49": (dict(heads=8, hd=64, ffn=768, layers=2, vocab=520, ple=32, gdn=False, flags=True), 49, 3, 200, 2),
 }
 
