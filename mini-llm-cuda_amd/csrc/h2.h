@@ -1,8 +1,10 @@
 // fp32 matrices as IEEE halves, for the prefill's products on the half-precision matrix cores at fp32 precision.
 //
 // A row is scaled by a power of two that brings its largest element into [2^14, 2^15).  An element x of it is hi + lo + tiny with hi = half(x),
-// lo = half(x - hi), tiny = half(x - hi - lo), each rounded to nearest even.  Weights keep the three (exact; elements below 2^-15 of the row's largest
-// to 2^-40 of it), activations hi and lo: x to 2^-23 of itself, every second value exactly, below 2^-18 of the row's largest to 2^-40 of that.  A product a.b is
+// lo = half(x - hi), tiny = half(x - hi - lo), each rounded to nearest even.  Weights keep the three: elements down to 2^-15 of the row's largest
+// exactly, smaller ones to 2^-39 of it.  Activations keep hi and lo: elements down to 2^-16 of the row's largest to 2^-23 of themselves, three in four of them
+// exactly, smaller ones to 2^-39 of the largest.  (Models whose rows spread far enough for that to matter multiply planes: operand_spread in
+// kernels_prefill.hip.)  A product a.b is
 // formed from hi.tiny, lo.hi, hi.lo and hi.hi, every one exact in the fp32 accumulator; lo.lo and lo.tiny, below 2^-22 of |a||b|, are left out.  That
 // moves a sum of normal terms by 6.2e-8 (rms, of |a||b| / sqrt(K)), whatever K is; what the accumulator rounds on the way is more, and grows with the
 // number of matrix instructions: four here for 32 columns where three bf16 planes (p3.h) take six.  Measured against float64 (rms, of the product's
@@ -15,7 +17,7 @@
 //
 // FFN units are written by many workgroups a row, and no pass finds their rows' scale: they have a scale per column instead, from a bound on what the
 // unit can be (k_unit_exps in kernels_prefill.hip), and W2's columns take it back before its rows are scaled.  Units are typically 2^-11 of
-// the bound; those of 2^-18 of it and more are kept to 2^-23, the rest to 2^-40 of the bound.
+// the bound; those of 2^-16 of it and more are kept to 2^-23, the rest to 2^-39 of the bound.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -1717,19 +1717,22 @@ static int operand_values(mlh_ctx* c, bool* within) {
     return 0;
 }
 
-// Whether scaled halves reach over an fp32 model's operands.  A row of halves ends 2^-40 below its largest element (h2.h), where floats and planes end
+// Whether scaled halves reach over an fp32 model's operands.  A row of halves ends 2^-39 below its largest element (h2.h), where floats and planes end
 // at 2^-126: elements far below the largest are kept in fewer bits, and where the large ones meet zeros the sum is made of those.  So
 //   - a row of weights has its typical element (mean of the exponents, zeros apart) within 2^12 of its largest: with its columns' scales in W2, whose
 //     columns the units' exponents go into;
 //   - the rows that are multiplied have theirs within 2^8, as far as that follows from the model: residual columns (E's columns, rows of [Wo | pleUp] and W2, each
 //     about its own mean) with the gain in front of a product; value rows and PLE columns (gate row and table) beside each other;
-//   - an FFN unit, whose scale comes from its bound, is dim below that on rows without a direction; on rows as uneven as the residual columns at most 2^6 more.
-// What ends at 2^-40 is then 2^-24 or less of what is typical in all of them.
+//   - an FFN unit, whose scale comes from its bound, is dim below that on rows without a direction; on rows as uneven as the residual columns at most 2^4 more.
+// What is lost at 2^-39 of the largest is then 2^-27 of a typical weight, 2^-31 of a typical element of a row, 2^-24 of a typical unit (dim 2048).
 // Models beyond multiply planes.  Random and trained weights have 3 to 6 in all of them.  Exponents and integer sums: the answer is the same at every finalize.
 #define SPREAD_WEIGHTS 12
 #define SPREAD_ROWS 8
-#define SPREAD_UNITS 6
+#define SPREAD_UNITS 4
 #define SPREAD_NONE (-100000)
+__device__ __forceinline__ void spread_worst(int* worst, int v) { // (a row that does not add to it leaves the word alone: one address for all)
+    if (v > __hip_atomic_load(worst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(worst, v);
+}
 // the exponents of rows of [W | U] with those of the columns: the largest of each row to rowMost, and the largest distance of one from its row's mean to worst
 __global__ void __launch_bounds__(PWG) k_spread_rows(const float* __restrict__ W, int cols, const float* __restrict__ U, int cols2, const int* __restrict__ colExps, int* rowMost, int* worst, int rows) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -1745,7 +1748,7 @@ __global__ void __launch_bounds__(PWG) k_spread_rows(const float* __restrict__ W
     for (int o = 32; o > 0; o >>= 1) { most = max(most, __shfl_xor(most, o, 64)); sum += __shfl_xor(sum, o, 64); count += __shfl_xor(count, o, 64); }
     if (lane) return;
     if (rowMost) rowMost[row] = most;
-    if (count) atomicMax(worst, most - (int)floorf((float)sum / (float)count));
+    if (count) spread_worst(worst, most - (int)floorf((float)sum / (float)count));
 }
 // ... the largest of each column to colMost (x: columns, y: strips of rows)
 __global__ void __launch_bounds__(PWG) k_spread_cols(const float* __restrict__ W, int rows, int cols, int* colMost) {
@@ -1771,7 +1774,7 @@ __global__ void __launch_bounds__(PWG) k_spread_units(const float* __restrict__ 
         for (int k = 0; k < 4; k++) s[k] += __shfl_xor(s[k], o, 64);
     if (lane || s[0] == 0.0 || s[1] == 0.0) return; // (a unit that is always 0)
     const double size = sqrt(s[2]) * sqrt(s[3]);
-    atomicMax(worst, size > 0.0 ? __builtin_amdgcn_frexp_exp(sqrt(s[0]) * sqrt(s[1]) / size) : -SPREAD_NONE);
+    spread_worst(worst, size > 0.0 ? __builtin_amdgcn_frexp_exp(sqrt(s[0]) * sqrt(s[1]) / size) : -SPREAD_NONE);
 }
 static int spread_mean(const int* v, int n) { // rounded down; of the elements there are
     long sum = 0, count = 0;
@@ -2128,6 +2131,7 @@ int mlh_run_prefill_gemm(mlh_ctx* c, int nseg, const int32_t* seqs, const int32_
     const int d_ = hp.dim, F = hp.ffnDim, dt = c->pfDtype;
     // Up to 64 rows of halves are one row of 64 x 64 tiles: their two groups of waves keep four stages in flight, where a wave of the weight-streaming kernel (what
     // mlh_gemm_tn_epi takes) has one chunk.  Whole prefills, 24 layers of width 2048, us: 33 rows 2237 -> 1756, 48 2406 -> 1819, 64 2707 -> 2002 (65: 2084).
+    // (FFN units go through the hardware's exp2 and reciprocal in tiles, through expf and a division in that kernel: both 2.085e-4 of their norm from float64, K 2048.)
     auto* const product = dt == MLH_GEMM_F16 && n <= 64 ? mlh_gemm_tile : mlh_gemm_tn_epi;
 #define GEMM(A, lda, eA, B, alpha, eB, ldb, C, ldc, R, ldr, M, N, K)                                                           \
     do {                                                                                                                     \

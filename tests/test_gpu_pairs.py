@@ -1,7 +1,7 @@
 """fp32 products as halves, pairs times triples with a scale per row (csrc/h2.h): edges of tiles and of K splits, rows longer than what the split keeps in
 registers, rows of any size, against float64.
 
-Bound: a pair holds an element to 2^-23 of itself (2^-40 of its row's largest below 2^-18 of it), a triple exactly; what is left out of a product is below
+Bound: a pair holds an element to 2^-23 of itself (to 2^-39 of its row's largest below 2^-16 of it), a triple exactly (to 2^-39 below 2^-15); what is left out of a product is below
 2^-22 of |a||b|; the accumulator takes four products per 32 columns and rounds each time, 2^-24 of at most the sum of the magnitudes, twice that for what a matrix
 instruction rounds inside: (2^-21 + (K / 8 + 8) 2^-23) sum |a||b|, and 2^-38 of the largest products for the small ones."""
 import numpy as np
