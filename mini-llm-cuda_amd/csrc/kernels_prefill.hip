@@ -120,17 +120,29 @@ template <typename AT> __device__ __forceinline__ void put_mix4(const PfArgs& P,
 // PLE columns of `rows` rows from row0 on, e[row][j] = silu(ple gate output) * P[tok][j], behind the mixing output (fp32 models' calls of more rows than the row
 // kernels take: k_pf_operand_rows).  Workgroups of their own in the launches that mix: a launch for them took 4.4 us a layer, whatever it did.  24 bf16 layers of width
 // 2048, us: 17 rows 1945 -> 1884, 70 2094 -> 2019, 300 3081 -> 3006, 777 4512 -> 4442; 16 384 rows the same.
-template <typename WT, typename AT> __device__ __forceinline__ void ple_columns(const PfArgs& P, const LayerDev& L, int row0, int rows, int tid, int threads) {
-    const int ple = P.a.ple;
-    for (int i = tid; i < rows * ple; i += threads) {
-        const int r = i / ple, j = i - r * ple;
-        const size_t row = (size_t)row0 + r;
-        put_mix<AT>(P, row, L.ad + j, pf_silu(P.QKV[row * P.qkvLd + L.offPle + j]) * getw<WT>((const WT*)L.pleTable + (size_t)P.ids[row] * ple + j));
+// AT_ONCE: elements of a thread on their way together; one after the other a chunk of 64 rows x 128 columns was a chain of 32 latencies, and what a
+// launch of few chunks ended with (8 bf16 layers of width 1024, us: 64 rows 588 -> 538, 600 820 -> 749, 1500 1340 -> 1262, 8 prompts of 1160 rows 1126 -> 1047).
+template <int AT_ONCE, typename WT, typename AT> __device__ __forceinline__ void ple_columns(const PfArgs& P, const LayerDev& L, int row0, int rows, int tid, int threads) {
+    const int ple = P.a.ple, total = rows * ple;
+    for (int i0 = tid; i0 < total; i0 += AT_ONCE * threads) {
+        float gate[AT_ONCE], emb[AT_ONCE];
+#pragma unroll
+        for (int k = 0; k < AT_ONCE; k++) {
+            const int i = min(i0 + k * threads, total - 1), r = i / ple, j = i - r * ple;
+            const size_t row = (size_t)row0 + r;
+            gate[k] = P.QKV[row * P.qkvLd + L.offPle + j];
+            emb[k] = getw<WT>((const WT*)L.pleTable + (size_t)P.ids[row] * ple + j);
+        }
+#pragma unroll
+        for (int k = 0; k < AT_ONCE; k++) {
+            const int i = i0 + k * threads, r = i / ple, j = i - r * ple;
+            if (i < total) put_mix<AT>(P, (size_t)row0 + r, L.ad + j, pf_silu(gate[k]) * emb[k]);
+        }
     }
 }
-__device__ __forceinline__ void ple_columns(const PfArgs& P, const LayerDev& L, int row0, int rows, int tid, int threads) {
-    if (P.half) ple_columns<bf16_t, f16_t>(P, L, row0, rows, tid, threads);
-    else ple_columns<float, float>(P, L, row0, rows, tid, threads);
+template <int AT_ONCE> __device__ __forceinline__ void ple_columns(const PfArgs& P, const LayerDev& L, int row0, int rows, int tid, int threads) {
+    if (P.half) ple_columns<AT_ONCE, bf16_t, f16_t>(P, L, row0, rows, tid, threads);
+    else ple_columns<AT_ONCE, float, float>(P, L, row0, rows, tid, threads);
 }
 
 // KEEP: 16-byte pieces a lane keeps, rows of up to 256 KEEP elements.  All loads of a row and of the gains go out at once: a load under a comparison, or the
@@ -198,7 +210,7 @@ __global__ void __launch_bounds__(64) k_pf_qk_rope_kv(PfArgs P, LayerDev L) {
     constexpr int EPL = HD / 64;
     const StepArgs& a = P.a;
     const int h = blockIdx.x, row = blockIdx.y, lane = threadIdx.x;
-    if (h == a.heads) { ple_columns(P, L, row, 1, lane, 64); return; }
+    if (h == a.heads) { ple_columns<1>(P, L, row, 1, lane, 64); return; }
     const int seq = P.rowSeq[row], pos = P.rowPos[row];
     float* qkv = P.QKV + (size_t)row * P.qkvLd;
     float qv[EPL], kv[EPL], vv[EPL];
@@ -693,7 +705,7 @@ __global__ void __launch_bounds__(PWG) k_pf_gdn(PfArgs P, LayerDev L, int skipFr
     if (len >= skipFrom) return; // taken by the chunk-parallel kernels
     if (h == a.gdnHeads) { // the segment's PLE columns, a share of its rows each
         const int share = (len + gridDim.z - 1) / gridDim.z, from = min((int)blockIdx.z * share, len);
-        ple_columns(P, L, row0 + from, min(share, len - from), tid, PWG);
+        ple_columns<8>(P, L, row0 + from, min(share, len - from), tid, PWG);
         return;
     }
     const int r = tid / TPR * RPT, cg = tid % TPR, c0 = cg * CPT;
@@ -902,7 +914,7 @@ __global__ void __launch_bounds__(2 * DK, 2) k_gdn_prep(PfArgs P, LayerDev L, co
     const int chunk = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int seg = chunkSeg[chunk], t0 = chunkT0[chunk];
     const int nv = min(GD_C, P.segLen[seg] - t0), row0 = P.segStart[seg] + t0;
-    if (h == a.gdnHeads) { ple_columns(P, L, row0, nv, tid, NT); return; }
+    if (h == a.gdnHeads) { ple_columns<8>(P, L, row0, nv, tid, NT); return; }
     unsigned char* img = ws + ((size_t)chunk * a.gdnHeads + h) * Lay::total;
     float* g = gs; float* beta = gs + GD_C; float* sp = gs + 2 * GD_C; float* rk = gs + 3 * GD_C; float* rq = gs + 4 * GD_C;
     float* part = gs + 5 * GD_C;
