@@ -3,7 +3,8 @@
 //
 //     C[M, N] = A[M, K] . B[N, K]^T  (+ R[M, N])        A, B: IEEE half, fp32 as scaled halves (h2.h), fp32 as bf16 planes (p3.h), or bf16
 //
-// (bf16 operands and planes: the GEMM self-test only; models with bf16 weights multiply halves, those with fp32 weights pairs of them by triples.)
+// (bf16 operands: the GEMM self-test only; models with bf16 weights multiply halves, those with fp32 weights pairs of them by triples, or planes where
+// their weights spread further than halves reach.)
 //
 // KG groups of 2 x NW waves own one TM x TN tile, 128 x 128 or 64 x 64, every wave WM x WN blocks of 16 x 16.  K goes by in slices of RA and RB bytes per row of A
 // and B: 64 two-byte elements (128 bytes), 32 elements of three planes or halves (192 bytes) or 32 of two (128).  Slices go global -> LDS directly into a ring

@@ -1,8 +1,8 @@
 """fp32 prefills of models whose weights, gains or tables spread over many octaves: halves do not reach that far (csrc/h2.h), and such models multiply planes; models
 just inside the rule stay with pairs.  Against the float64 oracle.
 
-Bound: the same context token by token multiplies in fp32; a product of planes or pairs rounds a few times less often, and the two differ by the order of their
-sums, so no more than twice its distance, and 1e-6 for what a short sum may hit by chance."""
+Bound: beside what the same context is off token by token (fp32 products), the accumulator of a product of planes rounds 6 K / 32 times, 2^-24 of a partial sum at most and
+evenly spread, which is 2^-24 sqrt(K / 16) of the product's norm (rms); four products a layer and the LM head add up in squares; twice that."""
 import numpy as np
 import pytest
 
@@ -12,8 +12,12 @@ pytestmark = pytest.mark.gpu
 TOKENS = 130
 
 
-def build(pkg, orc, change, **kw):
-    hp = config(pkg, heads=4, hd=64, ffn=512, layers=4, vocab=700, ple=64, maxSeqs=2, maxL=200, **kw)
+def bound(hp):
+    return 2 * 2.0 ** -24 * np.sqrt(hp.dim / 16) * np.sqrt(4 * hp.transformers + 1)
+
+
+def build(pkg, orc, change, heads=4, layers=4):
+    hp = config(pkg, heads=heads, hd=64, ffn=512, layers=layers, vocab=700, ple=64, maxSeqs=2, maxL=200)
     model = pkg.Model.generate(hp, 11).randomize_gains(11)
     change(pkg, model, hp)
     return hp, model, orc.Weights.from_model(model)
@@ -70,10 +74,10 @@ CASES = {"plain": (plain, "PREFILL_PAIRS"), "gains inside": (gains(4), "PREFILL_
          "column": (column, "PREFILL_PLANES"), "table": (table, "PREFILL_PLANES")}
 
 
-@pytest.mark.parametrize("case", list(CASES))
-def test_distance_from_float64(pkg, orc, case):
+@pytest.mark.parametrize("case,heads,layers", [(c, 4, 4) for c in CASES] + [("gains", 18, 2), ("gains", 34, 2), ("plain", 34, 2)])  # rows of up to 1024, 2048 and more
+def test_distance_from_float64(pkg, orc, case, heads, layers):
     change, route = CASES[case]
-    hp, model, w = build(pkg, orc, change)
+    hp, model, w = build(pkg, orc, change, heads, layers)
     ids = pkg.random_tokens(5, 0, hp.vocabSize, TOKENS)
     dec = orc.Decoder(w, "f64")
     want = np.array([dec.step(int(t))[1] for t in ids])
@@ -88,14 +92,14 @@ def test_distance_from_float64(pkg, orc, case):
         got = dev.forward_full(0, ids, want_probs=False)[0]
         err[mode] = float(np.linalg.norm(got - want) / np.linalg.norm(want))
     print(f"{case}: prefill {err[0]:.2e}, token by token {err[1]:.2e}")
-    assert err[0] <= 2 * err[1] + 1e-6
+    assert err[0] <= err[1] + bound(hp)
     # prompts of two sequences in one call, and a second call behind cached rows
     dev.set_prefill_mode(0)
     dev.reset()
     dev.prefill_batch([0, 1], [ids[:40], ids[:50]])
     dev.prefill_batch([1, 0], [ids[50:], ids[40:]])
     for s in range(2):
-        assert np.linalg.norm(dev.logits(s) - want[-1]) <= (2 * err[1] + 2e-6) * np.linalg.norm(want[-1]) * 2
+        assert np.linalg.norm(dev.logits(s) - want[-1]) <= 2 * (err[1] + bound(hp)) * np.linalg.norm(want[-1])  # (one row: twice the rms of all)
     dev.close()
 
 
@@ -114,5 +118,5 @@ def test_a_finalize_changes_the_form(pkg, orc):
         dec.close()
         dev.reset()
         dev.prefill(0, ids)
-        assert np.linalg.norm(dev.logits(0) - want) <= 1e-5 * np.linalg.norm(want)
+        assert np.linalg.norm(dev.logits(0) - want) <= 4 * bound(hp) * np.linalg.norm(want)
     dev.close()
