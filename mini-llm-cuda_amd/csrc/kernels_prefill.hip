@@ -1737,7 +1737,7 @@ static int operand_values(mlh_ctx* c, bool* within) {
 //     about its own mean) with the gain in front of a product; value rows and PLE columns (gate row and table) beside each other;
 //   - an FFN unit, whose scale comes from its bound, is dim below that on rows without a direction; on rows as uneven as the residual columns at most 2^4 more.
 // What is lost at 2^-39 of the largest is then 2^-27 of a typical weight, 2^-31 of a typical element of a row, 2^-24 of a typical unit (dim 2048).
-// Models beyond multiply planes.  Normally distributed weights have 3 or 4, 3 and 1 octaves.  Exponents and integer sums: the answer is the same at every finalize.
+// Models beyond multiply planes.  Normally distributed weights have 4 or 5, 1 and 1 octaves.  Exponents and integer sums: the answer is the same at every finalize.
 #define SPREAD_WEIGHTS 12
 #define SPREAD_ROWS 8
 #define SPREAD_UNITS 4
